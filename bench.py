@@ -73,8 +73,8 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "all_ops_baseline_shapes_hbm_traff
 # rocprofv3 prints it (a prefix; {T} = float / double). Used to label the
 # per-kernel figures and to find the kernel in the counter summary.
 MAIN_KERNELS = {
-    ("hpe", "forward"): "hpe::forward_ordered_kernel<{T}, 4>",
-    ("hpe", "vjp"): "hpe::vjp_ordered_kernel<{T}, 4, true>",
+    ("hpe", "forward"): "hpe_tiles::forward_kernel<{T}, 4, 1>",
+    ("hpe", "vjp"): "hpe::vjp_ordered_kernel<{T}, 4>",
     ("sap", "forward"): "sap_mfma::forward_kernel<{T}, 2, 2, false, 2>",
     ("sap", "vjp"): "sap_mfma::vjp_kernel<{T}, 5, 2>",
     ("opsa", "forward"): "opsa::forward_kernel<{T}, 2, false, true, true>",

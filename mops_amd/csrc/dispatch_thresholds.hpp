@@ -12,16 +12,14 @@
 namespace mops::amd::thresholds {
 
 // ---- HPE (hpe.hip) ---------------------------------------------------------
-/// Rows from which the vjp goes by feature (the table turned round by a launch
-/// in front, accumulators in registers) instead of a workgroup per few rows
-/// with accumulators in LDS, which with thousands of rows is bound by its LDS
-/// add instructions. At 1000 rows by feature is the slower way (the extra
-/// launch). 8192 rows, 2000 monomials of order 4: 169 -> 64 us.
-constexpr int32_t HPE_VJP_BY_FEATURE_ROWS = 4096;
-/// Rows from which the forward pass has a lane per row (a workgroup per 64 or
-/// 128 rows): fewer workgroups than about one per compute unit leave the
-/// kernel with a workgroup per few rows ahead (8192 rows: 24 us against 35).
-constexpr int32_t HPE_FORWARD_LANE_PER_ROW_ROWS = 200 * 64;
+/// Factors of all monomials times rows from which the gradients go by feature
+/// (hpe_tiles.hip: two launches in front turn the table round) instead of a
+/// workgroup per few rows with accumulators in LDS. Whole vjp, LDS
+/// accumulators / by feature, in double: 8.0e6 (1000 rows, 2000 monomials of
+/// order 4, 100 features) 15.0 / 23 us, 1.15e7 (100 x 28 794 x 4, 53 features)
+/// 58 / 32, 2.9e7 (673 x 14 572 x 3, 23 features) 38.6 / 27, 6.6e7 (8192 x 2000
+/// x 4) 65 / 50; second order 20 / 39, 88 / 51, 49 / 47, 113 / 85.
+constexpr int64_t HPE_TILES_WORK = 10 * 1000 * 1000;
 
 // ---- SAP (sap_mfma.hip) ----------------------------------------------------
 /// Tiles of 16 rows per wavefront of the device from which a launch has as many

@@ -31,17 +31,14 @@
 #include "dispatch_thresholds.hpp"
 #include "index_validation.hpp"
 #include "elementwise.hpp"
+#include "hpe_tiles.hpp"
 #include "runtime.hpp"
-#include "sender_buckets.hpp"
 
 namespace mops::amd {
 namespace hpe { // a name of its own for this file's kernels: profilers print it
 namespace {
 
 constexpr size_t LDS_BUDGET = 60 * 1024;
-constexpr int32_t MANY_ROWS = thresholds::HPE_VJP_BY_FEATURE_ROWS;            // from here on the vjp goes by feature
-constexpr int32_t FORWARD_MANY_ROWS = thresholds::HPE_FORWARD_LANE_PER_ROW_ROWS; // from here on the forward pass has a lane per row
-constexpr size_t BY_FEATURE_LDS_BUDGET = 140 * 1024;    // its two tiles, of the 160 KB of a compute unit
 
 // ---------------------------------------------------------------------------
 // forward. LDS: a[nA][R] partial[G][R]
@@ -307,7 +304,7 @@ __global__ __launch_bounds__(WAVE) void vjp_kernel(
 // ---------------------------------------------------------------------------
 constexpr int ORDERED_VJP_THREADS = 4 * WAVE; // one wavefront that walks the monomials and three helpers
 
-template <typename T, int ORDER, bool ALL_FEATURES>
+template <typename T, int ORDER>
 __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
     T* __restrict__ grad_A,
     const T* __restrict__ grad_output,
@@ -317,21 +314,16 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
     int32_t n_rows,
     int32_t nA,
     int32_t n_monomials,
-    int32_t log2_R,
-    int32_t span
+    int32_t log2_R
 ) {
-    // LDS: a[nA + 1][R] accumulator[G][feature_count + 1][R]. The extra row of
-    // `a` stays zero and the extra accumulator row is never read: a factor
-    // outside [0, nA) reads the one, a term that is not to be kept (a feature
-    // of another range, a monomial beyond the last) goes to the other, and
-    // the loop over the monomials has no branch in it.
-    // ALL_FEATURES: span == nA, the workgroup keeps the terms of all features.
+    // LDS: a[nA + 1][R] accumulator[G][nA + 1][R]. The extra row of `a` stays zero
+    // and the extra accumulator row is never read: a factor outside [0, nA)
+    // reads the one, its term and those of a monomial beyond the last go to the
+    // other, and the loop over the monomials has no branch in it.
     extern __shared__ __align__(16) unsigned char lds_bytes[];
     const int32_t R = 1 << log2_R;
     T* a_stage = reinterpret_cast<T*>(lds_bytes);
     T* accumulator = a_stage + static_cast<size_t>(nA + 1) * R;
-    const int32_t feature_begin = ALL_FEATURES ? 0 : blockIdx.y * span;
-    const int32_t feature_count = ALL_FEATURES ? nA : min(span, nA - feature_begin);
 
     // Thread (r, g) of the FIRST wavefront walks the monomials; the other
     // wavefronts of the workgroup only help to stage the rows, to clear the
@@ -400,27 +392,27 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
     if (tid < R) {
         a_stage[nA * R + tid] = T(0);
     }
-    // (G * R = 64: the accumulators are feature_count + 1 rows of 64 values, one
+    // (G * R = 64: the accumulators are nA + 1 rows of 64 values, one
     // per lane; wavefront w clears rows w, w + 4, ...; unrolled, because a
     // wavefront pays for every instruction of the loop around a store)
     {
         constexpr int HELPERS = ORDERED_VJP_THREADS / WAVE;
         T* clear = accumulator + (tid & (WAVE - 1));
         int32_t k = tid >> 6;
-        for (; k + 7 * HELPERS < feature_count + 1; k += 8 * HELPERS) {
+        for (; k + 7 * HELPERS < nA + 1; k += 8 * HELPERS) {
 #pragma unroll
             for (int u = 0; u < 8; u++) {
                 clear[(k + u * HELPERS) * WAVE] = T(0);
             }
         }
-        for (; k < feature_count + 1; k += HELPERS) {
+        for (; k < nA + 1; k += HELPERS) {
             clear[k * WAVE] = T(0);
         }
     }
     __syncthreads();
 
     if (walks && r < rows) {
-        T* mine = accumulator + static_cast<size_t>(g) * (feature_count + 1) * R + r;
+        T* mine = accumulator + static_cast<size_t>(g) * (nA + 1) * R + r;
         const T* my_a = a_stage + r;
         // a feature's distance in bytes as a shift: address = base + (feature << shift), one
         // instruction (shift-and-add) per LDS access instead of a shift, a scaling and an add
@@ -431,7 +423,6 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
             return reinterpret_cast<Pointer>(reinterpret_cast<Bytes>(base) + (feature << byte_shift));
         };
         const uint32_t features = static_cast<uint32_t>(nA);
-        const uint32_t kept = static_cast<uint32_t>(feature_count);
         // `whole`: all monomials of the batch exist
         auto batch = [&](int32_t j0, auto whole) {
             constexpr bool WHOLE = decltype(whole)::value;
@@ -475,12 +466,8 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
                 const bool exists = WHOLE || j0 + d * G < n_monomials;
 #pragma unroll
                 for (int f = ORDER - 1; f >= 0; f--) {
-                    uint32_t slot = static_cast<uint32_t>(now[d].factor[f]);
-                    if constexpr (!ALL_FEATURES) {
-                        slot -= static_cast<uint32_t>(feature_begin);
-                    }
-                    slot = min(slot, kept);
-                    T* to = at(mine, exists ? slot : kept);
+                    const uint32_t slot = min(static_cast<uint32_t>(now[d].factor[f]), features);
+                    T* to = at(mine, exists ? slot : features);
                     // a slot of my own. In f64 the LDS add instruction, which saves the
                     // round trip of read, add, write; in f32 that instruction is the
                     // slower way here (53 us against 21)
@@ -506,9 +493,9 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
     // sums over the copies g = 0, 4, ... / 1, 5, ... / 2, 6, ... / 3, 7, ...
     // and then (s0 + s1) + (s2 + s3): one fixed order, and chains of additions
     // a quarter as long as one sum over all copies would be.
-    T* dst = grad_A + static_cast<size_t>(row0) * nA + feature_begin;
-    const int32_t copy_stride = (feature_count + 1) * R;
-    for (int32_t entry = tid; entry < feature_count * R; entry += ORDERED_VJP_THREADS) {
+    T* dst = grad_A + static_cast<size_t>(row0) * nA;
+    const int32_t copy_stride = (nA + 1) * R;
+    for (int32_t entry = tid; entry < nA * R; entry += ORDERED_VJP_THREADS) {
         const int32_t row = entry & (R - 1);
         const int32_t feature = entry >> log2_R;
         const T* from = accumulator + entry;
@@ -526,299 +513,6 @@ __global__ __launch_bounds__(ORDERED_VJP_THREADS) void vjp_ordered_kernel(
         if (row < rows) {
             dst[static_cast<size_t>(row) * nA + feature] = (partial[0] + partial[1]) + (partial[2] + partial[3]);
         }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// vjp for MANY rows, by feature. With thousands of rows the kernel above is
-// bound by its LDS add instructions (one per factor of every monomial and
-// row). Here nothing is scattered: the table is first turned round on the
-// device (sender_buckets.hpp, the same counting sort that orders edges by
-// sender: for every feature a the list of pairs q = j * ORDER + f with
-// P[j, f] = a, in ascending q), and then a wavefront owns (64 rows, one
-// feature at a time): a lane is a row, walks the feature's list, multiplies
-// up the OTHER factors of its row from an LDS tile of A and adds the terms in
-// a register:
-//
-//   grad_A[i, a] = gO[i] * sum over (j, f) in list(a) of C[j] * prod_{k != f} A[i, P[j, k]]
-//
-// The list entries are read 64 at a time, one per lane, and handed out to all
-// lanes through readlane. One fixed order (ascending q), no atomics.
-// LDS: a[nA][ROW_PITCH] out[64][out_pitch]
-// ---------------------------------------------------------------------------
-constexpr int FEATURE_WAVES = 16;
-/// Rows per workgroup when a lane has RPL rows (lane, lane + 64, ...: the table entry a
-/// wavefront is at then serves RPL rows per lane for the same readlanes and address)
-__host__ __device__ constexpr int feature_rows(int rpl) { return WAVE * rpl; }
-/// Distance between features in the tile of A
-__host__ __device__ constexpr int feature_row_pitch(int rpl) { return WAVE * rpl + 1; }
-
-template <typename T, int ORDER, int RPL>
-__global__ __launch_bounds__(FEATURE_WAVES* WAVE) void vjp_by_feature_kernel(
-    T* __restrict__ grad_A,
-    const T* __restrict__ grad_output,
-    const T* __restrict__ A,
-    const T* __restrict__ C,
-    const int32_t* __restrict__ P,
-    const int32_t* __restrict__ list_begin, // [nA + 1]
-    const int32_t* __restrict__ list,       // pairs q = j * ORDER + f, grouped by feature
-    int32_t n_rows,
-    int32_t nA,
-    int32_t features_per_group, // blockIdx.y takes the features [y, y + 1) * features_per_group
-    int32_t out_pitch
-) {
-    extern __shared__ __align__(16) unsigned char lds_bytes[];
-    T* a_stage = reinterpret_cast<T*>(lds_bytes);
-    T* out = a_stage + static_cast<size_t>(nA) * feature_row_pitch(RPL);
-    const int32_t first_feature = blockIdx.y * features_per_group;
-    const int32_t n_features = min(features_per_group, nA - first_feature);
-    constexpr int THREADS = FEATURE_WAVES * WAVE;
-    constexpr int FEATURE_ROWS = feature_rows(RPL);
-    constexpr int FEATURE_ROW_PITCH = feature_row_pitch(RPL);
-    constexpr int OTHERS = ORDER - 1;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int32_t row0 = blockIdx.x * FEATURE_ROWS;
-    const int32_t rows = min(FEATURE_ROWS, n_rows - row0);
-
-    const T* a_src = A + static_cast<size_t>(row0) * nA;
-    constexpr int STAGE_LOADS = 4;
-    for (int32_t i0 = tid; i0 < FEATURE_ROWS * nA; i0 += STAGE_LOADS * THREADS) {
-        T value[STAGE_LOADS];
-#pragma unroll
-        for (int u = 0; u < STAGE_LOADS; u++) {
-            const int32_t i = i0 + u * THREADS;
-            value[u] = load_or_zero(a_src, static_cast<size_t>(i), i < rows * nA); // rows beyond the end: zeros
-        }
-#pragma unroll
-        for (int u = 0; u < STAGE_LOADS; u++) {
-            const int32_t i = i0 + u * THREADS;
-            if (i < FEATURE_ROWS * nA) {
-                const int32_t row = i / nA;
-                a_stage[(i - row * nA) * FEATURE_ROW_PITCH + row] = value[u];
-            }
-        }
-    }
-    T upstream[RPL];
-#pragma unroll
-    for (int r = 0; r < RPL; r++) {
-        upstream[r] = load_or_zero(grad_output, static_cast<size_t>(row0 + lane + r * WAVE), lane + r * WAVE < rows);
-    }
-    __syncthreads();
-
-    const T* mine = a_stage + lane;
-    for (int32_t local = wave; local < n_features; local += FEATURE_WAVES) {
-        const int32_t feature = first_feature + local;
-        const int32_t begin = list_begin[feature];
-        const int32_t end = list_begin[feature + 1];
-        T sum[RPL];
-#pragma unroll
-        for (int r = 0; r < RPL; r++) {
-            sum[r] = T(0);
-        }
-        for (int32_t p0 = begin; p0 < end; p0 += WAVE) {
-            const int32_t n = min(WAVE, end - p0);
-            // my entry of the batch: coefficient (zero: no entry, or a factor out of range) and
-            // where the other factors' values are in the tile
-            const int32_t q = lane < n ? list[p0 + lane] : 0;
-            const int32_t j = q / ORDER;
-            const int32_t f = q - j * ORDER;
-            T coefficient = lane < n ? C[j] : T(0);
-            int32_t other[OTHERS > 0 ? OTHERS : 1];
-#pragma unroll
-            for (int k = 0; k < OTHERS; k++) {
-                const int32_t factor = P[static_cast<size_t>(j) * ORDER + (k < f ? k : k + 1)];
-                const bool valid = in_bounds(factor, nA);
-                other[k] = (valid ? factor : 0) * FEATURE_ROW_PITCH;
-                coefficient = valid ? coefficient : T(0);
-            }
-            int32_t words[sizeof(T) / 4];
-            __builtin_memcpy(words, &coefficient, sizeof(T));
-            // BATCH entries at a time: first every LDS read, then the products (a read that
-            // is waited for before the next one is asked for costs its whole latency)
-            constexpr int BATCH = 8;
-            for (int32_t u0 = 0; u0 < n; u0 += BATCH) {
-                T term[BATCH];
-                T value[BATCH][OTHERS > 0 ? OTHERS : 1][RPL];
-#pragma unroll
-                for (int b = 0; b < BATCH; b++) {
-                    // entries beyond n: lanes beyond n hold coefficient zero and a place that exists
-                    const int32_t u = min(u0 + b, WAVE - 1);
-                    int32_t uniform[sizeof(T) / 4];
-#pragma unroll
-                    for (int w = 0; w < static_cast<int>(sizeof(T) / 4); w++) {
-                        uniform[w] = __builtin_amdgcn_readlane(words[w], u);
-                    }
-                    __builtin_memcpy(&term[b], uniform, sizeof(T));
-                    if (u0 + b >= WAVE) {
-                        term[b] = T(0);
-                    }
-#pragma unroll
-                    for (int k = 0; k < OTHERS; k++) {
-                        const T* at = mine + __builtin_amdgcn_readlane(other[k], u);
-#pragma unroll
-                        for (int r = 0; r < RPL; r++) {
-                            value[b][k][r] = at[r * WAVE];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int b = 0; b < BATCH; b++) {
-#pragma unroll
-                    for (int r = 0; r < RPL; r++) {
-                        T product = term[b];
-#pragma unroll
-                        for (int k = 0; k < OTHERS; k++) {
-                            product *= value[b][k][r];
-                        }
-                        sum[r] += product;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < RPL; r++) {
-            out[(lane + r * WAVE) * out_pitch + local] = upstream[r] * sum[r];
-        }
-    }
-    __syncthreads();
-    // row by row, this group's features next to each other (all of them: one contiguous piece)
-    T* target = grad_A + static_cast<size_t>(row0) * nA + first_feature;
-    for (int32_t i = tid; i < rows * n_features; i += THREADS) {
-        const int32_t row = i / n_features;
-        const int32_t local = i - row * n_features;
-        target[static_cast<size_t>(row) * nA + local] = out[row * out_pitch + local];
-    }
-}
-
-// ---------------------------------------------------------------------------
-// forward for MANY rows, the same way: a lane is RPL rows, all lanes of a
-// wavefront are at the same monomial. The wavefronts of a workgroup share the
-// rows and take contiguous shares of the monomials, 64 at a time (lane u
-// loads monomial u of the batch, readlane hands it out); their partial sums
-// meet in LDS in wave order.
-// LDS: a[nA][pitch] partial[FEATURE_WAVES][rows]
-// ---------------------------------------------------------------------------
-template <typename T, int ORDER, int RPL>
-__global__ __launch_bounds__(FEATURE_WAVES* WAVE) void forward_rows_kernel(
-    T* __restrict__ output,
-    const T* __restrict__ A,
-    const T* __restrict__ C,
-    const int32_t* __restrict__ P,
-    int32_t n_rows,
-    int32_t nA,
-    int32_t n_monomials
-) {
-    extern __shared__ __align__(16) unsigned char lds_bytes[];
-    constexpr int THREADS = FEATURE_WAVES * WAVE;
-    constexpr int ROWS = feature_rows(RPL);
-    constexpr int PITCH = feature_row_pitch(RPL);
-    T* a_stage = reinterpret_cast<T*>(lds_bytes);
-    T* partial = a_stage + static_cast<size_t>(nA) * PITCH;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int32_t row0 = blockIdx.x * ROWS;
-    const int32_t rows = min(ROWS, n_rows - row0);
-
-    const T* a_src = A + static_cast<size_t>(row0) * nA;
-    constexpr int STAGE_LOADS = 4;
-    for (int32_t i0 = tid; i0 < ROWS * nA; i0 += STAGE_LOADS * THREADS) {
-        T value[STAGE_LOADS];
-#pragma unroll
-        for (int u = 0; u < STAGE_LOADS; u++) {
-            const int32_t i = i0 + u * THREADS;
-            value[u] = load_or_zero(a_src, static_cast<size_t>(i), i < rows * nA); // rows beyond the end: zeros
-        }
-#pragma unroll
-        for (int u = 0; u < STAGE_LOADS; u++) {
-            const int32_t i = i0 + u * THREADS;
-            if (i < ROWS * nA) {
-                const int32_t row = i / nA;
-                a_stage[(i - row * nA) * PITCH + row] = value[u];
-            }
-        }
-    }
-    __syncthreads();
-
-    const int32_t per_wave = (n_monomials + FEATURE_WAVES - 1) / FEATURE_WAVES;
-    const int32_t begin = min(wave * per_wave, n_monomials);
-    const int32_t end = min(begin + per_wave, n_monomials);
-    const T* mine = a_stage + lane;
-    T sum[RPL];
-#pragma unroll
-    for (int r = 0; r < RPL; r++) {
-        sum[r] = T(0);
-    }
-    for (int32_t j0 = begin; j0 < end; j0 += WAVE) {
-        const int32_t n = min(WAVE, end - j0);
-        // my monomial of the batch: coefficient (zero: none, or a factor out of range) and where
-        // its factors' values are in the tile
-        const int32_t j = lane < n ? j0 + lane : 0;
-        T coefficient = lane < n ? C[j] : T(0);
-        int32_t place[ORDER];
-#pragma unroll
-        for (int k = 0; k < ORDER; k++) {
-            const int32_t factor = P[static_cast<size_t>(j) * ORDER + k];
-            const bool valid = in_bounds(factor, nA);
-            place[k] = (valid ? factor : 0) * PITCH;
-            coefficient = valid ? coefficient : T(0);
-        }
-        int32_t words[sizeof(T) / 4];
-        __builtin_memcpy(words, &coefficient, sizeof(T));
-        constexpr int BATCH = 8;
-        for (int32_t u0 = 0; u0 < n; u0 += BATCH) {
-            T term[BATCH];
-            T value[BATCH][ORDER][RPL];
-#pragma unroll
-            for (int b = 0; b < BATCH; b++) {
-                const int32_t u = min(u0 + b, WAVE - 1);
-                int32_t uniform[sizeof(T) / 4];
-#pragma unroll
-                for (int w = 0; w < static_cast<int>(sizeof(T) / 4); w++) {
-                    uniform[w] = __builtin_amdgcn_readlane(words[w], u);
-                }
-                __builtin_memcpy(&term[b], uniform, sizeof(T));
-                if (u0 + b >= WAVE) {
-                    term[b] = T(0);
-                }
-#pragma unroll
-                for (int k = 0; k < ORDER; k++) {
-                    const T* at = mine + __builtin_amdgcn_readlane(place[k], u);
-#pragma unroll
-                    for (int r = 0; r < RPL; r++) {
-                        value[b][k][r] = at[r * WAVE];
-                    }
-                }
-            }
-#pragma unroll
-            for (int b = 0; b < BATCH; b++) {
-#pragma unroll
-                for (int r = 0; r < RPL; r++) {
-                    T product = term[b];
-#pragma unroll
-                    for (int k = 0; k < ORDER; k++) {
-                        product *= value[b][k][r];
-                    }
-                    sum[r] += product;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < RPL; r++) {
-        partial[wave * ROWS + lane + r * WAVE] = sum[r];
-    }
-    __syncthreads();
-    if (tid < rows) {
-        T total = T(0);
-        for (int w = 0; w < FEATURE_WAVES; w++) {
-            total += partial[w * ROWS + tid];
-        }
-        output[row0 + tid] = total;
     }
 }
 
@@ -1357,59 +1051,25 @@ void homogeneous_polynomial_evaluation(MOPS_HPE_PARAMS(MOPS_CXX_FIRST, MOPS_CXX_
         return;
     }
     hipStream_t stream = current_stream();
-    constexpr int THREADS = 256;
-    // many rows: a lane per row (forward_rows_kernel), two where the tile of 128 rows fits
-    auto rows_bytes = [&](int rpl) {
-        return (static_cast<size_t>(nA) * feature_row_pitch(rpl) + static_cast<size_t>(FEATURE_WAVES) * feature_rows(rpl)) *
-               sizeof(scalar_t);
-    };
-    // (a workgroup per 64 or 128 rows: fewer workgroups than about one per compute unit leave the
-    // kernel below ahead, 8192 rows: 24 us against 35)
-    if (n_rows >= FORWARD_MANY_ROWS && order >= 1 && order <= 6 && n_monomials > 0 &&
-        rows_bytes(1) <= BY_FEATURE_LDS_BUDGET) {
-        // (two rows per lane also where that halves the workgroups: 20 000 rows, 51 us against 65)
-        const int rows_per_lane = rows_bytes(2) <= BY_FEATURE_LDS_BUDGET ? 2 : 1;
-        const size_t lds = rows_bytes(rows_per_lane);
-        const unsigned blocks =
-            static_cast<unsigned>(ceil_div(static_cast<size_t>(n_rows), static_cast<size_t>(feature_rows(rows_per_lane))));
-#define MOPS_LAUNCH_ROWS(ORDER)                                                                     \
-    {                                                                                              \
-        auto kernel = rows_per_lane == 2 ? forward_rows_kernel<scalar_t, ORDER, 2>                 \
-                                         : forward_rows_kernel<scalar_t, ORDER, 1>;                \
-        if (lds > 64 * 1024) {                                                                     \
-            MOPS_HIP_CHECK(hipFuncSetAttribute(                                                    \
-                reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                static_cast<int>(lds)                                                              \
-            ));                                                                                    \
-        }                                                                                          \
-        kernel<<<blocks, FEATURE_WAVES * WAVE, lds, stream>>>(                                     \
-            output.data, A.data, C.data, indices_A.data, n_rows, nA, n_monomials                   \
-        );                                                                                         \
-    }
-        switch (order) {
-        case 1:
-            MOPS_LAUNCH_ROWS(1);
-            break;
-        case 2:
-            MOPS_LAUNCH_ROWS(2);
-            break;
-        case 3:
-            MOPS_LAUNCH_ROWS(3);
-            break;
-        case 4:
-            MOPS_LAUNCH_ROWS(4);
-            break;
-        case 5:
-            MOPS_LAUNCH_ROWS(5);
-            break;
-        default:
-            MOPS_LAUNCH_ROWS(6);
-            break;
+    const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
+    if (const auto plan = hpe_tiles::plan_forward(shape, sizeof(scalar_t)); plan.values > 0) {
+        const size_t bytes = hpe_tiles::forward_bytes(shape, plan, sizeof(scalar_t));
+        void* workspace = bytes > 0 ? scratch(bytes) : nullptr;
+        auto launch = [&](int32_t* counters) {
+            hpe_tiles::forward<scalar_t>(
+                output.data, A.data, C.data, indices_A.data, shape, plan, workspace, counters, stream
+            );
+        };
+        if (bytes > 0) {
+            ScratchCounters counters;
+            launch(counters.data());
+        } else {
+            launch(nullptr);
         }
-#undef MOPS_LAUNCH_ROWS
         finish_call(operation);
         return;
     }
+    constexpr int THREADS = 256;
     // per row: its A values plus one partial sum per group (G <= THREADS)
     int R = pick_rows(n_rows, (static_cast<size_t>(nA) + 1 + THREADS) * sizeof(scalar_t));
     if (R > 0) {
@@ -1477,74 +1137,19 @@ void homogeneous_polynomial_evaluation_vjp(MOPS_HPE_VJP_PARAMS(MOPS_CXX_FIRST, M
         return;
     }
     hipStream_t stream = current_stream();
-    // many rows: by feature (vjp_by_feature_kernel), after the table has been turned round
-    // workgroup = (64 rows, a group of features): groups of 16 features (one per wavefront)
-    // while that brings the launch to a few hundred workgroups, all features in one otherwise
-    auto by_feature_bytes = [&](int rpl, int32_t pitch) {
-        return (static_cast<size_t>(nA) * feature_row_pitch(rpl) + static_cast<size_t>(feature_rows(rpl)) * pitch) *
-               sizeof(scalar_t);
-    };
-    // two rows per lane where the tiles of 128 rows fit
-    const int rows_per_lane = by_feature_bytes(2, (FEATURE_WAVES * 4) | 1) <= BY_FEATURE_LDS_BUDGET ? 2 : 1;
-    const size_t row_groups = ceil_div(static_cast<size_t>(n_rows), static_cast<size_t>(feature_rows(rows_per_lane)));
-    const size_t wanted_groups = std::max<size_t>(1, ceil_div(512, row_groups));
-    const size_t feature_groups = std::min(wanted_groups, ceil_div(static_cast<size_t>(nA), FEATURE_WAVES));
-    const int32_t features_per_group = static_cast<int32_t>(
-        ceil_div(ceil_div(static_cast<size_t>(nA), feature_groups), FEATURE_WAVES) * FEATURE_WAVES
-    );
-    const int32_t out_pitch = features_per_group | 1;
-    const size_t by_feature_lds = by_feature_bytes(rows_per_lane, out_pitch);
-    const size_t n_pairs = static_cast<size_t>(n_monomials) * static_cast<size_t>(std::max(order, 0));
-    if (n_rows >= MANY_ROWS && order >= 1 && order <= 6 && n_pairs > 0 && n_pairs < (size_t(1) << 30) &&
-        by_feature_lds <= BY_FEATURE_LDS_BUDGET) {
-        void* workspace = scratch(edges_by_sender_bytes(nA, static_cast<int32_t>(n_pairs)));
-        const EdgesBySender lists =
-            order_edges_by_sender(indices_A.data, static_cast<int32_t>(n_pairs), nA, workspace, stream);
-        const dim3 blocks(
-            static_cast<unsigned>(row_groups),
-            static_cast<unsigned>(ceil_div(static_cast<size_t>(nA), static_cast<size_t>(features_per_group)))
+    // accumulators of every feature for each of the 64 lanes that walk the monomials
+    const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
+    const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
+    const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), false);
+    if (plan.values > 0 && (hpe_tiles::large(shape) || accumulator_bytes > LDS_BUDGET)) {
+        void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), false));
+        hpe_tiles::vjp<scalar_t>(
+            grad_A.data, grad_output.data, A.data, C.data, indices_A.data, shape, plan, workspace, stream
         );
-#define MOPS_LAUNCH_BY_FEATURE(ORDER)                                                               \
-    {                                                                                              \
-        auto kernel = rows_per_lane == 2 ? vjp_by_feature_kernel<scalar_t, ORDER, 2>               \
-                                         : vjp_by_feature_kernel<scalar_t, ORDER, 1>;              \
-        if (by_feature_lds > 64 * 1024) {                                                          \
-            MOPS_HIP_CHECK(hipFuncSetAttribute(                                                    \
-                reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, \
-                static_cast<int>(by_feature_lds)                                                   \
-            ));                                                                                    \
-        }                                                                                          \
-        kernel<<<blocks, FEATURE_WAVES * WAVE, by_feature_lds, stream>>>(                          \
-            grad_A.data, grad_output.data, A.data, C.data, indices_A.data, lists.offsets, lists.edge, \
-            n_rows, nA, features_per_group, out_pitch                                              \
-        );                                                                                         \
-    }
-        switch (order) {
-        case 1:
-            MOPS_LAUNCH_BY_FEATURE(1);
-            break;
-        case 2:
-            MOPS_LAUNCH_BY_FEATURE(2);
-            break;
-        case 3:
-            MOPS_LAUNCH_BY_FEATURE(3);
-            break;
-        case 4:
-            MOPS_LAUNCH_BY_FEATURE(4);
-            break;
-        case 5:
-            MOPS_LAUNCH_BY_FEATURE(5);
-            break;
-        default:
-            MOPS_LAUNCH_BY_FEATURE(6);
-            break;
-        }
-#undef MOPS_LAUNCH_BY_FEATURE
         finish_call(operation);
         return;
     }
-    // LDS holds R rows of A and WAVE private accumulator rows, whatever R is
-    const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
+    // LDS holds R rows of A and the accumulators, whatever R is
     // Rows per workgroup: the fewest for which all workgroups are on the
     // device at once (256 CUs, as many workgroups per CU as the 160 KB of LDS
     // hold): a second round of workgroups costs more than rows twice as long
@@ -1591,18 +1196,12 @@ void homogeneous_polynomial_evaluation_vjp(MOPS_HPE_VJP_PARAMS(MOPS_CXX_FIRST, M
         );
         MainKernelTimer timer(stream);
 #define MOPS_LAUNCH_ORDERED(ORDER)                                                                  \
-    if (span == nA) {                                                                              \
-        vjp_ordered_kernel<scalar_t, ORDER, true><<<blocks, ORDERED_VJP_THREADS, lds, stream>>>(                  \
-            grad_A.data, grad_output.data, A.data, C.data, indices_A.data, n_rows, nA,             \
-            n_monomials, log2_R, span                                                              \
-        );                                                                                         \
-    } else {                                                                                       \
-        vjp_ordered_kernel<scalar_t, ORDER, false><<<blocks, ORDERED_VJP_THREADS, lds, stream>>>(                 \
-            grad_A.data, grad_output.data, A.data, C.data, indices_A.data, n_rows, nA,             \
-            n_monomials, log2_R, span                                                              \
-        );                                                                                         \
-    }
-        switch (n_monomials > 0 ? order : 0) {
+    vjp_ordered_kernel<scalar_t, ORDER><<<blocks, ORDERED_VJP_THREADS, lds, stream>>>(             \
+        grad_A.data, grad_output.data, A.data, C.data, indices_A.data, n_rows, nA, n_monomials,    \
+        log2_R                                                                                     \
+    )
+        // (features in ranges: kernels of any order)
+        switch (n_monomials > 0 && span == nA ? order : 0) {
         case 1:
             MOPS_LAUNCH_ORDERED(1);
             break;
@@ -1671,10 +1270,22 @@ void homogeneous_polynomial_evaluation_vjp_vjp(MOPS_HPE_VJP_VJP_PARAMS(MOPS_CXX_
         finish_call(operation);
         return;
     }
+    const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
+    const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
+    const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), true);
+    if (plan.values > 0 && (hpe_tiles::large(shape) || accumulator_bytes > LDS_BUDGET)) {
+        void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), true));
+        ScratchCounters counters;
+        hpe_tiles::vjp_vjp<scalar_t>(
+            grad_grad_output.data, grad_A_2.data, grad_grad_A.data, grad_output.data, A.data, C.data, indices_A.data,
+            shape, plan, workspace, counters.data(), stream
+        );
+        finish_call(operation);
+        return;
+    }
     // order known at compile time: the tiles of vjp_ordered_kernel and one more of grad_grad_A;
     // rows per workgroup as there (the fewest for which all workgroups are on the device at once)
     if (order >= 1 && order <= 6 && n_monomials > 0) {
-        const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
         auto ordered_lds = [&](int rows) {
             return accumulator_bytes + 2 * (static_cast<size_t>(nA) + 1) * rows * sizeof(scalar_t);
         };
