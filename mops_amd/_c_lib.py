@@ -12,6 +12,7 @@ from ._c_api import Library
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIBRARY_PATH = os.path.join(_HERE, "lib", "libmops.so")
+ARRAY_FUNCTIONS_PATH = os.path.join(_HERE, "lib", "_array_ops.so")
 
 _device = None
 _host = None
@@ -68,3 +69,26 @@ def host_library():
 
         _host = Library(LIBRARY_PATH, "mops_", "mops_get_last_error_message")
     return _host
+
+
+class _NoFunctions:
+    def __getattr__(self, name):
+        return lambda *arguments: None
+
+
+def array_functions():
+    """The functions of ``mops_amd/csrc/array_ops.cpp`` (built by ``build_torch_ops.py``), or functions
+    that leave every call to their caller where that has not been built or
+    ``MOPS_AMD_ARRAY_PYTHON=1`` is set."""
+    if not os.path.exists(ARRAY_FUNCTIONS_PATH) or os.environ.get("MOPS_AMD_ARRAY_PYTHON", "0") not in ("", "0"):
+        return _NoFunctions()
+    _require_built()
+    import importlib.machinery
+    import importlib.util
+
+    import torch  # noqa: F401  (see device_library)
+
+    loader = importlib.machinery.ExtensionFileLoader("_array_ops", ARRAY_FUNCTIONS_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_array_ops", loader))
+    loader.exec_module(module)
+    return module

@@ -23,14 +23,15 @@
 #include <string>
 #include <vector>
 
-#include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/script.h>
 
 #include "mops.hpp"
-#include "mops/amd.h"
+
+#include "torch_tensors.hpp"
 
 namespace {
+
+using namespace mops::amd::torch_tensors;
 
 using torch::autograd::AutogradContext;
 using torch::autograd::Function;
@@ -70,43 +71,19 @@ at::Tensor indices(const at::Tensor& tensor, const at::Tensor& like, const char*
     return tensor.to(at::kInt).contiguous();
 }
 
-template <typename T, size_t N> mops::Tensor<T, N> view(const at::Tensor& tensor, const char* name) {
-    mops::Tensor<T, N> result{nullptr, {}};
-    for (size_t d = 0; d < N; d++) {
-        result.shape[d] = 0;
+/// Whether a call on these tensors has to leave something for autograd. Without it (inference, and
+/// a backward pass that is not itself differentiated) an operator calls the library directly: a
+/// Function and its context cost 1 us, of a call of 6.
+bool recorded(std::initializer_list<const at::Tensor*> tensors) {
+    for (const at::Tensor* tensor : tensors) {
+        if (!tensor->defined() || tensor->unsafeGetTensorImpl()->autograd_meta() == nullptr) {
+            continue;
+        }
+        if ((at::GradMode::is_enabled() && tensor->requires_grad()) || tensor->_fw_grad(0).defined()) {
+            return true; // (forward-mode gradients: Function says that there are none)
+        }
     }
-    if (!tensor.defined()) {
-        return result; // "not wanted" / "not given": a null view
-    }
-    if (static_cast<size_t>(tensor.dim()) != N) {
-        throw std::runtime_error(
-            std::string(name) + " must have " + std::to_string(N) + " dimensions, got " + std::to_string(tensor.dim())
-        );
-    }
-    result.data = tensor.data_ptr<T>();
-    for (size_t d = 0; d < N; d++) {
-        result.shape[d] = static_cast<size_t>(tensor.size(static_cast<int64_t>(d)));
-    }
-    return result;
-}
-
-/// The library's launches go to PyTorch's current stream of the tensors' device, without blocking.
-/// (In a ROCm build of PyTorch the HIP device type goes under the name of CUDA: these are the
-/// guard and the stream of that build.)
-struct OnTorchStream {
-    c10::hip::HIPGuardMasqueradingAsCUDA guard;
-    explicit OnTorchStream(const at::Tensor& tensor) : guard(tensor.device()) {
-        mops_amd_set_stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
-        mops_amd_set_synchronous(0);
-    }
-};
-
-template <typename Body> void by_dtype(const at::Tensor& like, Body&& body) {
-    if (like.scalar_type() == at::kFloat) {
-        body(float{});
-    } else {
-        body(double{});
-    }
+    return false;
 }
 
 at::Tensor nothing(const at::Tensor& like) { return at::empty({0}, like.options()); }
@@ -117,7 +94,7 @@ at::Tensor hpe_forward(const at::Tensor& A_, const at::Tensor& C_, const at::Ten
     const char* op = "homogeneous_polynomial_evaluation";
     const at::Tensor A = values(A_, A_, "A", op), C = values(C_, A_, "C", op), P = indices(P_, A_, "indices_A", op);
     OnTorchStream stream(A);
-    at::Tensor output = at::empty({A.dim() == 2 ? A.size(0) : 0}, A.options());
+    at::Tensor output = new_tensor({A.dim() == 2 ? A.size(0) : 0}, A);
     by_dtype(A, [&](auto zero) {
         using T = decltype(zero);
         mops::cuda::homogeneous_polynomial_evaluation<T>(
@@ -132,7 +109,7 @@ at::Tensor hpe_vjp(const at::Tensor& gO_, const at::Tensor& A_, const at::Tensor
     const at::Tensor A = values(A_, A_, "A", op), C = values(C_, A_, "C", op), P = indices(P_, A_, "indices_A", op);
     const at::Tensor gO = values(gO_, A_, "grad_output", op);
     OnTorchStream stream(A);
-    at::Tensor grad_A = at::empty_like(A);
+    at::Tensor grad_A = new_like(A);
     by_dtype(A, [&](auto zero) {
         using T = decltype(zero);
         mops::cuda::homogeneous_polynomial_evaluation_vjp<T>(
@@ -152,8 +129,8 @@ std::array<at::Tensor, 2> hpe_vjp_vjp(
     const at::Tensor gO = values(gO_, A_, "grad_output", op);
     const at::Tensor ggA = ggA_.defined() ? values(ggA_, A_, "grad_grad_A", op) : at::Tensor();
     OnTorchStream stream(A);
-    at::Tensor ggO = want_ggO ? at::empty_like(gO) : at::Tensor();
-    at::Tensor A2 = want_A2 ? at::empty_like(A) : at::Tensor();
+    at::Tensor ggO = want_ggO ? new_like(gO) : at::Tensor();
+    at::Tensor A2 = want_A2 ? new_like(A) : at::Tensor();
     by_dtype(A, [&](auto zero) {
         using T = decltype(zero);
         mops::cuda::homogeneous_polynomial_evaluation_vjp_vjp<T>(
@@ -192,7 +169,8 @@ struct Hpe : public Function<Hpe> {
         }
         at::Tensor grad_A;
         if (ctx->needs_input_grad(0)) {
-            grad_A = HpeVjp::apply(grads[0], saved[0], saved[1], saved[2]);
+            grad_A = recorded({&grads[0], &saved[0], &saved[1]}) ? HpeVjp::apply(grads[0], saved[0], saved[1], saved[2])
+                                                                 : hpe_vjp(grads[0], saved[0], saved[1], saved[2]);
         }
         return {grad_A, at::Tensor(), at::Tensor()};
     }
@@ -209,7 +187,7 @@ struct Opsa {
         return {indices(extra[0], A, "indices_output", op)};
     }
     static at::Tensor output_like(const at::Tensor& A, const at::Tensor& B, int64_t output_size) {
-        return at::empty({output_size, A.dim() == 2 ? A.size(1) : 0, B.dim() == 2 ? B.size(1) : 0}, A.options());
+        return new_tensor({output_size, A.dim() == 2 ? A.size(1) : 0, B.dim() == 2 ? B.size(1) : 0}, A);
     }
     template <typename T>
     static void forward(at::Tensor& O, const at::Tensor& A, const at::Tensor& B, const std::vector<at::Tensor>& e) {
@@ -252,7 +230,7 @@ struct Sap {
             indices(extra[3], A, "indices_output", op)};
     }
     static at::Tensor output_like(const at::Tensor& A, const at::Tensor&, int64_t output_size) {
-        return at::empty({A.dim() == 2 ? A.size(0) : 0, output_size}, A.options());
+        return new_tensor({A.dim() == 2 ? A.size(0) : 0, output_size}, A);
     }
     template <typename T>
     static void forward(at::Tensor& O, const at::Tensor& A, const at::Tensor& B, const std::vector<at::Tensor>& e) {
@@ -298,8 +276,8 @@ std::array<at::Tensor, 2> bilinear_vjp(
     const at::Tensor gO = values(gO_, A_, "grad_output", op.c_str());
     const std::vector<at::Tensor> extra = Op::prepare(extra_, A, op.c_str());
     OnTorchStream stream(A);
-    at::Tensor gA = want_A ? at::empty_like(A) : at::Tensor();
-    at::Tensor gB = want_B ? at::empty_like(B) : at::Tensor();
+    at::Tensor gA = want_A ? new_like(A) : at::Tensor();
+    at::Tensor gB = want_B ? new_like(B) : at::Tensor();
     by_dtype(A, [&](auto zero) { Op::template vjp<decltype(zero)>(gA, gB, gO, A, B, extra); });
     return {gA, gB};
 }
@@ -342,9 +320,9 @@ template <typename Op> struct BilinearVjp : public Function<BilinearVjp<Op>> {
         const at::Tensor ggB = have_B ? values(grads[1], A_, "grad_grad_B", op.c_str()) : at::Tensor();
         const std::vector<at::Tensor> extra = Op::prepare(extra_, A, op.c_str());
         OnTorchStream stream(A);
-        at::Tensor ggO = want_ggO ? at::empty_like(gO) : at::Tensor();
-        at::Tensor A2 = want_A2 ? at::empty_like(A) : at::Tensor();
-        at::Tensor B2 = want_B2 ? at::empty_like(B) : at::Tensor();
+        at::Tensor ggO = want_ggO ? new_like(gO) : at::Tensor();
+        at::Tensor A2 = want_A2 ? new_like(A) : at::Tensor();
+        at::Tensor B2 = want_B2 ? new_like(B) : at::Tensor();
         by_dtype(A, [&](auto zero) {
             Op::template vjp_vjp<decltype(zero)>(ggO, A2, B2, ggA, ggB, gO, A, B, extra);
         });
@@ -354,6 +332,18 @@ template <typename Op> struct BilinearVjp : public Function<BilinearVjp<Op>> {
     }
 };
 
+template <typename Op>
+at::Tensor bilinear_forward(
+    const at::Tensor& A_, const at::Tensor& B_, const std::vector<at::Tensor>& extra_, int64_t output_size
+) {
+    const at::Tensor A = values(A_, A_, "A", Op::name), B = values(B_, A_, "B", Op::name);
+    const std::vector<at::Tensor> extra = Op::prepare(extra_, A, Op::name);
+    OnTorchStream stream(A);
+    at::Tensor output = Op::output_like(A, B, output_size);
+    by_dtype(A, [&](auto zero) { Op::template forward<decltype(zero)>(output, A, B, extra); });
+    return output;
+}
+
 template <typename Op> struct Bilinear : public Function<Bilinear<Op>> {
     static at::Tensor forward(
         AutogradContext* ctx, at::Tensor A_, at::Tensor B_, at::TensorList extra_list, int64_t output_size
@@ -362,12 +352,7 @@ template <typename Op> struct Bilinear : public Function<Bilinear<Op>> {
         variable_list saved = {A_, B_};
         saved.insert(saved.end(), extra_.begin(), extra_.end());
         ctx->save_for_backward(saved);
-        const at::Tensor A = values(A_, A_, "A", Op::name), B = values(B_, A_, "B", Op::name);
-        const std::vector<at::Tensor> extra = Op::prepare(extra_, A, Op::name);
-        OnTorchStream stream(A);
-        at::Tensor output = Op::output_like(A, B, output_size);
-        by_dtype(A, [&](auto zero) { Op::template forward<decltype(zero)>(output, A, B, extra); });
-        return output;
+        return bilinear_forward<Op>(A_, B_, extra_, output_size);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
@@ -380,10 +365,16 @@ template <typename Op> struct Bilinear : public Function<Bilinear<Op>> {
         const bool want_A = ctx->needs_input_grad(0), want_B = ctx->needs_input_grad(1);
         variable_list result(2 + Op::n_extra + 1);
         if (want_A || want_B) {
-            const auto gradients =
-                BilinearVjp<Op>::apply(grads[0], saved[0], saved[1], at::TensorList(extra), want_A, want_B);
-            result[0] = or_undefined(gradients[0], want_A);
-            result[1] = or_undefined(gradients[1], want_B);
+            if (recorded({&grads[0], &saved[0], &saved[1]})) {
+                const auto gradients =
+                    BilinearVjp<Op>::apply(grads[0], saved[0], saved[1], at::TensorList(extra), want_A, want_B);
+                result[0] = or_undefined(gradients[0], want_A);
+                result[1] = or_undefined(gradients[1], want_B);
+            } else {
+                const auto gradients = bilinear_vjp<Op>(grads[0], saved[0], saved[1], extra, want_A, want_B);
+                result[0] = gradients[0];
+                result[1] = gradients[1];
+            }
         }
         return result;
     }
@@ -392,26 +383,31 @@ template <typename Op> struct Bilinear : public Function<Bilinear<Op>> {
 // ------------------------------------------------------- OPSAW, SASAW --
 // Three differentiable inputs (A, B, W), no second derivative (the reference has none:
 // mops/src/opsaw/cpu.tpp:133-150, mops/src/sasaw/cpu.tpp:173-194).
+at::Tensor opsaw_forward(
+    const at::Tensor& A_, const at::Tensor& B_, const at::Tensor& W_, const at::Tensor& PW_, const at::Tensor& PO_
+) {
+    const char* op = "outer_product_scatter_add_with_weights";
+    const at::Tensor A = values(A_, A_, "A", op), B = values(B_, A_, "B", op), W = values(W_, A_, "W", op);
+    const at::Tensor PW = indices(PW_, A_, "indices_W", op), PO = indices(PO_, A_, "indices_output", op);
+    OnTorchStream stream(A);
+    at::Tensor output =
+        new_tensor({W.dim() == 2 ? W.size(0) : 0, A.dim() == 2 ? A.size(1) : 0, B.dim() == 2 ? B.size(1) : 0}, A);
+    by_dtype(A, [&](auto zero) {
+        using T = decltype(zero);
+        mops::cuda::outer_product_scatter_add_with_weights<T>(
+            view<T, 3>(output, "output"), view<T, 2>(A, "A"), view<T, 2>(B, "B"), view<T, 2>(W, "W"),
+            view<int32_t, 1>(PW, "indices_W"), view<int32_t, 1>(PO, "indices_output")
+        );
+    });
+    return output;
+}
+
 struct OpsawFunction : public Function<OpsawFunction> {
     static at::Tensor forward(
         AutogradContext* ctx, at::Tensor A_, at::Tensor B_, at::Tensor W_, at::Tensor PW_, at::Tensor PO_
     ) {
-        const char* op = "outer_product_scatter_add_with_weights";
         ctx->save_for_backward({A_, B_, W_, PW_, PO_});
-        const at::Tensor A = values(A_, A_, "A", op), B = values(B_, A_, "B", op), W = values(W_, A_, "W", op);
-        const at::Tensor PW = indices(PW_, A_, "indices_W", op), PO = indices(PO_, A_, "indices_output", op);
-        OnTorchStream stream(A);
-        at::Tensor output = at::empty(
-            {W.dim() == 2 ? W.size(0) : 0, A.dim() == 2 ? A.size(1) : 0, B.dim() == 2 ? B.size(1) : 0}, A.options()
-        );
-        by_dtype(A, [&](auto zero) {
-            using T = decltype(zero);
-            mops::cuda::outer_product_scatter_add_with_weights<T>(
-                view<T, 3>(output, "output"), view<T, 2>(A, "A"), view<T, 2>(B, "B"), view<T, 2>(W, "W"),
-                view<int32_t, 1>(PW, "indices_W"), view<int32_t, 1>(PO, "indices_output")
-            );
-        });
-        return output;
+        return opsaw_forward(A_, B_, W_, PW_, PO_);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const char* op = "outer_product_scatter_add_with_weights_vjp";
@@ -424,9 +420,9 @@ struct OpsawFunction : public Function<OpsawFunction> {
                          PO = indices(saved[4], saved[0], "indices_output", op);
         const at::Tensor gO = values(grads[0], saved[0], "grad_output", op);
         OnTorchStream stream(A);
-        at::Tensor gA = want_A ? at::empty_like(A) : at::Tensor();
-        at::Tensor gB = want_B ? at::empty_like(B) : at::Tensor();
-        at::Tensor gW = want_W ? at::empty_like(W) : at::Tensor();
+        at::Tensor gA = want_A ? new_like(A) : at::Tensor();
+        at::Tensor gB = want_B ? new_like(B) : at::Tensor();
+        at::Tensor gW = want_W ? new_like(W) : at::Tensor();
         by_dtype(A, [&](auto zero) {
             using T = decltype(zero);
             mops::cuda::outer_product_scatter_add_with_weights_vjp<T>(
@@ -439,31 +435,38 @@ struct OpsawFunction : public Function<OpsawFunction> {
     }
 };
 
+at::Tensor sasaw_forward(
+    const at::Tensor& A_, const at::Tensor& B_, const at::Tensor& C_, const at::Tensor& W_, const at::Tensor& PA_,
+    const at::Tensor& PW1_, const at::Tensor& PW2_, const at::Tensor& PO1_, const at::Tensor& PO2_, int64_t output_size
+) {
+    const char* op = "sparse_accumulation_scatter_add_with_weights";
+    const at::Tensor A = values(A_, A_, "A", op), B = values(B_, A_, "B", op), C = values(C_, A_, "C", op),
+                     W = values(W_, A_, "W", op);
+    const at::Tensor PA = indices(PA_, A_, "indices_A", op), PW1 = indices(PW1_, A_, "indices_W_1", op),
+                     PW2 = indices(PW2_, A_, "indices_W_2", op), PO1 = indices(PO1_, A_, "indices_output_1", op),
+                     PO2 = indices(PO2_, A_, "indices_output_2", op);
+    OnTorchStream stream(A);
+    at::Tensor output =
+        new_tensor({W.dim() == 3 ? W.size(0) : 0, output_size, B.dim() == 2 ? B.size(1) : 0}, A);
+    by_dtype(A, [&](auto zero) {
+        using T = decltype(zero);
+        mops::cuda::sparse_accumulation_scatter_add_with_weights<T>(
+            view<T, 3>(output, "output"), view<T, 2>(A, "A"), view<T, 2>(B, "B"), view<T, 1>(C, "C"),
+            view<T, 3>(W, "W"), view<int32_t, 1>(PA, "indices_A"), view<int32_t, 1>(PW1, "indices_W_1"),
+            view<int32_t, 1>(PW2, "indices_W_2"), view<int32_t, 1>(PO1, "indices_output_1"),
+            view<int32_t, 1>(PO2, "indices_output_2")
+        );
+    });
+    return output;
+}
+
 struct SasawFunction : public Function<SasawFunction> {
     static at::Tensor forward(
         AutogradContext* ctx, at::Tensor A_, at::Tensor B_, at::Tensor C_, at::Tensor W_, at::Tensor PA_,
         at::Tensor PW1_, at::Tensor PW2_, at::Tensor PO1_, at::Tensor PO2_, int64_t output_size
     ) {
-        const char* op = "sparse_accumulation_scatter_add_with_weights";
         ctx->save_for_backward({A_, B_, C_, W_, PA_, PW1_, PW2_, PO1_, PO2_});
-        const at::Tensor A = values(A_, A_, "A", op), B = values(B_, A_, "B", op), C = values(C_, A_, "C", op),
-                         W = values(W_, A_, "W", op);
-        const at::Tensor PA = indices(PA_, A_, "indices_A", op), PW1 = indices(PW1_, A_, "indices_W_1", op),
-                         PW2 = indices(PW2_, A_, "indices_W_2", op), PO1 = indices(PO1_, A_, "indices_output_1", op),
-                         PO2 = indices(PO2_, A_, "indices_output_2", op);
-        OnTorchStream stream(A);
-        at::Tensor output =
-            at::empty({W.dim() == 3 ? W.size(0) : 0, output_size, B.dim() == 2 ? B.size(1) : 0}, A.options());
-        by_dtype(A, [&](auto zero) {
-            using T = decltype(zero);
-            mops::cuda::sparse_accumulation_scatter_add_with_weights<T>(
-                view<T, 3>(output, "output"), view<T, 2>(A, "A"), view<T, 2>(B, "B"), view<T, 1>(C, "C"),
-                view<T, 3>(W, "W"), view<int32_t, 1>(PA, "indices_A"), view<int32_t, 1>(PW1, "indices_W_1"),
-                view<int32_t, 1>(PW2, "indices_W_2"), view<int32_t, 1>(PO1, "indices_output_1"),
-                view<int32_t, 1>(PO2, "indices_output_2")
-            );
-        });
-        return output;
+        return sasaw_forward(A_, B_, C_, W_, PA_, PW1_, PW2_, PO1_, PO2_, output_size);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         const char* op = "sparse_accumulation_scatter_add_with_weights_vjp";
@@ -482,9 +485,9 @@ struct SasawFunction : public Function<SasawFunction> {
                          PO2 = indices(saved[8], like, "indices_output_2", op);
         const at::Tensor gO = values(grads[0], like, "grad_output", op);
         OnTorchStream stream(A);
-        at::Tensor gA = want_A ? at::empty_like(A) : at::Tensor();
-        at::Tensor gB = want_B ? at::empty_like(B) : at::Tensor();
-        at::Tensor gW = want_W ? at::empty_like(W) : at::Tensor();
+        at::Tensor gA = want_A ? new_like(A) : at::Tensor();
+        at::Tensor gB = want_B ? new_like(B) : at::Tensor();
+        at::Tensor gW = want_W ? new_like(W) : at::Tensor();
         by_dtype(A, [&](auto zero) {
             using T = decltype(zero);
             mops::cuda::sparse_accumulation_scatter_add_with_weights_vjp<T>(
@@ -504,36 +507,47 @@ struct SasawFunction : public Function<SasawFunction> {
 };
 
 // ------------------------------------------------------------ operators --
-at::Tensor homogeneous_polynomial_evaluation(at::Tensor A, at::Tensor C, at::Tensor indices_A) {
-    return Hpe::apply(A, C, indices_A);
+at::Tensor homogeneous_polynomial_evaluation(const at::Tensor& A, const at::Tensor& C, const at::Tensor& indices_A) {
+    return recorded({&A, &C}) ? Hpe::apply(A, C, indices_A) : hpe_forward(A, C, indices_A);
 }
 
-at::Tensor outer_product_scatter_add(at::Tensor A, at::Tensor B, at::Tensor indices_output, int64_t output_size) {
+at::Tensor outer_product_scatter_add(
+    const at::Tensor& A, const at::Tensor& B, const at::Tensor& indices_output, int64_t output_size
+) {
     const variable_list extra = {indices_output};
-    return Bilinear<Opsa>::apply(A, B, at::TensorList(extra), output_size);
+    return recorded({&A, &B}) ? Bilinear<Opsa>::apply(A, B, at::TensorList(extra), output_size)
+                              : bilinear_forward<Opsa>(A, B, extra, output_size);
 }
 
 at::Tensor sparse_accumulation_of_products(
-    at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor indices_A, at::Tensor indices_B, at::Tensor indices_output,
-    int64_t output_size
+    const at::Tensor& A, const at::Tensor& B, const at::Tensor& C, const at::Tensor& indices_A,
+    const at::Tensor& indices_B, const at::Tensor& indices_output, int64_t output_size
 ) {
     const variable_list extra = {C, indices_A, indices_B, indices_output};
-    return Bilinear<Sap>::apply(A, B, at::TensorList(extra), output_size);
+    return recorded({&A, &B, &C}) ? Bilinear<Sap>::apply(A, B, at::TensorList(extra), output_size)
+                                  : bilinear_forward<Sap>(A, B, extra, output_size);
 }
 
 at::Tensor outer_product_scatter_add_with_weights(
-    at::Tensor A, at::Tensor B, at::Tensor W, at::Tensor indices_W, at::Tensor indices_output
+    const at::Tensor& A, const at::Tensor& B, const at::Tensor& W, const at::Tensor& indices_W,
+    const at::Tensor& indices_output
 ) {
-    return OpsawFunction::apply(A, B, W, indices_W, indices_output);
+    return recorded({&A, &B, &W}) ? OpsawFunction::apply(A, B, W, indices_W, indices_output)
+                                  : opsaw_forward(A, B, W, indices_W, indices_output);
 }
 
 at::Tensor sparse_accumulation_scatter_add_with_weights(
-    at::Tensor A, at::Tensor B, at::Tensor C, at::Tensor W, at::Tensor indices_A, at::Tensor indices_W_1,
-    at::Tensor indices_W_2, at::Tensor indices_output_1, at::Tensor indices_output_2, int64_t output_size
+    const at::Tensor& A, const at::Tensor& B, const at::Tensor& C, const at::Tensor& W, const at::Tensor& indices_A,
+    const at::Tensor& indices_W_1, const at::Tensor& indices_W_2, const at::Tensor& indices_output_1,
+    const at::Tensor& indices_output_2, int64_t output_size
 ) {
-    return SasawFunction::apply(
-        A, B, C, W, indices_A, indices_W_1, indices_W_2, indices_output_1, indices_output_2, output_size
-    );
+    return recorded({&A, &B, &C, &W})
+               ? SasawFunction::apply(
+                     A, B, C, W, indices_A, indices_W_1, indices_W_2, indices_output_1, indices_output_2, output_size
+                 )
+               : sasaw_forward(
+                     A, B, C, W, indices_A, indices_W_1, indices_W_2, indices_output_1, indices_output_2, output_size
+                 );
 }
 
 } // namespace

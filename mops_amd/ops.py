@@ -12,8 +12,12 @@ current PyTorch stream of the tensors' device without blocking the host.
 """
 from . import _dispatch
 from ._c_api import SIGNATURES
-from ._c_lib import device_library, host_library
+from ._c_lib import array_functions, device_library, host_library
 from .checks import check_arguments, check_scalar
+
+
+#: the same functions natively, for plain ROCm tensors; each returns None where this file has to do the call
+_native = array_functions()
 
 
 def _call(function, reference, tensors):
@@ -67,6 +71,9 @@ def _optional(requested, like):
 
 # ------------------------------------------------------------------- HPE ----
 def homogeneous_polynomial_evaluation(A, C, indices_A):
+    result = _native.homogeneous_polynomial_evaluation(A, C, indices_A)
+    if result is not None:
+        return result
     function = "homogeneous_polynomial_evaluation"
     check_arguments(function, {"A": A, "C": C, "indices_A": indices_A})
     A, C = _floats(A, C)
@@ -77,6 +84,9 @@ def homogeneous_polynomial_evaluation(A, C, indices_A):
 
 
 def homogeneous_polynomial_evaluation_vjp(grad_output, A, C, indices_A, compute_grad_A=True):
+    result = _native.homogeneous_polynomial_evaluation_vjp(grad_output, A, C, indices_A, compute_grad_A)
+    if result is not None:
+        return result
     function = "homogeneous_polynomial_evaluation_vjp"
     check_arguments(
         function, {"grad_output": grad_output, "A": A, "C": C, "indices_A": indices_A}
@@ -97,6 +107,11 @@ def homogeneous_polynomial_evaluation_vjp_vjp(
     compute_grad_grad_output=True,
     compute_grad_A_2=True,
 ):
+    result = _native.homogeneous_polynomial_evaluation_vjp_vjp(
+        grad_grad_A, grad_output, A, C, indices_A, compute_grad_grad_output, compute_grad_A_2,
+    )
+    if result is not None:
+        return result
     function = "homogeneous_polynomial_evaluation_vjp_vjp"
     check_arguments(
         function,
@@ -112,6 +127,9 @@ def homogeneous_polynomial_evaluation_vjp_vjp(
 
 # ------------------------------------------------------------------- SAP ----
 def sparse_accumulation_of_products(A, B, C, indices_A, indices_B, indices_output, output_size):
+    result = _native.sparse_accumulation_of_products(A, B, C, indices_A, indices_B, indices_output, output_size)
+    if result is not None:
+        return result
     function = "sparse_accumulation_of_products"
     check_arguments(
         function,
@@ -137,6 +155,11 @@ def sparse_accumulation_of_products_vjp(
     compute_grad_A=True,
     compute_grad_B=True,
 ):
+    result = _native.sparse_accumulation_of_products_vjp(
+        grad_output, A, B, C, indices_A, indices_B, indices_output, compute_grad_A, compute_grad_B,
+    )
+    if result is not None:
+        return result
     function = "sparse_accumulation_of_products_vjp"
     check_arguments(
         function,
@@ -165,6 +188,12 @@ def sparse_accumulation_of_products_vjp_vjp(
     compute_grad_A_2=True,
     compute_grad_B_2=True,
 ):
+    result = _native.sparse_accumulation_of_products_vjp_vjp(
+        grad_grad_A, grad_grad_B, grad_output, A, B, C, indices_A, indices_B, indices_output,
+        compute_grad_grad_output, compute_grad_A_2, compute_grad_B_2,
+    )
+    if result is not None:
+        return result
     function = "sparse_accumulation_of_products_vjp_vjp"
     check_arguments(
         function,
@@ -190,6 +219,9 @@ def sparse_accumulation_of_products_vjp_vjp(
 
 # ------------------------------------------------------------------ OPSA ----
 def outer_product_scatter_add(A, B, indices_output, output_size):
+    result = _native.outer_product_scatter_add(A, B, indices_output, output_size)
+    if result is not None:
+        return result
     function = "outer_product_scatter_add"
     check_arguments(function, {"A": A, "B": B, "indices_output": indices_output})
     check_scalar(output_size, function, "output_size")
@@ -203,6 +235,9 @@ def outer_product_scatter_add(A, B, indices_output, output_size):
 def outer_product_scatter_add_vjp(
     grad_output, A, B, indices_output, compute_grad_A=True, compute_grad_B=True
 ):
+    result = _native.outer_product_scatter_add_vjp(grad_output, A, B, indices_output, compute_grad_A, compute_grad_B)
+    if result is not None:
+        return result
     function = "outer_product_scatter_add_vjp"
     check_arguments(
         function, {"grad_output": grad_output, "A": A, "B": B, "indices_output": indices_output}
@@ -226,6 +261,12 @@ def outer_product_scatter_add_vjp_vjp(
     compute_grad_A_2=True,
     compute_grad_B_2=True,
 ):
+    result = _native.outer_product_scatter_add_vjp_vjp(
+        grad_grad_A, grad_grad_B, grad_output, A, B, indices_output, compute_grad_grad_output, compute_grad_A_2,
+        compute_grad_B_2,
+    )
+    if result is not None:
+        return result
     function = "outer_product_scatter_add_vjp_vjp"
     check_arguments(
         function,
@@ -247,6 +288,9 @@ def outer_product_scatter_add_vjp_vjp(
 
 # ----------------------------------------------------------------- OPSAW ----
 def outer_product_scatter_add_with_weights(A, B, W, indices_W, indices_output):
+    result = _native.outer_product_scatter_add_with_weights(A, B, W, indices_W, indices_output)
+    if result is not None:
+        return result
     function = "outer_product_scatter_add_with_weights"
     check_arguments(
         function, {"A": A, "B": B, "W": W, "indices_W": indices_W, "indices_output": indices_output}
@@ -269,6 +313,11 @@ def outer_product_scatter_add_with_weights_vjp(
     compute_grad_B=True,
     compute_grad_W=True,
 ):
+    result = _native.outer_product_scatter_add_with_weights_vjp(
+        grad_output, A, B, W, indices_W, indices_output, compute_grad_A, compute_grad_B, compute_grad_W,
+    )
+    if result is not None:
+        return result
     function = "outer_product_scatter_add_with_weights_vjp"
     check_arguments(
         function,
@@ -336,6 +385,11 @@ def sparse_accumulation_scatter_add_with_weights(
     indices_output_2,
     output_size,
 ):
+    result = _native.sparse_accumulation_scatter_add_with_weights(
+        A, B, C, W, indices_A, indices_W_1, indices_W_2, indices_output_1, indices_output_2, output_size,
+    )
+    if result is not None:
+        return result
     function = "sparse_accumulation_scatter_add_with_weights"
     check_arguments(
         function,
@@ -373,6 +427,12 @@ def sparse_accumulation_scatter_add_with_weights_vjp(
     compute_grad_C=True,
     compute_grad_W=True,
 ):
+    result = _native.sparse_accumulation_scatter_add_with_weights_vjp(
+        grad_output, A, B, C, W, indices_A, indices_W_1, indices_W_2, indices_output_1, indices_output_2,
+        compute_grad_A, compute_grad_B, compute_grad_W,
+    )
+    if result is not None:
+        return result
     # compute_grad_C is accepted for signature compatibility and ignored, as
     # in the reference: there is no gradient with respect to C.
     function = "sparse_accumulation_scatter_add_with_weights_vjp"
