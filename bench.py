@@ -81,23 +81,14 @@ MAIN_KERNELS = {
     ("opsa", "vjp"): "opsa::edge_rows_vjp_kernel<{T}, 1, 2, false, true, false, false>",
     ("opsaw", "forward"): "opsa::forward_kernel<{T}, 2, true, true, true>",
     ("opsaw", "vjp"): "opsa::edge_rows_vjp_kernel<{T}, 1, 2, true, true, false, true>",
-    ("sasaw", "forward"): {
-        "float": "sasaw_segments::contract_kernel<float, 9, true, 32, false>",
-        "double": "sasaw_segments::contract_kernel<double, 9, true, 64, false>",
-    },
-    ("sasaw", "vjp"): {
-        "float": "sasaw_segments::gradients_kernel<float, 9, true, true, false, false>",
-        "double": "sasaw_segments::gradients_kernel<double, 9, true, true, false, false>",
-    },
+    ("sasaw", "forward"): "sasaw_columns::contract_kernel<{T}, 9, 32, 0>",
+    ("sasaw", "vjp"): "sasaw_columns::edge_kernel<{T}, 9, 32>",
 }
 
 
 def main_kernel_name(op, kind, type_name):
     """Name of the main kernel of ``op``'s ``kind`` call for elements of C++ type ``type_name``."""
-    entry = MAIN_KERNELS.get((op, kind), "?")
-    if isinstance(entry, dict):
-        return entry[type_name]
-    return entry.format(T=type_name)
+    return MAIN_KERNELS.get((op, kind), "?").format(T=type_name)
 
 
 def nbytes(arrays):

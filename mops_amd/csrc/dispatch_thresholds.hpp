@@ -70,6 +70,18 @@ constexpr int32_t ARRIVAL_MEAN_EDGES = 64;
 /// / 255, 20 000: 682 / 820. OPSAW f32 vjp: 2000 senders 27.6 / 22.6, 3000:
 /// 33.4 / 29.6, 4000: 37.6 / 39.3, 6000: 48 / 75, 20 000: 156 / 212.
 constexpr int32_t ARRIVAL_NODES = 4000;
+/// Edges x nodes from which a counting sort of the edges by sender replaces the
+/// slots where the kernels of sasaw_columns.hip use them (four lookers at the
+/// index per 16 nodes against three short launches). grad_W alone, f32, 9
+/// components, 32 columns, slots / sort: 4000 nodes of 30 edges 44.7 / 52.0 us,
+/// of 46 edges 56.0 / 64.5, 6000 of 30 70.8 / about 66, 11 000 of 10 65.5 / 59.
+constexpr size_t SLOT_PRODUCT = 1000u * 1000 * 1000;
+
+// ---- SASAW (sasaw_columns.hip) ------------------------------------------------
+/// Edges from which the forward pass of a shape that fills the matrix cores (16
+/// components, at most 16 columns, f32) stays with them: 300 000 edges 65 us
+/// against 81; 60 000 edges 31 against 22.
+constexpr int32_t COLUMNS_EDGES_AT_16 = 150000;
 
 // ---- SASAW (sasaw_segments.hip) ----------------------------------------------
 /// Values of a component index that one launch of the matrix-core kernels

@@ -895,15 +895,14 @@ __global__ __launch_bounds__(WAVE) void vjp_kernel(
 // ---------------------------------------------------------------------------
 template <typename T>
 __global__ __launch_bounds__(256) void gather_weights_kernel(
-    T* __restrict__ grad_W, const T* __restrict__ edge_W, SenderBuckets buckets, int32_t L
+    T* __restrict__ grad_W, const T* __restrict__ edge_W, EdgesBySender lists, int32_t L
 ) {
-    __shared__ int32_t bucket_lds[BUCKET_LDS_CAPACITY];
     const int32_t node = blockIdx.x;
-    SortedBucket bucket = sorted_bucket(buckets, node, bucket_lds);
+    const int32_t begin = lists.offsets[node], end = lists.offsets[node + 1];
     for (int32_t l = threadIdx.x; l < L; l += blockDim.x) {
         T sum = 0;
-        for (int32_t i = 0; i < bucket.count; i++) {
-            sum += edge_W[static_cast<size_t>(bucket.edges[i]) * L + l];
+        for (int32_t i = begin; i < end; i++) {
+            sum += edge_W[static_cast<size_t>(lists.edge[i]) * L + l];
         }
         grad_W[static_cast<size_t>(node) * L + l] = sum;
     }
@@ -1863,14 +1862,13 @@ void launch_vjp(
     const bool slotted = want_W && gather_in_kernel && sparse && !by_arrival;
     const size_t slots_bytes = slotted ? sender_slots_bytes(n_output) : by_arrival ? sender_arrivals_bytes(n_output) : 0;
     const size_t buckets_bytes =
-        want_W && !gather_in_kernel && !by_arrival ? edges_by_sender_bytes(n_output, n_edges) : slots_bytes;
+        want_W && !gather_in_kernel && !by_arrival ? edges_by_sender_bytes(n_output, n_edges, false) : slots_bytes;
     char* workspace =
         want_W ? static_cast<char*>(scratch(edge_w_bytes + buckets_bytes)) : nullptr;
     T* edge_W = want_W ? reinterpret_cast<T*>(workspace) : nullptr;
 
     // the lists of edges per sender do not depend on the kernels below: they are
     // built beside them, on a side stream that joins before the lists are used
-    SenderBuckets buckets{};
     EdgesBySender by_sender{};
     SenderSlots slots{};
     std::optional<ScratchCounters> taken; // (until the end of this call, finish_call included)
@@ -1884,11 +1882,7 @@ void launch_vjp(
     bool listed = false; // the slots are being filled by a kernel that is already enqueued
     if (use_buckets) {
         beside = std::make_unique<SideStream>(stream);
-        if (narrow_rows) {
-            by_sender = order_edges_by_sender(indices_W, n_edges, n_output, workspace + edge_w_bytes, beside->get());
-        } else {
-            buckets = build_sender_buckets(indices_W, n_edges, n_output, workspace + edge_w_bytes, beside->get());
-        }
+        by_sender = order_edges_by_sender(indices_W, n_edges, n_output, false, workspace + edge_w_bytes, beside->get());
     }
 
     // degenerate shapes: a gradient that sums over an empty axis is zero
@@ -2087,7 +2081,7 @@ void launch_vjp(
             );
         } else {
             int threads = std::min(256, round_up_wave(L));
-            gather_weights_kernel<T><<<n_output, threads, 0, stream>>>(grad_W.data, edge_W, buckets, L);
+            gather_weights_kernel<T><<<n_output, threads, 0, stream>>>(grad_W.data, edge_W, by_sender, L);
         }
     }
     finish_call(operation);

@@ -466,7 +466,7 @@ __global__ __launch_bounds__(MAX_THREADS) void vjp_weights_kernel(
     const T* __restrict__ B,
     const int32_t* __restrict__ PO1,
     CouplingPlan<T> plan,
-    SenderBuckets buckets,
+    EdgesBySender lists,
     int32_t n_nodes,
     int32_t nA,
     int32_t L,
@@ -475,7 +475,6 @@ __global__ __launch_bounds__(MAX_THREADS) void vjp_weights_kernel(
     int32_t chunk
 ) {
     extern __shared__ __align__(16) unsigned char lds_bytes[];
-    __shared__ int32_t bucket_lds[BUCKET_LDS_CAPACITY];
     const int32_t node = blockIdx.x;
     const int tid = threadIdx.x;
     const int nthreads = blockDim.x;
@@ -486,7 +485,7 @@ __global__ __launch_bounds__(MAX_THREADS) void vjp_weights_kernel(
     T* t_stage = a_stage + static_cast<size_t>(chunk) * nA;       // [chunk, n_cells]
     T* gb_stage = t_stage + static_cast<size_t>(chunk) * n_cells; // [chunk, n3, L]
 
-    SortedBucket bucket = sorted_bucket(buckets, node, bucket_lds);
+    const int32_t begin = lists.offsets[node], count = lists.offsets[node + 1] - begin;
     const int32_t row_elements = n2 * L;
     T* out_row = grad_W + static_cast<size_t>(node) * row_elements;
 
@@ -497,19 +496,19 @@ __global__ __launch_bounds__(MAX_THREADS) void vjp_weights_kernel(
         const int32_t l = active ? element - m2 * L : 0;
         T sum = 0;
 
-        for (int32_t c0 = 0; c0 < bucket.count; c0 += chunk) {
-            const int32_t n = min(chunk, bucket.count - c0);
+        for (int32_t c0 = 0; c0 < count; c0 += chunk) {
+            const int32_t n = min(chunk, count - c0);
             __syncthreads();
             for (int32_t i = tid; i < n * nA; i += nthreads) {
                 int32_t e = i / nA;
-                int32_t edge = bucket.edges[c0 + e];
+                int32_t edge = lists.edge[begin + c0 + e];
                 a_stage[i] = A[static_cast<size_t>(edge) * nA + (i - e * nA)];
             }
             for (int32_t i = tid; i < n * g_per_edge; i += nthreads) {
                 int32_t e = i / g_per_edge;
                 int32_t rest = i - e * g_per_edge; // m3 * L + col
                 int32_t col = rest % L;
-                int32_t edge = bucket.edges[c0 + e];
+                int32_t edge = lists.edge[begin + c0 + e];
                 int32_t receiver = PO1[edge];
                 T value = T(0);
                 if (in_bounds(receiver, n_nodes)) {
@@ -759,7 +758,7 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
         const sasaw_mfma::Indices indices{
             indices_A.data, indices_W_1.data, indices_W_2.data, indices_output_1.data, indices_output_2.data
         };
-        const size_t bytes = sasaw_segments::vjp_workspace_bytes(shape, want_W);
+        const size_t bytes = sasaw_segments::vjp_workspace_bytes(shape, sizeof(scalar_t), want_W);
         void* workspace = bytes > 0 ? scratch(bytes) : nullptr;
         std::optional<ScratchCounters> taken; // (until the end of this call, finish_call included)
         if (bytes > 0) {
@@ -788,7 +787,7 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
 
     const size_t segments_bytes = align256(static_cast<size_t>(s.n_nodes) * 2 * sizeof(int32_t));
     const size_t table_bytes = plan_bytes<scalar_t>(s.N, s.n_cells, s.nA);
-    const size_t buckets_bytes = want_W ? sender_buckets_bytes(s.n_nodes, s.n_edges) : 0;
+    const size_t buckets_bytes = want_W ? edges_by_sender_bytes(s.n_nodes, s.n_edges, false) : 0;
     char* workspace = static_cast<char*>(scratch(segments_bytes + table_bytes + buckets_bytes));
     auto* segments = reinterpret_cast<int32_t*>(workspace);
     CouplingPlan<scalar_t> plan = enqueue_plan<scalar_t>(
@@ -815,8 +814,8 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
     }
 
     if (want_W && s.n_nodes > 0 && s.n2 > 0 && s.L > 0) {
-        SenderBuckets buckets = build_sender_buckets(
-            indices_W_1.data, s.n_edges, s.n_nodes, workspace + segments_bytes + table_bytes, stream
+        const EdgesBySender lists = order_edges_by_sender(
+            indices_W_1.data, s.n_edges, s.n_nodes, false, workspace + segments_bytes + table_bytes, stream
         );
         const size_t per_edge =
             static_cast<size_t>(s.nA) + s.n_cells + static_cast<size_t>(s.n3) * s.L;
@@ -827,7 +826,7 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
         size_t lds = static_cast<size_t>(chunk) * per_edge * sizeof(scalar_t);
         int threads = std::min(MAX_THREADS, round_up_wave(std::min(s.n2 * s.L, MAX_THREADS)));
         vjp_weights_kernel<scalar_t><<<s.n_nodes, threads, lds, stream>>>(
-            grad_W.data, grad_output.data, A.data, B.data, indices_output_1.data, plan, buckets,
+            grad_W.data, grad_output.data, A.data, B.data, indices_output_1.data, plan, lists,
             s.n_nodes, s.nA, s.L, s.n2, s.n3, chunk
         );
     }
@@ -948,8 +947,8 @@ void sasaw_vjp_no_alloc(
         // (the same kernels as the existing entry point takes for these shapes)
         // (the places of the senders' edges, then their counters; the array is shared with the
         // kernels of other shapes, so the counters are cleared by a launch in front)
-        const size_t places = sasaw_segments::vjp_workspace_bytes(shape, want_W);
-        const size_t needed = places + sasaw_segments::vjp_counters(shape, want_W) * sizeof(int32_t);
+        const size_t places = sasaw_segments::vjp_workspace_bytes(shape, sizeof(float), want_W);
+        const size_t needed = places + sasaw_segments::vjp_counters(shape, sizeof(float), want_W) * sizeof(int32_t);
         if (needed > NO_ALLOC_SCRATCH_BYTES) {
             throw std::runtime_error(
                 std::string(who) + "these shapes need " + std::to_string(needed) + " bytes of temporary memory, the "

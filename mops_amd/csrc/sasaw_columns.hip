@@ -1,0 +1,986 @@
+// SASAW with a lane per feature column, for gfx950.
+//
+//   Z_i[m1, m2, l] = sum over edges e of i of  A[e, m1] * (B[e, l] * W[PW1[e], m2, l])
+//   O[i, m3, l]    = sum_{m1, m2} D[m3, m2, m1] * Z_i[m1, m2, l]
+//
+// (D: the coupling table made dense, see sasaw_segments.hip.) A lane stands for
+// a column l and keeps sums of Z_i[:, :, l] of a node in registers; an edge is
+// then a multiply-add per sum, whose operands are the edge's row of A, the same
+// for all lanes and therefore in scalar registers, and the lane's own elements
+// of B and of the rows of W. No lane works on padding but where the columns or
+// the block rows do not fill a wavefront, nothing is exchanged between lanes
+// until the node's edges are done, and the addresses of an edge are scalar
+// arithmetic. The f32 matrix cores do the same products at the same rate per
+// useful operation only if all 16 rows of an instruction are useful (9 of 16 at
+// l <= 2), and the f64 ones at half of it.
+//
+// The 64 lanes are (part, column): tiles of 16, 32 or 64 columns, and 4, 2 or 1
+// parts that share the block rows m2. What bounds these kernels is the
+// multiply-adds and the latency of the gathered rows of W; several edges are on
+// their way while one is worked on. O = D Z then goes through LDS and the
+// matrix cores, a few components of A at a time.
+//
+// grad_A and grad_B of an edge need
+//
+//   U[m1, l]     = sum_m2 G_i[m1, m2, l] * W[PW1[e], m2, l],   G_i = D^T grad_output_i
+//   grad_B[e, l] = sum_m1 A[e, m1] U[m1, l],   grad_A[e, m1] = sum_l B[e, l] U[m1, l]
+//
+// with G_i[:, :, l] of the receiver in the registers of the lane: both come from
+// the same multiply-adds and ONE look at the rows of W; the sum over the columns
+// is taken across lanes (DPP and permlane swaps). grad_W is the sum of the
+// forward pass over the edges of a sender, with the roles of W and grad_output,
+// m2 and m3 exchanged.
+//
+// Whole calls against one per-node sum on the matrix cores each, 9 components, 32
+// columns, f32 / f64, us: 1 000 000 edges, forward 316 -> 199 / 390 -> 386, vjp
+// 1160 -> 530 / 1360 -> 950; 60 000 edges, 21.5 -> 20.3 / 30 -> 27 and 60 -> 56 /
+// 99 -> 74; 128 columns there, vjp 247 -> 121 / 360 -> 223. At a million edges the
+// forward pass in float gathers 1.15 GB of rows at 6.8 TB/s with everything else
+// it reads, which is what the Infinity Cache gives for rows in no order.
+//
+// Every sum has one fixed order; no atomics on floating point.
+#include "sasaw_columns.hpp"
+
+#include <algorithm>
+#include <type_traits>
+
+#include "device_common.hpp"
+#include "mfma.hpp"
+#include "runtime.hpp"
+#include "sasaw_table.hpp"
+#include "sender_buckets.hpp"
+
+namespace mops::amd::sasaw_columns {
+namespace {
+
+using namespace mops::amd::sasaw;
+
+constexpr int THREADS = 256;
+constexpr int WAVES = THREADS / WAVE;
+
+/// The sums of a lane for N components of A and N block rows: all components
+/// times M2 block rows, a PARTS-th of them: part, part + PARTS, ... (so that the
+/// parts together load consecutive rows).
+template <int N, int COLUMNS> struct Sums {
+    static constexpr int PARTS = WAVE / COLUMNS;
+    static constexpr int M2 = (N + PARTS - 1) / PARTS;
+    static constexpr bool EXACT = PARTS * M2 == N;
+    static constexpr int MC = N == 4 ? 4 : N == 9 ? 3 : 2; // components of A that go through LDS at a time
+    static constexpr int CHUNKS = (N + MC - 1) / MC;
+    static constexpr int VALUES = MC * M2;       // of a lane at a time
+    static constexpr int PAIRS = PARTS * VALUES; // of a column at a time
+    static constexpr int STEPS = (PAIRS + 3) / 4, TILES = (PAIRS + 15) / 16;
+};
+
+/// A tile of COLUMNS columns: an LDS row a little longer, so that four rows of
+/// 16 columns, which a matrix instruction takes at a time, lie on different banks.
+template <int COLUMNS> constexpr int pitch() { return COLUMNS == 16 ? 16 : COLUMNS + 16; }
+
+// ------------------------------------------------------------------- table --
+/// The dense table in LDS as operands of matrix instructions. Component m1 and
+/// block row m2 are pair (m2 % PARTS) * VALUES + (m1 % MC) * M2 + m2 / PARTS of chunk m1 / MC.
+///   SPREAD false (D as left operand of D * Z), step ks of 4 pairs:
+///     table[(chunk * STEPS + ks) * 64 + 16 * (pair % 4) + o]
+///   SPREAD (D^T as left operand of D^T * grad_output), tile zt of 16 pairs, step s3 of 4 rows:
+///     table[((chunk * TILES + zt) * 4 + s3) * 64 + 16 * (o % 4) + pair % 16]
+struct Dense {
+    const int32_t* PA;   // [N]
+    const int32_t* Pred; // [N] block row
+    const int32_t* Pout; // [N] row of the result
+    int32_t entries, n_out;
+};
+template <int N, int COLUMNS, bool SPREAD> constexpr int table_slots() {
+    using S = Sums<N, COLUMNS>;
+    return S::CHUNKS * (SPREAD ? S::TILES * 4 : S::STEPS) * WAVE;
+}
+template <int N, int COLUMNS, bool SPREAD> __device__ __forceinline__ int32_t slot_of(int32_t m1, int32_t m2, int32_t o) {
+    using S = Sums<N, COLUMNS>;
+    const int32_t chunk = m1 / S::MC;
+    const int32_t pair = m2 % S::PARTS * S::VALUES + m1 % S::MC * S::M2 + m2 / S::PARTS;
+    return SPREAD ? ((chunk * S::TILES + (pair >> 4)) * 4 + (o >> 2)) * WAVE + 16 * (o & 3) + (pair & 15)
+                  : (chunk * S::STEPS + (pair >> 2)) * WAVE + 16 * (pair & 3) + o;
+}
+
+/// Called by all threads of a workgroup, which is in step afterwards. The
+/// entries of one slot are added in ascending order: every round the smallest
+/// pending one of each slot (`owner`: as many integers as the table has slots).
+template <typename T, int N, int COLUMNS, bool SPREAD>
+__device__ void build(T* __restrict__ table, int32_t* __restrict__ owner, const T* __restrict__ C, const Dense& t) {
+    constexpr int ENTRIES = 4; // of a thread at a time
+    for (int32_t s = threadIdx.x; s < table_slots<N, COLUMNS, SPREAD>(); s += THREADS) {
+        table[s] = T(0);
+        owner[s] = NOBODY;
+    }
+    for (int32_t first = 0; first < t.entries; first += THREADS * ENTRIES) {
+        int32_t m1[ENTRIES], c[ENTRIES], o[ENTRIES], slot[ENTRIES];
+        T coefficient[ENTRIES];
+#pragma unroll
+        for (int k = 0; k < ENTRIES; k++) {
+            const int32_t safe = min(static_cast<int32_t>(first + threadIdx.x + k * THREADS), t.entries - 1);
+            m1[k] = t.PA[safe];
+            c[k] = t.Pred[safe];
+            o[k] = t.Pout[safe];
+            coefficient[k] = C[safe];
+        }
+        uint32_t pending = 0;
+#pragma unroll
+        for (int k = 0; k < ENTRIES; k++) {
+            const int32_t n = first + threadIdx.x + k * THREADS;
+            const bool inside =
+                n < t.entries && in_bounds(m1[k], N) && in_bounds(c[k], N) && in_bounds(o[k], t.n_out);
+            slot[k] = slot_of<N, COLUMNS, SPREAD>(m1[k], c[k], o[k]);
+            pending |= inside ? 1u << k : 0u;
+        }
+        __syncthreads();
+        do {
+#pragma unroll
+            for (int k = 0; k < ENTRIES; k++) {
+                if (pending >> k & 1) {
+                    atomicMin(&owner[slot[k]], static_cast<int32_t>(first + threadIdx.x + k * THREADS));
+                }
+            }
+            __syncthreads();
+            uint32_t winners = 0;
+#pragma unroll
+            for (int k = 0; k < ENTRIES; k++) {
+                if ((pending >> k & 1) && owner[slot[k]] == static_cast<int32_t>(first + threadIdx.x + k * THREADS)) {
+                    winners |= 1u << k;
+                    table[slot[k]] += coefficient[k];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < ENTRIES; k++) {
+                if (winners >> k & 1) {
+                    owner[slot[k]] = NOBODY;
+                }
+            }
+            pending &= ~winners;
+        } while (__syncthreads_or(static_cast<int>(pending)));
+    }
+    __syncthreads();
+}
+
+// ---------------------------------------------------------------- wavefront --
+template <typename T> __device__ __forceinline__ void swap_rows(T& x, T& y) { // odd rows of 16 lanes of x, even ones of y
+    uint32_t a[sizeof(T) / 4], b[sizeof(T) / 4];
+    __builtin_memcpy(a, &x, sizeof(T));
+    __builtin_memcpy(b, &y, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; i++) {
+        const auto swapped = __builtin_amdgcn_permlane16_swap(a[i], b[i], false, false);
+        a[i] = swapped[0];
+        b[i] = swapped[1];
+    }
+    __builtin_memcpy(&x, a, sizeof(T));
+    __builtin_memcpy(&y, b, sizeof(T));
+}
+template <typename T> __device__ __forceinline__ void swap_halves(T& x, T& y) { // upper half of x, lower half of y
+    uint32_t a[sizeof(T) / 4], b[sizeof(T) / 4];
+    __builtin_memcpy(a, &x, sizeof(T));
+    __builtin_memcpy(b, &y, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; i++) {
+        const auto swapped = __builtin_amdgcn_permlane32_swap(a[i], b[i], false, false);
+        a[i] = swapped[0];
+        b[i] = swapped[1];
+    }
+    __builtin_memcpy(&x, a, sizeof(T));
+    __builtin_memcpy(&y, b, sizeof(T));
+}
+/// Lanes 0-31: the two halves of x added up; lanes 32-63: those of y.
+template <typename T> __device__ __forceinline__ T sum_halves(T x, T y) {
+    swap_halves(x, y);
+    return x + y;
+}
+/// Rows 0 and 2 of 16 lanes: row pairs of x added up; rows 1 and 3: those of y.
+template <typename T> __device__ __forceinline__ T sum_rows(T x, T y) {
+    swap_rows(x, y);
+    return x + y;
+}
+/// The sum over the 16 lanes of a row, in all of them.
+template <int CONTROL, typename T> __device__ __forceinline__ T rotated(T x) {
+    uint32_t a[sizeof(T) / 4];
+    __builtin_memcpy(a, &x, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; i++) {
+        a[i] = static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(a[i]), CONTROL, 0xf, 0xf, true));
+    }
+    __builtin_memcpy(&x, a, sizeof(T));
+    return x;
+}
+template <typename T> __device__ __forceinline__ T sum_of_row(T x) {
+    x += rotated<0x128>(x); // row_ror:8, 4, 2, 1
+    x += rotated<0x124>(x);
+    x += rotated<0x122>(x);
+    x += rotated<0x121>(x);
+    return x;
+}
+
+/// First position of the sorted index (n entries) whose value is not below `value`.
+__device__ __forceinline__ int32_t lower_bound(const int32_t* __restrict__ index, int32_t n, int32_t value, int lane) {
+    int32_t low = 0, high = n;
+    while (high - low > WAVE) {
+        const int32_t step = (high - low + WAVE - 1) / WAVE;
+        const int32_t probe = low + (lane + 1) * step - 1;
+        const bool below = probe < high && index[min(probe, n - 1)] < value;
+        const int32_t passed = __popcll(__ballot(below));
+        low += passed * step;
+        high = min(high, low + step);
+    }
+    const bool below = low + lane < high && index[min(low + lane, n - 1)] < value;
+    return low + __popcll(__ballot(below));
+}
+
+template <typename T> struct Walk {
+    const T* A;    // [n_edges][N]
+    const T* B;    // [n_edges][L]
+    const T* rows; // [n_blocks][N][L]  (forward: W)
+    const T* C;    // [entries]
+    int32_t n_edges, n_blocks, L;
+    int32_t column_tiles;
+    int32_t ranges; // of nodes, a wavefront each (and tile)
+    const int32_t* sorted; // [n_edges] node of every position, non-decreasing
+    const int32_t* gather; // [n_edges] block of `rows` of every edge
+    Dense table;
+};
+
+/// The next 64 positions of the sorted index, one per lane, asked for while the
+/// ones before are worked on.
+template <typename T> struct Window {
+    int32_t receiver, source;
+    bool inside;
+
+    __device__ __forceinline__ Window(const Walk<T>& p, int32_t at, int32_t lane) {
+        const int32_t position = min(at + lane, p.n_edges - 1);
+        inside = at + lane < p.n_edges;
+        receiver = p.sorted[position];
+        source = p.gather[position];
+    }
+    /// How many of them, from the first on, name `node`.
+    __device__ __forceinline__ int32_t edges_of(int32_t node) const {
+        const unsigned long long others = __ballot(!inside || receiver != node);
+        return others == 0 ? WAVE : __ffsll(others) - 1;
+    }
+};
+
+/// A lane's place, and the rows of an edge it works on.
+template <typename T, int N, int COLUMNS> struct Columns {
+    using S = Sums<N, COLUMNS>;
+    static constexpr int M2 = S::M2;
+    /// Edges whose operands are on their way while one is worked on.
+    static constexpr int AHEAD = (M2 + 1) * sizeof(T) <= 32 ? 4 : 2;
+
+    const Walk<T>& p;
+    int lane, c, part;
+    int32_t column;
+    bool column_inside;
+    uint32_t column_bytes;
+    uint32_t row_at[M2]; // byte offset of the lane's element of its rows in a block (a row there is not: the last)
+    uint32_t row_bytes, block_bytes;
+    BufferOf<T> B;
+
+    /// What a lane loads for an edge. The row of A is the same for all lanes: a scalar load.
+    struct Operands {
+        T b;
+        T w[M2];
+        T more; // (edge_kernel)
+    };
+    typedef const __attribute__((address_space(4))) T* Uniform;
+
+    __device__ __forceinline__ explicit Columns(const Walk<T>& walk) : p(walk) {
+        lane = threadIdx.x & (WAVE - 1);
+        c = lane & (COLUMNS - 1);
+        part = lane / COLUMNS;
+        row_bytes = static_cast<uint32_t>(p.L) * sizeof(T);
+        block_bytes = N * row_bytes;
+        B.set(p.B, static_cast<uint32_t>(p.n_edges) * row_bytes);
+    }
+
+    __device__ __forceinline__ void set_tile(int32_t tile) {
+        column = tile * COLUMNS + c;
+        column_inside = column < p.L;
+        column_bytes = static_cast<uint32_t>(min(column, p.L - 1)) * sizeof(T);
+#pragma unroll
+        for (int m = 0; m < M2; m++) {
+            row_at[m] = column_bytes + static_cast<uint32_t>(min(m * S::PARTS + part, N - 1)) * row_bytes;
+        }
+    }
+
+    /// Whether the lane's row m exists (the others repeat the last one).
+    __device__ __forceinline__ bool has_row(int m) const { return S::EXACT || m * S::PARTS + part < N; }
+
+    /// Asks for the operands of an edge (edge and source are uniform). The rows of a source outside
+    /// the tensor are those of a tensor of no bytes, which reads as zeros.
+    __device__ __forceinline__ void load(Operands& to, int32_t edge, int32_t source) const {
+        to.b = B.load(column_bytes, static_cast<uint32_t>(edge) * row_bytes);
+        const bool exists = in_bounds(source, p.n_blocks);
+        const uint32_t block = exists ? static_cast<uint32_t>(source) * block_bytes : 0;
+        BufferOf<T> rows;
+        rows.set(p.rows, exists ? static_cast<uint32_t>(p.n_blocks) * block_bytes : 0);
+#pragma unroll
+        for (int m = 0; m < M2; m++) {
+            to.w[m] = rows.load(row_at[m], block);
+        }
+    }
+    __device__ __forceinline__ void load_row_of_A(T (&to)[N], int32_t edge) const {
+        const Uniform row = (Uniform)(p.A + static_cast<size_t>(static_cast<uint32_t>(edge)) * N);
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            to[i] = row[i];
+        }
+    }
+
+    /// `each(row of A, operands, k)` for the edges k < n <= 64 of a list: edge k is `edge_of(k)`, lane k
+    /// holds its source (of one outside the tensor, everything counts as zero). `ask(operands, k)`:
+    /// what else `each` wants loaded for an edge.
+    ///
+    /// What makes the operands of AHEAD edges be on their way: no branch between the asking and the
+    /// waiting (the compiler counts the loads of both ways and takes the smaller number), the order of
+    /// the asking kept, stores without a branch around them (they count as well), and the row of A
+    /// asked for only when the one before has arrived (scalar loads come back in any order, so that a
+    /// wait is for all of them).
+    template <typename EdgeOf, typename Ask, typename Each>
+    __device__ __forceinline__ void
+    over(int32_t sources, int32_t n, EdgeOf&& edge_of, Ask&& ask_more, Each&& each) const {
+        Operands ring[AHEAD];
+        auto ask = [&](Operands& to, int32_t k) {
+            k = min(k, n - 1);
+            load(to, edge_of(k), __builtin_amdgcn_readlane(sources, k));
+            ask_more(to, k);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        T a[2][N];
+        load_row_of_A(a[0], edge_of(0));
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+            ask(ring[d], d);
+        }
+        auto step = [&](int d, int32_t k) {
+            arrived(a[d & 1]);
+            load_row_of_A(a[~d & 1], edge_of(min(k + 1, n - 1)));
+            __builtin_amdgcn_sched_barrier(0);
+            each(a[d & 1], ring[d], k);
+        };
+        int32_t first = 0;
+        for (; first + AHEAD <= n; first += AHEAD) {
+#pragma unroll
+            for (int d = 0; d < AHEAD; d++) {
+                step(d, first + d);
+                ask(ring[d], first + d + AHEAD);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < AHEAD - 1; d++) {
+            if (first + d < n) { // (uniform)
+                step(d, first + d);
+            }
+        }
+    }
+
+    /// Waits for a row of A.
+    static __device__ __forceinline__ void arrived(T (&a)[N]) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            asm volatile("" : "+s"(a[i]));
+        }
+    }
+};
+
+// -------------------------------------------------------------- contraction --
+template <typename T> struct ContractArgs {
+    Walk<T> walk;
+    T* result; // [n_blocks][n_out][L]
+    // the edges of every sender: LISTS == SLOTS, and what they were made from
+    SenderSlots slots;
+    const int32_t* senders; // [n_edges]
+    // LISTS == ORDERED
+    EdgesBySender ordered;
+};
+
+/// Where the edges of a node are: next to each other in the (sorted) index, or in lists.
+enum Lists { SEGMENTS, SLOTS, ORDERED };
+
+/// The next 64 edges, one per lane: at positions of the index, or of the ordered lists.
+template <typename T, Lists LISTS> struct ContractWindow : Window<T> {
+    __device__ __forceinline__ ContractWindow(const ContractArgs<T>& args, int32_t at, int32_t lane)
+        : Window<T>(args.walk, at, lane) {}
+    __device__ __forceinline__ int32_t edges_of(const ContractArgs<T>&, int32_t node, int32_t) const {
+        return Window<T>::edges_of(node);
+    }
+    static __device__ __forceinline__ int32_t edge(int32_t at, int32_t k) { return at + k; }
+};
+template <typename T> struct ContractWindow<T, ORDERED> {
+    int32_t listed, source;
+
+    __device__ __forceinline__ ContractWindow(const ContractArgs<T>& args, int32_t at, int32_t lane) {
+        listed = args.ordered.edge[min(at + lane, args.walk.n_edges - 1)];
+        source = args.walk.gather[listed];
+    }
+    __device__ __forceinline__ int32_t edges_of(const ContractArgs<T>& args, int32_t node, int32_t at) const {
+        return min(args.ordered.offsets[node + 1] - at, WAVE);
+    }
+    __device__ __forceinline__ int32_t edge(int32_t, int32_t k) const { return __builtin_amdgcn_readlane(listed, k); }
+};
+
+/// Wavefronts per SIMD.
+template <typename T, int N, int COLUMNS> constexpr int contract_waves() {
+    constexpr int REGISTERS = (N * Sums<N, COLUMNS>::M2 + 34) * static_cast<int>(sizeof(T)) / 4;
+    return REGISTERS <= 90 ? 4 : REGISTERS <= 130 ? 3 : 2;
+}
+template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
+    using S = Sums<N, COLUMNS>;
+    return table_slots<N, COLUMNS, false>() * sizeof(T) +
+           std::max(table_slots<N, COLUMNS, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
+}
+
+template <typename T, int N, int COLUMNS, Lists LISTS>
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contract_kernel(const ContractArgs<T> args) {
+    using M = Mfma<T>;
+    using S = Sums<N, COLUMNS>;
+    constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::STEPS * 4 * PITCH;
+    const Walk<T>& p = args.walk;
+    extern __shared__ __align__(16) char lds[];
+    T* table = reinterpret_cast<T*>(lds);
+    T* stages = table + table_slots<N, COLUMNS, false>();
+    int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
+    T* stage = stages + wave * STAGE;
+
+    Columns<T, N, COLUMNS> columns_of(p);
+    const int lane = columns_of.lane;
+    build<T, N, COLUMNS, false>(table, owner, p.C, p.table);
+    for (int32_t k = lane; k < STAGE; k += WAVE) {
+        stage[k] = T(0); // (rows of a step that stand for no pair stay zero)
+    }
+    wave_sync();
+
+    const int32_t unit = blockIdx.x * WAVES + wave;
+    const int32_t tile = unit % p.column_tiles, range = unit / p.column_tiles;
+    if (range >= p.ranges) {
+        return;
+    }
+    columns_of.set_tile(tile);
+    const int32_t node0 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * range / p.ranges);
+    const int32_t node1 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * (range + 1) / p.ranges);
+
+    T z[N * M2];
+    auto add = [&](const T (&a)[N], const auto& operands, int32_t) {
+        T bw[M2];
+#pragma unroll
+        for (int m = 0; m < M2; m++) {
+            bw[m] = operands.b * operands.w[m];
+        }
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+#pragma unroll
+            for (int m = 0; m < M2; m++) {
+                z[i * M2 + m] += a[i] * bw[m];
+            }
+        }
+    };
+
+    auto nothing = [](auto&, int32_t) {};
+
+    // O = D Z, MC components of A at a time through LDS
+    const int row16 = lane >> 4;
+    T* mine = stage + columns_of.part * S::VALUES * PITCH + columns_of.c;
+    const T* right = stage + row16 * PITCH + (lane & 15);
+    auto finish = [&](int32_t node) {
+        typename M::Acc acc[COLUMNS / 16];
+#pragma unroll
+        for (int t = 0; t < COLUMNS / 16; t++) {
+            acc[t] = M::zero();
+        }
+#pragma unroll
+        for (int chunk = 0; chunk < S::CHUNKS; chunk++) {
+#pragma unroll
+            for (int k = 0; k < S::VALUES; k++) { // pair k of the lane's part
+                if (chunk * S::VALUES + k < N * M2) {
+                    const T sum = z[chunk * S::VALUES + k];
+                    mine[k * PITCH] = columns_of.has_row(k % M2) ? sum : T(0);
+                }
+            }
+            wave_sync();
+#pragma unroll
+            for (int ks = 0; ks < S::STEPS; ks++) {
+                const T left = table[(chunk * S::STEPS + ks) * WAVE + lane];
+#pragma unroll
+                for (int t = 0; t < COLUMNS / 16; t++) {
+                    acc[t] = M::mma(left, right[4 * ks * PITCH + 16 * t], acc[t]);
+                }
+            }
+            wave_sync();
+        }
+        T* target = args.result + static_cast<size_t>(node) * p.table.n_out * p.L;
+#pragma unroll
+        for (int t = 0; t < COLUMNS / 16; t++) {
+            const int32_t column = tile * COLUMNS + 16 * t + (lane & 15);
+            if (column < p.L) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int row = M::row(lane, r);
+                    if (row < p.table.n_out) {
+                        target[static_cast<size_t>(row) * p.L + column] = acc[t][r];
+                    }
+                }
+            }
+        }
+    };
+    auto clear = [&] {
+#pragma unroll
+        for (int k = 0; k < N * M2; k++) {
+            z[k] = T(0);
+        }
+    };
+
+    if constexpr (LISTS != SLOTS) {
+        int32_t at = LISTS == SEGMENTS ? lower_bound(p.sorted, p.n_edges, node0, lane) : args.ordered.offsets[node0];
+        // positions at .. at + 64 of the index or of the lists, and the blocks of their edges
+        ContractWindow<T, LISTS> window(args, at, lane);
+        for (int32_t node = node0; node < node1; node++) {
+            clear();
+            int32_t n;
+            do {
+                n = window.edges_of(args, node, at);
+                const ContractWindow<T, LISTS> next(args, at + n, lane);
+                if (n > 0) {
+                    columns_of.over(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, add);
+                }
+                at += n;
+                window = next;
+            } while (n == WAVE);
+            finish(node);
+        }
+    } else {
+        for (int32_t node = node0; node < node1; node++) {
+            clear();
+            auto hand_on = [&](int32_t edge, int32_t n) {
+                const int32_t sources = p.gather[edge];
+                columns_of.over(
+                    sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, add
+                );
+            };
+            const int32_t* places = args.slots.edges + static_cast<size_t>(node) * SLOT_CAPACITY;
+            int32_t first_half = places[lane], second_half = places[lane + WAVE];
+            static_assert(SLOT_PARTS == 4 && SLOT_CAPACITY == 2 * WAVE, "four parts of a node's places in two registers");
+            const int4 counts = reinterpret_cast<const int4*>(args.slots.counts)[node];
+            const int32_t c0 = __builtin_amdgcn_readfirstlane(counts.x), c1 = __builtin_amdgcn_readfirstlane(counts.y);
+            const int32_t c2 = __builtin_amdgcn_readfirstlane(counts.z), c3 = __builtin_amdgcn_readfirstlane(counts.w);
+            const int32_t count = c0 + c1 + c2 + c3;
+            const bool listed = max(max(c0, c1), max(c2, c3)) <= SLOT_PART_CAPACITY;
+            // the parts moved together: position k of the list is in part `part`, place k - before
+            const int32_t low = first_half, high = second_half;
+            auto edge_at = [&](int32_t position) {
+                const int32_t part =
+                    (position >= c0 ? 1 : 0) + (position >= c0 + c1 ? 1 : 0) + (position >= c0 + c1 + c2 ? 1 : 0);
+                const int32_t before = part == 0 ? 0 : part == 1 ? c0 : part == 2 ? c0 + c1 : c0 + c1 + c2;
+                const int32_t place = part * SLOT_PART_CAPACITY + position - before;
+                const int32_t from_low = __shfl(low, place & (WAVE - 1));
+                const int32_t from_high = __shfl(high, place & (WAVE - 1));
+                return place < WAVE ? from_low : from_high;
+            };
+            if (listed) {
+                first_half = edge_at(lane);
+                second_half = count > WAVE ? edge_at(lane + WAVE) : 0;
+            }
+            if (listed) {
+                if (count > 0) {
+                    hand_on(lane < count ? first_half : 0, min(count, WAVE));
+                }
+                if (count > WAVE) {
+                    hand_on(lane + WAVE < count ? second_half : 0, count - WAVE);
+                }
+            } else {
+                // more edges than places (a hub of a sparse graph): this wavefront reads the index itself
+                const unsigned long long below = (1ull << lane) - 1ull;
+                for (int32_t base = 0; base < p.n_edges; base += WAVE) {
+                    const int32_t e = base + lane;
+                    const bool named = e < p.n_edges && args.senders[min(e, p.n_edges - 1)] == node;
+                    const unsigned long long mask = __ballot(named);
+                    if (mask != 0) {
+                        const int32_t n = __popcll(mask);
+                        const int32_t named_below = __popcll(mask & below);
+                        const int32_t place = named ? named_below : n + lane - named_below;
+                        const int32_t edges = __builtin_amdgcn_ds_permute(place << 2, e);
+                        hand_on(lane < n ? edges : 0, n);
+                    }
+                }
+            }
+            finish(node);
+        }
+    }
+}
+
+// ---------------------------------------------------------------- gradients --
+template <typename T> struct EdgeArgs {
+    Walk<T> walk;
+    const T* grad_output; // [n_nodes][n_out][L]
+    T* grad_A;            // [n_edges][nA], may be null
+    T* grad_B;            // [n_edges][L], may be null
+    int32_t shares;       // wavefronts per range, each with a share of a node's edges
+};
+
+/// Wavefronts per SIMD.
+template <typename T, int N, int COLUMNS> constexpr int edge_waves() {
+    constexpr int REGISTERS = (N * Sums<N, COLUMNS>::M2 + N + 44) * static_cast<int>(sizeof(T)) / 4;
+    return REGISTERS <= 100 ? 4 : REGISTERS <= 140 ? 3 : 2;
+}
+template <typename T, int N, int COLUMNS> constexpr size_t edge_lds() {
+    return table_slots<N, COLUMNS, true>() * sizeof(T) +
+           std::max(table_slots<N, COLUMNS, true>() * sizeof(int32_t), WAVES * Sums<N, COLUMNS>::TILES * 16 * pitch<COLUMNS>() * sizeof(T));
+}
+
+template <typename T, int N, int COLUMNS>
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kernel(const EdgeArgs<T> args) {
+    using M = Mfma<T>;
+    using S = Sums<N, COLUMNS>;
+    constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::TILES * 16 * PITCH;
+    const Walk<T>& p = args.walk;
+    extern __shared__ __align__(16) char lds[];
+    T* table = reinterpret_cast<T*>(lds);
+    T* stages = table + table_slots<N, COLUMNS, true>();
+    int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
+    T* stage = stages + wave * STAGE;
+
+    Columns<T, N, COLUMNS> columns_of(p);
+    const int lane = columns_of.lane;
+    build<T, N, COLUMNS, true>(table, owner, p.C, p.table);
+
+    const int32_t unit = blockIdx.x * WAVES + wave;
+    const int32_t range = unit / args.shares, share = unit % args.shares;
+    if (range >= p.ranges) {
+        return;
+    }
+    const int32_t node0 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * range / p.ranges);
+    const int32_t node1 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * (range + 1) / p.ranges);
+    BufferOf<T> G;
+    const uint32_t g_block_bytes = static_cast<uint32_t>(p.table.n_out) * columns_of.row_bytes;
+    G.set(args.grad_output, static_cast<uint32_t>(p.n_blocks) * g_block_bytes);
+    const int row16 = lane >> 4, sub = lane & 15;
+    constexpr int FOLDED = (N + 3) / 4;
+    constexpr uint32_t A_ROW_BYTES = N * sizeof(T);
+    const int32_t component = 4 * sub + ((row16 & 1) << 1 | row16 >> 1);
+    const uint32_t a_at =
+        static_cast<uint32_t>(component) * static_cast<uint32_t>(sizeof(T)) | unless(sub < FOLDED && component < N);
+    // (a gradient that is not wanted: a tensor of no bytes, which stores do not reach)
+    BufferOf<T> to_A, to_B;
+    to_A.set(args.grad_A, args.grad_A != nullptr ? static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES : 0);
+    to_B.set(args.grad_B, args.grad_B != nullptr ? static_cast<uint32_t>(p.n_edges) * columns_of.row_bytes : 0);
+    const T* spread_from = stage + columns_of.part * S::VALUES * PITCH + columns_of.c;
+    const int32_t start = lower_bound(p.sorted, p.n_edges, node0, lane);
+
+    for (int32_t tile = 0; tile < p.column_tiles; tile++) {
+        columns_of.set_tile(tile);
+        // what this lane stores of an edge's gradients, if anything: an element of grad_B, and a
+        // component of grad_A, to which the columns of the tiles before are added
+        const uint32_t b_at = columns_of.column_bytes | unless(columns_of.part == 0 && columns_of.column_inside);
+        BufferOf<T> from_A;
+        from_A.set(args.grad_A, tile == 0 || args.grad_A == nullptr ? 0 : static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES);
+        int32_t at = start;
+        Window<T> window(p, at, lane);
+        for (int32_t node = node0; node < node1; node++) {
+            T g[N * M2];
+            bool have = false;
+            // G = D^T grad_output of the node, MC components of A at a time through LDS
+            auto spread = [&] {
+                T upstream[COLUMNS / 16][4];
+#pragma unroll
+                for (int t = 0; t < COLUMNS / 16; t++) {
+#pragma unroll
+                    for (int s3 = 0; s3 < 4; s3++) {
+                        const int32_t o = 4 * s3 + row16, column = tile * COLUMNS + 16 * t + sub;
+                        upstream[t][s3] = G.load(
+                            (static_cast<uint32_t>(node) * g_block_bytes + static_cast<uint32_t>(o) * columns_of.row_bytes +
+                             static_cast<uint32_t>(column) * static_cast<uint32_t>(sizeof(T))) |
+                                unless(o < p.table.n_out && column < p.L),
+                            0
+                        );
+                    }
+                }
+#pragma unroll
+                for (int chunk = 0; chunk < S::CHUNKS; chunk++) {
+#pragma unroll
+                    for (int zt = 0; zt < S::TILES; zt++) {
+                        typename M::Acc acc[COLUMNS / 16];
+#pragma unroll
+                        for (int t = 0; t < COLUMNS / 16; t++) {
+                            acc[t] = M::zero();
+                        }
+#pragma unroll
+                        for (int s3 = 0; s3 < 4; s3++) {
+                            if (4 * s3 < p.table.n_out) { // (uniform)
+                                const T left = table[((chunk * S::TILES + zt) * 4 + s3) * WAVE + lane];
+#pragma unroll
+                                for (int t = 0; t < COLUMNS / 16; t++) {
+                                    acc[t] = M::mma(left, upstream[t][s3], acc[t]);
+                                }
+                            }
+                        }
+#pragma unroll
+                        for (int t = 0; t < COLUMNS / 16; t++) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                stage[(zt * 16 + M::row(lane, r)) * PITCH + 16 * t + sub] = acc[t][r];
+                            }
+                        }
+                    }
+                    wave_sync();
+#pragma unroll
+                    for (int k = 0; k < S::VALUES; k++) {
+                        if (chunk * S::VALUES + k < N * M2) {
+                            g[chunk * S::VALUES + k] = spread_from[k * PITCH];
+                        }
+                    }
+                    wave_sync();
+                }
+                if constexpr (!S::EXACT) { // (what the last part has no row for)
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        g[i * M2 + M2 - 1] = columns_of.has_row(M2 - 1) ? g[i * M2 + M2 - 1] : T(0);
+                    }
+                }
+            };
+            auto gradients = [&](int32_t first) {
+                return [&, first](const T (&a)[N], const auto& operands, int32_t k) {
+                    T u[N];
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        u[i] = g[i * M2] * operands.w[0];
+#pragma unroll
+                        for (int m = 1; m < M2; m++) {
+                            u[i] += g[i * M2 + m] * operands.w[m];
+                        }
+                    }
+                    const uint32_t edge = static_cast<uint32_t>(first + k);
+                    T sum = a[0] * u[0];
+#pragma unroll
+                    for (int i = 1; i < N; i++) {
+                        sum += a[i] * u[i];
+                    }
+                    // over the parts: rows of 16 lanes, or halves
+                    if constexpr (S::PARTS == 4) {
+                        sum = sum_rows(sum, sum);
+                    }
+                    if constexpr (S::PARTS > 1) {
+                        sum = sum_halves(sum, sum);
+                    }
+                    to_B.store(sum, b_at, edge * columns_of.row_bytes);
+                    const T b = columns_of.column_inside ? operands.b : T(0);
+                    auto term = [&](int i) { return i < N ? u[i < N ? i : 0] * b : T(0); };
+                    // the sum over columns and parts: four values folded together across the halves
+                    // and the rows of the wavefront, so that a row of 16 lanes sums one
+                    T mine = T(0);
+#pragma unroll
+                    for (int i = 0; i < FOLDED; i++) {
+                        const T low = sum_halves(term(4 * i), term(4 * i + 1));
+                        const T folded =
+                            sum_of_row(sum_rows(low, 4 * i + 2 < N ? sum_halves(term(4 * i + 2), term(4 * i + 3)) : T(0)));
+                        mine = sub == i ? folded : mine;
+                    }
+                    to_A.store(mine + operands.more, a_at, edge * A_ROW_BYTES);
+                };
+            };
+            int32_t n;
+            do {
+                n = window.edges_of(node);
+                const Window<T> next(p, at + n, lane);
+                const int32_t from = n * share / args.shares, to = n * (share + 1) / args.shares;
+                if (to > from) {
+                    if (!have) {
+                        spread();
+                        have = true;
+                    }
+                    const int32_t first = at + from;
+                    columns_of.over(
+                        __shfl(window.source, min(from + lane, to - 1)), to - from, [&](int32_t k) { return first + k; },
+                        [&](auto& operands, int32_t k) {
+                            operands.more = from_A.load(a_at, static_cast<uint32_t>(first + k) * A_ROW_BYTES);
+                        },
+                        gradients(first)
+                    );
+                }
+                at += n;
+                window = next;
+            } while (n == WAVE);
+        }
+    }
+}
+
+// --------------------------------------------------------------------- host --
+/// What a tile of columns costs: the multiply-adds of a lane, and some eight
+/// instructions' worth of everything else.
+template <int N, int COLUMNS> constexpr int cost() { return (N + 1) * Sums<N, COLUMNS>::M2 + 8; }
+
+/// body(N, COLUMNS): the cheapest tiles.
+template <typename T, typename Body> void with_layout(const Shape& s, bool narrow, Body&& body) {
+    auto with_columns = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        // (sums that fit the registers of a lane)
+        constexpr int MOST = N == 16 ? (sizeof(T) == 4 ? 32 : 16) : 64;
+        int best = 16, least = (s.L + 15) / 16 * cost<N, 16>();
+        if (const int c = (s.L + 31) / 32 * cost<N, 32>(); MOST >= 32 && c <= least) {
+            best = 32;
+            least = c;
+        }
+        if (const int c = (s.L + 63) / 64 * cost<N, 64>(); MOST >= 64 && c <= least) {
+            best = 64;
+        }
+        // (few nodes: more, narrower tiles, which the contraction takes as wavefronts of their own)
+        if (narrow && static_cast<int64_t>(s.n_nodes) * ((s.L + best - 1) / best) < 4 * compute_units()) {
+            best = 16;
+        }
+        if (best == 16) {
+            body(n, std::integral_constant<int, 16>{});
+        }
+        if constexpr (MOST >= 32) {
+            if (best == 32) {
+                body(n, std::integral_constant<int, 32>{});
+            }
+        }
+        if constexpr (MOST >= 64) {
+            if (best == 64) {
+                body(n, std::integral_constant<int, 64>{});
+            }
+        }
+    };
+    if (s.nA == 4) {
+        with_columns(std::integral_constant<int, 4>{});
+    } else if (s.nA == 9) {
+        with_columns(std::integral_constant<int, 9>{});
+    } else {
+        with_columns(std::integral_constant<int, 16>{});
+    }
+}
+
+template <typename Kernel> void allow_lds(Kernel kernel, size_t lds) {
+    if (lds > 64 * 1024) {
+        MOPS_HIP_CHECK(hipFuncSetAttribute(
+            reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)
+        ));
+    }
+}
+
+template <typename T>
+Walk<T> walk_of(
+    const Shape& s, const T* A, const T* B, const T* rows, const T* C, const int32_t* sorted, const int32_t* gather,
+    const Dense& table
+) {
+    Walk<T> w{};
+    w.A = A;
+    w.B = B;
+    w.rows = rows;
+    w.C = C;
+    w.n_edges = s.n_edges;
+    w.n_blocks = s.n_nodes;
+    w.L = s.L;
+    w.sorted = sorted;
+    w.gather = gather;
+    w.table = table;
+    return w;
+}
+
+template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Shape& s, hipStream_t stream) {
+    with_layout<T>(s, true, [&](auto n, auto columns) {
+        constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
+        Walk<T>& w = args.walk;
+        constexpr size_t lds = contract_lds<T, N, COLUMNS>();
+        w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
+        const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * contract_waves<T, N, COLUMNS>();
+        w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, std::max<int64_t>(1, resident / w.column_tiles)));
+        const size_t units = static_cast<size_t>(w.ranges) * w.column_tiles;
+        auto kernel = contract_kernel<T, N, COLUMNS, LISTS>;
+        allow_lds(kernel, lds);
+        kernel<<<static_cast<unsigned>(ceil_div(units, WAVES)), THREADS, lds, stream>>>(args);
+    });
+    MOPS_HIP_CHECK(hipGetLastError());
+}
+
+} // namespace
+
+bool covers(int32_t nA, int32_t block_rows, int32_t result_rows) {
+    return (nA == 4 || nA == 9 || nA == 16) && block_rows == nA && result_rows <= MAX_INDEX;
+}
+
+template <typename T>
+void forward(
+    T* output, const T* A, const T* B, const T* C, const T* W, const Indices& indices, const Shape& s, hipStream_t stream
+) {
+    ContractArgs<T> args{};
+    args.walk = walk_of(
+        s, A, B, W, C, indices.output_1, indices.W_1, Dense{indices.A, indices.W_2, indices.output_2, s.N, s.n3}
+    );
+    args.result = output;
+    MainKernelTimer timer(stream);
+    contract<T, SEGMENTS>(args, s, stream);
+}
+
+template <typename T>
+void weight_gradient(
+    T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& s,
+    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+) {
+    ContractArgs<T> args{};
+    args.walk = walk_of<T>(
+        s, A, B, grad_output, C, nullptr, indices.output_1, Dense{indices.A, indices.output_2, indices.W_2, s.N, s.n2}
+    );
+    args.result = grad_W;
+    if (slots != nullptr) {
+        args.slots = *slots;
+        args.senders = indices.W_1;
+        contract<T, SLOTS>(args, s, stream);
+    } else {
+        args.ordered = *ordered;
+        contract<T, ORDERED>(args, s, stream);
+    }
+}
+
+template <typename T>
+void edge_gradients(
+    T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
+    const Shape& s, hipStream_t stream
+) {
+    EdgeArgs<T> args{};
+    args.walk = walk_of(
+        s, A, B, W, C, indices.output_1, indices.W_1, Dense{indices.A, indices.W_2, indices.output_2, s.N, s.n3}
+    );
+    args.grad_output = grad_output;
+    args.grad_A = grad_A;
+    args.grad_B = grad_B;
+    MainKernelTimer timer(stream);
+    with_layout<T>(s, false, [&](auto components, auto columns) {
+        constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
+        Walk<T>& w = args.walk;
+        constexpr size_t lds = edge_lds<T, N, COLUMNS>();
+        w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
+        const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * edge_waves<T, N, COLUMNS>();
+        w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, resident));
+        // (a node's edges shared out where there are fewer nodes than wavefronts, in shares of four or more)
+        const int64_t shares = std::min<int64_t>(s.n_edges / (4 * static_cast<int64_t>(s.n_nodes)), resident / s.n_nodes);
+        args.shares = static_cast<int32_t>(std::max<int64_t>(1, shares));
+        const size_t units = static_cast<size_t>(w.ranges) * args.shares;
+        auto kernel = edge_kernel<T, N, COLUMNS>;
+        allow_lds(kernel, lds);
+        kernel<<<static_cast<unsigned>(ceil_div(units, WAVES)), THREADS, lds, stream>>>(args);
+    });
+    MOPS_HIP_CHECK(hipGetLastError());
+}
+
+#define MOPS_INSTANTIATE(T)                                                                         \
+    template void forward<T>(                                                                      \
+        T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t      \
+    );                                                                                             \
+    template void edge_gradients<T>(                                                               \
+        T*, T*, const T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t \
+    );                                                                                             \
+    template void weight_gradient<T>(                                                              \
+        T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, const SenderSlots*, const EdgesBySender*, hipStream_t \
+    );
+MOPS_INSTANTIATE(float)
+MOPS_INSTANTIATE(double)
+#undef MOPS_INSTANTIATE
+
+} // namespace mops::amd::sasaw_columns

@@ -1,0 +1,56 @@
+// SASAW with a lane per feature column (sasaw_columns.hip): the numbers of
+// components of equivariant message passing. sasaw_segments.hip calls these for
+// them and keeps its own kernels for other numbers.
+#ifndef MOPS_AMD_SASAW_COLUMNS_HPP
+#define MOPS_AMD_SASAW_COLUMNS_HPP
+
+#include <cstddef>
+#include <cstdint>
+
+#include <hip/hip_runtime.h>
+
+#include "dispatch_thresholds.hpp"
+#include "sasaw_mfma.hpp"
+#include "sender_buckets.hpp"
+
+namespace mops::amd::sasaw_columns {
+
+using sasaw_mfma::Indices;
+using sasaw_mfma::Shape;
+
+/// Whether these kernels cover sums over `nA` components and `block_rows` block
+/// rows with `result_rows` rows of the result: 4, 9 or 16 of the first two (the
+/// components of spherical harmonics up to some degree), at most 16 of the last.
+bool covers(int32_t nA, int32_t block_rows, int32_t result_rows);
+
+/// Where the matrix cores (sasaw_segments.hip) stay ahead in the forward pass:
+/// 16 components in float leave none of their rows unused, and up to 16 columns
+/// leave these kernels their narrowest tiles.
+inline bool slower_forward(const Shape& shape, size_t element_size) {
+    return element_size == 4 && shape.nA == 16 && shape.L <= 16 && shape.n_edges > thresholds::COLUMNS_EDGES_AT_16;
+}
+
+template <typename T>
+void forward(
+    T* output, const T* A, const T* B, const T* C, const T* W, const Indices& indices, const Shape& shape,
+    hipStream_t stream
+);
+
+/// grad_A, grad_B: either may be null.
+template <typename T>
+void edge_gradients(
+    T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
+    const Shape& shape, hipStream_t stream
+);
+
+/// The edges of every sender in slots, or in the order of their senders: one of
+/// the two is null.
+template <typename T>
+void weight_gradient(
+    T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& shape,
+    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+);
+
+} // namespace mops::amd::sasaw_columns
+
+#endif

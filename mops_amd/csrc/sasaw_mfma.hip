@@ -1353,7 +1353,7 @@ bool lists_edges_in_slots(const Shape& s) {
 
 size_t workspace_bytes(const Shape& s, size_t element_size) {
     return align256(dense_bytes(dense_layout(s), element_size)) +
-           (orders_edges_by_sender(s, element_size) ? edges_by_sender_bytes(s.n_nodes, s.n_edges)
+           (orders_edges_by_sender(s, element_size) ? edges_by_sender_bytes(s.n_nodes, s.n_edges, true)
             : lists_edges_in_slots(s)               ? sender_slots_bytes(s.n_nodes)
                                                     : 0);
 }
@@ -1534,7 +1534,7 @@ void vjp(
         SideStream side(stream);
         EdgesBySender order{};
         if (by_sender) {
-            order = order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, order_workspace, side.get());
+            order = order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, true, order_workspace, side.get());
         }
         for_each_column_block(s, [&](int32_t first, const Shape& block) {
             if (by_sender) {
@@ -1549,7 +1549,7 @@ void vjp(
     } else if (grad_W != nullptr) {
         EdgesBySender order{};
         if (by_sender) {
-            order = order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, order_workspace, stream);
+            order = order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, true, order_workspace, stream);
         }
         for_each_column_block(s, [&](int32_t first, const Shape& block) {
             if (by_sender) {

@@ -35,8 +35,8 @@ void forward(
 /// 32-bit counters (see SenderArrivals in sender_buckets.hpp). vjp() makes no
 /// allocation and uses no second stream.
 bool vjp_supported(const Shape& shape, size_t element_size, bool want_grad_W);
-size_t vjp_workspace_bytes(const Shape& shape, bool want_grad_W);
-size_t vjp_counters(const Shape& shape, bool want_grad_W);
+size_t vjp_workspace_bytes(const Shape& shape, size_t element_size, bool want_grad_W);
+size_t vjp_counters(const Shape& shape, size_t element_size, bool want_grad_W);
 
 /// Any of grad_A, grad_B, grad_W may be null (not all). `counters`: the
 /// vjp_counters() counters; they are zero again when the kernels have run.

@@ -8,247 +8,333 @@ namespace mops::amd {
 
 namespace {
 
-constexpr int THREADS = 256;
-constexpr int SCAN_THREADS = 1024;
+// A stable counting sort of the edges by sender, in two levels where there are
+// more senders than MOST_BUCKETS: into buckets of 2^shift consecutive senders,
+// then every bucket by a workgroup of its own. Nothing is counted or placed by
+// atomics on global memory (a returning atomic per edge, 1 000 000 of them over
+// eight L2 caches, took 90 us): a workgroup counts its share of the edges, and
+// the next launch finds out from all counts where its share of every bucket
+// begins. 1 000 000 edges over 33 000 senders: 49 us for the three launches (5, 17
+// and 27; what they wait for is one dependent load after the other), 300 000 over
+// 10 000: 27.
+constexpr int SORT_THREADS = 1024;
+constexpr int32_t MOST_BUCKETS = 512;
+constexpr int32_t MOST_SHARES = 256;         // workgroups of the first level
+constexpr int32_t SENDERS_AT_A_TIME = 4096;  // of the second level: counters in LDS
 
-__global__ __launch_bounds__(THREADS) void clear_kernel(int32_t* __restrict__ data, int32_t count) {
-    int32_t i = blockIdx.x * THREADS + threadIdx.x;
-    if (i < count) {
-        data[i] = 0;
+constexpr int BATCH = 4;                     // positions a lane asks for at once
+
+/// What lies at a position: an edge, its sender, and what it is sorted by (negative: it is not).
+struct Item {
+    int32_t key, edge, sender;
+};
+
+/// The lanes of a wavefront with the same key, and how many of them are below this one.
+struct Ranked {
+    uint64_t same;
+    uint32_t before;
+};
+__device__ __forceinline__ Ranked rank_in_wave(int32_t key, bool valid, int bits, int lane) {
+    uint64_t same = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+        const bool set = (key >> b & 1) != 0;
+        const uint64_t with = __ballot(set);
+        same &= set ? with : ~with;
     }
+    return Ranked{same, static_cast<uint32_t>(__popcll(same & ((uint64_t(1) << lane) - 1)))};
 }
 
-// integer atomics: the final counts do not depend on the order of arrival
-__global__ __launch_bounds__(THREADS) void count_kernel(
-    const int32_t* __restrict__ senders, int32_t n_edges, int32_t n_nodes, int32_t* __restrict__ counts
-) {
-    int32_t e = blockIdx.x * THREADS + threadIdx.x;
-    if (e < n_edges) {
-        int32_t node = senders[e];
-        if (in_bounds(node, n_nodes)) {
-            atomicAdd(&counts[node], 1);
-        }
+/// A wavefront's share [begin, end) of the positions a workgroup has.
+struct Share {
+    int32_t begin, end;
+    __device__ __forceinline__ Share(int32_t first, int32_t last, int wave, int waves) {
+        const int32_t each = ((last - first + waves - 1) / waves + WAVE - 1) / WAVE * WAVE;
+        begin = min(first + wave * each, last);
+        end = min(begin + each, last);
     }
-}
+};
 
-// one workgroup: exclusive prefix sum of counts -> offsets (and a copy of the
-// offsets in `cursor`, the running insertion point of each list)
-__global__ __launch_bounds__(SCAN_THREADS) void scan_kernel(
-    const int32_t* __restrict__ counts,
-    int32_t n_nodes,
-    int32_t* __restrict__ offsets,
-    int32_t* __restrict__ cursor
-) {
-    __shared__ int32_t tile[SCAN_THREADS];
-    __shared__ int32_t carry;
-    const int tid = threadIdx.x;
-    if (tid == 0) {
-        carry = 0;
+/// counters[wavefront][key] := how many of the wavefront's items have the key.
+template <typename ItemAt>
+__device__ __forceinline__ void
+count_keys(int32_t* counters, int32_t keys, const Share& share, int wave, int waves, int lane, ItemAt&& item_at) {
+    for (int32_t i = threadIdx.x; i < waves * keys; i += blockDim.x) {
+        counters[i] = 0;
     }
     __syncthreads();
-    for (int32_t base = 0; base < n_nodes; base += SCAN_THREADS) {
-        int32_t i = base + tid;
-        int32_t value = i < n_nodes ? counts[i] : 0;
-        tile[tid] = value;
-        __syncthreads();
-        for (int distance = 1; distance < SCAN_THREADS; distance <<= 1) {
-            int32_t add = tid >= distance ? tile[tid - distance] : 0;
-            __syncthreads();
-            tile[tid] += add;
-            __syncthreads();
+    for (int32_t at = share.begin + lane; at - lane < share.end; at += BATCH * WAVE) {
+        int32_t key[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            key[u] = item_at(min(at + u * WAVE, share.end - 1)).key;
         }
-        int32_t exclusive = carry + tile[tid] - value;
-        if (i < n_nodes) {
-            offsets[i] = exclusive;
-            cursor[i] = exclusive;
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            if (at + u * WAVE < share.end && key[u] >= 0) {
+                atomicAdd(&counters[wave * keys + key[u]], 1);
+            }
         }
-        __syncthreads();
-        if (tid == SCAN_THREADS - 1) {
-            carry += tile[tid];
-        }
-        __syncthreads();
     }
-    if (tid == 0) {
-        offsets[n_nodes] = carry;
+    __syncthreads();
+}
+
+/// put(place, item) for every item that has a key, items of one key in ascending places:
+/// counters[wavefront][key] is the place of the wavefront's first one.
+template <typename ItemAt, typename Put>
+__device__ __forceinline__ void place_keys(
+    int32_t* counters, int32_t keys, int bits, const Share& share, int wave, int lane, ItemAt&& item_at, Put&& put
+) {
+    int32_t* mine = counters + static_cast<size_t>(wave) * keys;
+    for (int32_t at = share.begin + lane; at - lane < share.end; at += BATCH * WAVE) {
+        Item item[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            item[u] = item_at(min(at + u * WAVE, share.end - 1));
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            const bool valid = at + u * WAVE < share.end && item[u].key >= 0;
+            const Ranked ranked = rank_in_wave(item[u].key, valid, bits, lane);
+            const int32_t place = valid ? mine[item[u].key] + static_cast<int32_t>(ranked.before) : 0;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (valid && ranked.before == 0) {
+                mine[item[u].key] += __popcll(ranked.same);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (valid) {
+                put(place, item[u]);
+            }
+        }
     }
 }
 
-// the position inside a list depends on the order of arrival; consumers sort
-// each list, so the arrival order never reaches a floating-point sum
-__global__ __launch_bounds__(THREADS) void fill_kernel(
-    const int32_t* __restrict__ senders,
-    int32_t n_edges,
-    int32_t n_nodes,
-    int32_t* __restrict__ cursor,
-    int32_t* __restrict__ order
-) {
-    int32_t e = blockIdx.x * THREADS + threadIdx.x;
-    if (e < n_edges) {
-        int32_t node = senders[e];
-        if (in_bounds(node, n_nodes)) {
-            int32_t slot = atomicAdd(&cursor[node], 1);
-            order[slot] = e;
+/// Turns counters[wavefront][key] into the place of the wavefront's first of each key:
+/// start_of(key, number of the workgroup's keys) and what the wavefronts before have. All threads.
+template <typename StartOf>
+__device__ __forceinline__ void starts_of_waves(int32_t* counters, int32_t keys, int waves, StartOf&& start_of) {
+    for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
+        int32_t total = 0;
+        for (int w = 0; w < waves; w++) {
+            total += counters[w * keys + key];
         }
+        int32_t place = start_of(key, total);
+        for (int w = 0; w < waves; w++) {
+            const int32_t here = counters[w * keys + key];
+            counters[w * keys + key] = place;
+            place += here;
+        }
+    }
+    __syncthreads();
+}
+
+/// values[0 .. n) := `first` + the sum of those before; returns `first` + the sum of all. All
+/// threads; `of_wave`: an integer per wavefront.
+__device__ __forceinline__ int32_t scan_in_place(int32_t* values, int32_t n, int32_t first, int32_t* of_wave) {
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, waves = blockDim.x / WAVE;
+    int32_t carry = first;
+    for (int32_t base = 0; base < n; base += blockDim.x) {
+        const int32_t i = base + threadIdx.x;
+        const int32_t value = i < n ? values[i] : 0;
+        int32_t sum = value;
+#pragma unroll
+        for (int step = 1; step < WAVE; step <<= 1) {
+            const int32_t other = __shfl_up(sum, step);
+            sum += lane >= step ? other : 0;
+        }
+        if (lane == WAVE - 1) {
+            of_wave[wave] = sum;
+        }
+        __syncthreads();
+        int32_t ahead = carry;
+        for (int w = 0; w < waves; w++) {
+            ahead += w < wave ? of_wave[w] : 0;
+            carry += of_wave[w];
+        }
+        if (i < n) {
+            values[i] = ahead + sum - value;
+        }
+        __syncthreads();
+    }
+    return carry;
+}
+
+/// counts[workgroup][pitch]: how many in every bucket of the workgroup's share of the edges.
+__global__ __launch_bounds__(SORT_THREADS) void count_buckets_kernel(
+    int32_t* __restrict__ counts, const int32_t* __restrict__ senders, int32_t n_edges, int32_t n_nodes, int shift,
+    int32_t pitch, int32_t share
+) {
+    __shared__ int32_t histogram[MOST_BUCKETS];
+    for (int32_t b = threadIdx.x; b < pitch; b += SORT_THREADS) {
+        histogram[b] = 0;
+    }
+    __syncthreads();
+    const int32_t begin = blockIdx.x * share, end = begin + min(share, n_edges - begin);
+    constexpr int AHEAD = 4;
+    for (int32_t e = begin + threadIdx.x; e < end; e += AHEAD * SORT_THREADS) {
+        int32_t sender[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            sender[u] = senders[min(e + u * SORT_THREADS, n_edges - 1)];
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            if (e + u * SORT_THREADS < end && in_bounds(sender[u], n_nodes)) {
+                atomicAdd(&histogram[sender[u] >> shift], 1);
+            }
+        }
+    }
+    __syncthreads();
+    for (int32_t b = threadIdx.x; b < pitch; b += SORT_THREADS) {
+        counts[static_cast<size_t>(blockIdx.x) * pitch + b] = histogram[b];
     }
 }
 
-// workgroup `node` writes its list, sorted, and its own number next to every
-// entry; workgroup n_nodes fills what is left after the last list
-// (threads, entries sorted in LDS; longer lists take the slow way through global memory):
-// small workgroups for the short lists of a graph, large ones where lists are long on average
-constexpr int SHORT_LIST_THREADS = 64;
-constexpr int SHORT_LIST_CAPACITY = BUCKET_LDS_CAPACITY;
-constexpr int LONG_LIST_THREADS = 256;
-constexpr int LONG_LIST_CAPACITY = 8192;
-
-template <int LIST_THREADS, int LIST_LDS_CAPACITY>
-__global__ __launch_bounds__(LIST_THREADS) void write_lists_kernel(
-    SenderBuckets buckets, int32_t n_nodes, int32_t n_edges, int32_t* __restrict__ sender_of_position,
-    int32_t* __restrict__ edge_of_position
+/// The edges into their buckets, in ascending order. With one sender per bucket this is the result;
+/// `offsets`: where every bucket begins, and where the last one ends. `pitch`: the buckets, rounded
+/// up to a multiple of four.
+/// LDS: counters[wavefronts][pitch], before[pitch], total[pitch], of_wave[wavefronts].
+__global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
+    int32_t* __restrict__ sender_of_place, int32_t* __restrict__ edge_of_place, int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ counts, const int32_t* __restrict__ senders, int32_t n_edges, int32_t n_nodes, int shift,
+    int32_t buckets, int32_t pitch, int bits, int32_t share
 ) {
-    __shared__ int32_t list[LIST_LDS_CAPACITY];
-    const int32_t node = blockIdx.x;
-    if (node == n_nodes) {
-        for (int32_t at = buckets.offsets[n_nodes] + threadIdx.x; at < n_edges; at += LIST_THREADS) {
-            sender_of_position[at] = n_nodes;
-            edge_of_position[at] = 0;
-        }
-        return;
-    }
-    const int32_t begin = buckets.offsets[node];
-    const SortedBucket sorted = sorted_bucket(buckets, node, list, LIST_LDS_CAPACITY);
-    for (int32_t at = threadIdx.x; at < sorted.count; at += LIST_THREADS) {
-        sender_of_position[begin + at] = node;
-        edge_of_position[begin + at] = sorted.edges[at];
-    }
-}
-
-// Small problems (a table of some thousands of entries over a few hundred values:
-// the monomial table of HPE turned round) in ONE workgroup, without atomics on
-// shared counters and without a sort afterwards: wavefront w looks after a
-// contiguous share of the edges; counts per (wavefront, value) in LDS, a scan
-// over them, and then every edge takes the next free place of its value, edges
-// of one group of 64 with the same value in lane order (ranks from ballots
-// over the bits of the value). The places are handed out in ascending edge
-// order, so every list comes out sorted.
-constexpr int SMALL_WAVES = 16;
-constexpr int SMALL_THREADS = SMALL_WAVES * WAVE;
-constexpr int32_t SMALL_MAX_NODES = 896; // (SMALL_WAVES + 1) counters per value in 64 KB of LDS
-constexpr int32_t SMALL_MAX_EDGES = 131072;
-
-/// LDS: counts[SMALL_WAVES][n_nodes] totals[n_nodes] (ints).
-__global__ __launch_bounds__(SMALL_THREADS) void order_small_kernel(
-    const int32_t* __restrict__ senders, int32_t n_edges, int32_t n_nodes, int32_t value_bits,
-    int32_t* __restrict__ offsets, int32_t* __restrict__ sender_of_position, int32_t* __restrict__ edge_of_position
-) {
-    extern __shared__ __align__(16) unsigned char lds_bytes[];
-    int32_t* counts = reinterpret_cast<int32_t*>(lds_bytes);
-    int32_t* totals = counts + SMALL_WAVES * n_nodes;
-    const int tid = threadIdx.x;
-    const int lane = tid & (WAVE - 1);
-    const int wave = tid >> 6;
-    const int32_t share = (n_edges + SMALL_THREADS - 1) / SMALL_THREADS * WAVE;
-    const int32_t my_begin = min(wave * share, n_edges);
-    const int32_t my_end = min(my_begin + share, n_edges);
-    // the value of edge e for this lane: negative if there is no such edge or the value is out of range
-    auto value_of = [&](int32_t e) {
-        const int32_t loaded = load_or_zero(senders, static_cast<size_t>(e), e < my_end);
-        return e < my_end && in_bounds(loaded, n_nodes) ? loaded : -1;
+    constexpr int WAVES = SORT_THREADS / WAVE;
+    extern __shared__ int32_t shared[];
+    int32_t* counters = shared;
+    int32_t* before = counters + WAVES * pitch;
+    int32_t* total = before + pitch;
+    int32_t* of_wave = total + pitch;
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int32_t first = blockIdx.x * share, last = first + min(share, n_edges - first);
+    const Share mine(first, last, wave, WAVES);
+    auto item_at = [&](int32_t e) {
+        const int32_t sender = senders[e];
+        return Item{in_bounds(sender, n_nodes) ? sender >> shift : -1, e, sender};
     };
+    for (int32_t b = threadIdx.x; b < pitch; b += SORT_THREADS) {
+        before[b] = 0;
+        total[b] = 0;
+    }
+    count_keys(counters, pitch, mine, wave, WAVES, lane, item_at);
+    // what the workgroups before have of every bucket, and all of them: several threads per bucket
+    // (of a single workgroup, the counts it has just made)
+    const int32_t* all_counts = gridDim.x > 1 ? counts : counters;
+    const int32_t rows = gridDim.x > 1 ? static_cast<int32_t>(gridDim.x) : WAVES;
+    const int32_t mine_from = gridDim.x > 1 ? static_cast<int32_t>(blockIdx.x) : 0;
+    const int32_t groups = pitch / 4; // (of four buckets)
+    const int32_t group = static_cast<int32_t>(threadIdx.x) % groups;
+    int4 ahead{0, 0, 0, 0}, all{0, 0, 0, 0};
+#pragma unroll 8
+    for (int32_t w = threadIdx.x / groups; w < rows; w += SORT_THREADS / groups) {
+        const int4 count = reinterpret_cast<const int4*>(all_counts)[w * groups + group];
+        const int32_t earlier = w < mine_from ? -1 : 0;
+        ahead.x += count.x & earlier;
+        ahead.y += count.y & earlier;
+        ahead.z += count.z & earlier;
+        ahead.w += count.w & earlier;
+        all.x += count.x;
+        all.y += count.y;
+        all.z += count.z;
+        all.w += count.w;
+    }
+    if (static_cast<int32_t>(threadIdx.x) < SORT_THREADS / groups * groups) {
+        int32_t* to = before + 4 * group;
+        atomicAdd(&to[0], ahead.x);
+        atomicAdd(&to[1], ahead.y);
+        atomicAdd(&to[2], ahead.z);
+        atomicAdd(&to[3], ahead.w);
+        to = total + 4 * group;
+        atomicAdd(&to[0], all.x);
+        atomicAdd(&to[1], all.y);
+        atomicAdd(&to[2], all.z);
+        atomicAdd(&to[3], all.w);
+    }
+    __syncthreads();
+    const int32_t listed = scan_in_place(total, buckets, 0, of_wave);
+    if (blockIdx.x == 0) {
+        for (int32_t bucket = threadIdx.x; bucket < buckets; bucket += SORT_THREADS) {
+            offsets[bucket] = total[bucket];
+        }
+        if (threadIdx.x == 0) {
+            offsets[buckets] = listed;
+        }
+    }
+    starts_of_waves(counters, pitch, WAVES, [&](int32_t bucket, int32_t) { return total[bucket] + before[bucket]; });
+    place_keys(counters, pitch, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+        edge_of_place[place] = item.edge;
+        if (sender_of_place != nullptr) {
+            sender_of_place[place] = item.sender;
+        }
+    });
+    // (places that no edge takes: as many as there are edges whose sender does not exist)
+    for (int32_t place = max(first, listed) + static_cast<int32_t>(threadIdx.x); place < last; place += SORT_THREADS) {
+        edge_of_place[place] = 0;
+        if (sender_of_place != nullptr) {
+            sender_of_place[place] = n_nodes;
+        }
+    }
+}
 
-    for (int32_t i = tid; i < SMALL_WAVES * n_nodes; i += SMALL_THREADS) {
-        counts[i] = 0;
-    }
-    __syncthreads();
-    constexpr int AHEAD = 8; // loads in flight
-    for (int32_t e0 = my_begin; e0 < my_end; e0 += AHEAD * WAVE) {
-        int32_t value[AHEAD];
-#pragma unroll
-        for (int c = 0; c < AHEAD; c++) {
-            value[c] = value_of(e0 + c * WAVE + lane);
-        }
-#pragma unroll
-        for (int c = 0; c < AHEAD; c++) {
-            if (value[c] >= 0) {
-                atomicAdd(&counts[wave * n_nodes + value[c]], 1); // integer counts in LDS: no order involved
+/// A workgroup per bucket puts its edges in the order of their senders: `senders` of the edges, or
+/// of the places (`of_place`).
+/// LDS: counters[wavefronts][at_a_time], start[at_a_time], of_wave[wavefronts].
+__global__ __launch_bounds__(SORT_THREADS) void sort_buckets_kernel(
+    int32_t* __restrict__ sender_of_place, int32_t* __restrict__ edge_of_place, int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ bucket_offsets, const int32_t* __restrict__ senders, const int32_t* __restrict__ edges,
+    bool of_place, int32_t n_edges, int32_t n_nodes, int shift, int32_t at_a_time, int bits
+) {
+    extern __shared__ int32_t shared[];
+    const int waves = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    int32_t* counters = shared;
+    int32_t* start = counters + waves * at_a_time;
+    int32_t* of_wave = start + at_a_time;
+    const int32_t begin = bucket_offsets[blockIdx.x], end = bucket_offsets[blockIdx.x + 1];
+    const Share mine(begin, end, wave, waves);
+    const int32_t node0 = static_cast<int32_t>(blockIdx.x) << shift;
+    const int32_t nodes = min(1 << shift, n_nodes - node0);
+    int32_t place0 = begin;
+    for (int32_t base = 0; base < nodes; base += at_a_time) {
+        const int32_t keys = min(at_a_time, nodes - base);
+        auto item_at = [&](int32_t place) {
+            const int32_t edge = edges[place], sender = senders[of_place ? place : edge];
+            const int32_t key = sender - node0 - base;
+            return Item{in_bounds(key, keys) ? key : -1, edge, sender};
+        };
+        count_keys(counters, keys, mine, wave, waves, lane, item_at);
+        for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
+            int32_t sum = 0;
+            for (int w = 0; w < waves; w++) {
+                sum += counters[w * keys + key];
             }
-        }
-    }
-    __syncthreads();
-    // counts[w][v] := edges of value v in the shares before w; totals[v] := all of them
-    if (tid < n_nodes) {
-        int32_t running = 0;
-        for (int w = 0; w < SMALL_WAVES; w++) {
-            const int32_t here = counts[w * n_nodes + tid];
-            counts[w * n_nodes + tid] = running;
-            running += here;
-        }
-        totals[tid] = running;
-    }
-    __syncthreads();
-    // inclusive scan of totals over the values (at most one per thread)
-    for (int32_t step = 1; step < n_nodes; step <<= 1) {
-        const int32_t mine = tid < n_nodes ? totals[tid] : 0;
-        const int32_t left = tid < n_nodes && tid >= step ? totals[tid - step] : 0;
-        __syncthreads();
-        if (tid < n_nodes) {
-            totals[tid] = mine + left;
+            start[key] = sum;
         }
         __syncthreads();
+        place0 = scan_in_place(start, keys, place0, of_wave);
+        for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
+            offsets[node0 + base + key] = start[key];
+        }
+        starts_of_waves(counters, keys, waves, [&](int32_t key, int32_t) { return start[key]; });
+        place_keys(counters, keys, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+            edge_of_place[place] = item.edge;
+            if (sender_of_place != nullptr) {
+                sender_of_place[place] = item.sender;
+            }
+        });
+        __syncthreads();
     }
-    const int32_t listed = totals[n_nodes - 1];
-    if (tid < n_nodes) {
-        const int32_t before = tid > 0 ? totals[tid - 1] : 0;
-        offsets[tid] = before;
-        if (tid == n_nodes - 1) {
-            offsets[n_nodes] = totals[tid];
+    if (blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x == 0) {
+            offsets[n_nodes] = end;
         }
-        for (int w = 0; w < SMALL_WAVES; w++) {
-            counts[w * n_nodes + tid] += before;
-        }
-    }
-    __syncthreads();
-    for (int32_t e0 = my_begin; e0 < my_end; e0 += AHEAD * WAVE) {
-        int32_t value[AHEAD];
-#pragma unroll
-        for (int c = 0; c < AHEAD; c++) {
-            value[c] = value_of(e0 + c * WAVE + lane);
-        }
-#pragma unroll
-        for (int c = 0; c < AHEAD; c++) {
-            if (e0 + c * WAVE < my_end) { // uniform
-                const bool valid = value[c] >= 0;
-                // the lanes with my value: agreement on every bit of it
-                unsigned long long match = __ballot(valid);
-                for (int32_t bit = 0; bit < value_bits; bit++) {
-                    const bool set = ((value[c] >> bit) & 1) != 0;
-                    const unsigned long long with_bit = __ballot(valid && set);
-                    match &= set ? with_bit : ~with_bit;
-                }
-                const int32_t rank = __popcll(match & ((1ull << lane) - 1ull));
-                const int32_t same = __popcll(match);
-                int32_t place = -1;
-                if (valid) {
-                    place = counts[wave * n_nodes + value[c]] + rank;
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                if (valid && rank == same - 1) {
-                    counts[wave * n_nodes + value[c]] += same; // one lane per value of the group
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                if (place >= 0) {
-                    sender_of_position[place] = value[c];
-                    edge_of_position[place] = e0 + c * WAVE + lane;
-                }
+        for (int32_t place = end + static_cast<int32_t>(threadIdx.x); place < n_edges; place += blockDim.x) {
+            edge_of_place[place] = 0;
+            if (sender_of_place != nullptr) {
+                sender_of_place[place] = n_nodes;
             }
         }
-    }
-    for (int32_t at = listed + tid; at < n_edges; at += SMALL_THREADS) {
-        sender_of_position[at] = n_nodes;
-        edge_of_position[at] = 0;
     }
 }
 
@@ -337,88 +423,96 @@ void clear_counters(int32_t* counters, size_t count, hipStream_t stream) {
     }
 }
 
-size_t edges_by_sender_bytes(int32_t n_nodes, int32_t n_edges) {
-    return sender_buckets_bytes(n_nodes, n_edges) + 2 * align256(static_cast<size_t>(n_edges) * 4);
+namespace {
+
+struct SortPlan {
+    int shift;       // senders per bucket: 2^shift
+    int32_t buckets, pitch;
+    int32_t share;   // edges per workgroup of the first level
+    int32_t shares;
+};
+SortPlan sort_plan(int32_t n_nodes, int32_t n_edges) {
+    SortPlan plan;
+    plan.shift = 0;
+    while ((n_nodes - 1) >> plan.shift >= MOST_BUCKETS) {
+        plan.shift++;
+    }
+    plan.buckets = ((n_nodes - 1) >> plan.shift) + 1;
+    plan.pitch = (plan.buckets + 3) / 4 * 4;
+    const size_t each = ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(SORT_THREADS) * MOST_SHARES);
+    plan.share = static_cast<int32_t>(each) * SORT_THREADS;
+    plan.shares = static_cast<int32_t>(ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(plan.share)));
+    return plan;
+}
+int bits_for(int32_t values) {
+    int bits = 0;
+    while ((int64_t(1) << bits) < values) {
+        bits++;
+    }
+    return bits;
+}
+
+} // namespace
+
+size_t edges_by_sender_bytes(int32_t n_nodes, int32_t n_edges, bool with_senders) {
+    if (n_nodes < 1) {
+        return 0;
+    }
+    return align256((static_cast<size_t>(n_nodes) + 1) * 4) + align256((MOST_BUCKETS + 1) * 4) +
+           (with_senders ? 4 : 2) * align256(static_cast<size_t>(n_edges) * 4);
 }
 
 EdgesBySender order_edges_by_sender(
-    const int32_t* senders, int32_t n_edges, int32_t n_nodes, void* workspace, hipStream_t stream
+    const int32_t* senders, int32_t n_edges, int32_t n_nodes, bool with_senders, void* workspace, hipStream_t stream
 ) {
-    if (n_nodes >= 1 && n_nodes <= SMALL_MAX_NODES && n_edges >= 1 && n_edges <= SMALL_MAX_EDGES) {
-        // same places in the workspace as below
-        char* at = static_cast<char*>(workspace);
-        int32_t* offsets = reinterpret_cast<int32_t*>(at + align256(static_cast<size_t>(n_nodes) * 4));
-        at += sender_buckets_bytes(n_nodes, n_edges);
-        int32_t* sender_of_position = reinterpret_cast<int32_t*>(at);
-        int32_t* edge_of_position = reinterpret_cast<int32_t*>(at + align256(static_cast<size_t>(n_edges) * 4));
-        int32_t value_bits = 0;
-        while ((1 << value_bits) < n_nodes) {
-            value_bits++;
-        }
-        const size_t lds = static_cast<size_t>(SMALL_WAVES + 1) * n_nodes * sizeof(int32_t);
-        order_small_kernel<<<1, SMALL_THREADS, lds, stream>>>(
-            senders, n_edges, n_nodes, value_bits, offsets, sender_of_position, edge_of_position
+    if (n_nodes < 1) {
+        return EdgesBySender{nullptr, nullptr, nullptr};
+    }
+    char* at = static_cast<char*>(workspace);
+    auto take = [&](size_t integers) {
+        int32_t* p = reinterpret_cast<int32_t*>(at);
+        at += align256(integers * 4);
+        return p;
+    };
+    int32_t* offsets = take(static_cast<size_t>(n_nodes) + 1);
+    int32_t* bucket_offsets = take(MOST_BUCKETS + 1);
+    int32_t* edge = take(static_cast<size_t>(n_edges));
+    int32_t* edge_in_buckets = take(static_cast<size_t>(n_edges));
+    int32_t* sender = with_senders ? take(static_cast<size_t>(n_edges)) : nullptr;
+    int32_t* sender_in_buckets = with_senders ? take(static_cast<size_t>(n_edges)) : nullptr;
+    if (n_edges < 1) {
+        clear_counters(offsets, static_cast<size_t>(n_nodes) + 1, stream);
+        return EdgesBySender{sender, edge, offsets};
+    }
+    const SortPlan plan = sort_plan(n_nodes, n_edges);
+    const bool two_levels = plan.shift > 0;
+    // The counts of several shares lie where nothing is written by the launch that reads them. They
+    // fit: a share is 1024 edges or more, and there are 512 buckets at most.
+    int32_t* counts = two_levels ? edge : edge_in_buckets;
+    if (plan.shares > 1) {
+        count_buckets_kernel<<<plan.shares, SORT_THREADS, 0, stream>>>(
+            counts, senders, n_edges, n_nodes, plan.shift, plan.pitch, plan.share
         );
-        MOPS_HIP_CHECK(hipGetLastError());
-        return EdgesBySender{sender_of_position, edge_of_position, offsets};
     }
-    const SenderBuckets buckets = build_sender_buckets(senders, n_edges, n_nodes, workspace, stream);
-    char* base = static_cast<char*>(workspace) + sender_buckets_bytes(n_nodes, n_edges);
-    int32_t* sender_of_position = reinterpret_cast<int32_t*>(base);
-    int32_t* edge_of_position = reinterpret_cast<int32_t*>(base + align256(static_cast<size_t>(n_edges) * 4));
-    if (static_cast<size_t>(n_edges) <= static_cast<size_t>(n_nodes) * 256) {
-        write_lists_kernel<SHORT_LIST_THREADS, SHORT_LIST_CAPACITY>
-            <<<static_cast<unsigned>(n_nodes) + 1, SHORT_LIST_THREADS, 0, stream>>>(
-                buckets, n_nodes, n_edges, sender_of_position, edge_of_position
-            );
-    } else {
-        write_lists_kernel<LONG_LIST_THREADS, LONG_LIST_CAPACITY>
-            <<<static_cast<unsigned>(n_nodes) + 1, LONG_LIST_THREADS, 0, stream>>>(
-                buckets, n_nodes, n_edges, sender_of_position, edge_of_position
-            );
-    }
-    MOPS_HIP_CHECK(hipGetLastError());
-    return EdgesBySender{sender_of_position, edge_of_position, buckets.offsets};
-}
-
-size_t sender_buckets_bytes(int32_t n_nodes, int32_t n_edges) {
-    size_t nodes = static_cast<size_t>(n_nodes);
-    size_t edges = static_cast<size_t>(n_edges);
-    return align256(nodes * 4) + align256((nodes + 1) * 4) + align256(nodes * 4) +
-           2 * align256(edges * 4);
-}
-
-SenderBuckets build_sender_buckets(
-    const int32_t* senders, int32_t n_edges, int32_t n_nodes, void* workspace, hipStream_t stream
-) {
-    char* base = static_cast<char*>(workspace);
-    size_t nodes = static_cast<size_t>(n_nodes);
-    size_t edges = static_cast<size_t>(n_edges);
-    int32_t* counts = reinterpret_cast<int32_t*>(base);
-    base += align256(nodes * 4);
-    int32_t* offsets = reinterpret_cast<int32_t*>(base);
-    base += align256((nodes + 1) * 4);
-    int32_t* cursor = reinterpret_cast<int32_t*>(base);
-    base += align256(nodes * 4);
-    int32_t* order = reinterpret_cast<int32_t*>(base);
-    base += align256(edges * 4);
-    int32_t* order_sorted = reinterpret_cast<int32_t*>(base);
-
-    unsigned node_blocks = static_cast<unsigned>(ceil_div(nodes, THREADS));
-    unsigned edge_blocks = static_cast<unsigned>(ceil_div(edges, THREADS));
-
-    if (node_blocks > 0) {
-        clear_kernel<<<node_blocks, THREADS, 0, stream>>>(counts, n_nodes);
-    }
-    if (edge_blocks > 0) {
-        count_kernel<<<edge_blocks, THREADS, 0, stream>>>(senders, n_edges, n_nodes, counts);
-    }
-    scan_kernel<<<1, SCAN_THREADS, 0, stream>>>(counts, n_nodes, offsets, cursor);
-    if (edge_blocks > 0) {
-        fill_kernel<<<edge_blocks, THREADS, 0, stream>>>(senders, n_edges, n_nodes, cursor, order);
+    constexpr int WAVES = SORT_THREADS / WAVE;
+    const size_t lds = (static_cast<size_t>(WAVES + 2) * plan.pitch + WAVES) * sizeof(int32_t);
+    fill_buckets_kernel<<<plan.shares, SORT_THREADS, lds, stream>>>(
+        two_levels ? sender_in_buckets : sender, two_levels ? edge_in_buckets : edge,
+        two_levels ? bucket_offsets : offsets, counts, senders, n_edges, n_nodes, plan.shift, plan.buckets,
+        plan.pitch, bits_for(plan.buckets), plan.share
+    );
+    if (two_levels) {
+        const int32_t at_a_time = std::min(int32_t(1) << plan.shift, SENDERS_AT_A_TIME);
+        // (the counters of all wavefronts within 64 KB)
+        const int waves = at_a_time <= 512 ? 16 : at_a_time <= 1024 ? 8 : at_a_time <= 2048 ? 4 : 2;
+        const size_t sort_lds = (static_cast<size_t>(waves + 1) * at_a_time + waves) * sizeof(int32_t);
+        sort_buckets_kernel<<<plan.buckets, waves * WAVE, sort_lds, stream>>>(
+            sender, edge, offsets, bucket_offsets, with_senders ? sender_in_buckets : senders, edge_in_buckets,
+            with_senders, n_edges, n_nodes, plan.shift, at_a_time, bits_for(at_a_time)
+        );
     }
     MOPS_HIP_CHECK(hipGetLastError());
-    return SenderBuckets{offsets, order, order_sorted};
+    return EdgesBySender{sender, edge, offsets};
 }
 
 } // namespace mops::amd

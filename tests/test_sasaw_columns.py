@@ -1,0 +1,92 @@
+"""SASAW with a lane per feature column (mops_amd/csrc/sasaw_columns.hip) against the oracle.
+
+4, 9 and 16 values of every component index; columns at the edges of its tiles of 16, 32 and 64 and
+just beside them; lists of edges around the number it asks for ahead and around 64; nodes without
+edges, a single node, and more nodes than wavefronts; senders outside the tensor; every way the edges
+of a sender are listed.
+"""
+import numpy as np
+import pytest
+
+from tests import support
+from tests.support import cpu_forward, cpu_vjp, hip_forward, hip_vjp, to_device
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # edges, nodes, components, entries, columns
+    (1, 1, 4, 10, 1),
+    (3, 2, 9, 40, 31),
+    (65, 1, 9, 250, 33),
+    (130, 2, 16, 300, 17),
+    (400, 300, 4, 24, 64),
+    (900, 30, 9, 250, 65),
+    (1000, 20, 16, 800, 48),
+    (1500, 50, 9, 1100, 100),
+    (2000, 40, 4, 30, 130),
+    (6000, 5000, 9, 100, 20),
+    (30000, 1000, 16, 100, 12),
+    # the senders' edges by a counting sort, in one level and in two
+    (9000, 3, 4, 12, 5),
+    (40000, 600, 4, 12, 3),
+]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_against_the_oracle(oracle, device, shape, dtype):
+    edges, nodes, n, entries, columns = shape
+    case = support.sasaw_case(
+        sum(shape), dtype, E=edges, nA=n, L=columns, n_nodes=nodes, n2=n, n3=n, N=entries, allow_empty=True
+    )
+    exact, absolute, on_device = support.in_float64(case), support.magnitudes(case), to_device(case, device)
+    single = dtype == np.float32
+
+    def check(name, run, actual):
+        support.assert_calibrated(
+            actual.cpu().numpy(), run(exact), dtype, f"{shape} {name}", run(case) if single else None,
+            None if single else run(absolute),
+        )  # fmt: skip
+
+    check("output", lambda c: cpu_forward(oracle, "sasaw", c), hip_forward("sasaw", on_device))
+    gradients = hip_vjp("sasaw", on_device)
+    for key, gradient in gradients.items():
+        check(f"grad_{key}", lambda c: cpu_vjp(oracle, "sasaw", c)[key], gradient)
+    again = hip_vjp("sasaw", on_device)
+    for key in gradients:  # the same bits twice, and alone
+        assert (gradients[key] == again[key]).all(), key
+        assert (gradients[key] == hip_vjp("sasaw", on_device, wanted=[key])[key]).all(), key
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_senders_outside_the_tensor_count_as_zero(oracle, device, dtype):
+    case = support.sasaw_case(7, dtype, E=300, nA=9, L=20, n_nodes=12, n2=9, n3=9, N=120)
+    lost = np.random.default_rng(1).integers(0, 300, 40)
+    with_zero = dict(case, B=case["B"].copy())
+    with_zero["B"][lost] = 0
+    case["indices_W_1"] = case["indices_W_1"].copy()
+    case["indices_W_1"][lost] = np.where(lost % 2 == 0, -1, 12)
+    on_device = to_device(case, device)
+    support.assert_close(
+        hip_forward("sasaw", on_device).cpu().numpy(), cpu_forward(oracle, "sasaw", with_zero), dtype, "output"
+    )
+    gradients = hip_vjp("sasaw", on_device)
+    expected = cpu_vjp(oracle, "sasaw", with_zero)
+    support.assert_close(gradients["W"].cpu().numpy(), expected["W"], dtype, "grad_W")
+    support.assert_close(gradients["A"].cpu().numpy(), expected["A"], dtype, "grad_A")
+    assert (gradients["B"][lost] == 0).all()
+
+
+def test_more_senders_than_the_counting_sort_counts_at_a_time(oracle, device):
+    small = support.sasaw_case(9, np.float64, E=2000, nA=4, L=1, n_nodes=30, n2=4, n3=4, N=12)
+    places = np.sort(np.random.default_rng(2).choice(2200000, 30, replace=False)).astype(np.int32)
+    case = dict(small)
+    for key in ("W", "grad_output"):
+        case[key] = np.zeros((2200000, 4, 1))
+        case[key][places] = small[key]
+    for key in ("indices_W_1", "indices_output_1"):
+        case[key] = places[small[key]]
+    expected = cpu_vjp(oracle, "sasaw", small)
+    actual = {key: value.cpu().numpy() for key, value in hip_vjp("sasaw", to_device(case, device)).items()}
+    support.assert_close(actual["W"][places], expected["W"], np.float64, "grad_W")
+    assert np.count_nonzero(actual["W"]) == np.count_nonzero(expected["W"])
+    support.assert_close(actual["A"], expected["A"], np.float64, "grad_A")
