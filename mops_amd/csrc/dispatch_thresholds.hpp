@@ -32,6 +32,22 @@ constexpr int64_t HPE_TILES_WORK = 10 * 1000 * 1000;
 constexpr int64_t SAP_FORWARD_WALK_TILES_PER_WAVE = 1;
 constexpr int64_t SAP_VJP_WALK_TILES_PER_WAVE = 2;
 
+/// Rows from which a lane per row (sap_rows.hip) takes the vjp, and the forward pass of two pairs; half
+/// as many in double where the table fits the scalar cache. vjp, matrix cores / a lane per row, us: nA, nB,
+/// nO = 13, 7, 20, 120 000 rows 28.9 / 23.6 (f32), 53.1 / 33.4 (f64), 60 000 rows 16.4 / 19.2, 28.1 / 24.1;
+/// 5, 4, 12, 120 000 rows 15.6 / 12.1, 22.9 / 15.0; a million rows of 13, 7, 20: 148 / 90, 280 / 129.
+constexpr int32_t SAP_ROWS_VJP = 100000;
+/// The same for the forward pass, which the matrix cores pad less: 13, 7, 20 in double, 250 000 rows 39.8 /
+/// 42.1, 500 000 68.7 / 62.5, a million 130 / 110; 16, 16, 8: 250 000 48.7 / 41.1, 500 000 86 / 61.
+constexpr int32_t SAP_ROWS_FORWARD = 300000;
+/// ... and for shapes that the matrix cores do not take (more than 64 columns, a table larger than the LDS).
+/// 4, 9, 90 with 1500 entries, forward, 30 000 rows 26.9 / 30.3, 60 000 42.2 / 31.2, 250 000 152 / 60 (f32),
+/// vjp 52.9 / 30.2, 81 / 31, 298 / 67; 10, 13, 30 in double, vjp, 30 000 rows 61 / 44, 500 000 823 / 290.
+constexpr int32_t SAP_ROWS_BEYOND_MATRIX_CORES = 50000;
+constexpr int32_t SAP_ROWS_BEYOND_MATRIX_CORES_VJP = 25000;
+/// Bytes of a table that stays in the scalar cache.
+constexpr int64_t SAP_ROWS_CACHED_TABLE = 16 * 1024;
+
 // ---- OPSA / OPSAW (opsa.hip) -----------------------------------------------
 /// Forward pass: segments are cut every so many positions of the sorted index,
 /// and the pieces added by a second launch, when the average segment is twice

@@ -46,6 +46,7 @@
 #include "elementwise.hpp"
 #include "runtime.hpp"
 #include "sap_mfma.hpp"
+#include "sap_rows.hpp"
 
 namespace mops::amd {
 namespace sap { // a name of its own for this file's kernels: profilers print it
@@ -685,6 +686,12 @@ void sparse_accumulation_of_products(MOPS_SAP_PARAMS(MOPS_CXX_FIRST, MOPS_CXX_NE
     }
     hipStream_t stream = current_stream();
     const sap_mfma::Shape dense_shape{n_rows, nA, nB, nO, n_products};
+    if (sap_rows::chosen_forward(dense_shape, sizeof(scalar_t))) {
+        const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
+        sap_rows::forward<scalar_t>(output.data, A.data, B.data, nullptr, nullptr, dense_table, dense_shape, stream);
+        finish_call(operation);
+        return;
+    }
     if (sap_mfma::supports_forward(dense_shape, sizeof(scalar_t))) {
         const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
         sap_mfma::forward<scalar_t>(output.data, A.data, B.data, dense_table, dense_shape, stream);
@@ -765,6 +772,14 @@ void sparse_accumulation_of_products_vjp(MOPS_SAP_VJP_PARAMS(MOPS_CXX_FIRST, MOP
     }
     hipStream_t stream = current_stream();
     const sap_mfma::Shape dense_shape{n_rows, nA, nB, nO, n_products};
+    if (sap_rows::chosen_vjp(dense_shape, sizeof(scalar_t))) {
+        const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
+        sap_rows::vjp<scalar_t>(
+            grad_A.data, grad_B.data, grad_output.data, A.data, B.data, dense_table, dense_shape, stream
+        );
+        finish_call(operation);
+        return;
+    }
     if (sap_mfma::supports_vjp(dense_shape, sizeof(scalar_t))) {
         const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
         sap_mfma::vjp<scalar_t>(
@@ -849,9 +864,13 @@ void sparse_accumulation_of_products_vjp_vjp(MOPS_SAP_VJP_VJP_PARAMS(MOPS_CXX_FI
             narrow_i32(A.shape[0], "A.shape[0]"), narrow_i32(A.shape[1], "A.shape[1]"),
             narrow_i32(B.shape[1], "B.shape[1]"), narrow_i32(grad_output.shape[1], "grad_output.shape[1]"),
             narrow_i32(C.shape[0], "C.shape[0]")};
-        if (have_A && have_B && sap_mfma::supports_forward_of_two_pairs(dense_shape, sizeof(scalar_t))) {
+        const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
+        if (have_A && have_B && output_count > 0 && sap_rows::chosen_forward_of_two_pairs(dense_shape, sizeof(scalar_t))) {
+            sap_rows::forward<scalar_t>(
+                grad_grad_output.data, grad_grad_A.data, B.data, A.data, grad_grad_B.data, dense_table, dense_shape, stream
+            );
+        } else if (have_A && have_B && sap_mfma::supports_forward_of_two_pairs(dense_shape, sizeof(scalar_t))) {
             // both terms in the sums of one launch
-            const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
             sap_mfma::forward_of_two_pairs<scalar_t>(
                 grad_grad_output.data, grad_grad_A.data, B.data, A.data, grad_grad_B.data, dense_table,
                 dense_shape, stream
