@@ -1,6 +1,7 @@
 #include "sender_buckets.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 #include "runtime.hpp"
 
@@ -14,15 +15,19 @@ namespace {
 // atomics on global memory (a returning atomic per edge, 1 000 000 of them over
 // eight L2 caches, took 90 us): a workgroup counts its share of the edges, and
 // the next launch finds out from all counts where its share of every bucket
-// begins. 1 000 000 edges over 33 000 senders: 49 us for the three launches (5, 17
-// and 27; what they wait for is one dependent load after the other), 300 000 over
-// 10 000: 27.
+// begins. Where edge and sender's place in its bucket fit into one word of 32 bits,
+// the second level looks at nothing else, and both levels keep a lane's first items
+// in registers from counting to placing. 1 000 000 edges over 33 000 senders: 35 us
+// for the three launches (5, 15 and 15; 46 with two looks at everything), 400 000
+// over 10 000: 27; what they wait for is one dependent load after the other.
 constexpr int SORT_THREADS = 1024;
 constexpr int32_t MOST_BUCKETS = 512;
 constexpr int32_t MOST_SHARES = 256;         // workgroups of the first level
 constexpr int32_t SENDERS_AT_A_TIME = 4096;  // of the second level: counters in LDS
 
-constexpr int BATCH = 4;                     // positions a lane asks for at once
+constexpr int HELD = 4;                      // positions a lane keeps from counting to placing
+constexpr int32_t STAGED = 5120;             // edges of a bucket that are put in order in LDS
+constexpr int BATCH = 4;                     // positions beyond those that it asks for at once
 
 /// What lies at a position: an edge, its sender, and what it is sorted by (negative: it is not).
 struct Item {
@@ -54,15 +59,32 @@ struct Share {
     }
 };
 
+/// The first HELD items of a lane: those of most shares all told, so that they are read once.
+template <int HELD, typename ItemAt>
+__device__ __forceinline__ void hold_items(Item (&held)[HELD], const Share& share, int lane, ItemAt&& item_at) {
+#pragma unroll
+    for (int u = 0; u < HELD; u++) {
+        held[u] = item_at(max(min(share.begin + u * WAVE + lane, share.end - 1), 0));
+    }
+}
+
 /// counters[wavefront][key] := how many of the wavefront's items have the key.
-template <typename ItemAt>
-__device__ __forceinline__ void
-count_keys(int32_t* counters, int32_t keys, const Share& share, int wave, int waves, int lane, ItemAt&& item_at) {
+template <int HELD, typename ItemAt>
+__device__ __forceinline__ void count_keys(
+    const Item (&held)[HELD], int32_t* counters, int32_t keys, const Share& share, int wave, int waves, int lane,
+    ItemAt&& item_at
+) {
     for (int32_t i = threadIdx.x; i < waves * keys; i += blockDim.x) {
         counters[i] = 0;
     }
     __syncthreads();
-    for (int32_t at = share.begin + lane; at - lane < share.end; at += BATCH * WAVE) {
+#pragma unroll
+    for (int u = 0; u < HELD; u++) {
+        if (share.begin + u * WAVE + lane < share.end && held[u].key >= 0) {
+            atomicAdd(&counters[wave * keys + held[u].key], 1);
+        }
+    }
+    for (int32_t at = share.begin + HELD * WAVE + lane; at - lane < share.end; at += BATCH * WAVE) {
         int32_t key[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; u++) {
@@ -80,12 +102,35 @@ count_keys(int32_t* counters, int32_t keys, const Share& share, int wave, int wa
 
 /// put(place, item) for every item that has a key, items of one key in ascending places:
 /// counters[wavefront][key] is the place of the wavefront's first one.
-template <typename ItemAt, typename Put>
+template <int HELD, typename ItemAt, typename Put>
 __device__ __forceinline__ void place_keys(
-    int32_t* counters, int32_t keys, int bits, const Share& share, int wave, int lane, ItemAt&& item_at, Put&& put
+    const Item (&held)[HELD], int32_t* counters, int32_t keys, int bits, const Share& share, int wave, int lane,
+    ItemAt&& item_at, Put&& put
 ) {
     int32_t* mine = counters + static_cast<size_t>(wave) * keys;
-    for (int32_t at = share.begin + lane; at - lane < share.end; at += BATCH * WAVE) {
+    auto place_one = [&](const Item& item, int32_t at) {
+        const bool valid = at < share.end && item.key >= 0;
+        const Ranked ranked = rank_in_wave(item.key, valid, bits, lane);
+        const int32_t place = valid ? mine[item.key] + static_cast<int32_t>(ranked.before) : 0;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && ranked.before == 0) {
+            mine[item.key] += __popcll(ranked.same);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (valid) {
+            put(place, item);
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < HELD; u++) {
+        if (share.begin + u * WAVE < share.end) { // (uniform)
+            place_one(held[u], share.begin + u * WAVE + lane);
+        }
+    }
+    for (int32_t at = share.begin + HELD * WAVE + lane; at - lane < share.end; at += BATCH * WAVE) {
         Item item[BATCH];
 #pragma unroll
         for (int u = 0; u < BATCH; u++) {
@@ -93,38 +138,26 @@ __device__ __forceinline__ void place_keys(
         }
 #pragma unroll
         for (int u = 0; u < BATCH; u++) {
-            const bool valid = at + u * WAVE < share.end && item[u].key >= 0;
-            const Ranked ranked = rank_in_wave(item[u].key, valid, bits, lane);
-            const int32_t place = valid ? mine[item[u].key] + static_cast<int32_t>(ranked.before) : 0;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (valid && ranked.before == 0) {
-                mine[item[u].key] += __popcll(ranked.same);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (valid) {
-                put(place, item[u]);
-            }
+            place_one(item[u], at + u * WAVE);
         }
     }
 }
 
 /// Turns counters[wavefront][key] into the place of the wavefront's first of each key:
-/// start_of(key, number of the workgroup's keys) and what the wavefronts before have. All threads.
-template <typename StartOf>
-__device__ __forceinline__ void starts_of_waves(int32_t* counters, int32_t keys, int waves, StartOf&& start_of) {
+/// start_of(key) and what the wavefronts before have. All threads.
+template <int WAVES, typename StartOf>
+__device__ __forceinline__ void starts_of_waves(int32_t* counters, int32_t keys, StartOf&& start_of) {
     for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
-        int32_t total = 0;
-        for (int w = 0; w < waves; w++) {
-            total += counters[w * keys + key];
+        int32_t here[WAVES];
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
+            here[w] = counters[w * keys + key];
         }
-        int32_t place = start_of(key, total);
-        for (int w = 0; w < waves; w++) {
-            const int32_t here = counters[w * keys + key];
+        int32_t place = start_of(key);
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
             counters[w * keys + key] = place;
-            place += here;
+            place += here[w];
         }
     }
     __syncthreads();
@@ -132,8 +165,9 @@ __device__ __forceinline__ void starts_of_waves(int32_t* counters, int32_t keys,
 
 /// values[0 .. n) := `first` + the sum of those before; returns `first` + the sum of all. All
 /// threads; `of_wave`: an integer per wavefront.
+template <int WAVES>
 __device__ __forceinline__ int32_t scan_in_place(int32_t* values, int32_t n, int32_t first, int32_t* of_wave) {
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE, waves = blockDim.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int32_t carry = first;
     for (int32_t base = 0; base < n; base += blockDim.x) {
         const int32_t i = base + threadIdx.x;
@@ -149,7 +183,8 @@ __device__ __forceinline__ int32_t scan_in_place(int32_t* values, int32_t n, int
         }
         __syncthreads();
         int32_t ahead = carry;
-        for (int w = 0; w < waves; w++) {
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) {
             ahead += w < wave ? of_wave[w] : 0;
             carry += of_wave[w];
         }
@@ -199,7 +234,7 @@ __global__ __launch_bounds__(SORT_THREADS) void count_buckets_kernel(
 __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
     int32_t* __restrict__ sender_of_place, int32_t* __restrict__ edge_of_place, int32_t* __restrict__ offsets,
     const int32_t* __restrict__ counts, const int32_t* __restrict__ senders, int32_t n_edges, int32_t n_nodes, int shift,
-    int32_t buckets, int32_t pitch, int bits, int32_t share
+    int32_t buckets, int32_t pitch, int bits, int32_t share, int packed_above
 ) {
     constexpr int WAVES = SORT_THREADS / WAVE;
     extern __shared__ int32_t shared[];
@@ -218,7 +253,9 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
         before[b] = 0;
         total[b] = 0;
     }
-    count_keys(counters, pitch, mine, wave, WAVES, lane, item_at);
+    Item held[HELD];
+    hold_items(held, mine, lane, item_at);
+    count_keys(held, counters, pitch, mine, wave, WAVES, lane, item_at);
     // what the workgroups before have of every bucket, and all of them: several threads per bucket
     // (of a single workgroup, the counts it has just made)
     const int32_t* all_counts = gridDim.x > 1 ? counts : counters;
@@ -253,7 +290,7 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
         atomicAdd(&to[3], all.w);
     }
     __syncthreads();
-    const int32_t listed = scan_in_place(total, buckets, 0, of_wave);
+    const int32_t listed = scan_in_place<WAVES>(total, buckets, 0, of_wave);
     if (blockIdx.x == 0) {
         for (int32_t bucket = threadIdx.x; bucket < buckets; bucket += SORT_THREADS) {
             offsets[bucket] = total[bucket];
@@ -262,9 +299,11 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
             offsets[buckets] = listed;
         }
     }
-    starts_of_waves(counters, pitch, WAVES, [&](int32_t bucket, int32_t) { return total[bucket] + before[bucket]; });
-    place_keys(counters, pitch, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
-        edge_of_place[place] = item.edge;
+    starts_of_waves<WAVES>(counters, pitch, [&](int32_t bucket) { return total[bucket] + before[bucket]; });
+    // (two levels: the sender's place in its bucket beside the edge, where both go into one word)
+    const int32_t of_bucket = (1 << shift) - 1;
+    place_keys(held, counters, pitch, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+        edge_of_place[place] = packed_above < 32 ? item.edge | (item.sender & of_bucket) << packed_above : item.edge;
         if (sender_of_place != nullptr) {
             sender_of_place[place] = item.sender;
         }
@@ -278,52 +317,77 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
     }
 }
 
-/// A workgroup per bucket puts its edges in the order of their senders: `senders` of the edges, or
-/// of the places (`of_place`).
-/// LDS: counters[wavefronts][at_a_time], start[at_a_time], of_wave[wavefronts].
-__global__ __launch_bounds__(SORT_THREADS) void sort_buckets_kernel(
+/// A workgroup per bucket puts its edges in the order of their senders. The sender of a place's edge
+/// is in the edge's word from bit `packed_above` on, or in `senders`. A bucket of up to `staged_room` edges
+/// is put in order in LDS and written in whole lines (1 000 000 edges, 33 000 senders: 26.5 us with
+/// two looks at `senders` by edge and stores of 64 words in 64 lines, 15.0 like this).
+/// LDS: counters[wavefronts][at_a_time], start[at_a_time], of_wave[wavefronts], staged[staged_room].
+template <int WAVES>
+__global__ __launch_bounds__(WAVES* WAVE) void sort_buckets_kernel(
     int32_t* __restrict__ sender_of_place, int32_t* __restrict__ edge_of_place, int32_t* __restrict__ offsets,
     const int32_t* __restrict__ bucket_offsets, const int32_t* __restrict__ senders, const int32_t* __restrict__ edges,
-    bool of_place, int32_t n_edges, int32_t n_nodes, int shift, int32_t at_a_time, int bits
+    int packed_above, int32_t n_edges, int32_t n_nodes, int shift, int32_t at_a_time, int bits, int32_t staged_room
 ) {
     extern __shared__ int32_t shared[];
-    const int waves = blockDim.x / WAVE, lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int32_t* counters = shared;
-    int32_t* start = counters + waves * at_a_time;
+    int32_t* start = counters + WAVES * at_a_time;
     int32_t* of_wave = start + at_a_time;
+    int32_t* staged = of_wave + WAVES;
     const int32_t begin = bucket_offsets[blockIdx.x], end = bucket_offsets[blockIdx.x + 1];
-    const Share mine(begin, end, wave, waves);
+    const Share mine(begin, end, wave, WAVES);
     const int32_t node0 = static_cast<int32_t>(blockIdx.x) << shift;
     const int32_t nodes = min(1 << shift, n_nodes - node0);
+    const bool packed = packed_above < 32;
+    const bool in_lds = packed && end - begin <= staged_room && nodes <= at_a_time;
+    const uint32_t edge_mask = packed ? (1u << packed_above) - 1 : ~0u;
     int32_t place0 = begin;
     for (int32_t base = 0; base < nodes; base += at_a_time) {
         const int32_t keys = min(at_a_time, nodes - base);
         auto item_at = [&](int32_t place) {
-            const int32_t edge = edges[place], sender = senders[of_place ? place : edge];
-            const int32_t key = sender - node0 - base;
-            return Item{in_bounds(key, keys) ? key : -1, edge, sender};
+            const uint32_t word = static_cast<uint32_t>(edges[place]);
+            const int32_t of_bucket =
+                packed ? static_cast<int32_t>(word >> packed_above) : senders[place] - node0;
+            const int32_t key = of_bucket - base;
+            return Item{in_bounds(key, keys) ? key : -1, static_cast<int32_t>(word & edge_mask), node0 + of_bucket};
         };
-        count_keys(counters, keys, mine, wave, waves, lane, item_at);
+        Item held[HELD];
+        hold_items(held, mine, lane, item_at);
+        count_keys(held, counters, keys, mine, wave, WAVES, lane, item_at);
         for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
             int32_t sum = 0;
-            for (int w = 0; w < waves; w++) {
+#pragma unroll
+            for (int w = 0; w < WAVES; w++) {
                 sum += counters[w * keys + key];
             }
             start[key] = sum;
         }
         __syncthreads();
-        place0 = scan_in_place(start, keys, place0, of_wave);
+        place0 = scan_in_place<WAVES>(start, keys, place0, of_wave);
         for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
             offsets[node0 + base + key] = start[key];
         }
-        starts_of_waves(counters, keys, waves, [&](int32_t key, int32_t) { return start[key]; });
-        place_keys(counters, keys, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
-            edge_of_place[place] = item.edge;
-            if (sender_of_place != nullptr) {
-                sender_of_place[place] = item.sender;
+        starts_of_waves<WAVES>(counters, keys, [&](int32_t key) { return start[key]; });
+        place_keys(held, counters, keys, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+            if (in_lds) {
+                staged[place - begin] = item.edge | item.key << packed_above;
+            } else {
+                edge_of_place[place] = item.edge;
+                if (sender_of_place != nullptr) {
+                    sender_of_place[place] = item.sender;
+                }
             }
         });
         __syncthreads();
+    }
+    if (in_lds) {
+        for (int32_t place = begin + static_cast<int32_t>(threadIdx.x); place < end; place += WAVES * WAVE) {
+            const uint32_t word = static_cast<uint32_t>(staged[place - begin]);
+            edge_of_place[place] = static_cast<int32_t>(word & edge_mask);
+            if (sender_of_place != nullptr) {
+                sender_of_place[place] = node0 + static_cast<int32_t>(word >> packed_above);
+            }
+        }
     }
     if (blockIdx.x == gridDim.x - 1) {
         if (threadIdx.x == 0) {
@@ -430,7 +494,15 @@ struct SortPlan {
     int32_t buckets, pitch;
     int32_t share;   // edges per workgroup of the first level
     int32_t shares;
+    int packed_above; // two levels: bits below the sender's place in its bucket, 32: not in one word
 };
+int bits_for(int32_t values) {
+    int bits = 0;
+    while ((int64_t(1) << bits) < values) {
+        bits++;
+    }
+    return bits;
+}
 SortPlan sort_plan(int32_t n_nodes, int32_t n_edges) {
     SortPlan plan;
     plan.shift = 0;
@@ -442,24 +514,19 @@ SortPlan sort_plan(int32_t n_nodes, int32_t n_edges) {
     const size_t each = ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(SORT_THREADS) * MOST_SHARES);
     plan.share = static_cast<int32_t>(each) * SORT_THREADS;
     plan.shares = static_cast<int32_t>(ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(plan.share)));
+    const int edge_bits = bits_for(n_edges);
+    plan.packed_above = plan.shift > 0 && edge_bits + plan.shift <= 32 ? edge_bits : 32;
     return plan;
 }
-int bits_for(int32_t values) {
-    int bits = 0;
-    while ((int64_t(1) << bits) < values) {
-        bits++;
-    }
-    return bits;
-}
-
 } // namespace
 
 size_t edges_by_sender_bytes(int32_t n_nodes, int32_t n_edges, bool with_senders) {
     if (n_nodes < 1) {
         return 0;
     }
+    const bool senders_in_buckets = n_edges > 0 && sort_plan(n_nodes, n_edges).packed_above == 32;
     return align256((static_cast<size_t>(n_nodes) + 1) * 4) + align256((MOST_BUCKETS + 1) * 4) +
-           (with_senders ? 4 : 2) * align256(static_cast<size_t>(n_edges) * 4);
+           (2 + with_senders + senders_in_buckets) * align256(static_cast<size_t>(n_edges) * 4);
 }
 
 EdgesBySender order_edges_by_sender(
@@ -479,13 +546,13 @@ EdgesBySender order_edges_by_sender(
     int32_t* edge = take(static_cast<size_t>(n_edges));
     int32_t* edge_in_buckets = take(static_cast<size_t>(n_edges));
     int32_t* sender = with_senders ? take(static_cast<size_t>(n_edges)) : nullptr;
-    int32_t* sender_in_buckets = with_senders ? take(static_cast<size_t>(n_edges)) : nullptr;
     if (n_edges < 1) {
         clear_counters(offsets, static_cast<size_t>(n_nodes) + 1, stream);
         return EdgesBySender{sender, edge, offsets};
     }
     const SortPlan plan = sort_plan(n_nodes, n_edges);
     const bool two_levels = plan.shift > 0;
+    int32_t* sender_in_buckets = plan.packed_above == 32 ? take(static_cast<size_t>(n_edges)) : nullptr;
     // The counts of several shares lie where nothing is written by the launch that reads them. They
     // fit: a share is 1024 edges or more, and there are 512 buckets at most.
     int32_t* counts = two_levels ? edge : edge_in_buckets;
@@ -499,17 +566,30 @@ EdgesBySender order_edges_by_sender(
     fill_buckets_kernel<<<plan.shares, SORT_THREADS, lds, stream>>>(
         two_levels ? sender_in_buckets : sender, two_levels ? edge_in_buckets : edge,
         two_levels ? bucket_offsets : offsets, counts, senders, n_edges, n_nodes, plan.shift, plan.buckets,
-        plan.pitch, bits_for(plan.buckets), plan.share
+        plan.pitch, bits_for(plan.buckets), plan.share, plan.packed_above
     );
     if (two_levels) {
         const int32_t at_a_time = std::min(int32_t(1) << plan.shift, SENDERS_AT_A_TIME);
         // (the counters of all wavefronts within 64 KB)
-        const int waves = at_a_time <= 512 ? 16 : at_a_time <= 1024 ? 8 : at_a_time <= 2048 ? 4 : 2;
-        const size_t sort_lds = (static_cast<size_t>(waves + 1) * at_a_time + waves) * sizeof(int32_t);
-        sort_buckets_kernel<<<plan.buckets, waves * WAVE, sort_lds, stream>>>(
-            sender, edge, offsets, bucket_offsets, with_senders ? sender_in_buckets : senders, edge_in_buckets,
-            with_senders, n_edges, n_nodes, plan.shift, at_a_time, bits_for(at_a_time)
-        );
+        auto sort = [&](auto with_waves) {
+            constexpr int WAVES = decltype(with_waves)::value;
+            const int32_t room = WAVES >= 4 ? STAGED : 0;
+            const size_t sort_lds = (static_cast<size_t>(WAVES + 1) * at_a_time + WAVES + room) * sizeof(int32_t);
+            sort_buckets_kernel<WAVES><<<plan.buckets, WAVES * WAVE, sort_lds, stream>>>(
+                sender, edge, offsets, bucket_offsets, sender_in_buckets, edge_in_buckets,
+                plan.packed_above, n_edges, n_nodes, plan.shift, at_a_time, bits_for(at_a_time), room
+            );
+        };
+        // (within 64 KB: the counters of all wavefronts, and the edges of a bucket where there is room)
+        if (at_a_time <= 512) {
+            sort(std::integral_constant<int, 16>{});
+        } else if (at_a_time <= 1024) {
+            sort(std::integral_constant<int, 8>{});
+        } else if (at_a_time <= 2048) {
+            sort(std::integral_constant<int, 4>{});
+        } else {
+            sort(std::integral_constant<int, 2>{});
+        }
     }
     MOPS_HIP_CHECK(hipGetLastError());
     return EdgesBySender{sender, edge, offsets};
