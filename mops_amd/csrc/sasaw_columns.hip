@@ -337,10 +337,12 @@ template <typename T, int N, int COLUMNS> struct Columns {
     ///
     /// What makes the operands of AHEAD edges be on their way: no branch between the asking and the
     /// waiting (the compiler counts the loads of both ways and takes the smaller number), the order of
-    /// the asking kept, stores without a branch around them (they count as well), and the row of A
-    /// asked for only when the one before has arrived (scalar loads come back in any order, so that a
+    /// the asking kept, stores without a branch around them (they count as well), and rows of A
+    /// asked for only when the ones before have arrived (scalar loads come back in any order, so that a
     /// wait is for all of them).
-    template <typename EdgeOf, typename Ask, typename Each>
+    ///
+    /// A_BATCH: the rows of A asked for at once, while as many are worked on.
+    template <int A_BATCH, typename EdgeOf, typename Ask, typename Each>
     __device__ __forceinline__ void
     over(int32_t sources, int32_t n, EdgeOf&& edge_of, Ask&& ask_more, Each&& each) const {
         Operands ring[AHEAD];
@@ -350,30 +352,47 @@ template <typename T, int N, int COLUMNS> struct Columns {
             ask_more(to, k);
             __builtin_amdgcn_sched_barrier(0);
         };
-        T a[2][N];
-        load_row_of_A(a[0], edge_of(0));
+        T a[2][A_BATCH][N];
+        auto ask_rows = [&](T (&to)[A_BATCH][N], int32_t k) {
+#pragma unroll
+            for (int r = 0; r < A_BATCH; r++) {
+                load_row_of_A(to[r], edge_of(min(k + r, n - 1)));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        ask_rows(a[0], 0);
 #pragma unroll
         for (int d = 0; d < AHEAD; d++) {
             ask(ring[d], d);
         }
         auto step = [&](int d, int32_t k) {
-            arrived(a[d & 1]);
-            load_row_of_A(a[~d & 1], edge_of(min(k + 1, n - 1)));
-            __builtin_amdgcn_sched_barrier(0);
-            each(a[d & 1], ring[d], k);
-        };
-        int32_t first = 0;
-        for (; first + AHEAD <= n; first += AHEAD) {
+            T(&rows)[A_BATCH][N] = a[d / A_BATCH & 1];
+            if (d % A_BATCH == 0) {
 #pragma unroll
-            for (int d = 0; d < AHEAD; d++) {
+                for (int r = 0; r < A_BATCH; r++) {
+                    arrived(rows[r]);
+                }
+                ask_rows(a[~(d / A_BATCH) & 1], k + A_BATCH);
+            }
+            each(rows[d % A_BATCH], ring[d % AHEAD], k);
+        };
+        constexpr int STEPS = AHEAD > 2 * A_BATCH ? AHEAD : 2 * A_BATCH;
+        int32_t first = 0;
+        for (; first + STEPS <= n; first += STEPS) {
+#pragma unroll
+            for (int d = 0; d < STEPS; d++) {
                 step(d, first + d);
-                ask(ring[d], first + d + AHEAD);
+                ask(ring[d % AHEAD], first + d + AHEAD);
             }
         }
 #pragma unroll
-        for (int d = 0; d < AHEAD - 1; d++) {
-            if (first + d < n) { // (uniform)
-                step(d, first + d);
+        for (int d = 0; d < STEPS - 1; d++) {
+            if (first + d >= n) { // (uniform; the two ways do not meet before the end)
+                return;
+            }
+            step(d, first + d);
+            if (d + AHEAD < STEPS - 1) {
+                ask(ring[d % AHEAD], first + d + AHEAD);
             }
         }
     }
@@ -423,6 +442,12 @@ template <typename T> struct ContractWindow<T, ORDERED> {
     __device__ __forceinline__ int32_t edge(int32_t, int32_t k) const { return __builtin_amdgcn_readlane(listed, k); }
 };
 
+/// Rows of A in scalar registers at once, where they fit without others being moved out of the way:
+/// 1 000 000 edges, 32 columns, 4 components, f32 / f64, 94.9 -> 92.7 / 198 -> 188 us, sums over
+/// senders 180 -> 170 / 273 -> 264; 9 in double 386 -> 371; 9 in float is slower by it.
+template <typename T, int N> constexpr int contract_rows_of_A() {
+    return N == 4 ? 4 : N == 9 && sizeof(T) == 8 ? 2 : 1;
+}
 /// Wavefronts per SIMD.
 template <typename T, int N, int COLUMNS> constexpr int contract_waves() {
     constexpr int REGISTERS = (N * Sums<N, COLUMNS>::M2 + 34) * static_cast<int>(sizeof(T)) / 4;
@@ -440,6 +465,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
     using M = Mfma<T>;
     using S = Sums<N, COLUMNS>;
     constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::STEPS * 4 * PITCH;
+    constexpr int ROWS_OF_A = contract_rows_of_A<T, N>();
     const Walk<T>& p = args.walk;
     extern __shared__ __align__(16) char lds[];
     T* table = reinterpret_cast<T*>(lds);
@@ -546,7 +572,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
                 n = window.edges_of(args, node, at);
                 const ContractWindow<T, LISTS> next(args, at + n, lane);
                 if (n > 0) {
-                    columns_of.over(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, add);
+                    columns_of.template over<ROWS_OF_A>(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, add);
                 }
                 at += n;
                 window = next;
@@ -558,7 +584,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
             clear();
             auto hand_on = [&](int32_t edge, int32_t n) {
                 const int32_t sources = p.gather[edge];
-                columns_of.over(
+                columns_of.template over<ROWS_OF_A>(
                     sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, add
                 );
             };
@@ -795,7 +821,7 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
                         have = true;
                     }
                     const int32_t first = at + from;
-                    columns_of.over(
+                    columns_of.template over<1>(
                         __shfl(window.source, min(from + lane, to - 1)), to - from, [&](int32_t k) { return first + k; },
                         [&](auto& operands, int32_t k) {
                             operands.more = from_A.load(a_at, static_cast<uint32_t>(first + k) * A_ROW_BYTES);
