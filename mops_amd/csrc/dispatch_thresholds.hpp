@@ -74,8 +74,8 @@ constexpr size_t SENDER_SCAN_LIMIT = 100u * 1000 * 1000;
 /// reading the whole index). OPSAW, 60 000 edges over 2000 senders, L = 32,
 /// f32: 33 -> 22 us for the whole vjp.
 constexpr int32_t SLOT_MEAN_EDGES = 48;
-/// Edges per sender on average up to which SASAW lists by arrival (128 places
-/// per sender): 1000 nodes x 60 edges, whole vjp 87.6 -> 76.6 us (f32), 143.8
+/// Edges per sender on average up to which lists are made by arrival (128 places
+/// per sender). SASAW, 1000 nodes x 60 edges, whole vjp 87.6 -> 76.6 us (f32), 143.8
 /// -> 115.3 (f64) against the kernels of sasaw_mfma.hip; at 100 per sender the
 /// lists overflow (375 against 101 us).
 constexpr int32_t ARRIVAL_MEAN_EDGES = 64;
@@ -86,6 +86,9 @@ constexpr int32_t ARRIVAL_MEAN_EDGES = 64;
 /// / 255, 20 000: 682 / 820. OPSAW f32 vjp: 2000 senders 27.6 / 22.6, 3000:
 /// 33.4 / 29.6, 4000: 37.6 / 39.3, 6000: 48 / 75, 20 000: 156 / 212.
 constexpr int32_t ARRIVAL_NODES = 4000;
+/// Edges up to which OPSAW lists by arrival; beyond, the counting sort (see
+/// opsa.hip).
+constexpr int32_t ARRIVAL_EDGES = 500000;
 /// Edges x nodes from which a counting sort of the edges by sender replaces the
 /// slots where the kernels of sasaw_columns.hip use them (four lookers at the
 /// index per 16 nodes against three short launches). grad_W alone, f32, 9

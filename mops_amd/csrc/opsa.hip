@@ -30,8 +30,8 @@
 // order is fixed (ascending edge number in steps of four), so results are
 // bit-reproducible.
 #include <algorithm>
-#include <optional>
 #include <cstdlib>
+#include <optional>
 #include <memory>
 
 #include "mops/opsa.hpp"
@@ -46,6 +46,7 @@
 #include "edge_order.hpp"
 #include "elementwise.hpp"
 #include "runtime.hpp"
+#include "opsa_edges.hpp"
 #include "segment_walk.hpp"
 #include "sender_buckets.hpp"
 #include "sender_gather.hpp"
@@ -1512,64 +1513,68 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
 }
 
 // The same sum over lists that are already there (sender_buckets.hpp: the edges in
-// the order of their senders, built beside the per-edge kernel on a side
-// stream): one wavefront per sender, sixteen rows in flight.
-
-template <typename T>
+// the order of their senders): one wavefront per sender, its lanes (part, column),
+// so that a load brings PARTS rows of up to 64 / PARTS columns (1: COLUMNS values
+// of a row per lane, any number of rows of columns). What bounds it is the gather
+// of the rows, BATCH loads in flight: 1 000 000 rows of 32 floats, 53.9 us with a
+// row per load, 26.4 us with two.
+template <typename T, int PARTS, int COLUMNS>
 __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_listed_rows_kernel(
     T* __restrict__ grad_W, const T* __restrict__ edge_W, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ edge_of_position, int32_t n_nodes, int32_t L
 ) {
-    const int lane = threadIdx.x & (WAVE - 1);
+    constexpr int WIDTH = WAVE / PARTS;
+    constexpr int BATCH = 16 / (COLUMNS * static_cast<int>(sizeof(T) / 4)); // (of PARTS rows)
+    const int lane = threadIdx.x & (WAVE - 1), part = lane / WIDTH;
     const int32_t node = __builtin_amdgcn_readfirstlane(blockIdx.x * LISTED_WAVES + (threadIdx.x >> 6));
     if (node >= n_nodes) {
         return;
     }
     const int32_t begin = offsets[node];
     const int32_t end = offsets[node + 1];
-    T sum[GATHER_COLUMNS];
-    uint32_t column[GATHER_COLUMNS];
+    T sum[COLUMNS];
+    int32_t column[COLUMNS];
 #pragma unroll
-    for (int c = 0; c < GATHER_COLUMNS; c++) {
+    for (int c = 0; c < COLUMNS; c++) {
         sum[c] = T(0);
-        column[c] = min(lane + c * WAVE, L - 1);
+        column[c] = min(lane % WIDTH + c * WIDTH, L - 1);
     }
-    constexpr int ROWS = sizeof(T) == 8 ? 8 : 16;
     for (int32_t p0 = begin; p0 < end; p0 += WAVE) {
         const int32_t n = min(WAVE, end - p0);
-        const int32_t my_edge = lane < n ? edge_of_position[p0 + lane] : 0;
+        const int32_t my_edge = edge_of_position[p0 + min(lane, n - 1)];
 #pragma unroll 1
-        for (int32_t k0 = 0; k0 < n; k0 += ROWS) {
-            T values[ROWS][GATHER_COLUMNS];
+        for (int32_t k0 = 0; k0 < n; k0 += BATCH * PARTS) {
+            T values[BATCH][COLUMNS];
 #pragma unroll
-            for (int k = 0; k < ROWS; k++) {
-                // beyond n: some row that exists, left out of the sum
-                const int32_t edge = __builtin_amdgcn_readlane(my_edge, min(k0 + k, WAVE - 1));
+            for (int k = 0; k < BATCH; k++) {
+                // beyond n: the last row once more, left out of the sum
+                const int32_t place = min(k0 + k * PARTS, WAVE - PARTS);
+                const int32_t edge = PARTS == 1 ? __builtin_amdgcn_readlane(my_edge, place)
+                                                : __builtin_amdgcn_ds_bpermute((place + part) << 2, my_edge);
                 const T* row = edge_W + static_cast<size_t>(edge) * L;
 #pragma unroll
-                for (int c = 0; c < GATHER_COLUMNS; c++) {
-                    if (c * WAVE < L) {
-                        values[k][c] = row[column[c]];
-                    }
+                for (int c = 0; c < COLUMNS; c++) {
+                    values[k][c] = row[column[c]];
                 }
             }
 #pragma unroll
-            for (int k = 0; k < ROWS; k++) {
-                if (k0 + k < n) {
+            for (int k = 0; k < BATCH; k++) {
+                const bool counts = k0 + k * PARTS + part < n;
 #pragma unroll
-                    for (int c = 0; c < GATHER_COLUMNS; c++) {
-                        if (c * WAVE < L) {
-                            sum[c] += values[k][c];
-                        }
-                    }
+                for (int c = 0; c < COLUMNS; c++) {
+                    sum[c] += counts ? values[k][c] : T(0);
                 }
             }
         }
     }
 #pragma unroll
-    for (int c = 0; c < GATHER_COLUMNS; c++) {
-        const int32_t l = lane + c * WAVE;
-        if (l < L) {
+    for (int c = 0; c < COLUMNS; c++) {
+#pragma unroll
+        for (int apart = WIDTH; apart < WAVE; apart *= 2) {
+            sum[c] += __shfl_xor(sum[c], apart);
+        }
+        const int32_t l = lane % WIDTH + c * WIDTH;
+        if (part == 0 && l < L) {
             grad_W[static_cast<size_t>(node) * L + l] = sum[c];
         }
     }
@@ -1807,6 +1812,36 @@ bool launch_forward_of_two_pairs(
     return true;
 }
 
+/// From how many edges on the per-edge gradients come from opsa_edges.hip (up to 32 columns of A and
+/// 64 of B) rather than from edge_rows_vjp_kernel. The latter has a wavefront for every 16 edges, which
+/// is done sooner on small graphs, but loads and stores the layout of its operands: full lines only
+/// where rows consist of aligned 16-byte pieces (`vectors`), and with more than 16 columns of A, or in
+/// double, few wavefronts per SIMD. Measured over 4 to 31 columns of A and 9 to 64 of B, 5000 to
+/// 1 000 000 edges, 30 per node; rows that are not vectors, this kernel / that one: OPSAW, f32, 400 000
+/// edges, 13 x 33 172 / 135 us, 31 x 37 344 / 165, f64 503 / 272 with 26 x 33; vectors, 1 000 000 edges,
+/// f32, 20 x 48 458 / 321, f64, 13 x 40 627 / 458, but 120 000 edges, f32, 13 x 32 42 / 45.
+template <typename T> int32_t tiles_from(int32_t K, int32_t L, bool weighted, bool vectors) {
+    constexpr int32_t NEVER = INT32_MAX;
+    const bool wide = K > 16;
+    if (L <= 16) {
+        return NEVER;
+    }
+    if constexpr (sizeof(T) == 4) {
+        if (vectors) {
+            return L > 32 ? (wide ? 350000 : 700000) : weighted ? 700000 : NEVER;
+        }
+        return L > 32 ? (wide ? 30000 : 100000) : wide ? 100000 : 400000;
+    } else {
+        if (vectors) {
+            return L > 32 && L <= 48 && !(weighted && wide && L < 40) ? 250000 : NEVER;
+        }
+        if (L > 48) {
+            return weighted ? (wide ? 60000 : 200000) : wide ? 600000 : 300000;
+        }
+        return L > 32 ? (weighted && !wide ? 100000 : 30000) : 300000;
+    }
+}
+
 template <typename T, bool WEIGHTED>
 void launch_vjp(
     Tensor<T, 2> grad_A,
@@ -1845,15 +1880,18 @@ void launch_vjp(
     const bool gather_in_kernel = narrow_rows && n_edges > 0 && index_reads <= SENDER_SCAN_LIMIT;
     const bool sparse = n_output > 0 && L > 0 &&
                         static_cast<size_t>(n_edges) <= static_cast<size_t>(n_output) * SLOT_MEAN_LIMIT;
-    // large sparse graphs: every edge takes the next of its sender's places in the per-edge
-    // kernel itself, an atomic each, and the sum puts the places in order. Whole vjp at 30 edges
-    // per sender, L = 32, f32, this way against the slots below (up to 4000 senders) or the
-    // counting sort beside the per-edge kernel (beyond): 2000 senders 27.6 / 22.6 us, 3000:
-    // 33.4 / 29.6, 4000: 37.6 / 39.3, 6000: 48 / 75, 20 000: 156 / 212
+    // sparse graphs: every edge takes the next of its sender's places in the per-edge kernel itself,
+    // an atomic each, and the sum puts the places in order. Whole vjp at 30 edges per sender,
+    // L = 32, f32, this way against the slots below (up to 4000 senders): 2000 senders 27.6 / 22.6
+    // us, 3000: 33.4 / 29.6, 4000: 37.6 / 39.3; against the counting sort of many edges: 200 000
+    // edges 48.7 / 62.8, 500 000: 129 / 122, 1 000 000: 231 / 204 (their lines cross between 400 000
+    // and 700 000, the shorter the rows the later)
     // (with no edges at all gather_in_kernel is false too: the per-edge kernel that would fill the
     // places is not launched then, so this way needs edges)
-    const bool by_arrival = want_W && narrow_rows && sparse && n_edges > 0 && K > 0 && K <= thresholds::OPSA_VJP_ROWS_IN_REGISTERS &&
-                            (n_output > thresholds::ARRIVAL_NODES || !gather_in_kernel) &&
+    const bool by_arrival = want_W && narrow_rows && n_output > 0 && L > 0 && n_edges > 0 && K > 0 &&
+                            K <= thresholds::OPSA_VJP_ROWS_IN_REGISTERS && n_edges <= thresholds::ARRIVAL_EDGES &&
+                            static_cast<size_t>(n_edges) <= static_cast<size_t>(n_output) * thresholds::ARRIVAL_MEAN_EDGES &&
+                            (n_output > thresholds::ARRIVAL_NODES || !gather_in_kernel || !sparse) &&
                             static_cast<size_t>(n_output) <= SCRATCH_COUNTERS;
     // small sparse graphs: the pass over the sender index is done by workgroups of the
     // per-edge kernel's launch and leaves every sender's edges in places of its own
@@ -1867,8 +1905,6 @@ void launch_vjp(
         want_W ? static_cast<char*>(scratch(edge_w_bytes + buckets_bytes)) : nullptr;
     T* edge_W = want_W ? reinterpret_cast<T*>(workspace) : nullptr;
 
-    // the lists of edges per sender do not depend on the kernels below: they are
-    // built beside them, on a side stream that joins before the lists are used
     EdgesBySender by_sender{};
     SenderSlots slots{};
     std::optional<ScratchCounters> taken; // (until the end of this call, finish_call included)
@@ -1878,11 +1914,10 @@ void launch_vjp(
         slots = SenderSlots{reinterpret_cast<int32_t*>(workspace + edge_w_bytes), taken->data()};
     }
     const bool use_buckets = want_W && n_output > 0 && L > 0 && !gather_in_kernel && !by_arrival;
-    std::unique_ptr<SideStream> beside;
     bool listed = false; // the slots are being filled by a kernel that is already enqueued
     if (use_buckets) {
-        beside = std::make_unique<SideStream>(stream);
-        by_sender = order_edges_by_sender(indices_W, n_edges, n_output, false, workspace + edge_w_bytes, beside->get());
+        // (beside the per-edge kernel on a stream of its own the sort gains nothing: both want all CUs)
+        by_sender = order_edges_by_sender(indices_W, n_edges, n_output, false, workspace + edge_w_bytes, stream);
     }
 
     // degenerate shapes: a gradient that sums over an empty axis is zero
@@ -1917,7 +1952,29 @@ void launch_vjp(
             return shift;
         };
         const unsigned waves = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_edges), CHUNK));
-        if (lds > 64 * 1024 && K > thresholds::OPSA_VJP_ROWS_IN_REGISTERS) {
+        // rows whose 16-byte pieces lie on 16-byte boundaries
+        const bool vectors = L % (16 / static_cast<int32_t>(sizeof(T))) == 0 &&
+                             reinterpret_cast<uintptr_t>(B.data) % 16 == 0 &&
+                             reinterpret_cast<uintptr_t>(grad_output.data) % 16 == 0 &&
+                             reinterpret_cast<uintptr_t>(grad_B.data) % 16 == 0 &&
+                             reinterpret_cast<uintptr_t>(edge_W) % 16 == 0 &&
+                             (!WEIGHTED || reinterpret_cast<uintptr_t>(W) % 16 == 0);
+        const bool by_tiles =
+            opsa_edges::covers(n_output, K, L, sizeof(T)) && n_edges >= tiles_from<T>(K, L, WEIGHTED, vectors);
+        if (by_tiles) {
+            const unsigned list_blocks = slotted ? sender_slots_blocks(n_output) : 0;
+            if (slotted) {
+                slots = sender_slots_in(workspace + edge_w_bytes, n_output);
+                listed = true;
+            }
+            MainKernelTimer timer(stream);
+            opsa_edges::launch<T>(
+                opsa_edges::Tensors<T>{
+                    grad_A.data, grad_B.data, edge_W, grad_output.data, A.data, B.data, W, indices_output.data, indices_W,
+                    n_edges, n_output, K, L},
+                const_cast<int32_t*>(slots.edges), const_cast<int32_t*>(slots.counts), list_blocks, stream
+            );
+        } else if (lds > 64 * 1024 && K > thresholds::OPSA_VJP_ROWS_IN_REGISTERS) {
             const unsigned blocks = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_edges), WIDE_WAVES));
             vjp_wide_kernel<T, WEIGHTED><<<blocks, WIDE_WAVES * WAVE, 0, stream>>>(
                 grad_A.data, grad_B.data, edge_W, grad_output.data, A.data, B.data, W, indices_W,
@@ -1926,12 +1983,6 @@ void launch_vjp(
         } else if (K <= thresholds::OPSA_VJP_ROWS_IN_REGISTERS) {
             const unsigned groups = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_edges), 16));
             MainKernelTimer timer(stream);
-            const bool vectors = L % (16 / static_cast<int32_t>(sizeof(T))) == 0 &&
-                                 reinterpret_cast<uintptr_t>(B.data) % 16 == 0 &&
-                                 reinterpret_cast<uintptr_t>(grad_output.data) % 16 == 0 &&
-                                 reinterpret_cast<uintptr_t>(grad_B.data) % 16 == 0 &&
-                                 reinterpret_cast<uintptr_t>(edge_W) % 16 == 0 &&
-                                 (!WEIGHTED || reinterpret_cast<uintptr_t>(W) % 16 == 0);
 #define MOPS_LAUNCH_ROWS_WITH(KT, NT, VECTORS, BLOCKS, LISTS, GRID, WAVES)                          \
     edge_rows_vjp_kernel<T, KT, NT, WEIGHTED, VECTORS, BLOCKS, LISTS><<<GRID, (WAVES) * WAVE, 0, stream>>>( \
         grad_A.data, grad_B.data, edge_W, grad_output.data, A.data, B.data, W, indices_W,          \
@@ -2073,12 +2124,24 @@ void launch_vjp(
             grad_W.data, edge_W, indices_W, n_edges, n_output, L, aligned
         );
     } else if (use_buckets) {
-        beside.reset(); // joins
         if (narrow_rows) {
             const unsigned blocks = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_output), LISTED_WAVES));
-            sum_listed_rows_kernel<T><<<blocks, LISTED_WAVES * WAVE, 0, stream>>>(
-                grad_W.data, edge_W, by_sender.offsets, by_sender.edge, n_output, L
-            );
+            auto sum = [&](auto kernel) {
+                kernel<<<blocks, LISTED_WAVES * WAVE, 0, stream>>>(
+                    grad_W.data, edge_W, by_sender.offsets, by_sender.edge, n_output, L
+                );
+            };
+            if (L <= 16) {
+                sum(sum_listed_rows_kernel<T, 4, 1>);
+            } else if (L <= 32) {
+                sum(sum_listed_rows_kernel<T, 2, 1>);
+            } else if (L <= WAVE) {
+                sum(sum_listed_rows_kernel<T, 1, 1>);
+            } else if (L <= 2 * WAVE) {
+                sum(sum_listed_rows_kernel<T, 1, 2>);
+            } else {
+                sum(sum_listed_rows_kernel<T, 1, 4>);
+            }
         } else {
             int threads = std::min(256, round_up_wave(L));
             gather_weights_kernel<T><<<n_output, threads, 0, stream>>>(grad_W.data, edge_W, by_sender, L);
