@@ -100,6 +100,13 @@ def test_setup_ships_library_headers_and_cmake_files(tmp_path):
     )
     assert built.returncode == 0, built.stdout + built.stderr
     package = tmp_path / "mops_amd"
-    for relative in ("lib/libmops.so", "lib/libmops_amd_torch.so", "include/mops.h", "include/mops/opsa.hpp", "cmake/mops/mops-config.cmake",
+    for relative in ("lib/libmops.so", "lib/libmops_amd_torch.so", "lib/_array_ops.so", "include/mops.h", "include/mops/opsa.hpp", "cmake/mops/mops-config.cmake",
                      "cmake/mops/mops-config-version.cmake", "torch.py"):
         assert (package / relative).exists(), relative
+    # the package as installed: its functions go the native way, without a message
+    probe = "from mops_amd import _c_lib, ops; print(ops.__file__); assert not isinstance(ops._native, _c_lib._NoFunctions)"
+    installed = subprocess.run(
+        [sys.executable, "-W", "error::RuntimeWarning", "-c", probe], cwd=str(tmp_path), capture_output=True, text=True
+    )
+    assert installed.returncode == 0, installed.stdout + installed.stderr
+    assert installed.stdout.startswith(str(package)), installed.stdout
