@@ -78,17 +78,30 @@ class _NoFunctions:
 
 def array_functions():
     """The functions of ``mops_amd/csrc/array_ops.cpp`` (built by ``build_torch_ops.py``), or functions
-    that leave every call to their caller where that has not been built or
-    ``MOPS_AMD_ARRAY_PYTHON=1`` is set."""
+    that leave every call to their caller (which goes through ctypes) where that has not been built,
+    cannot be loaded (PyTorch is not there; the file was built for another PyTorch or Python: a
+    warning says so) or ``MOPS_AMD_ARRAY_PYTHON=1`` is set."""
     if not os.path.exists(ARRAY_FUNCTIONS_PATH) or os.environ.get("MOPS_AMD_ARRAY_PYTHON", "0") not in ("", "0"):
         return _NoFunctions()
-    _require_built()
     import importlib.machinery
     import importlib.util
+    import warnings
 
-    import torch  # noqa: F401  (see device_library)
-
-    loader = importlib.machinery.ExtensionFileLoader("_array_ops", ARRAY_FUNCTIONS_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_array_ops", loader))
-    loader.exec_module(module)
+    try:
+        import torch  # noqa: F401  (see device_library)
+    except ImportError:
+        return _NoFunctions()
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_array_ops", ARRAY_FUNCTIONS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_array_ops", loader))
+        loader.exec_module(module)
+    except ImportError as error:
+        warnings.warn(
+            f"{ARRAY_FUNCTIONS_PATH} cannot be loaded ({error}): the functions of mops_amd go through ctypes, which "
+            "takes about 17 us more of the host per call; build it again for this PyTorch and Python with "
+            "`python mops_amd/csrc/build_torch_ops.py`",
+            RuntimeWarning,
+            stacklevel=2,
+        )
+        return _NoFunctions()
     return module
