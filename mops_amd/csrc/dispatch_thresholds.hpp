@@ -12,14 +12,79 @@
 namespace mops::amd::thresholds {
 
 // ---- HPE (hpe.hip) ---------------------------------------------------------
-/// Factors of all monomials times rows from which the gradients go by feature
-/// (hpe_tiles.hip: two launches in front turn the table round) instead of a
-/// workgroup per few rows with accumulators in LDS. Whole vjp, LDS
-/// accumulators / by feature, in double: 8.0e6 (1000 rows, 2000 monomials of
-/// order 4, 100 features) 15.0 / 23 us, 1.15e7 (100 x 28 794 x 4, 53 features)
-/// 58 / 32, 2.9e7 (673 x 14 572 x 3, 23 features) 38.6 / 27, 6.6e7 (8192 x 2000
-/// x 4) 65 / 50; second order 20 / 39, 88 / 51, 49 / 47, 113 / 85.
-constexpr int64_t HPE_TILES_WORK = 10 * 1000 * 1000;
+/// The three families of kernels: a tile of 4 to 16 rows in LDS and the monomials
+/// spread over a workgroup of 1024 threads (hpe_tiles.hip), a lane per row
+/// (hpe_rows.hip), and a few rows per workgroup of 256 threads (hpe.hip; in the
+/// gradients with accumulators in LDS).
+enum class HpeKernels { TILES, ROWS, FEW };
+
+/// Forward pass. The tiles pay for filling LDS, a reduction over 256 teams and
+/// two barriers per 16 rows (fewer where rows are wide), whatever the length of
+/// the table; a lane per row pays a readlane per factor; a few rows per
+/// workgroup read the table once for every few rows, from the caches. By
+/// `factors` of the table (monomials x order), measured at 1370 points (64 to
+/// 100 000 rows, 10 to 2000 features, 30 to 90 000 factors; the rule is on
+/// average 1.3 % above the best of the three there, always tiles 30 %), us,
+/// tiles / rows / few: 100 000 rows x 10 features, 150 factors, f32 27.5 / 8.0 /
+/// 7.7, f64 41.6 / 11.4 / 10.4, 2000 factors f32 34.7 / 24.0 / 62.8, 9000 60.7 /
+/// 87.8 / 174; 100 000 x 100, 600: 40.2 / 19.8 / 31.8, f64 66 / 32 / 40; 13 000 x
+/// 30, 300: 6.8 / 4.6 / 4.9; 4000 x 250, 600, f64: 16.7 / 7.7 / 5.8; 1000 x 100,
+/// 9000: 7.1 / 27.9 / 5.2, 30 000: 10.2 / 80 / 9.7, 90 000: 13.5 / 230 / 21.8.
+inline HpeKernels hpe_forward(int64_t rows, int64_t features, int64_t factors, int64_t element_size) {
+    const int64_t row_bytes = features * element_size;
+    const bool single = element_size == 4;
+    const int64_t rows_factors =
+        (single ? (rows / 10 < 5000 ? rows / 10 : 5000) : (rows * 3 / 20 < 3000 ? rows * 3 / 20 : 3000)) + 2 * row_bytes;
+    if (rows >= 10000 && row_bytes <= (single ? 850 : 2100) && factors <= rows_factors) {
+        return HpeKernels::ROWS;
+    }
+    bool few;
+    if (rows < 3000) {
+        few = rows * factors <= 30 * 1000 * 1000 &&
+              (factors >= (single && row_bytes > 2500 ? row_bytes : 2500) || (!single && row_bytes >= 400));
+    } else if (single) {
+        few = row_bytes >= 300 && row_bytes <= 1000 && factors <= 1000;
+    } else {
+        const int64_t more = rows >= 5000 ? row_bytes * 5 / 4 : row_bytes * 4 < 7000 ? row_bytes * 4 : 7000;
+        few = row_bytes >= 200 && row_bytes <= 10000 && factors <= 1000 + more;
+    }
+    return few ? HpeKernels::FEW : HpeKernels::TILES;
+}
+
+/// Gradients. Tiles and a lane per row turn the table round first (one or two
+/// launches in front); the accumulators in LDS of a few rows per workgroup are
+/// cleared and added up for every group of rows, which is work per feature, and
+/// take an LDS addition per factor. The rule is on average 2 % above the best of
+/// the three at 370 points (1000 to 100 000 rows, 10 to 250 features, 30 to 9000
+/// factors); tiles from 10^7 factors of all rows on and few rows below are 16 %. us,
+/// tiles / rows / few: 1000 rows x 100 features, 8000 factors, f32 18.0 / 27.6 /
+/// 11.5; 13 000 x 30, 300: 13.7 / 10.4 / 9.0; 100 000 x 10, 150: 42.5 / 15.2 /
+/// 22.6, f64 87 / 17.7 / 25.4, 2000: 48.0 / 40.4 / 113, 9000: 121 / 218 / 497;
+/// 40 000 x 100, 300: 30.0 / 31.1 / 42.4, 3000: 42.6 / 55.1 / 159.
+inline HpeKernels hpe_vjp(int64_t rows, int64_t features, int64_t factors, int64_t element_size) {
+    const bool single = element_size == 4;
+    const bool little = rows * factors < 10 * 1000 * 1000;
+    if (features > 16 && little && rows * features < 3 * 1000 * 1000) {
+        return HpeKernels::FEW;
+    }
+    const int64_t by_table = features <= 64 ? 3000 - 20 * features : features <= 120 ? 600 : 0;
+    const int64_t rows_factors = (rows / 10 < by_table ? rows / 10 : by_table) * (single ? 5 : 8) / 5;
+    if (rows >= 8000 + 100 * features && factors <= rows_factors) {
+        return HpeKernels::ROWS;
+    }
+    const bool few = little || (features > 16 && factors < 500 && rows >= 10000 && rows * features < 2500 * 1000);
+    return few ? HpeKernels::FEW : HpeKernels::TILES;
+}
+
+/// Second order: tiles or few rows (a lane per row has no second-order kernel).
+/// us, tiles / few: 100 000 rows x 10 features, 150 factors, f32 102 / 23.3, f64
+/// 165 / 26.7, 900: 121 / 77, 200 / 100; 100 000 x 30, 900: 143 / 131, 225 / 157;
+/// 100 000 x 100, 300: 123 / 110, 600: 132 / 160; 1000 x 100, 8000, f64 45 / 17.
+inline HpeKernels hpe_vjp_vjp(int64_t rows, int64_t features, int64_t factors, int64_t element_size) {
+    const bool few = rows * factors < (element_size == 4 ? 16 : 24) * int64_t(1000 * 1000) ||
+                     (rows >= 10000 && factors < 1500 - 10 * features);
+    return few ? HpeKernels::FEW : HpeKernels::TILES;
+}
 
 // ---- SAP (sap_mfma.hip) ----------------------------------------------------
 /// Tiles of 16 rows per wavefront of the device from which a launch has as many

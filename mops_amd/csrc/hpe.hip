@@ -31,6 +31,7 @@
 #include "dispatch_thresholds.hpp"
 #include "index_validation.hpp"
 #include "elementwise.hpp"
+#include "hpe_rows.hpp"
 #include "hpe_tiles.hpp"
 #include "runtime.hpp"
 
@@ -1052,7 +1053,14 @@ void homogeneous_polynomial_evaluation(MOPS_HPE_PARAMS(MOPS_CXX_FIRST, MOPS_CXX_
     }
     hipStream_t stream = current_stream();
     const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
-    if (const auto plan = hpe_tiles::plan_forward(shape, sizeof(scalar_t)); plan.values > 0) {
+    const auto kernels = thresholds::hpe_forward(n_rows, nA, static_cast<int64_t>(n_monomials) * order, sizeof(scalar_t));
+    if (kernels == thresholds::HpeKernels::ROWS && hpe_rows::covers_forward(shape, sizeof(scalar_t))) {
+        hpe_rows::forward<scalar_t>(output.data, A.data, C.data, indices_A.data, shape, stream);
+        finish_call(operation);
+        return;
+    }
+    if (const auto plan = hpe_tiles::plan_forward(shape, sizeof(scalar_t));
+        plan.values > 0 && kernels != thresholds::HpeKernels::FEW) {
         const size_t bytes = hpe_tiles::forward_bytes(shape, plan, sizeof(scalar_t));
         void* workspace = bytes > 0 ? scratch(bytes) : nullptr;
         auto launch = [&](int32_t* counters) {
@@ -1140,8 +1148,17 @@ void homogeneous_polynomial_evaluation_vjp(MOPS_HPE_VJP_PARAMS(MOPS_CXX_FIRST, M
     // accumulators of every feature for each of the 64 lanes that walk the monomials
     const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
     const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
+    const auto kernels = thresholds::hpe_vjp(n_rows, nA, static_cast<int64_t>(n_monomials) * order, sizeof(scalar_t));
+    if (kernels == thresholds::HpeKernels::ROWS && hpe_rows::covers_vjp(shape, sizeof(scalar_t))) {
+        void* workspace = scratch(hpe_tiles::table_bytes(shape, sizeof(scalar_t)));
+        hpe_rows::vjp<scalar_t>(
+            grad_A.data, grad_output.data, A.data, C.data, indices_A.data, shape, workspace, stream
+        );
+        finish_call(operation);
+        return;
+    }
     const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), false);
-    if (plan.values > 0 && (hpe_tiles::large(shape) || accumulator_bytes > LDS_BUDGET)) {
+    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET)) {
         void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), false));
         hpe_tiles::vjp<scalar_t>(
             grad_A.data, grad_output.data, A.data, C.data, indices_A.data, shape, plan, workspace, stream
@@ -1272,8 +1289,9 @@ void homogeneous_polynomial_evaluation_vjp_vjp(MOPS_HPE_VJP_VJP_PARAMS(MOPS_CXX_
     }
     const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
     const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
+    const auto kernels = thresholds::hpe_vjp_vjp(n_rows, nA, static_cast<int64_t>(n_monomials) * order, sizeof(scalar_t));
     const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), true);
-    if (plan.values > 0 && (hpe_tiles::large(shape) || accumulator_bytes > LDS_BUDGET)) {
+    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET)) {
         void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), true));
         ScratchCounters counters;
         hpe_tiles::vjp_vjp<scalar_t>(

@@ -29,7 +29,6 @@
 #include "hpe_tiles.hpp"
 
 #include "device_common.hpp"
-#include "dispatch_thresholds.hpp"
 #include "runtime.hpp"
 
 namespace mops::amd {
@@ -42,7 +41,6 @@ constexpr int TEAM = 4;
 constexpr int TEAMS = THREADS / TEAM;
 constexpr size_t LDS_LIMIT = 156 * 1024; // of the 160 KB of a compute unit
 constexpr int MOST_VALUES = 4;           // per lane: one 16-byte load of floats, two of doubles
-constexpr int32_t MAX_FEATURES = 10000;  // of the counting sort
 
 /// Values of T that one LDS load of a lane brings: V of them, 16 bytes at most.
 template <typename T, int V> constexpr int chunk_values() { return V * sizeof(T) < 16 ? V : 16 / sizeof(T); }
@@ -711,35 +709,43 @@ Sort sort_of(const Shape& s) {
     return sort;
 }
 
+/// Carves `bytes` of scratch memory; with no memory given, adds them up.
+struct Carver {
+    char* base;
+    size_t used = 0;
+    void* take(size_t bytes) {
+        void* p = base + used;
+        used += align256(bytes);
+        return p;
+    }
+};
+TurnedTable carve_table(const Shape& s, size_t element_size, Carver& carver) {
+    const size_t n_pairs = static_cast<size_t>(s.n_monomials) * s.order;
+    const Sort sort = sort_of(s);
+    TurnedTable table;
+    table.lists = static_cast<int32_t*>(carver.take((static_cast<size_t>(s.nA) + 1) * sizeof(int32_t)));
+    table.counts = static_cast<int32_t*>(
+        carver.take(sort.blocks > 1 ? static_cast<size_t>(sort.blocks) * s.nA * sizeof(int32_t) : 0)
+    );
+    table.records = static_cast<uint32_t*>(carver.take(
+        (n_pairs + static_cast<size_t>(TEAM) * (s.nA + 1)) * (s.order - 1 + element_size / 4) * sizeof(uint32_t)
+    ));
+    return table;
+}
+
 struct Workspace {
-    int32_t* lists;
-    int32_t* counts;
-    uint32_t* records;
+    TurnedTable table;
     void* partial;
     size_t bytes;
 };
 Workspace carve(const Shape& s, const Plan& plan, size_t element_size, bool second, void* at) {
-    const size_t n_pairs = static_cast<size_t>(s.n_monomials) * s.order;
-    const Sort sort = sort_of(s);
-    char* base = static_cast<char*>(at);
-    size_t used = 0;
-    auto take = [&](size_t bytes) {
-        char* p = base + used;
-        used += align256(bytes);
-        return p;
-    };
+    Carver carver{static_cast<char*>(at)};
     Workspace w;
-    w.lists = reinterpret_cast<int32_t*>(take((static_cast<size_t>(s.nA) + 1) * sizeof(int32_t)));
-    w.counts = reinterpret_cast<int32_t*>(
-        take(sort.blocks > 1 ? static_cast<size_t>(sort.blocks) * s.nA * sizeof(int32_t) : 0)
-    );
-    w.records = reinterpret_cast<uint32_t*>(
-        take((n_pairs + static_cast<size_t>(TEAM) * (s.nA + 1)) * (s.order - 1 + element_size / 4) * sizeof(uint32_t))
-    );
-    w.partial = take(
+    w.table = carve_table(s, element_size, carver);
+    w.partial = carver.take(
         second && plan.groups > 1 ? static_cast<size_t>(plan.tiles) * plan.groups * TEAM * plan.values * element_size : 0
     );
-    w.bytes = used;
+    w.bytes = carver.used;
     return w;
 }
 
@@ -784,7 +790,7 @@ template <typename Body> void with_values(int values, Body&& body) {
 }
 
 template <typename T, int ORDER>
-void turn_table(const Workspace& w, const T* C, const int32_t* P, const Shape& s, int32_t stride, hipStream_t stream) {
+void enqueue_table(const TurnedTable& w, const T* C, const int32_t* P, const Shape& s, int32_t stride, hipStream_t stream) {
     const int32_t n_pairs = s.n_monomials * s.order;
     const Sort sort = sort_of(s);
     if (sort.blocks > 1) {
@@ -820,14 +826,14 @@ void gradient(
     with_order(s.order, [&](auto order) {
         constexpr int ORDER = decltype(order)::value;
         const int32_t stride = (SECOND ? 2 : 1) * TEAM * plan.values * static_cast<int32_t>(sizeof(T));
-        turn_table<T, ORDER>(w, C, P, s, stride, stream);
+        enqueue_table<T, ORDER>(w.table, C, P, s, stride, stream);
         with_values(plan.values, [&](auto values) {
             auto kernel = gradient_kernel<T, ORDER, decltype(values)::value, SECOND>;
             allow_lds(kernel, plan.lds);
             MainKernelTimer timer(stream);
             kernel<<<blocks_of(plan), THREADS, plan.lds, stream>>>(
-                grad_A, grad_grad_output, static_cast<T*>(w.partial), counters, grad_grad_A, grad_output, A, w.lists,
-                w.records, s.n_rows, s.nA, share, plan.log2_parts, plan.tiles, plan.groups
+                grad_A, grad_grad_output, static_cast<T*>(w.partial), counters, grad_grad_A, grad_output, A, w.table.lists,
+                w.table.records, s.n_rows, s.nA, share, plan.log2_parts, plan.tiles, plan.groups
             );
         });
     });
@@ -844,7 +850,7 @@ void gradient(
 /// features, 314 monomials of order 3, forward, 4 / 2 values in float 33 / 24
 /// us, 2 / 1 in double 66 / 52).
 template <typename Bytes> Plan choose(const Shape& s, size_t most_groups, Bytes&& lds) {
-    constexpr size_t UNITS = 256;
+    const size_t units = static_cast<size_t>(compute_units());
     const bool light = static_cast<size_t>(s.n_monomials) * s.order < 4 * static_cast<size_t>(s.nA);
     Plan plan;
     for (int values = MOST_VALUES; values >= 1; values >>= 1) {
@@ -855,24 +861,34 @@ template <typename Bytes> Plan choose(const Shape& s, size_t most_groups, Bytes&
         plan.values = values;
         plan.lds = bytes;
         plan.tiles = static_cast<int32_t>(ceil_div(static_cast<size_t>(s.n_rows), static_cast<size_t>(TEAM * values)));
-        const size_t resident = UNITS * (bytes <= LDS_LIMIT / 2 ? 2 : 1);
+        const size_t resident = units * (bytes <= LDS_LIMIT / 2 ? 2 : 1);
         plan.groups = static_cast<int32_t>(std::min(most_groups, std::max<size_t>(1, resident / plan.tiles)));
-        if (plan.tiles * most_groups >= UNITS && !(light && bytes > LDS_LIMIT / 3)) {
+        if (plan.tiles * most_groups >= units && !(light && bytes > LDS_LIMIT / 3)) {
             break;
         }
     }
     return plan;
 }
 
+} // namespace
+
 bool covered(const Shape& s) {
     return s.order >= 1 && s.order <= 6 && s.n_monomials > 0 && s.n_rows > 0 && s.nA > 0 &&
            static_cast<size_t>(s.n_monomials) * s.order < (size_t(1) << 28);
 }
 
-} // namespace
+size_t table_bytes(const Shape& s, size_t element_size) {
+    Carver carver{nullptr};
+    carve_table(s, element_size, carver);
+    return carver.used;
+}
 
-bool large(const Shape& s) {
-    return static_cast<int64_t>(s.n_rows) * s.n_monomials * s.order >= thresholds::HPE_TILES_WORK;
+template <typename T>
+TurnedTable turn_table(const T* C, const int32_t* P, const Shape& s, int32_t stride, void* workspace, hipStream_t stream) {
+    Carver carver{static_cast<char*>(workspace)};
+    const TurnedTable table = carve_table(s, sizeof(T), carver);
+    with_order(s.order, [&](auto order) { enqueue_table<T, decltype(order)::value>(table, C, P, s, stride, stream); });
+    return table;
 }
 
 Plan plan_forward(const Shape& s, size_t element_size) {
@@ -963,7 +979,8 @@ void vjp_vjp(
     template void vjp_vjp<T>(                                                                      \
         T*, T*, const T*, const T*, const T*, const T*, const int32_t*, const Shape&, const Plan&, void*, int32_t*, \
         hipStream_t                                                                                \
-    );
+    );                                                                                             \
+    template TurnedTable turn_table<T>(const T*, const int32_t*, const Shape&, int32_t, void*, hipStream_t);
 MOPS_INSTANTIATE(float)
 MOPS_INSTANTIATE(double)
 #undef MOPS_INSTANTIATE

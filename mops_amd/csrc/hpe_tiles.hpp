@@ -1,8 +1,7 @@
 // HPE with the values of a few rows in LDS and the monomials spread over a
-// workgroup in teams of four lanes: the kernels of large problems (hpe_tiles.hip).
+// workgroup in teams of four lanes: the kernels of long tables (hpe_tiles.hip).
 // hpe.hip calls them when `plan_*` finds a layout (orders 1 to 6, tiles that fit
-// in LDS), for gradients when the problem is large, and keeps its own kernels
-// for everything else.
+// in LDS) and they are ahead of the others (thresholds::hpe_*).
 #ifndef MOPS_AMD_HPE_TILES_HPP
 #define MOPS_AMD_HPE_TILES_HPP
 
@@ -31,9 +30,28 @@ struct Plan {
     size_t lds = 0;
 };
 
-/// Whether the gradients are ahead of the kernels of hpe.hip where both could
-/// serve (the forward pass always is).
-bool large(const Shape& shape);
+/// Whether the kernels here and in hpe_rows.hip cover the table (orders 1 to 6, something to do).
+bool covered(const Shape& shape);
+
+/// Features up to which the table can be turned round (counters of the sort in LDS).
+constexpr int32_t MAX_FEATURES = 10000;
+
+/// The table turned round: for every feature the terms of its gradient. The
+/// records of feature f are those from 4 lists[f] up to 4 lists[f + 1], each
+/// the byte offsets of the order - 1 other factors (feature * stride; a factor
+/// out of range counts as feature nA) and the coefficient behind them; lists
+/// are filled up to four records with terms that are zero. For covered()
+/// shapes of at most MAX_FEATURES features.
+struct TurnedTable {
+    int32_t* lists;
+    int32_t* counts; // of the sort
+    uint32_t* records;
+};
+size_t table_bytes(const Shape& shape, size_t element_size);
+template <typename T>
+TurnedTable turn_table(
+    const T* C, const int32_t* P, const Shape& shape, int32_t stride, void* workspace, hipStream_t stream
+);
 
 Plan plan_forward(const Shape& shape, size_t element_size);
 /// `second`: the second-order pass, which keeps two values per row and feature.
