@@ -1382,9 +1382,14 @@ constexpr int SLOT_MEAN_LIMIT = thresholds::SLOT_MEAN_EDGES;
 
 // The sum over the slots: one wavefront per sender, ascending edge order, as
 // many rows in flight as 32 registers hold (COLUMNS values of a row per lane).
-// A sender with more edges than places (rare by the choice of SLOT_MEAN_LIMIT)
-// is looked after by its wavefront alone, which then reads the whole sender
-// index itself.
+// A sender with more edges than places (rare by the choice of SLOT_MEAN_LIMIT
+// and ARRIVAL_MEAN_EDGES) is looked after by the whole workgroup, each
+// wavefront with a quarter of the sender index (edges_of_sender); the four sums
+// are added in the order of the quarters. Whole OPSAW vjp, f32, L = 32, with one
+// sender of 300 edges among 1000 of 60, 3000 of 60 and 2000 of 46: 69, 105 and 68
+// us (without it 35.5, 44.7 and 27.4; by one wavefront, a load at a time, 552, 1141
+// and 702); with all of 3000 x 60 edges drawn with a density that falls along the
+// senders (every eighteenth has more than 128): 304 us against 2260.
 constexpr int LISTED_WAVES = 4;
 
 /// ARRIVALS: the places hold the sender's edges in the order of arrival, with one
@@ -1396,11 +1401,16 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
     int32_t n_nodes, int32_t L
 ) {
     __shared__ int32_t sorting_areas[ARRIVALS ? LISTED_WAVES : 1][ARRIVALS ? SLOT_CAPACITY : 1];
+    __shared__ int32_t hubs[LISTED_WAVES];
+    __shared__ T hub_sums[LISTED_WAVES][COLUMNS * WAVE];
     const int lane = threadIdx.x & (WAVE - 1);
-    const int32_t node = __builtin_amdgcn_readfirstlane(blockIdx.x * LISTED_WAVES + (threadIdx.x >> 6));
-    if (node >= n_nodes) {
-        return;
-    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // (neighbouring senders in different workgroups, and others a multiple of the number of workgroups
+    // apart too: those with many edges are often next to each other, or a fixed distance apart)
+    const int32_t own = wave * gridDim.x + (blockIdx.x + 17 * wave) % gridDim.x;
+    // (a wavefront beyond the last sender has no edges and nothing to store, but helps with the others)
+    const bool exists = own < n_nodes;
+    const int32_t node = exists ? own : n_nodes - 1;
     const int32_t* mine = slots + static_cast<size_t>(node) * SLOT_CAPACITY;
     // all places asked for before the counts are known
     int32_t first_half = mine[lane];
@@ -1411,8 +1421,9 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
     int32_t count;
     if constexpr (ARRIVALS) {
         count = max(__builtin_amdgcn_readfirstlane(counts[node]), 0);
-        if (lane == 0) {
-            counts[node] = 0; // (nobody else reads it: zero again for the next launch)
+        count = exists ? count : 0;
+        if (lane == 0 && exists) {
+            counts[node] = 0; // (nobody else uses it: zero again for the next launch)
         }
         listed = count <= SLOT_CAPACITY;
     } else {
@@ -1421,8 +1432,8 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
         c1 = __builtin_amdgcn_readfirstlane(part_counts.y);
         c2 = __builtin_amdgcn_readfirstlane(part_counts.z);
         c3 = __builtin_amdgcn_readfirstlane(part_counts.w);
-        listed = max(max(c0, c1), max(c2, c3)) <= SLOT_PART_CAPACITY;
-        count = c0 + c1 + c2 + c3;
+        listed = !exists || max(max(c0, c1), max(c2, c3)) <= SLOT_PART_CAPACITY;
+        count = exists ? c0 + c1 + c2 + c3 : 0;
     }
     T sum[COLUMNS];
     uint32_t column[COLUMNS];
@@ -1431,9 +1442,9 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
         sum[c] = T(0);
         column[c] = min(lane + c * WAVE, L - 1);
     }
-    constexpr int ROWS = 32 / (COLUMNS * static_cast<int>(sizeof(T) / 4));
-    // adds the rows of the first n <= 64 edges held by the lanes of `my_edge`
-    auto add_rows = [&](int32_t my_edge, int32_t n) {
+    // adds the rows of the first n <= 64 edges held by the lanes of `my_edge`, ROWS of them in flight
+    auto add_rows = [&](auto rows_in_flight, int32_t my_edge, int32_t n) {
+        constexpr int ROWS = decltype(rows_in_flight)::value;
 #pragma unroll 1
         for (int32_t k0 = 0; k0 < n; k0 += ROWS) {
             T values[ROWS][COLUMNS];
@@ -1458,6 +1469,9 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
             }
         }
     };
+    constexpr std::integral_constant<int, 32 / (COLUMNS * static_cast<int>(sizeof(T) / 4))> many{};
+    // (fewer for the hubs: the kernel takes no more registers for them)
+    constexpr std::integral_constant<int, std::max(many.value / 4, 1)> few{};
     if (listed) {
         // the parts moved together: position p of the list is in part `part`, place p - before
         auto edge_at = [&](int32_t position) {
@@ -1480,35 +1494,56 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
             second_half = min(max(second_half, 0), n_edges - 1);
         }
         const int32_t first = ARRIVALS ? first_half : edge_at(lane);
-        add_rows(lane < n_first ? first : 0, n_first);
+        add_rows(many, lane < n_first ? first : 0, n_first);
         if (count > WAVE) {
             const int32_t n_second = count - WAVE;
             const int32_t second = ARRIVALS ? second_half : edge_at(lane + WAVE);
-            add_rows(lane < n_second ? second : 0, n_second);
+            add_rows(many, lane < n_second ? second : 0, n_second);
         }
-    } else {
-        const unsigned long long below = (1ull << lane) - 1ull;
-        for (int32_t base = 0; base < n_edges; base += WAVE) {
-            const int32_t e = base + lane;
-            const bool named = e < n_edges && senders[min(e, n_edges - 1)] == node;
-            const unsigned long long mask = __ballot(named);
-            if (mask != 0) {
-                // the matches moved to the first lanes, in edge order
-                // (a permutation of the lanes: the others follow, in their order)
-                const int32_t n = __popcll(mask);
-                const int32_t named_below = __popcll(mask & below);
-                const int32_t place = named ? named_below : n + lane - named_below;
-                const int32_t packed = __builtin_amdgcn_ds_permute(place << 2, e);
-                add_rows(lane < n ? packed : 0, n);
+    }
+    if (listed && exists) {
+#pragma unroll
+        for (int c = 0; c < COLUMNS; c++) {
+            const int32_t l = lane + c * WAVE;
+            if (l < L) {
+                grad_W[static_cast<size_t>(node) * L + l] = sum[c];
             }
         }
     }
-#pragma unroll
-    for (int c = 0; c < COLUMNS; c++) {
-        const int32_t l = lane + c * WAVE;
-        if (l < L) {
-            grad_W[static_cast<size_t>(node) * L + l] = sum[c];
+    if (lane == 0) {
+        hubs[wave] = listed ? -1 : node;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int w = 0; w < LISTED_WAVES; w++) {
+        const int32_t hub = __builtin_amdgcn_readfirstlane(hubs[w]); // (the same in all wavefronts)
+        if (hub < 0) {
+            continue;
         }
+#pragma unroll
+        for (int c = 0; c < COLUMNS; c++) {
+            sum[c] = T(0);
+        }
+        const int32_t quarter = n_edges / LISTED_WAVES + 1;
+        const int32_t begin = min(wave * quarter, n_edges);
+        constexpr int AHEAD = sizeof(T) == 8 && COLUMNS > 1 ? 4 : 8; // (as many as cost no wavefront of the SIMD)
+        edges_of_sender<AHEAD>(
+            senders, n_edges, begin, min(begin + quarter, n_edges), hub, lane,
+            [&](int32_t edge, int32_t n) { add_rows(few, edge, n); }
+        );
+#pragma unroll
+        for (int c = 0; c < COLUMNS; c++) {
+            hub_sums[wave][lane + c * WAVE] = sum[c];
+        }
+        __syncthreads();
+        for (int32_t l = threadIdx.x; l < L; l += LISTED_WAVES * WAVE) {
+            T total = hub_sums[0][l];
+            for (int of = 1; of < LISTED_WAVES; of++) {
+                total += hub_sums[of][l];
+            }
+            grad_W[static_cast<size_t>(hub) * L + l] = total;
+        }
+        __syncthreads(); // (the next hub's sums go to the same place)
     }
 }
 

@@ -620,19 +620,8 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
                 }
             } else {
                 // more edges than places (a hub of a sparse graph): this wavefront reads the index itself
-                const unsigned long long below = (1ull << lane) - 1ull;
-                for (int32_t base = 0; base < p.n_edges; base += WAVE) {
-                    const int32_t e = base + lane;
-                    const bool named = e < p.n_edges && args.senders[min(e, p.n_edges - 1)] == node;
-                    const unsigned long long mask = __ballot(named);
-                    if (mask != 0) {
-                        const int32_t n = __popcll(mask);
-                        const int32_t named_below = __popcll(mask & below);
-                        const int32_t place = named ? named_below : n + lane - named_below;
-                        const int32_t edges = __builtin_amdgcn_ds_permute(place << 2, e);
-                        hand_on(lane < n ? edges : 0, n);
-                    }
-                }
+                // (3000 nodes of 30 edges, one of them of 300, f32, whole vjp 250 us; a load at a time 674; without it 71)
+                edges_of_sender<4>(args.senders, p.n_edges, 0, p.n_edges, node, lane, hand_on);
             }
             finish(node);
         }

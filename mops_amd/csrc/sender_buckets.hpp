@@ -307,6 +307,77 @@ __device__ __forceinline__ void arrivals_in_order(
     __builtin_amdgcn_wave_barrier();
 }
 
+/// The edges of [begin, end) that name `sender`, in ascending order, found by one wavefront that
+/// reads this piece of the index itself: for a sender with more edges than it has places.
+/// `hand_on(edge, n)` gets up to 64 of them at a time, lane k < n holding the k-th (the other lanes
+/// hold 0). AHEAD loads of 256 positions are on their way together, and the edges wait in a register
+/// until there are 64, so that neither the index nor the rows are read one round trip at a time.
+template <int AHEAD, typename HandOn>
+__device__ __forceinline__ void edges_of_sender(
+    const int32_t* __restrict__ senders, int32_t n_edges, int32_t begin, int32_t end, int32_t sender, int lane,
+    HandOn&& hand_on
+) {
+    // (four values at any address of an integer)
+    typedef int32_t Four __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int GROUP = 4 * WAVE;
+    int32_t waiting = 0, n_waiting = 0;
+    auto wait = [&](int32_t edge) { // (the same in all lanes)
+        waiting = lane == n_waiting ? edge : waiting;
+        n_waiting++;
+        if (n_waiting == WAVE) {
+            hand_on(waiting, WAVE);
+            n_waiting = 0;
+        }
+    };
+    if (n_edges < 4) {
+        return; // (no sender has more edges than places then)
+    }
+    for (int32_t base = begin; base < end; base += AHEAD * GROUP) {
+        // a lane looks at four positions of every group, moved to the front where the index ends
+        auto first = [&](int u) { return base + u * GROUP + 4 * lane; };
+        auto load = [&](int u) { return *reinterpret_cast<const Four*>(senders + min(first(u), n_edges - 4)); };
+        auto named = [&](const Four& value, int u, int c) {
+            const int32_t position = min(first(u), n_edges - 4) + c;
+            return value[c] == sender && position >= first(u) && position < end;
+        };
+        Four value[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            value[u] = load(u);
+        }
+        uint32_t with_matches = 0;
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const bool any = named(value[u], u, 0) || named(value[u], u, 1) || named(value[u], u, 2) || named(value[u], u, 3);
+            with_matches |= __ballot(any) != 0 ? 1u << u : 0u;
+        }
+        while (with_matches != 0) { // (the same in all lanes)
+            const int u = __builtin_ctz(with_matches);
+            with_matches &= with_matches - 1;
+            const Four again = load(u);
+            uint32_t mine = 0;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                mine |= named(again, u, c) ? 1u << c : 0u;
+            }
+            unsigned long long lanes = __ballot(mine != 0);
+            while (lanes != 0) {
+                const int from = __builtin_ctzll(lanes);
+                lanes &= lanes - 1;
+                uint32_t matches = __builtin_amdgcn_readlane(static_cast<int>(mine), from);
+                const int32_t position = min(base + u * GROUP + 4 * from, n_edges - 4);
+                while (matches != 0) {
+                    wait(position + __builtin_ctz(matches));
+                    matches &= matches - 1;
+                }
+            }
+        }
+    }
+    if (n_waiting > 0) {
+        hand_on(lane < n_waiting ? waiting : 0, n_waiting);
+    }
+}
+
 } // namespace mops::amd
 
 #endif
