@@ -99,8 +99,8 @@ MOPS_EXPORT int64_t mops_amd_scratch_capacity(void);
  *
  * No counterpart in lab-cosmo/mops. It is for callers that cannot allocate
  * device memory: code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc. Same arguments, checks, results (bit for bit) and
- * return convention as
+ * that forbid hipMalloc. Same arguments, checks, results (bit for bit but for the
+ * last limit below) and return convention as
  * mops_cuda_sparse_accumulation_scatter_add_with_weights_vjp_f32, but the
  * temporaries of its kernels (the dense coupling table and the list of every
  * sender's edges) live in an array of 4 MiB that is part of the library's
@@ -110,11 +110,14 @@ MOPS_EXPORT int64_t mops_amd_scratch_capacity(void);
  * it is off inside this call, whatever the thread's setting). Shapes whose
  * sums are empty (no column, table entry, edge or node) give zero gradients,
  * as there. Limits, reported as status 1 with a message: A.shape[1],
- * W.shape[1], output.shape[1] at most 16; temporaries within 4 MiB (about
- * 7800 nodes); when grad_W is asked for together with grad_A or grad_B, at
- * most 48 edges per node on average and W.shape[1], output.shape[1] in the
- * same multiple of four; no grad_W at all for graphs so large and dense that
- * the edges are first sorted by sender; indices_output_1 sorted
+ * W.shape[1], output.shape[1] at most 16; temporaries within 4 MiB: about
+ * 7800 nodes, or about 516 000 edges where grad_W has them put in the order of
+ * their senders (A.shape[1] = W.shape[1] = output.shape[1] = 4, 9 or 16 and
+ * more than 48 edges per node on average, or edges x nodes above 10^9); with
+ * other components, when grad_W is asked for together with grad_A or grad_B, at
+ * most 64 edges per node on average. Beyond these grad_W alone, in a call of
+ * its own, is served while edges x nodes / 4 is at most 10^8 (the sums in
+ * another order than the existing entry point's). indices_output_1 sorted
  * (mops_amd_accept_unsorted_indices does not apply). With
  * MOPS_AMD_CHECK_INDICES=1 the indices are copied to the host and checked as
  * in the existing entry point, which waits for the stream and allocates host

@@ -943,29 +943,39 @@ void sasaw_vjp_no_alloc(
     const sasaw_mfma::Indices indices{
         indices_A.data, indices_W_1.data, indices_W_2.data, indices_output_1.data, indices_output_2.data
     };
+    const bool mfma = sasaw_mfma::supports(shape, sizeof(float));
+    // grad_W alone by the in-kernel gather over the whole sender index: nothing but the dense table in the array
+    const bool gathers = !want_edges && mfma && sasaw_mfma::vjp_allocates_nothing(shape, sizeof(float), false, true) &&
+                         sasaw_mfma::workspace_bytes(shape, sizeof(float)) <= NO_ALLOC_SCRATCH_BYTES;
     if (s.L > 0 && sasaw_segments::vjp_supported(shape, sizeof(float), want_W)) {
         // (the same kernels as the existing entry point takes for these shapes)
-        // (the places of the senders' edges, then their counters; the array is shared with the
-        // kernels of other shapes, so the counters are cleared by a launch in front)
+        // (the places of the senders' edges or their order, then the counters; the array is shared with
+        // the kernels of other shapes, so the counters are cleared by a launch in front)
         const size_t places = sasaw_segments::vjp_workspace_bytes(shape, sizeof(float), want_W);
         const size_t needed = places + sasaw_segments::vjp_counters(shape, sizeof(float), want_W) * sizeof(int32_t);
-        if (needed > NO_ALLOC_SCRATCH_BYTES) {
+        if (needed <= NO_ALLOC_SCRATCH_BYTES) {
+            char* const array = static_cast<char*>(no_alloc_scratch_of_current_device());
+            sasaw_segments::vjp<float>(
+                grad_A.data, grad_B.data, grad_W.data, grad_output.data, A.data, B.data, C.data, W.data, indices, shape,
+                array, reinterpret_cast<int32_t*>(array + places), false, stream
+            );
+            finish_call(operation);
+            return;
+        }
+        if (!gathers) {
             throw std::runtime_error(
                 std::string(who) + "these shapes need " + std::to_string(needed) + " bytes of temporary memory, the "
                 "built-in array holds " + std::to_string(NO_ALLOC_SCRATCH_BYTES) + " (about " +
-                std::to_string(NO_ALLOC_SCRATCH_BYTES / 528 - 64) + " nodes); use "
-                "mops_cuda_sparse_accumulation_scatter_add_with_weights_vjp_f32"
+                std::to_string(NO_ALLOC_SCRATCH_BYTES / 528 - 64) + " nodes, and " +
+                std::to_string(NO_ALLOC_SCRATCH_BYTES / 8 - 8192) + " edges where they are put in the order of their "
+                "senders); use mops_cuda_sparse_accumulation_scatter_add_with_weights_vjp_f32"
+                + (want_edges && want_W && mfma && sasaw_mfma::vjp_allocates_nothing(shape, sizeof(float), false, true)
+                       ? ", or ask for grad_W in a call of its own" : "")
             );
         }
-        char* const array = static_cast<char*>(no_alloc_scratch_of_current_device());
-        sasaw_segments::vjp<float>(
-            grad_A.data, grad_B.data, grad_W.data, grad_output.data, A.data, B.data, C.data, W.data, indices, shape,
-            array, reinterpret_cast<int32_t*>(array + places), false, stream
-        );
-        finish_call(operation);
-        return;
+        // (a dense graph of so many edges that their order does not fit: as the shapes below)
     }
-    if (!sasaw_mfma::supports(shape, sizeof(float))) {
+    if (!mfma) {
         throw std::runtime_error(
             std::string(who) + "only the shapes of the matrix-core kernels are served without allocation (at least "
             "one node, edge and table entry; A.shape[1], W.shape[1] and output.shape[1] between 1 and 16); use "

@@ -124,10 +124,14 @@ def test_shapes_beyond_the_built_in_array_are_refused(device):
     [
         # the senders' edges in slots
         dict(E=6000, nA=9, L=32, n_nodes=200),
-        # more than 4000 nodes: listed by arrival, on counters inside the built-in array
+        # more than 4000 nodes, components 4, 4, 4: in slots too
         dict(E=30000, nA=4, L=16, n_nodes=6000, n2=4, n3=4, N=30),
+        # ... and with other components: listed by arrival, on counters inside the built-in array
+        dict(E=30000, nA=4, L=16, n_nodes=6000, n2=3, n3=4, N=30),
+        # a dense graph: the edges put in the order of their senders inside the array
+        dict(E=30000, nA=4, L=16, n_nodes=300, n2=4, n3=4, N=30),
     ],
-    ids=["slots", "by_arrival"],
+    ids=["slots", "many_nodes", "by_arrival", "in_order"],
 )
 def test_captured_into_a_graph_and_free_of_allocations(device, shape):
     """Asynchronous calls inside a stream capture (where an allocation, a stream or event creation
@@ -209,3 +213,27 @@ def test_degenerate_shapes_give_zero_gradients(device):
         for name in ("A", "B", "W"):
             assert torch.equal(got[name], want[name]), (shape, name)
             assert not torch.isnan(got[name]).any()
+
+
+def test_grad_W_alone_of_a_dense_graph_beyond_the_array(oracle, device):
+    """The order of so many edges does not fit the array, but the kernel that reads the whole sender
+    index needs none: grad_W alone is served (the same sums in another order than the existing entry
+    point's: to the float32 bar), all three gradients are refused with a message that says so."""
+    import torch
+
+    from mops_amd._c_lib import device_library
+    from mops_amd.status import MopsError
+
+    library = device_library()
+    support._bind_stream(library, device)
+    host_case = support.sasaw_case(47, np.float32, E=540000, nA=4, L=8, n_nodes=700, n2=4, n3=4, N=24)
+    case = support.to_device(host_case, device)
+    got = gradients_of(library, case, "no_alloc", ("W",))["W"]
+    support.assert_close(got.cpu().numpy(), support.cpu_vjp(oracle, "sasaw", host_case)["W"], np.float32, "grad_W")
+    assert torch.equal(got, gradients_of(library, case, "no_alloc", ("W",))["W"])
+    with pytest.raises(MopsError, match="edges where they are put in the order.*grad_W in a call of its own"):
+        gradients_of(library, case, "no_alloc")
+    without_W = gradients_of(library, case, "no_alloc", ("A", "B"))
+    want = gradients_of(library, case, "existing", ("A", "B"))
+    for name in ("A", "B"):
+        assert torch.equal(without_W[name], want[name]), name
