@@ -30,6 +30,8 @@ CASES = {
     "sasaw_many_columns": lambda d: support.sasaw_case(27, d, E=1500, nA=9, L=160, n_nodes=50, allow_empty=True),
     # more than 4000 nodes: the senders' edges listed by arrival, on counters that every replay must find at zero
     "opsaw_many_senders": lambda d: support.opsaw_case(29, d, E=30000, K=4, L=16, n_nodes=9000, allow_empty=True),
+    # (components that are not all 4, 9 or 16: the others have their edges ordered without counters)
+    "sasaw_many_senders_by_arrival": lambda d: support.sasaw_case(30, d, E=30000, nA=4, L=16, n_nodes=16000, n2=3, n3=4, N=30, allow_empty=True),
     "sasaw_many_senders": lambda d: support.sasaw_case(28, d, E=30000, nA=4, L=16, n_nodes=16000, n2=4, n3=4, N=30, allow_empty=True),
 }
 
@@ -265,7 +267,12 @@ def test_a_block_that_a_graph_names_outlives_a_later_growth(device):
 
 
 @pytest.mark.parametrize(
-    "op,point", [("opsaw_many_senders", "opsaw_vjp_after_listing"), ("sasaw_many_senders", "sasaw_vjp_after_listing")]
+    "op,point",
+    [
+        ("opsaw_many_senders", "opsaw_vjp_after_listing"),
+        ("sasaw_many_senders_by_arrival", "sasaw_vjp_after_listing"),
+        ("sasaw_many_senders", "sasaw_vjp_after_listing"),  # (without counters: nothing is left behind)
+    ],
 )
 def test_a_call_that_fails_between_two_launches_does_not_spoil_the_next(device, monkeypatch, op, point):
     """The senders' edges of large graphs are listed by a launch that counts in counters which the
@@ -288,3 +295,40 @@ def test_a_call_that_fails_between_two_launches_does_not_spoil_the_next(device, 
         torch.cuda.synchronize()
         for got, want in zip(again, good):
             assert torch.equal(got, want), (op, attempt)
+
+
+def test_another_stream_waits_for_a_call_on_the_default_stream(device):
+    """Nothing is recorded behind a call on the default stream; a call on another stream that takes the
+    same scratch block over records there first and waits. Both streams are the library's business
+    alone here: no wait is enqueued by PyTorch, and its streams do not wait for the default one by
+    themselves. The call on the default stream sits behind work that takes some milliseconds."""
+    from mops_amd._c_lib import device_library
+
+    library = device_library()
+    case = support.to_device(CASES["opsaw"](np.float32), device)
+    expected = [t.clone() for t in _call("opsaw", case)]
+    side = torch.cuda.Stream(device=device)
+    busy = torch.randn((4096, 4096), device=device)
+    default = torch.cuda.default_stream(device)
+    assert default.cuda_stream == 0
+    with torch.cuda.stream(side):  # (memory of that stream, so that the call below allocates none)
+        _call("opsaw", case)
+    torch.cuda.synchronize()
+    first = second = None
+    with torch.cuda.stream(default):
+        for _ in range(20):
+            busy = (busy @ busy).clamp(-1.0, 1.0)
+        first = _call("opsaw", case)
+        behind = torch.cuda.Event()
+        behind.record(default)
+    with torch.cuda.stream(side):
+        second = _call("opsaw", case)
+        done = torch.cuda.Event()
+        done.record(side)
+    assert not behind.query(), "the work on the default stream ended before the other call was enqueued"
+    done.synchronize()
+    assert behind.query(), "the call on the other stream did not wait for the one on the default stream"
+    torch.cuda.synchronize()
+    for got, again, want in zip(first, second, expected):
+        assert torch.equal(got, want) and torch.equal(again, want)
+    support._bind_stream(library, device)
