@@ -1059,9 +1059,9 @@ void homogeneous_polynomial_evaluation(MOPS_HPE_PARAMS(MOPS_CXX_FIRST, MOPS_CXX_
         finish_call(operation);
         return;
     }
-    if (const auto plan = hpe_tiles::plan_forward(shape, sizeof(scalar_t));
-        plan.values > 0 && kernels != thresholds::HpeKernels::FEW) {
-        const size_t bytes = hpe_tiles::forward_bytes(shape, plan, sizeof(scalar_t));
+    const auto plan = hpe_tiles::plan_forward(shape, sizeof(scalar_t));
+    const size_t bytes = hpe_tiles::forward_bytes(shape, plan, sizeof(scalar_t));
+    if (plan.values > 0 && kernels != thresholds::HpeKernels::FEW && (bytes == 0 || scratch_ready(bytes))) {
         void* workspace = bytes > 0 ? scratch(bytes) : nullptr;
         auto launch = [&](int32_t* counters) {
             hpe_tiles::forward<scalar_t>(
@@ -1149,7 +1149,8 @@ void homogeneous_polynomial_evaluation_vjp(MOPS_HPE_VJP_PARAMS(MOPS_CXX_FIRST, M
     const size_t accumulator_bytes = (static_cast<size_t>(nA) + 1) * WAVE * sizeof(scalar_t);
     const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
     const auto kernels = thresholds::hpe_vjp(n_rows, nA, static_cast<int64_t>(n_monomials) * order, sizeof(scalar_t));
-    if (kernels == thresholds::HpeKernels::ROWS && hpe_rows::covers_vjp(shape, sizeof(scalar_t))) {
+    if (kernels == thresholds::HpeKernels::ROWS && hpe_rows::covers_vjp(shape, sizeof(scalar_t)) &&
+        scratch_ready(hpe_tiles::table_bytes(shape, sizeof(scalar_t)))) {
         void* workspace = scratch(hpe_tiles::table_bytes(shape, sizeof(scalar_t)));
         hpe_rows::vjp<scalar_t>(
             grad_A.data, grad_output.data, A.data, C.data, indices_A.data, shape, workspace, stream
@@ -1158,8 +1159,10 @@ void homogeneous_polynomial_evaluation_vjp(MOPS_HPE_VJP_PARAMS(MOPS_CXX_FIRST, M
         return;
     }
     const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), false);
-    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET)) {
-        void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), false));
+    const size_t bytes = plan.values > 0 ? hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), false) : 0;
+    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET) &&
+        scratch_ready(bytes)) {
+        void* workspace = scratch(bytes);
         hpe_tiles::vjp<scalar_t>(
             grad_A.data, grad_output.data, A.data, C.data, indices_A.data, shape, plan, workspace, stream
         );
@@ -1291,8 +1294,10 @@ void homogeneous_polynomial_evaluation_vjp_vjp(MOPS_HPE_VJP_VJP_PARAMS(MOPS_CXX_
     const hpe_tiles::Shape shape{n_rows, nA, n_monomials, order};
     const auto kernels = thresholds::hpe_vjp_vjp(n_rows, nA, static_cast<int64_t>(n_monomials) * order, sizeof(scalar_t));
     const auto plan = hpe_tiles::plan_gradient(shape, sizeof(scalar_t), true);
-    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET)) {
-        void* workspace = scratch(hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), true));
+    const size_t bytes = plan.values > 0 ? hpe_tiles::gradient_bytes(shape, plan, sizeof(scalar_t), true) : 0;
+    if (plan.values > 0 && (kernels != thresholds::HpeKernels::FEW || accumulator_bytes > LDS_BUDGET) &&
+        scratch_ready(bytes)) {
+        void* workspace = scratch(bytes);
         ScratchCounters counters;
         hpe_tiles::vjp_vjp<scalar_t>(
             grad_grad_output.data, grad_A_2.data, grad_grad_A.data, grad_output.data, A.data, C.data, indices_A.data,

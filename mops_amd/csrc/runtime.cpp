@@ -362,6 +362,14 @@ void* scratch(size_t bytes) {
     return static_cast<char*>(res.block) + SCRATCH_COUNTERS * sizeof(int32_t);
 }
 
+bool scratch_ready(size_t bytes) {
+    auto& st = state();
+    const Resources& res = st.res();
+    int device = 0;
+    MOPS_HIP_CHECK(hipGetDevice(&device));
+    return (res.block != nullptr && device == res.device && bytes <= res.capacity) || !is_capturing(st.stream);
+}
+
 ScratchCounters::ScratchCounters() : exceptions_(std::uncaught_exceptions()) {
     auto& st = state();
     if (!st.used_scratch || st.resources == nullptr || st.resources->block == nullptr) {

@@ -45,6 +45,10 @@ void finish_call(const char* operation);
 /// share the block at the same time. A thread that ends leaves its block to
 /// the next new thread.
 void* scratch(size_t bytes);
+/// Whether scratch(bytes) gives memory: false only while the thread's stream is being captured and
+/// the thread has no block of that size. For kernels that are the faster ones for a shape which
+/// others serve without scratch memory: a call that is captured first thing must not fail for them.
+bool scratch_ready(size_t bytes);
 /// Bytes of the calling thread's scratch block (0: none yet).
 size_t scratch_capacity();
 

@@ -686,7 +686,8 @@ void sparse_accumulation_of_products(MOPS_SAP_PARAMS(MOPS_CXX_FIRST, MOPS_CXX_NE
     }
     hipStream_t stream = current_stream();
     const sap_mfma::Shape dense_shape{n_rows, nA, nB, nO, n_products};
-    if (sap_rows::chosen_forward(dense_shape, sizeof(scalar_t))) {
+    if (sap_rows::chosen_forward(dense_shape, sizeof(scalar_t)) &&
+        scratch_ready(sap_rows::scratch_bytes(dense_shape, sizeof(scalar_t)))) {
         const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
         sap_rows::forward<scalar_t>(output.data, A.data, B.data, nullptr, nullptr, dense_table, dense_shape, stream);
         finish_call(operation);
@@ -772,7 +773,8 @@ void sparse_accumulation_of_products_vjp(MOPS_SAP_VJP_PARAMS(MOPS_CXX_FIRST, MOP
     }
     hipStream_t stream = current_stream();
     const sap_mfma::Shape dense_shape{n_rows, nA, nB, nO, n_products};
-    if (sap_rows::chosen_vjp(dense_shape, sizeof(scalar_t))) {
+    if (sap_rows::chosen_vjp(dense_shape, sizeof(scalar_t)) &&
+        scratch_ready(sap_rows::scratch_bytes(dense_shape, sizeof(scalar_t)))) {
         const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
         sap_rows::vjp<scalar_t>(
             grad_A.data, grad_B.data, grad_output.data, A.data, B.data, dense_table, dense_shape, stream
@@ -865,7 +867,8 @@ void sparse_accumulation_of_products_vjp_vjp(MOPS_SAP_VJP_VJP_PARAMS(MOPS_CXX_FI
             narrow_i32(B.shape[1], "B.shape[1]"), narrow_i32(grad_output.shape[1], "grad_output.shape[1]"),
             narrow_i32(C.shape[0], "C.shape[0]")};
         const sap_mfma::Table dense_table{C.data, indices_A.data, indices_B.data, indices_output.data};
-        if (have_A && have_B && output_count > 0 && sap_rows::chosen_forward_of_two_pairs(dense_shape, sizeof(scalar_t))) {
+        if (have_A && have_B && output_count > 0 && sap_rows::chosen_forward_of_two_pairs(dense_shape, sizeof(scalar_t)) &&
+            scratch_ready(sap_rows::scratch_bytes(dense_shape, sizeof(scalar_t)))) {
             sap_rows::forward<scalar_t>(
                 grad_grad_output.data, grad_grad_A.data, B.data, A.data, grad_grad_B.data, dense_table, dense_shape, stream
             );

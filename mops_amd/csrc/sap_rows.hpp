@@ -84,6 +84,14 @@ inline bool chosen_forward_of_two_pairs(const Shape& s, size_t element_size) {
            (covers(s) && sap_mfma::supports_forward(s, element_size) && s.n_rows >= thresholds::SAP_ROWS_VJP);
 }
 
+/// Scratch memory of a call: M, and a row that is only asked for.
+inline size_t scratch_bytes(const Shape& s, size_t element_size) {
+    const Tiles tiles = tiles_of(s.nO, element_size);
+    const bool A_inside = inner_is_A(s);
+    const size_t cells = static_cast<size_t>(padded(A_inside ? s.nA : s.nB)) * tiles.columns;
+    return (static_cast<size_t>(tiles.count) * (A_inside ? s.nB : s.nA) * cells + tiles.columns) * element_size;
+}
+
 /// output = sap(A, B), or sap(A, B) + sap(A2, B2) when A2 is not null.
 template <typename T>
 void forward(

@@ -560,7 +560,7 @@ Arguments<T> prepare(const Table& table, const Shape& s, bool A_inside, int32_t 
     p.last_tile_columns = Columns::make(s.nO - (tiles.count - 1) * tiles.columns);
     const size_t cells = static_cast<size_t>(inner_pad) * tiles.columns;
     const size_t blocks = static_cast<size_t>(tiles.count) * p.n_outer;
-    T* dense = static_cast<T*>(scratch((blocks * cells + tiles.columns) * sizeof(T))); // (and a row that is only asked for)
+    T* dense = static_cast<T*>(scratch(scratch_bytes(s, sizeof(T))));
     p.dense = dense;
     p.touched = static_cast<int32_t>(blocks * cells * sizeof(T));
     const size_t lds = cells * (sizeof(T) + sizeof(int32_t));

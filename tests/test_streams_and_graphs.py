@@ -332,3 +332,84 @@ def test_another_stream_waits_for_a_call_on_the_default_stream(device):
     for got, again, want in zip(first, second, expected):
         assert torch.equal(got, want) and torch.equal(again, want)
     support._bind_stream(library, device)
+
+
+FIRST_CALLS_CAPTURED = """
+import ctypes, sys
+import numpy as np
+import torch
+from tests import support
+from mops_amd._c_lib import device_library
+
+device = torch.device("cuda:0")
+library = device_library()
+library.cdll.mops_amd_scratch_capacity.restype = ctypes.c_int64
+hpe, sap = support.hpe_case, support.sap_case
+CASES = {  # shapes whose kernels need scratch memory; others serve them without
+    "hpe_shares_of_the_monomials": (0, "hpe", np.float32, hpe(1, np.float32, I=100, nA=20, J=2100, K=1)),
+    "hpe_long_table": (0, "hpe", np.float64, hpe(2, np.float64, I=700, nA=30, J=20000, K=3)),
+    "hpe_gradients": (1, "hpe", np.float32, hpe(3, np.float32, I=1200, nA=40, J=3000, K=3)),
+    "hpe_gradients_by_rows": (1, "hpe", np.float64, hpe(4, np.float64, I=10001, nA=12, J=50, K=3)),
+    "hpe_second": (2, "hpe", np.float64, hpe(5, np.float64, I=1700, nA=40, J=5000, K=3)),
+    "sap_forward": (0, "sap", np.float64, sap(6, np.float64, I=300001, nA=13, nB=7, K=900, nO=20)),
+    "sap_gradients": (1, "sap", np.float32, sap(7, np.float32, I=100001, nA=13, nB=7, K=900, nO=20)),
+}
+
+def call(level, op, case):
+    library.cdll.mops_amd_set_stream(ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream))
+    library.cdll.mops_amd_set_synchronous(0)
+    spec = support.OPS[op]
+    inputs = [case[name] for name in spec.inputs]
+    if level == 0:
+        shape = (case["A"].shape[0],) + ((case["output_size"],) if "output_size" in case else ())
+        outputs = {"output": torch.full(shape, float("nan"), dtype=case["A"].dtype, device=device)}
+        library.call(spec.function, outputs["output"], *inputs)
+    elif level == 1:
+        outputs = {name: torch.full_like(case[name], float("nan")) for name in spec.differentiable}
+        library.call(spec.function + "_vjp", *outputs.values(), case["grad_output"], *inputs)
+    else:
+        outputs, arguments = support._vjp_vjp_arguments(spec, case, None, None, lambda x: torch.full_like(x, float("nan")))
+        library.call(spec.function + "_vjp_vjp", *arguments)
+    return outputs
+
+stream = torch.cuda.Stream(device=device)
+on_device = {
+    name: support.to_device(support.add_cotangents(case, op) if level == 2 else case, device)
+    for name, (level, op, _, case) in CASES.items()
+}
+torch.cuda.synchronize()
+captured = {}
+for name, (level, op, dtype, _) in CASES.items():
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        captured[name] = graph, call(level, op, on_device[name])
+    assert library.cdll.mops_amd_scratch_capacity() == 0, name
+torch.cuda.synchronize()
+for name, (level, op, dtype, _) in CASES.items():
+    graph, got = captured[name]
+    with torch.cuda.stream(stream):
+        want = call(level, op, on_device[name])  # (eager: with scratch memory)
+        stream.synchronize()
+        for replay in range(2):
+            for tensor in got.values():
+                tensor.fill_(float("nan"))
+            graph.replay()
+            stream.synchronize()
+            for key in want:
+                support.assert_close(got[key].cpu().numpy(), want[key].cpu().numpy(), dtype, f"{name} {key}")
+    print("ok", name, flush=True)
+assert library.cdll.mops_amd_scratch_capacity() > 0
+"""
+
+
+def test_calls_captured_before_any_eager_call(device):
+    """A thread that has no scratch memory yet and whose stream is being captured gets none: shapes that
+    have kernels without scratch memory take those. In a process of its own, where nothing ran before."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    done = subprocess.run([sys.executable, "-c", FIRST_CALLS_CAPTURED], cwd=root, capture_output=True, text=True, timeout=100)
+    assert done.returncode == 0, done.stdout + done.stderr[-3000:]
+    assert done.stdout.count("ok ") == 7, done.stdout
