@@ -2,10 +2,12 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--extra-shapes] [--no-per-op]
 
-Prints ONE JSON line. One "step" is the forward pass followed by the vjp of
-ALL eight operation x dtype combinations of the BASELINE configurations
-(configs[0] HPE f64; configs[1] SAP f32, f64; configs[2] OPSA f32, f64;
-configs[3] OPSAW f32; configs[4] SASAW f32, f64): sixteen calls. ``value`` is
+Prints ONE JSON line, short enough (a few kilobytes) for whoever reads it through a limited buffer: the
+rows per call hold the figures that ``per_op_columns`` names; ``--details FILE`` writes them in full, as
+described below. One "step" is the forward pass followed by the vjp of
+ALL eight operation x dtype combinations of the headline workload (c0: HPE
+f64; c1: SAP f32, f64; c2: OPSA f32, f64; c3: OPSAW f32; c4: SASAW f32, f64):
+sixteen calls. ``value`` is
 the algorithmic bytes of a step (every input read once, every output written
 once, index tensors included) divided by the wall time per step, inputs
 resident in HBM and rotated over buffer sets of more than 256 MB per operation
@@ -18,7 +20,7 @@ being exactly ``--steps`` steps between two host synchronisations;
 ``ms_per_step`` and ``value`` are the MEDIAN repetition, ``repetitions`` holds
 the minimum, median and maximum.
 
-``per_op`` has one entry per function: the device time of a call (every kernel
+``per_op`` has one entry per function (in full in the details, as every list below): the device time of a call (every kernel
 the call launches; HIP-graph replays between HIP events), the same with the
 same buffers every call (``device_us_same_buffers``), two copy yardsticks timed
 the same way (``copy_spans_us``: a copy kernel that reads and writes exactly
@@ -73,7 +75,7 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "all_ops_baseline_shapes_hbm_traff
 # rocprofv3 prints it (a prefix; {T} = float / double). Used to label the
 # per-kernel figures and to find the kernel in the counter summary.
 MAIN_KERNELS = {
-    ("hpe", "forward"): "hpe_tiles::forward_kernel<{T}, 4, 1>",
+    ("hpe", "forward"): "hpe::forward_ordered_kernel<{T}, 4>",
     ("hpe", "vjp"): "hpe::vjp_ordered_kernel<{T}, 4>",
     ("sap", "forward"): "sap_mfma::forward_kernel<{T}, 2, 2, false, 2>",
     ("sap", "vjp"): "sap_mfma::vjp_kernel<{T}, 5, 2>",
@@ -483,6 +485,15 @@ def largest_divisor(n, limit):
     return 1
 
 
+def call_name(entry):
+    return f"{entry['config']} {entry['op']} {entry['dtype'].replace('float', 'f')} {entry['function']}"
+
+
+def short_row(entry):
+    """An entry of per_op as the line that is printed holds it (see per_op_columns)."""
+    return [call_name(entry), *(entry[key] for key in ("device_us", "bound", "frac", "copy_us", "frac_of_copy"))]
+
+
 def main():
     parser = argparse.ArgumentParser()
     parser.add_argument("--gpus", type=int, default=1)
@@ -504,13 +515,13 @@ def main():
         "calls each, every call followed by the flat copy of the same number of bytes",
     )  # fmt: skip
     parser.add_argument("--repetitions", type=int, default=25, help="how often the region of --steps steps is timed")
+    parser.add_argument("--details", metavar="FILE", help="write the whole rows of every call there (JSON)")
     parser.add_argument("--no-scaled", action="store_true", help="leave per_op_scaled out")
     args = parser.parse_args()
 
     if args.gpus != 1:
         sys.stderr.write(
-            "bench.py measures one GPU: every box of this build has a single MI355X and the five "
-            "operations have no multi-GPU path (they would shard over rows / receivers, one gather and one "
+            "bench.py measures one GPU: the five operations have no multi-GPU path (they would shard over rows / receivers, one gather and one "
             "reduce-scatter of the weights per call). "
             "Run with --gpus 1.\n"
         )
@@ -839,12 +850,19 @@ def main():
         },
         "roofline": roofline,
         "cpu_baseline": cpu_baseline,
-        "roofline_per_op": roofline_per_op,
-        "per_op": per_op,
-        "per_op_scaled": per_op_scaled,
-        "per_op_second_order": per_op_second_order,
+        "per_op_columns": ["call", "device_us", "bound", "frac", "copy_us", "frac_of_copy"],
+        "per_op": [short_row(e) for e in per_op],
+        "per_op_scaled": [short_row(e) for e in per_op_scaled],
+        "per_op_second_order": [[call_name(e), e["device_us"]] for e in per_op_second_order],
         "device": torch.cuda.get_device_name(0),
     }
+    if args.details:
+        rows = {
+            "roofline_per_op": roofline_per_op, "per_op": per_op, "per_op_scaled": per_op_scaled,
+            "per_op_second_order": per_op_second_order,
+        }  # fmt: skip
+        with open(args.details, "w") as file:
+            json.dump({**result, **rows}, file, indent=1)
     print(json.dumps(result))
 
 
