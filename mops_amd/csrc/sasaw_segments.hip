@@ -1453,8 +1453,6 @@ void forward(
     }
 }
 
-/// Whether the persistent gradient kernel serves this vjp: the senders' edges
-/// fit the slots on average (sparse graphs), which grad_W needs.
 /// Whether the senders' edges are listed by arrival (one look at every edge,
 /// an atomic for each) rather than in slots (every 16 senders look at the whole
 /// index, which costs edges x nodes). Measured at 30 edges per node, whole vjp
@@ -1479,21 +1477,24 @@ static bool lists_by_arrival(const Shape& s) {
 /// 9 rows 60 us per launch; in double the 16-tile kernel spills and is four times slower still).
 constexpr int32_t GRADIENT_PART_ROWS = thresholds::SASAW_GRADIENT_PART_ROWS;
 
-/// Whether the vjp is one launch on the whole index ranges. In double, also a shape with at most
-/// 16 values of every index goes in parts when W or grad_output have more than 9 rows: the
-/// 16-tile kernel spills its accumulators, and four launches on 9 and 7 rows take 0.83 of its
-/// time (16 x 16 x 16 components, 64 columns, 60 000 edges: 784 against 950 us).
 /// Whether all three gradients are taken with a lane per column (sasaw_columns.hip).
 static bool vjp_by_columns(const Shape& s, size_t element_size) {
     return sasaw_segments::supports(s, element_size) && sasaw_columns::covers(s.nA, s.n2, s.n3) &&
            sasaw_columns::covers(s.nA, s.n3, s.n2);
 }
 
+/// Whether the vjp is one pass over the whole index ranges: with a lane per column, or one launch of
+/// gradients_kernel. In double, a shape with at most 16 values of every index that is not of the first
+/// kind goes in parts when W or grad_output have more than 9 rows: the 16-tile kernel spills its
+/// accumulators, and four launches on 9 and 7 rows take 0.83 of its time (16 x 16 x 16 components, 64
+/// columns, 60 000 edges: 784 against 950 us).
 static bool vjp_in_one_launch(const Shape& s, size_t element_size) {
     return vjp_by_columns(s, element_size) || (sasaw_segments::supports(s, element_size) &&
            !(element_size == 8 && std::max(s.n2, s.n3) > GRADIENT_PART_ROWS));
 }
 
+/// Whether the kernels here or those of sasaw_columns.hip serve this vjp. grad_W of gradients_kernel
+/// needs the senders' edges to fit their places on average.
 bool vjp_supported(const Shape& s, size_t element_size, bool want_grad_W) {
     if (vjp_by_columns(s, element_size)) {
         return true;
