@@ -99,11 +99,11 @@ constexpr int64_t SAP_VJP_WALK_TILES_PER_WAVE = 2;
 
 /// Rows from which a lane per row (sap_rows.hip) takes the vjp, and the forward pass of two pairs; half
 /// as many in double where the table fits the scalar cache. vjp, matrix cores / a lane per row, us: nA, nB,
-/// nO = 13, 7, 20, 120 000 rows 28.9 / 23.6 (f32), 53.1 / 33.4 (f64), 60 000 rows 16.4 / 19.2, 28.1 / 24.1;
-/// 5, 4, 12, 120 000 rows 15.6 / 12.1, 22.9 / 15.0; a million rows of 13, 7, 20: 148 / 90, 280 / 129.
+/// nO = 13, 7, 20, 120 000 rows 26.4 / 22.0 (f32), 50.0 / 30.5 (f64), 60 000 rows 16.4 / 19.2, 28.1 / 24.1;
+/// 5, 4, 12, 120 000 rows 15.6 / 12.1, 22.9 / 15.0; a million rows of 13, 7, 20: 133 / 83, 272 / 133.
 constexpr int32_t SAP_ROWS_VJP = 100000;
 /// The same for the forward pass, which the matrix cores pad less: 13, 7, 20 in double, 250 000 rows 39.8 /
-/// 42.1, 500 000 68.7 / 62.5, a million 130 / 110; 16, 16, 8: 250 000 48.7 / 41.1, 500 000 86 / 61.
+/// 42.1, 500 000 64.5 / 58.6, a million 132 / 113; 16, 16, 8: 250 000 48.7 / 41.1, 500 000 86 / 61.
 constexpr int32_t SAP_ROWS_FORWARD = 300000;
 /// ... and for shapes that the matrix cores do not take (more than 64 columns, a table larger than the LDS).
 /// 4, 9, 90 with 1500 entries, forward, 30 000 rows 26.9 / 30.3, 60 000 42.2 / 31.2, 250 000 152 / 60 (f32),

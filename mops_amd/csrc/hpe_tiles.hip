@@ -19,8 +19,8 @@
 // shared counters: a stable counting sort (8 us for 400 000 factors).
 //
 // 1000 rows, 2000 features, 100 000 monomials of order 4, whole calls: forward
-// 97 -> 39 us (float), 100 -> 66 (double), of which LDS at 128 bytes per clock
-// and compute unit needs 20 and 41; vjp 8040 -> 124 and 18 500 -> 205 (61 and
+// 91 -> 37 us (float), 98 -> 61 (double), of which LDS at 128 bytes per clock
+// and compute unit needs 20 and 41; vjp 8050 -> 118 and 18 560 -> 207 (61 and
 // 122); second order 1.46 s -> 414 us and 1.54 s -> 816 us, against the kernels
 // that keep the accumulators of a few features, or nothing, in LDS.
 #include <algorithm>

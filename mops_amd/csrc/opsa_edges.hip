@@ -17,8 +17,8 @@
 // asked of a tensor of no bytes.
 //
 // What bounds it on many edges is memory: 1 000 000 edges over 33 000 nodes, 13 x 32,
-// f32, OPSAW, 136 us for 551 MB (4.05 TB/s; 155 us with the operands' layout loaded
-// as it is), OPSA with 13 x 33 202 -> 121 us, 31 x 45 506 -> 202. Few tiles per
+// f32, OPSAW, 134 us for 701 MB at the memory side of L2 (5.2 TB/s; the tensors have
+// 551 MB; 155 us with the operands' layout loaded as it is), OPSA with 13 x 33 202 -> 121 us, 31 x 45 506 -> 202. Few tiles per
 // wavefront (below 30 000 to 400 000 edges, by shape) are the other kernel's: this one
 // has a start of some microseconds and as many wavefronts as are resident at most.
 #include "opsa_edges.hpp"

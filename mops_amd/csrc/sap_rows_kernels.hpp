@@ -26,11 +26,13 @@
 // columns (6 us of the calls below).
 //
 // A million rows of 13, 7 and 20 values, 900 entries, whole calls, matrix cores ->
-// this: vjp 277 -> 129 us in double, 148 -> 90 in float; second order 606 -> 277
-// and 338 -> 178; forward pass in double 130 -> 110. The vector units are busy for
-// three quarters of that (counters; 98 rows of M, 20 multiply-adds each and 15 % of
-// other work); rows in and out alone would take 101 us (vjp, double) and 67
-// (forward) at the rate of a large copy.
+// this, the same buffers every call: vjp 272 -> 133 us in double, 133 -> 83 in
+// float; second order 606 -> 277 and 338 -> 178; forward pass in double 132 -> 113.
+// Vector instructions occupy 0.77 (vjp, float), 0.55 (vjp, double) and 0.62
+// (forward, double) of the SIMDs' clocks at 2.4 GHz in these kernels (98 rows of M,
+// 20 multiply-adds each and 15 % of other work) and memory moves at 2.7 to 3.6
+// TB/s; rows in and out alone would take 109 us (vjp, double) and 73 (forward) at
+// the rate of a large copy.
 #include "sap_rows.hpp"
 
 #include <algorithm>

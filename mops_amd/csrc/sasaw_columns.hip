@@ -32,11 +32,13 @@
 // m2 and m3 exchanged.
 //
 // Whole calls against one per-node sum on the matrix cores each, 9 components, 32
-// columns, f32 / f64, us: 1 000 000 edges, forward 316 -> 199 / 390 -> 386, vjp
-// 1160 -> 530 / 1360 -> 950; 60 000 edges, 21.5 -> 20.3 / 30 -> 27 and 60 -> 56 /
-// 99 -> 74; 128 columns there, vjp 247 -> 121 / 360 -> 223. At a million edges the
-// forward pass in float gathers 1.15 GB of rows at 6.8 TB/s with everything else
-// it reads, which is what the Infinity Cache gives for rows in no order.
+// columns, the same buffers every call, f32 / f64, us: 1 000 000 edges, forward 315
+// -> 202 / 391 -> 377, vjp 1184 -> 521 / 1397 -> 926; 60 000 edges, 20.2 -> 20.2 /
+// 29.2 -> 24.5 and 58.5 -> 54.7 / 99 -> 71.5; 128 columns there, vjp 247 -> 121 / 360
+// -> 223; 600 edges, 12.6 -> 10.3 / 14.0 -> 11.5 and 25.1 -> 27.0 / 31.7 -> 29.5. At a
+// million edges 1.3 GB (float; 2.6 in double) come through the memory side of L2 in
+// the forward pass, rows of W in no order for the most part, at 6.2 (7.1) TB/s, 1.6
+// (3.0) GB at 7.0 (7.4) for grad_W: what the Infinity Cache gives for such rows.
 //
 // Every sum has one fixed order; no atomics on floating point.
 #include "sasaw_columns.hpp"
