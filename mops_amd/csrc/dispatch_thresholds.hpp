@@ -34,13 +34,13 @@ inline HpeKernels hpe_forward(int64_t rows, int64_t features, int64_t factors, i
     const int64_t row_bytes = features * element_size;
     const bool single = element_size == 4;
     const int64_t rows_factors =
-        (single ? (rows / 10 < 5000 ? rows / 10 : 5000) : (rows * 3 / 20 < 3000 ? rows * 3 / 20 : 3000)) + 2 * row_bytes;
+        (single ? (rows / 12 < 5000 ? rows / 12 : 5000) : (rows * 3 / 20 < 3000 ? rows * 3 / 20 : 3000)) + 2 * row_bytes;
     if (rows >= 10000 && row_bytes <= (single ? 850 : 2100) && factors <= rows_factors) {
         return HpeKernels::ROWS;
     }
     bool few;
     if (rows < 3000) {
-        few = rows * factors <= 30 * 1000 * 1000 &&
+        few = rows * factors <= 30 * 1000 * 1000 && (row_bytes >= 200 || 6 * rows < factors) &&
               (factors >= (single && row_bytes > 2500 ? row_bytes : 2500) || (!single && row_bytes >= 400));
     } else if (single) {
         few = row_bytes >= 300 && row_bytes <= 1000 && factors <= 1000;
@@ -81,8 +81,9 @@ inline HpeKernels hpe_vjp(int64_t rows, int64_t features, int64_t factors, int64
 /// 165 / 26.7, 900: 121 / 77, 200 / 100; 100 000 x 30, 900: 143 / 131, 225 / 157;
 /// 100 000 x 100, 300: 123 / 110, 600: 132 / 160; 1000 x 100, 8000, f64 45 / 17.
 inline HpeKernels hpe_vjp_vjp(int64_t rows, int64_t features, int64_t factors, int64_t element_size) {
-    const bool few = rows * factors < (element_size == 4 ? 16 : 24) * int64_t(1000 * 1000) ||
-                     (rows >= 10000 && factors < 1500 - 10 * features);
+    const bool narrow = element_size == 4 && features <= 16 && rows < 30000;
+    const int64_t millions = narrow ? 11 : element_size == 4 ? 16 : 24;
+    const bool few = rows * factors < millions * 1000 * 1000 || (!narrow && rows >= 10000 && factors < 1500 - 10 * features);
     return few ? HpeKernels::FEW : HpeKernels::TILES;
 }
 

@@ -19,10 +19,11 @@ SHAPES = [  # rows, features, monomials, order
     (10000, 1, 1, 1),
     (10049, 10, 50, 3),
     (10111, 16, 65, 2),
-    (10240, 4, 300, 3),
+    (11240, 4, 300, 3),
     (12801, 33, 100, 2),
     (13000, 30, 150, 4),
     (14001, 20, 31, 6),
+    (16001, 33, 330, 2),
     (16447, 7, 129, 5),
     (18001, 100, 200, 3),
     (20000, 119, 70, 2),
