@@ -33,12 +33,12 @@
 //
 // Whole calls against one per-node sum on the matrix cores each, 9 components, 32
 // columns, the same buffers every call, f32 / f64, us: 1 000 000 edges, forward 315
-// -> 202 / 391 -> 377, vjp 1184 -> 521 / 1397 -> 926; 60 000 edges, 20.2 -> 20.2 /
-// 29.2 -> 24.5 and 58.5 -> 54.7 / 99 -> 71.5; 128 columns there, vjp 247 -> 121 / 360
-// -> 223; 600 edges, 12.6 -> 10.3 / 14.0 -> 11.5 and 25.1 -> 27.0 / 31.7 -> 29.5. At a
+// -> 200 / 391 -> 366, vjp 1184 -> 507 / 1397 -> 895; 60 000 edges, 20.2 -> 19.6 /
+// 29.2 -> 25.1 and 58.5 -> 54 / 99 -> 69; 128 columns there, vjp 247 -> 114 / 360
+// -> 223; 600 edges, 12.6 -> 7.5 / 14.0 -> 8.5 and 25.1 -> 24.0 / 31.7 -> 26.6. At a
 // million edges 1.3 GB (float; 2.6 in double) come through the memory side of L2 in
-// the forward pass, rows of W in no order for the most part, at 6.2 (7.1) TB/s, 1.6
-// (3.0) GB at 7.0 (7.4) for grad_W: what the Infinity Cache gives for such rows.
+// the forward pass, rows of W in no order for the most part, at 6.4 (7.1) TB/s: the
+// same loads with nothing done to what they bring take 175 of the 200 us.
 //
 // Every sum has one fixed order; no atomics on floating point.
 #include "sasaw_columns.hpp"
@@ -241,7 +241,7 @@ template <typename T> struct Walk {
     const T* C;    // [entries]
     int32_t n_edges, n_blocks, L;
     int32_t column_tiles;
-    int32_t ranges; // of nodes, a wavefront each (and tile)
+    int32_t ranges; // of nodes or edges, a wavefront each (and tile)
     const int32_t* sorted; // [n_edges] node of every position, non-decreasing
     const int32_t* gather; // [n_edges] block of `rows` of every edge
     Dense table;
@@ -444,6 +444,16 @@ template <typename T> struct ContractWindow<T, ORDERED> {
     __device__ __forceinline__ int32_t edge(int32_t, int32_t k) const { return __builtin_amdgcn_readlane(listed, k); }
 };
 
+/// Where the edges of a node begin.
+template <typename T, Lists LISTS>
+__device__ __forceinline__ int32_t begin_of_node(const ContractArgs<T>& args, int32_t node, int lane) {
+    if constexpr (LISTS == ORDERED) {
+        return args.ordered.offsets[node];
+    } else {
+        return lower_bound(args.walk.sorted, args.walk.n_edges, node, lane);
+    }
+}
+
 /// Rows of A in scalar registers at once, where they fit without others being moved out of the way:
 /// 1 000 000 edges, 32 columns, 4 components, f32 / f64, 94.9 -> 92.7 / 198 -> 188 us, sums over
 /// senders 180 -> 170 / 273 -> 264; 9 in double 386 -> 371; 9 in float is slower by it.
@@ -461,7 +471,13 @@ template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
            std::max(table_slots<N, COLUMNS, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
 }
 
-template <typename T, int N, int COLUMNS, Lists LISTS>
+/// SHARED: a workgroup has one node, whose edges its wavefronts share; else every wavefront has a range of
+/// nodes. Bound by the rows it gathers (many edges), by the chain of a node's edges (few). With no more
+/// nodes than workgroups at a time, a node's 30 edges are a chain of eight: 600 edges, 9 components, 32
+/// columns, f32 / f64, 11.3 -> 7.5 / 12.0 -> 8.5 us, 5000 edges 10.6 -> 9.0 / 11.7 -> 10.8. Beyond, the
+/// same share-out of a range of nodes costs a table and a wait more for each share: 60 000 edges 19.3 -> 20.5.
+/// (Ranges of equal edges instead of equal nodes: within 3 % either way from 100 000 to 1 000 000 edges.)
+template <typename T, int N, int COLUMNS, Lists LISTS, bool SHARED>
 __global__ __launch_bounds__(THREADS)
 __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contract_kernel(const ContractArgs<T> args) {
     using M = Mfma<T>;
@@ -484,7 +500,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
     }
     wave_sync();
 
-    const int32_t unit = blockIdx.x * WAVES + wave;
+    const int32_t unit = SHARED ? blockIdx.x : blockIdx.x * WAVES + wave;
     const int32_t tile = unit % p.column_tiles, range = unit / p.column_tiles;
     if (range >= p.ranges) {
         return;
@@ -541,6 +557,27 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
             }
             wave_sync();
         }
+        if constexpr (SHARED) { // the sum over the wavefronts, in their order, by the first
+            constexpr int VALUES = 4 * (COLUMNS / 16);
+            static_assert(VALUES * WAVE <= STAGE, "a result fits a stage");
+            if (wave > 0) {
+#pragma unroll
+                for (int k = 0; k < VALUES; k++) {
+                    stage[k * WAVE + lane] = acc[k / 4][k % 4];
+                }
+            }
+            __syncthreads();
+            if (wave > 0) {
+                return;
+            }
+#pragma unroll
+            for (int other = 1; other < WAVES; other++) {
+#pragma unroll
+                for (int k = 0; k < VALUES; k++) {
+                    acc[k / 4][k % 4] += stages[other * STAGE + k * WAVE + lane];
+                }
+            }
+        }
         T* target = args.result + static_cast<size_t>(node) * p.table.n_out * p.L;
 #pragma unroll
         for (int t = 0; t < COLUMNS / 16; t++) {
@@ -564,14 +601,19 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
     };
 
     if constexpr (LISTS != SLOTS) {
-        int32_t at = LISTS == SEGMENTS ? lower_bound(p.sorted, p.n_edges, node0, lane) : args.ordered.offsets[node0];
+        int32_t at = begin_of_node<T, LISTS>(args, node0, lane), to = INT32_MAX;
+        if constexpr (SHARED) { // the wavefront's quarter of the node's edges
+            const int32_t first = at, n = begin_of_node<T, LISTS>(args, node0 + 1, lane) - first;
+            at = first + static_cast<int32_t>(static_cast<int64_t>(n) * wave / WAVES);
+            to = first + static_cast<int32_t>(static_cast<int64_t>(n) * (wave + 1) / WAVES);
+        }
         // positions at .. at + 64 of the index or of the lists, and the blocks of their edges
         ContractWindow<T, LISTS> window(args, at, lane);
         for (int32_t node = node0; node < node1; node++) {
             clear();
             int32_t n;
             do {
-                n = window.edges_of(args, node, at);
+                n = SHARED ? min(WAVE, to - at) : window.edges_of(args, node, at);
                 const ContractWindow<T, LISTS> next(args, at + n, lane);
                 if (n > 0) {
                     columns_of.template over<ROWS_OF_A>(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, add);
@@ -613,13 +655,25 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
                 first_half = edge_at(lane);
                 second_half = count > WAVE ? edge_at(lane + WAVE) : 0;
             }
-            if (listed) {
+            if (listed && SHARED) {
+                // (at most 32 of the 128 places)
+                const int32_t from = count * wave / WAVES, n = count * (wave + 1) / WAVES - from;
+                const int32_t place = from + lane;
+                const int32_t low = __shfl(first_half, place & (WAVE - 1)), high = __shfl(second_half, place & (WAVE - 1));
+                if (n > 0) {
+                    hand_on(lane < n ? (place < WAVE ? low : high) : 0, n);
+                }
+            } else if (listed) {
                 if (count > 0) {
                     hand_on(lane < count ? first_half : 0, min(count, WAVE));
                 }
                 if (count > WAVE) {
                     hand_on(lane + WAVE < count ? second_half : 0, count - WAVE);
                 }
+            } else if (SHARED) {
+                const int32_t share = (p.n_edges + WAVES - 1) / WAVES;
+                const int32_t begin = min(wave * share, p.n_edges);
+                edges_of_sender<4>(args.senders, p.n_edges, begin, min(begin + share, p.n_edges), node, lane, hand_on);
             } else {
                 // more edges than places (a hub of a sparse graph): this wavefront reads the index itself
                 // (3000 nodes of 30 edges, one of them of 300, f32, whole vjp 250 us; a load at a time 674; without it 71)
@@ -636,7 +690,7 @@ template <typename T> struct EdgeArgs {
     const T* grad_output; // [n_nodes][n_out][L]
     T* grad_A;            // [n_edges][nA], may be null
     T* grad_B;            // [n_edges][L], may be null
-    int32_t shares;       // wavefronts per range, each with a share of a node's edges
+    int32_t shares;       // wavefronts per node, each with a share of its edges (0: a share of all edges)
 };
 
 /// Wavefronts per SIMD.
@@ -667,13 +721,19 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
     const int lane = columns_of.lane;
     build<T, N, COLUMNS, true>(table, owner, p.C, p.table);
 
-    const int32_t unit = blockIdx.x * WAVES + wave;
-    const int32_t range = unit / args.shares, share = unit % args.shares;
+    const int32_t range = blockIdx.x * WAVES + wave;
     if (range >= p.ranges) {
         return;
     }
-    const int32_t node0 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * range / p.ranges);
-    const int32_t node1 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * (range + 1) / p.ranges);
+    int32_t first = 0, n_all = p.n_edges, share = range, shares = p.ranges;
+    if (args.shares > 0) {
+        share = range % args.shares;
+        shares = args.shares;
+        first = lower_bound(p.sorted, p.n_edges, range / args.shares, lane);
+        n_all = lower_bound(p.sorted, p.n_edges, range / args.shares + 1, lane) - first;
+    }
+    const int32_t begin = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * share / shares);
+    const int32_t end = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * (share + 1) / shares);
     BufferOf<T> G;
     const uint32_t g_block_bytes = static_cast<uint32_t>(p.table.n_out) * columns_of.row_bytes;
     G.set(args.grad_output, static_cast<uint32_t>(p.n_blocks) * g_block_bytes);
@@ -688,7 +748,6 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
     to_A.set(args.grad_A, args.grad_A != nullptr ? static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES : 0);
     to_B.set(args.grad_B, args.grad_B != nullptr ? static_cast<uint32_t>(p.n_edges) * columns_of.row_bytes : 0);
     const T* spread_from = stage + columns_of.part * S::VALUES * PITCH + columns_of.c;
-    const int32_t start = lower_bound(p.sorted, p.n_edges, node0, lane);
 
     for (int32_t tile = 0; tile < p.column_tiles; tile++) {
         columns_of.set_tile(tile);
@@ -697,11 +756,11 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
         const uint32_t b_at = columns_of.column_bytes | unless(columns_of.part == 0 && columns_of.column_inside);
         BufferOf<T> from_A;
         from_A.set(args.grad_A, tile == 0 || args.grad_A == nullptr ? 0 : static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES);
-        int32_t at = start;
+        int32_t at = begin;
         Window<T> window(p, at, lane);
-        for (int32_t node = node0; node < node1; node++) {
+        while (at < end) {
+            const int32_t node = __builtin_amdgcn_readfirstlane(window.receiver);
             T g[N * M2];
-            bool have = false;
             // G = D^T grad_output of the node, MC components of A at a time through LDS
             auto spread = [&] {
                 T upstream[COLUMNS / 16][4];
@@ -801,19 +860,18 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
                     to_A.store(mine + operands.more, a_at, edge * A_ROW_BYTES);
                 };
             };
+            const bool exists = in_bounds(node, p.n_blocks);
+            if (exists) {
+                spread();
+            }
             int32_t n;
             do {
-                n = window.edges_of(node);
+                n = min(window.edges_of(node), end - at);
                 const Window<T> next(p, at + n, lane);
-                const int32_t from = n * share / args.shares, to = n * (share + 1) / args.shares;
-                if (to > from) {
-                    if (!have) {
-                        spread();
-                        have = true;
-                    }
-                    const int32_t first = at + from;
+                if (exists && n > 0) {
+                    const int32_t first = at;
                     columns_of.template over<1>(
-                        __shfl(window.source, min(from + lane, to - 1)), to - from, [&](int32_t k) { return first + k; },
+                        window.source, n, [&](int32_t k) { return first + k; },
                         [&](auto& operands, int32_t k) {
                             operands.more = from_A.load(a_at, static_cast<uint32_t>(first + k) * A_ROW_BYTES);
                         },
@@ -906,12 +964,18 @@ template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Sha
         Walk<T>& w = args.walk;
         constexpr size_t lds = contract_lds<T, N, COLUMNS>();
         w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
-        const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * contract_waves<T, N, COLUMNS>();
-        w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, std::max<int64_t>(1, resident / w.column_tiles)));
-        const size_t units = static_cast<size_t>(w.ranges) * w.column_tiles;
-        auto kernel = contract_kernel<T, N, COLUMNS, LISTS>;
-        allow_lds(kernel, lds);
-        kernel<<<static_cast<unsigned>(ceil_div(units, WAVES)), THREADS, lds, stream>>>(args);
+        const int64_t resident = static_cast<int64_t>(compute_units()) * contract_waves<T, N, COLUMNS>(); // workgroups
+        auto launch = [&](auto kernel, int64_t ranges, int waves_per_range) {
+            w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, std::max<int64_t>(1, ranges)));
+            const size_t waves = static_cast<size_t>(w.ranges) * w.column_tiles * waves_per_range;
+            allow_lds(kernel, lds);
+            kernel<<<static_cast<unsigned>(ceil_div(waves, WAVES)), THREADS, lds, stream>>>(args);
+        };
+        if (static_cast<int64_t>(s.n_nodes) * w.column_tiles <= resident) {
+            launch(contract_kernel<T, N, COLUMNS, LISTS, true>, s.n_nodes, WAVES);
+        } else {
+            launch(contract_kernel<T, N, COLUMNS, LISTS, false>, resident * WAVES / w.column_tiles, 1);
+        }
     });
     MOPS_HIP_CHECK(hipGetLastError());
 }
@@ -974,11 +1038,19 @@ void edge_gradients(
         constexpr size_t lds = edge_lds<T, N, COLUMNS>();
         w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
         const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * edge_waves<T, N, COLUMNS>();
-        w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, resident));
-        // (a node's edges shared out where there are fewer nodes than wavefronts, in shares of four or more)
+        // Every wavefront has as many edges as the next, whatever nodes they are of, and makes G of each
+        // (against a range of nodes each, 9 components, 32 columns, f32 / f64, whole vjp: 60 000 edges of 2000
+        // nodes 74 -> 69 us in double, 200 000 of 6600 134 -> 125 / 212 -> 195; 91 000 of 3000, 16 components,
+        // 64 columns, 239 -> 219 / 464 -> 398). Where two wavefronts or more share a node, with four edges each
+        // at least, that is only more of G (600 edges of 20 nodes 24.0 -> 24.8; for 16 components in float, of
+        // which G is the most work, also with one: 50 000 of 2000 85.2 -> 87.1).
         const int64_t shares = std::min<int64_t>(s.n_edges / (4 * static_cast<int64_t>(s.n_nodes)), resident / s.n_nodes);
-        args.shares = static_cast<int32_t>(std::max<int64_t>(1, shares));
-        const size_t units = static_cast<size_t>(w.ranges) * args.shares;
+        const int64_t least = N == 16 && sizeof(T) == 4 ? 1 : 2;
+        args.shares = shares >= least ? static_cast<int32_t>(shares) : 0;
+        w.ranges = static_cast<int32_t>(
+            shares >= least ? s.n_nodes * shares : std::max<int64_t>(1, std::min<int64_t>(s.n_edges / 4, resident))
+        );
+        const size_t units = w.ranges;
         auto kernel = edge_kernel<T, N, COLUMNS>;
         allow_lds(kernel, lds);
         kernel<<<static_cast<unsigned>(ceil_div(units, WAVES)), THREADS, lds, stream>>>(args);

@@ -58,6 +58,43 @@ def test_against_the_oracle(oracle, device, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize(
+    "shape",
+    [  # edges, nodes, components, columns: a node by a workgroup (up to 512 to 1024 nodes), a range of them by a wavefront
+        (7, 3, 9, 32),
+        (700, 3, 9, 33),
+        (5000, 2, 4, 20),
+        (1100, 512, 16, 16),
+        (1030, 1024, 4, 16),
+        (1030, 1025, 4, 16),
+        (9000, 4500, 9, 40),
+        (9000, 4500, 16, 24),
+    ],
+    ids=lambda s: "x".join(map(str, s)),
+)
+def test_one_node_has_a_third_of_the_edges(oracle, device, shape, dtype):
+    """The edges of one node go to several wavefronts, those of many small ones to one."""
+    edges, nodes, n, columns = shape
+    case = support.sasaw_case(
+        sum(shape), dtype, E=edges, nA=n, L=columns, n_nodes=nodes, n2=n, n3=n, N=100, allow_empty=True
+    )
+    receivers = np.random.default_rng(sum(shape)).integers(0, nodes, edges)
+    receivers[: edges // 3] = nodes // 2
+    receivers.sort()
+    case["indices_output_1"] = receivers.astype(np.int32)
+    exact, absolute, on_device = support.in_float64(case), support.magnitudes(case), to_device(case, device)
+    other = case if dtype == np.float32 else absolute
+
+    def check(name, run, actual):
+        same, terms = (run(other), None) if dtype == np.float32 else (None, run(other))
+        support.assert_calibrated(actual.cpu().numpy(), run(exact), dtype, f"{shape} {name}", same, terms)
+
+    check("output", lambda c: cpu_forward(oracle, "sasaw", c), hip_forward("sasaw", on_device))
+    for key, gradient in hip_vjp("sasaw", on_device).items():
+        check(f"grad_{key}", lambda c: cpu_vjp(oracle, "sasaw", c)[key], gradient)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_senders_outside_the_tensor_count_as_zero(oracle, device, dtype):
     case = support.sasaw_case(7, dtype, E=300, nA=9, L=20, n_nodes=12, n2=9, n3=9, N=120)
     lost = np.random.default_rng(1).integers(0, 300, 40)
