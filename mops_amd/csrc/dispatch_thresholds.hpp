@@ -140,6 +140,12 @@ constexpr size_t SENDER_SCAN_LIMIT = 100u * 1000 * 1000;
 /// reading the whole index). OPSAW, 60 000 edges over 2000 senders, L = 32,
 /// f32: 33 -> 22 us for the whole vjp.
 constexpr int32_t SLOT_MEAN_EDGES = 48;
+/// Edges up to which SASAW's gradients with a lane per column are one launch, where every node's workgroup
+/// looks through the whole index of senders (with up to two nodes and 32 columns per compute unit). 9
+/// components, 32 columns, that / a launch that lists the edges and one for each kind of gradient, f32, f64:
+/// 600 edges of 20 nodes 11.8 / 24.0, 12.8 / 26.6 us; 8000 of 260 15.4 / 29, 26.7 / 33; 8000 of 700 22.5 / 28,
+/// 36.1 / 34.5; 16 000 of 500 27.6 / 34, 36.0 / 38.5 (4 components, 100 columns 30.8 / 35.0, 45.3 / 43.0).
+constexpr int32_t COLUMNS_EDGES_AS_THEY_ARE = 8192;
 /// Edges per sender on average up to which lists are made by arrival (128 places
 /// per sender). SASAW, 1000 nodes x 60 edges, whole vjp 87.6 -> 76.6 us (f32), 143.8
 /// -> 115.3 (f64) against the kernels of sasaw_mfma.hip; at 100 per sender the

@@ -35,7 +35,7 @@
 // columns, the same buffers every call, f32 / f64, us: 1 000 000 edges, forward 315
 // -> 200 / 391 -> 366, vjp 1184 -> 507 / 1397 -> 895; 60 000 edges, 20.2 -> 19.6 /
 // 29.2 -> 25.1 and 58.5 -> 54 / 99 -> 69; 128 columns there, vjp 247 -> 114 / 360
-// -> 223; 600 edges, 12.6 -> 7.5 / 14.0 -> 8.5 and 25.1 -> 24.0 / 31.7 -> 26.6. At a
+// -> 223; 600 edges, 12.6 -> 7.5 / 14.0 -> 8.5 and 25.1 -> 11.8 / 31.7 -> 12.8. At a
 // million edges 1.3 GB (float; 2.6 in double) come through the memory side of L2 in
 // the forward pass, rows of W in no order for the most part, at 6.4 (7.1) TB/s: the
 // same loads with nothing done to what they bring take 175 of the 200 us.
@@ -478,14 +478,12 @@ template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
 /// same share-out of a range of nodes costs a table and a wait more for each share: 60 000 edges 19.3 -> 20.5.
 /// (Ranges of equal edges instead of equal nodes: within 3 % either way from 100 000 to 1 000 000 edges.)
 template <typename T, int N, int COLUMNS, Lists LISTS, bool SHARED>
-__global__ __launch_bounds__(THREADS)
-__attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contract_kernel(const ContractArgs<T> args) {
+__device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds, const int32_t block) {
     using M = Mfma<T>;
     using S = Sums<N, COLUMNS>;
     constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::STEPS * 4 * PITCH;
     constexpr int ROWS_OF_A = contract_rows_of_A<T, N>();
     const Walk<T>& p = args.walk;
-    extern __shared__ __align__(16) char lds[];
     T* table = reinterpret_cast<T*>(lds);
     T* stages = table + table_slots<N, COLUMNS, false>();
     int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
@@ -500,7 +498,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
     }
     wave_sync();
 
-    const int32_t unit = SHARED ? blockIdx.x : blockIdx.x * WAVES + wave;
+    const int32_t unit = SHARED ? block : block * WAVES + wave;
     const int32_t tile = unit % p.column_tiles, range = unit / p.column_tiles;
     if (range >= p.ranges) {
         return;
@@ -632,6 +630,17 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
                     sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, add
                 );
             };
+            auto look_through_index = [&] {
+                const int32_t share = (p.n_edges + WAVES - 1) / WAVES, begin = min(wave * share, p.n_edges);
+                edges_of_sender<4>(args.senders, p.n_edges, begin, min(begin + share, p.n_edges), node, lane, hand_on);
+            };
+            if constexpr (SHARED) {
+                if (args.slots.edges == nullptr) { // a short index: its quarters looked at as they are
+                    look_through_index();
+                    finish(node);
+                    continue;
+                }
+            }
             const int32_t* places = args.slots.edges + static_cast<size_t>(node) * SLOT_CAPACITY;
             int32_t first_half = places[lane], second_half = places[lane + WAVE];
             static_assert(SLOT_PARTS == 4 && SLOT_CAPACITY == 2 * WAVE, "four parts of a node's places in two registers");
@@ -671,9 +680,7 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
                     hand_on(lane + WAVE < count ? second_half : 0, count - WAVE);
                 }
             } else if (SHARED) {
-                const int32_t share = (p.n_edges + WAVES - 1) / WAVES;
-                const int32_t begin = min(wave * share, p.n_edges);
-                edges_of_sender<4>(args.senders, p.n_edges, begin, min(begin + share, p.n_edges), node, lane, hand_on);
+                look_through_index();
             } else {
                 // more edges than places (a hub of a sparse graph): this wavefront reads the index itself
                 // (3000 nodes of 30 edges, one of them of 300, f32, whole vjp 250 us; a load at a time 674; without it 71)
@@ -682,6 +689,13 @@ __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contr
             finish(node);
         }
     }
+}
+
+template <typename T, int N, int COLUMNS, Lists LISTS, bool SHARED>
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contract_kernel(const ContractArgs<T> args) {
+    extern __shared__ __align__(16) char lds[];
+    contract<T, N, COLUMNS, LISTS, SHARED>(args, lds, blockIdx.x);
 }
 
 // ---------------------------------------------------------------- gradients --
@@ -704,13 +718,11 @@ template <typename T, int N, int COLUMNS> constexpr size_t edge_lds() {
 }
 
 template <typename T, int N, int COLUMNS>
-__global__ __launch_bounds__(THREADS)
-__attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kernel(const EdgeArgs<T> args) {
+__device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* lds, const int32_t block) {
     using M = Mfma<T>;
     using S = Sums<N, COLUMNS>;
     constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::TILES * 16 * PITCH;
     const Walk<T>& p = args.walk;
-    extern __shared__ __align__(16) char lds[];
     T* table = reinterpret_cast<T*>(lds);
     T* stages = table + table_slots<N, COLUMNS, true>();
     int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
@@ -721,7 +733,7 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
     const int lane = columns_of.lane;
     build<T, N, COLUMNS, true>(table, owner, p.C, p.table);
 
-    const int32_t range = blockIdx.x * WAVES + wave;
+    const int32_t range = block * WAVES + wave;
     if (range >= p.ranges) {
         return;
     }
@@ -885,6 +897,30 @@ __attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kern
     }
 }
 
+template <typename T, int N, int COLUMNS>
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kernel(const EdgeArgs<T> args) {
+    extern __shared__ __align__(16) char lds[];
+    edge_gradients<T, N, COLUMNS>(args, lds, blockIdx.x);
+}
+
+/// All gradients of a small graph in one launch: the first `nodes` workgroups have a node and a tile of
+/// columns of grad_W each, and look through the index for its edges themselves; the others grad_A and grad_B.
+/// Bound by the launch and one chain of loads. Against the listing of the edges, grad_A and grad_B, and grad_W
+/// one after the other, 9 components, 32 columns, f32 / f64: 600 edges 24.0 -> 11.8 / 26.6 -> 12.8 us, 5000 edges
+/// of 200 nodes 27.0 -> 14.9 / 31.3 -> 17.0.
+template <typename T, int N, int COLUMNS>
+__global__ __launch_bounds__(THREADS)
+__attribute__((amdgpu_waves_per_eu(std::min(contract_waves<T, N, COLUMNS>(), edge_waves<T, N, COLUMNS>())))) void
+small_kernel(const ContractArgs<T> of_nodes, const EdgeArgs<T> of_edges, int32_t nodes) {
+    extern __shared__ __align__(16) char lds[];
+    if (static_cast<int32_t>(blockIdx.x) < nodes) { // (uniform)
+        contract<T, N, COLUMNS, SLOTS, true>(of_nodes, lds, blockIdx.x);
+    } else {
+        edge_gradients<T, N, COLUMNS>(of_edges, lds, blockIdx.x - nodes);
+    }
+}
+
 // --------------------------------------------------------------------- host --
 /// What a tile of columns costs: the multiply-adds of a lane, and some eight
 /// instructions' worth of everything else.
@@ -999,19 +1035,66 @@ void forward(
     contract<T, SEGMENTS>(args, s, stream);
 }
 
+namespace {
+
 template <typename T>
-void weight_gradient(
-    T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& s,
-    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+ContractArgs<T> of_senders(
+    T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& s
 ) {
     ContractArgs<T> args{};
     args.walk = walk_of<T>(
         s, A, B, grad_output, C, nullptr, indices.output_1, Dense{indices.A, indices.output_2, indices.W_2, s.N, s.n2}
     );
     args.result = grad_W;
+    args.senders = indices.W_1;
+    return args;
+}
+
+template <typename T>
+EdgeArgs<T> of_edges(
+    T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
+    const Shape& s
+) {
+    EdgeArgs<T> args{};
+    args.walk = walk_of(
+        s, A, B, W, C, indices.output_1, indices.W_1, Dense{indices.A, indices.W_2, indices.output_2, s.N, s.n3}
+    );
+    args.grad_output = grad_output;
+    args.grad_A = grad_A;
+    args.grad_B = grad_B;
+    return args;
+}
+
+/// The wavefronts' shares of the edges; returns the workgroups that takes.
+template <typename T, int N, int COLUMNS> size_t share_out(EdgeArgs<T>& args, const Shape& s) {
+    Walk<T>& w = args.walk;
+    w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
+    const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * edge_waves<T, N, COLUMNS>();
+    // Every wavefront has as many edges as the next, whatever nodes they are of, and makes G of each
+    // (against a range of nodes each, 9 components, 32 columns, f32 / f64, whole vjp: 60 000 edges of 2000
+    // nodes 74 -> 69 us in double, 200 000 of 6600 134 -> 125 / 212 -> 195; 91 000 of 3000, 16 components,
+    // 64 columns, 239 -> 219 / 464 -> 398). Where two wavefronts or more share a node, with four edges each
+    // at least, that is only more of G (600 edges of 20 nodes, listing and grad_W with it, 24.0 -> 24.8; for 16 components in float, of
+    // which G is the most work, also with one: 50 000 of 2000 85.2 -> 87.1).
+    const int64_t shares = std::min<int64_t>(s.n_edges / (4 * static_cast<int64_t>(s.n_nodes)), resident / s.n_nodes);
+    const int64_t least = N == 16 && sizeof(T) == 4 ? 1 : 2;
+    args.shares = shares >= least ? static_cast<int32_t>(shares) : 0;
+    w.ranges = static_cast<int32_t>(
+        shares >= least ? s.n_nodes * shares : std::max<int64_t>(1, std::min<int64_t>(s.n_edges / 4, resident))
+    );
+    return ceil_div(static_cast<size_t>(w.ranges), WAVES);
+}
+
+} // namespace
+
+template <typename T>
+void weight_gradient(
+    T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& s,
+    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+) {
+    ContractArgs<T> args = of_senders(grad_W, grad_output, A, B, C, indices, s);
     if (slots != nullptr) {
         args.slots = *slots;
-        args.senders = indices.W_1;
         contract<T, SLOTS>(args, s, stream);
     } else {
         args.ordered = *ordered;
@@ -1024,36 +1107,42 @@ void edge_gradients(
     T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
     const Shape& s, hipStream_t stream
 ) {
-    EdgeArgs<T> args{};
-    args.walk = walk_of(
-        s, A, B, W, C, indices.output_1, indices.W_1, Dense{indices.A, indices.W_2, indices.output_2, s.N, s.n3}
-    );
-    args.grad_output = grad_output;
-    args.grad_A = grad_A;
-    args.grad_B = grad_B;
+    EdgeArgs<T> args = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
     MainKernelTimer timer(stream);
     with_layout<T>(s, false, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
-        Walk<T>& w = args.walk;
         constexpr size_t lds = edge_lds<T, N, COLUMNS>();
-        w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
-        const int64_t resident = static_cast<int64_t>(compute_units()) * 4 * edge_waves<T, N, COLUMNS>();
-        // Every wavefront has as many edges as the next, whatever nodes they are of, and makes G of each
-        // (against a range of nodes each, 9 components, 32 columns, f32 / f64, whole vjp: 60 000 edges of 2000
-        // nodes 74 -> 69 us in double, 200 000 of 6600 134 -> 125 / 212 -> 195; 91 000 of 3000, 16 components,
-        // 64 columns, 239 -> 219 / 464 -> 398). Where two wavefronts or more share a node, with four edges each
-        // at least, that is only more of G (600 edges of 20 nodes 24.0 -> 24.8; for 16 components in float, of
-        // which G is the most work, also with one: 50 000 of 2000 85.2 -> 87.1).
-        const int64_t shares = std::min<int64_t>(s.n_edges / (4 * static_cast<int64_t>(s.n_nodes)), resident / s.n_nodes);
-        const int64_t least = N == 16 && sizeof(T) == 4 ? 1 : 2;
-        args.shares = shares >= least ? static_cast<int32_t>(shares) : 0;
-        w.ranges = static_cast<int32_t>(
-            shares >= least ? s.n_nodes * shares : std::max<int64_t>(1, std::min<int64_t>(s.n_edges / 4, resident))
-        );
-        const size_t units = w.ranges;
+        const size_t blocks = share_out<T, N, COLUMNS>(args, s);
         auto kernel = edge_kernel<T, N, COLUMNS>;
         allow_lds(kernel, lds);
-        kernel<<<static_cast<unsigned>(ceil_div(units, WAVES)), THREADS, lds, stream>>>(args);
+        kernel<<<static_cast<unsigned>(blocks), THREADS, lds, stream>>>(args);
+    });
+    MOPS_HIP_CHECK(hipGetLastError());
+}
+
+bool small(const Shape& s) {
+    return s.n_edges <= thresholds::COLUMNS_EDGES_AS_THEY_ARE &&
+           static_cast<int64_t>(s.n_nodes) * ((s.L + 31) / 32) <= 2 * compute_units();
+}
+
+template <typename T>
+void small_vjp(
+    T* grad_A, T* grad_B, T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const T* W,
+    const Indices& indices, const Shape& s, hipStream_t stream
+) {
+    ContractArgs<T> nodes = of_senders(grad_W, grad_output, A, B, C, indices, s);
+    EdgeArgs<T> edges = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
+    MainKernelTimer timer(stream);
+    with_layout<T>(s, false, [&](auto components, auto columns) {
+        constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
+        constexpr size_t lds = std::max(edge_lds<T, N, COLUMNS>(), contract_lds<T, N, COLUMNS>());
+        nodes.walk.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
+        nodes.walk.ranges = s.n_nodes;
+        const size_t of_nodes = grad_W != nullptr ? static_cast<size_t>(s.n_nodes) * nodes.walk.column_tiles : 0;
+        const size_t of_edges = grad_A != nullptr || grad_B != nullptr ? share_out<T, N, COLUMNS>(edges, s) : 0;
+        auto kernel = small_kernel<T, N, COLUMNS>;
+        allow_lds(kernel, lds);
+        kernel<<<static_cast<unsigned>(of_nodes + of_edges), THREADS, lds, stream>>>(nodes, edges, static_cast<int32_t>(of_nodes));
     });
     MOPS_HIP_CHECK(hipGetLastError());
 }
@@ -1067,6 +1156,9 @@ void edge_gradients(
     );                                                                                             \
     template void weight_gradient<T>(                                                              \
         T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, const SenderSlots*, const EdgesBySender*, hipStream_t \
+    );                                                                                             \
+    template void small_vjp<T>(                                                                    \
+        T*, T*, T*, const T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t \
     );
 MOPS_INSTANTIATE(float)
 MOPS_INSTANTIATE(double)

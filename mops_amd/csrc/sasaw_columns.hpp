@@ -51,6 +51,17 @@ void weight_gradient(
     const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
 );
 
+/// Whether a graph is small enough that all its gradients are one launch, in which every sender's edges are
+/// looked for in the index as it is.
+bool small(const Shape& shape);
+
+/// Of a small graph: any of grad_A, grad_B, grad_W may be null, but not all.
+template <typename T>
+void small_vjp(
+    T* grad_A, T* grad_B, T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const T* W,
+    const Indices& indices, const Shape& shape, hipStream_t stream
+);
+
 } // namespace mops::amd::sasaw_columns
 
 #endif

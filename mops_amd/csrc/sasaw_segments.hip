@@ -1523,6 +1523,9 @@ static bool columns_in_order(const Shape& s) {
 }
 
 size_t vjp_workspace_bytes(const Shape& s, size_t element_size, bool want_grad_W) {
+    if (vjp_by_columns(s, element_size) && sasaw_columns::small(s)) {
+        return 0;
+    }
     if (want_grad_W && vjp_by_columns(s, element_size) && columns_in_order(s)) {
         return edges_by_sender_bytes(s.n_nodes, s.n_edges, false);
     }
@@ -1678,6 +1681,10 @@ void vjp(
     args.lda = s.nA;
     args.w_stride_rows = s.n2;
     args.g_stride_rows = s.n3;
+    if (vjp_by_columns(s, sizeof(T)) && sasaw_columns::small(s)) {
+        sasaw_columns::small_vjp<T>(grad_A, grad_B, grad_W, grad_output, A, B, C, W, indices, s, stream);
+        return;
+    }
     if (vjp_by_columns(s, sizeof(T))) {
         if (grad_A != nullptr || grad_B != nullptr) {
             sasaw_columns::edge_gradients<T>(grad_A, grad_B, grad_output, A, B, C, W, indices, s, stream);

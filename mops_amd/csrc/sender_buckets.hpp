@@ -329,10 +329,14 @@ __device__ __forceinline__ void edges_of_sender(
             n_waiting = 0;
         }
     };
-    if (n_edges < 4) {
-        return; // (no sender has more edges than places then)
+    if (n_edges < 4) { // (too short for a load of four)
+        for (int32_t position = begin; position < end; position++) {
+            if (senders[position] == sender) {
+                wait(position);
+            }
+        }
     }
-    for (int32_t base = begin; base < end; base += AHEAD * GROUP) {
+    for (int32_t base = n_edges < 4 ? end : begin; base < end; base += AHEAD * GROUP) {
         // a lane looks at four positions of every group, moved to the front where the index ends
         auto first = [&](int u) { return base + u * GROUP + 4 * lane; };
         auto load = [&](int u) { return *reinterpret_cast<const Four*>(senders + min(first(u), n_edges - 4)); };
