@@ -141,11 +141,14 @@ constexpr size_t SENDER_SCAN_LIMIT = 100u * 1000 * 1000;
 /// f32: 33 -> 22 us for the whole vjp.
 constexpr int32_t SLOT_MEAN_EDGES = 48;
 /// Edges up to which SASAW's gradients with a lane per column are one launch, where every node's workgroup
-/// looks through the whole index of senders (with up to two nodes and 32 columns per compute unit). 9
-/// components, 32 columns, that / a launch that lists the edges and one for each kind of gradient, f32, f64:
-/// 600 edges of 20 nodes 11.8 / 24.0, 12.8 / 26.6 us; 8000 of 260 15.4 / 29, 26.7 / 33; 8000 of 700 22.5 / 28,
-/// 36.1 / 34.5; 16 000 of 500 27.6 / 34, 36.0 / 38.5 (4 components, 100 columns 30.8 / 35.0, 45.3 / 43.0).
-constexpr int32_t COLUMNS_EDGES_AS_THEY_ARE = 8192;
+/// looks through the whole index of senders (with up to two nodes and 32 columns per compute unit). That / a
+/// launch that lists the edges and one for each kind of gradient, f32, f64, 9 components unless it says
+/// otherwise: 600 edges of 20 nodes, 32 columns 11.8 / 24.0, 12.8 / 26.6 us; 8000 of 260 15.4 / 29, 26.7 / 33;
+/// 16 000 of 500 27.7 / 34.1, 36.0 / 39.3; 16 000 of 250, 64 columns 28.5 / 39.1, 54.7 / 60.7; 24 000 of 500
+/// 30.5 / 37.1, 43.6 / 46.7. Half as many where nodes have more than SLOT_MEAN_EDGES each (24 000 of 40 63.7 /
+/// 52.2, 67.6 / 59.0), and for 16 components in double, then also half as many nodes (12 000 of 500 70 / 62;
+/// 5000 of 200 40.8 / 53).
+constexpr int32_t COLUMNS_EDGES_AS_THEY_ARE = 16384;
 /// Edges per sender on average up to which lists are made by arrival (128 places
 /// per sender). SASAW, 1000 nodes x 60 edges, whole vjp 87.6 -> 76.6 us (f32), 143.8
 /// -> 115.3 (f64) against the kernels of sasaw_mfma.hip; at 100 per sender the

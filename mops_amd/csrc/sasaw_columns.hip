@@ -1120,9 +1120,12 @@ void edge_gradients(
     MOPS_HIP_CHECK(hipGetLastError());
 }
 
-bool small(const Shape& s) {
-    return s.n_edges <= thresholds::COLUMNS_EDGES_AS_THEY_ARE &&
-           static_cast<int64_t>(s.n_nodes) * ((s.L + 31) / 32) <= 2 * compute_units();
+bool small(const Shape& s, size_t element_size) {
+    const bool sums_fill_the_registers = s.nA == 16 && element_size == 8;
+    const bool dense = s.n_edges > static_cast<int64_t>(s.n_nodes) * thresholds::SLOT_MEAN_EDGES;
+    const int32_t edges = thresholds::COLUMNS_EDGES_AS_THEY_ARE / (sums_fill_the_registers || dense ? 2 : 1);
+    return s.n_edges <= edges &&
+           static_cast<int64_t>(s.n_nodes) * ((s.L + 31) / 32) <= (sums_fill_the_registers ? 1 : 2) * compute_units();
 }
 
 template <typename T>

@@ -53,7 +53,7 @@ void weight_gradient(
 
 /// Whether a graph is small enough that all its gradients are one launch, in which every sender's edges are
 /// looked for in the index as it is.
-bool small(const Shape& shape);
+bool small(const Shape& shape, size_t element_size);
 
 /// Of a small graph: any of grad_A, grad_B, grad_W may be null, but not all.
 template <typename T>

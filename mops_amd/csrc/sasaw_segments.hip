@@ -1523,7 +1523,7 @@ static bool columns_in_order(const Shape& s) {
 }
 
 size_t vjp_workspace_bytes(const Shape& s, size_t element_size, bool want_grad_W) {
-    if (vjp_by_columns(s, element_size) && sasaw_columns::small(s)) {
+    if (vjp_by_columns(s, element_size) && sasaw_columns::small(s, element_size)) {
         return 0;
     }
     if (want_grad_W && vjp_by_columns(s, element_size) && columns_in_order(s)) {
@@ -1681,7 +1681,7 @@ void vjp(
     args.lda = s.nA;
     args.w_stride_rows = s.n2;
     args.g_stride_rows = s.n3;
-    if (vjp_by_columns(s, sizeof(T)) && sasaw_columns::small(s)) {
+    if (vjp_by_columns(s, sizeof(T)) && sasaw_columns::small(s, sizeof(T))) {
         sasaw_columns::small_vjp<T>(grad_A, grad_B, grad_W, grad_output, A, B, C, W, indices, s, stream);
         return;
     }

@@ -67,11 +67,13 @@ def test_against_the_oracle(oracle, device, shape, dtype):
         (1100, 512, 16, 16),
         (1030, 1024, 4, 16),
         (1030, 1025, 4, 16),
-        # one launch for all gradients up to 8192 edges
+        # one launch for all gradients up to 16 384 edges, 8192 of nodes with many
         (3, 1, 4, 5),
         (4, 2, 4, 5),
         (8192, 40, 9, 32),
         (8193, 40, 9, 32),
+        (16384, 400, 9, 20),
+        (16385, 400, 9, 20),
         (9000, 4500, 9, 40),
         (9000, 4500, 16, 24),
     ],
