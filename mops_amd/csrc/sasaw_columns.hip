@@ -234,6 +234,34 @@ __device__ __forceinline__ int32_t lower_bound(const int32_t* __restrict__ index
     return low + __popcll(__ballot(below));
 }
 
+/// The first positions whose values are not below `value` and not below `value` + 1: both searches at once, so
+/// that they wait together (few nodes, forward, f32: 7.6 -> 7.4 us at 600 edges, 16.3 -> 15.8 at 8000 of 30).
+__device__ __forceinline__ void bounds_of(
+    const int32_t* __restrict__ index, int32_t n, int32_t value, int lane, int32_t& first, int32_t& end
+) {
+    int32_t low[2] = {0, 0}, high[2] = {n, n};
+    bool more;
+    do {
+        int32_t step[2], probe[2], found[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            step[k] = max((high[k] - low[k] + WAVE - 1) / WAVE, 1);
+            probe[k] = low[k] + (lane + 1) * step[k] - 1;
+            found[k] = index[min(probe[k], n - 1)];
+        }
+        more = false;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int32_t passed = __popcll(__ballot(probe[k] < high[k] && found[k] < value + k));
+            low[k] += passed * step[k];
+            high[k] = min(high[k], low[k] + step[k]);
+            more = more || step[k] > 1;
+        }
+    } while (more); // (after a step of one place, `low` is the answer)
+    first = low[0];
+    end = low[1];
+}
+
 template <typename T> struct Walk {
     const T* A;    // [n_edges][N]
     const T* B;    // [n_edges][L]
@@ -444,16 +472,6 @@ template <typename T> struct ContractWindow<T, ORDERED> {
     __device__ __forceinline__ int32_t edge(int32_t, int32_t k) const { return __builtin_amdgcn_readlane(listed, k); }
 };
 
-/// Where the edges of a node begin.
-template <typename T, Lists LISTS>
-__device__ __forceinline__ int32_t begin_of_node(const ContractArgs<T>& args, int32_t node, int lane) {
-    if constexpr (LISTS == ORDERED) {
-        return args.ordered.offsets[node];
-    } else {
-        return lower_bound(args.walk.sorted, args.walk.n_edges, node, lane);
-    }
-}
-
 /// Rows of A in scalar registers at once, where they fit without others being moved out of the way:
 /// 1 000 000 edges, 32 columns, 4 components, f32 / f64, 94.9 -> 92.7 / 198 -> 188 us, sums over
 /// senders 180 -> 170 / 273 -> 264; 9 in double 386 -> 371; 9 in float is slower by it.
@@ -474,7 +492,7 @@ template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
 /// SHARED: a workgroup has one node, whose edges its wavefronts share; else every wavefront has a range of
 /// nodes. Bound by the rows it gathers (many edges), by the chain of a node's edges (few). With no more
 /// nodes than workgroups at a time, a node's 30 edges are a chain of eight: 600 edges, 9 components, 32
-/// columns, f32 / f64, 11.3 -> 7.5 / 12.0 -> 8.5 us, 5000 edges 10.6 -> 9.0 / 11.7 -> 10.8. Beyond, the
+/// columns, f32 / f64, 11.3 -> 7.4 / 12.0 -> 8.2 us, 5000 edges 10.6 -> 8.8 / 11.7 -> 10.6. Beyond, the
 /// same share-out of a range of nodes costs a table and a wait more for each share: 60 000 edges 19.3 -> 20.5.
 /// (Ranges of equal edges instead of equal nodes: within 3 % either way from 100 000 to 1 000 000 edges.)
 template <typename T, int N, int COLUMNS, Lists LISTS, bool SHARED>
@@ -599,11 +617,19 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
     };
 
     if constexpr (LISTS != SLOTS) {
-        int32_t at = begin_of_node<T, LISTS>(args, node0, lane), to = INT32_MAX;
+        int32_t at, to = INT32_MAX;
         if constexpr (SHARED) { // the wavefront's quarter of the node's edges
-            const int32_t first = at, n = begin_of_node<T, LISTS>(args, node0 + 1, lane) - first;
-            at = first + static_cast<int32_t>(static_cast<int64_t>(n) * wave / WAVES);
-            to = first + static_cast<int32_t>(static_cast<int64_t>(n) * (wave + 1) / WAVES);
+            int32_t first, last;
+            if constexpr (LISTS == ORDERED) {
+                first = args.ordered.offsets[node0];
+                last = args.ordered.offsets[node0 + 1];
+            } else {
+                bounds_of(p.sorted, p.n_edges, node0, lane, first, last);
+            }
+            at = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * wave / WAVES);
+            to = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * (wave + 1) / WAVES);
+        } else {
+            at = LISTS == ORDERED ? args.ordered.offsets[node0] : lower_bound(p.sorted, p.n_edges, node0, lane);
         }
         // positions at .. at + 64 of the index or of the lists, and the blocks of their edges
         ContractWindow<T, LISTS> window(args, at, lane);
@@ -741,8 +767,9 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
     if (args.shares > 0) {
         share = range % args.shares;
         shares = args.shares;
-        first = lower_bound(p.sorted, p.n_edges, range / args.shares, lane);
-        n_all = lower_bound(p.sorted, p.n_edges, range / args.shares + 1, lane) - first;
+        int32_t last;
+        bounds_of(p.sorted, p.n_edges, range / args.shares, lane, first, last);
+        n_all = last - first;
     }
     const int32_t begin = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * share / shares);
     const int32_t end = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * (share + 1) / shares);
