@@ -83,7 +83,7 @@ MAIN_KERNELS = {
     ("opsa", "vjp"): "opsa::edge_rows_vjp_kernel<{T}, 1, 2, false, true, false, false>",
     ("opsaw", "forward"): "opsa::forward_kernel<{T}, 2, true, true, true>",
     ("opsaw", "vjp"): "opsa::edge_rows_vjp_kernel<{T}, 1, 2, true, true, false, true>",
-    ("sasaw", "forward"): "sasaw_columns::contract_kernel<{T}, 9, 32, (sasaw_columns::Lists)0>",
+    ("sasaw", "forward"): "sasaw_columns::contract_kernel<{T}, 9, 32, (sasaw_columns::Lists)0, false>",
     ("sasaw", "vjp"): "sasaw_columns::edge_kernel<{T}, 9, 32>",
 }
 
