@@ -102,6 +102,47 @@ def test_one_node_has_a_third_of_the_edges(oracle, device, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("components", [4, 9, 16])
+def test_listed_senders_shared_by_a_workgroup(oracle, device, components, dtype):
+    """Lists in slots whose entries the wavefronts of a workgroup share (more than 16 384 edges, no more nodes
+    than workgroups at a time): around 64 and 128 entries, parts that overflow, senders outside the tensor."""
+    import torch
+
+    edges, nodes, columns = 17003, 401, 16
+    case = support.sasaw_case(
+        components, dtype, E=edges, nA=components, L=columns, n_nodes=nodes, n2=components, n3=components, N=60,
+        allow_empty=True,
+    )  # fmt: skip
+    rng = np.random.default_rng(components)
+    # (a quarter of the index each, away from the ends of the quarters)
+    quarters = [rng.permutation(np.arange(edges // 4 * q + 8, edges // 4 * (q + 1) - 8)) for q in range(4)]
+    senders = rng.integers(8, nodes, edges).astype(np.int32)
+    counts = {
+        0: (16, 16, 16, 16), 1: (17, 16, 16, 16), 2: (32, 32, 32, 31), 3: (32, 32, 32, 32), 4: (0, 0, 32, 32),
+        5: (33, 0, 0, 0), 6: (3, 30, 33, 5), 7: (0, 0, 0, 300), nodes: (9, 9, 9, 9), -1: (5, 0, 5, 0),
+    }  # fmt: skip
+    for q, places in enumerate(quarters):
+        at = 0
+        for sender, of_quarter in counts.items():
+            senders[places[at : at + of_quarter[q]]] = sender
+            at += of_quarter[q]
+    inside = (senders >= 0) & (senders < nodes)
+    assert np.bincount(senders[inside], minlength=nodes)[:8].tolist() == [sum(counts[k]) for k in range(8)]
+    on_device = to_device(dict(case, indices_W_1=senders), device)
+    # (for the oracle, an edge that does not count is one without B)
+    case["indices_W_1"] = np.where(inside, senders, 0).astype(np.int32)
+    case["B"] = np.where(inside[:, None], case["B"], 0).astype(dtype)
+    exact = cpu_vjp(oracle, "sasaw", support.in_float64(case))["W"]
+    other = cpu_vjp(oracle, "sasaw", case if dtype == np.float32 else support.magnitudes(case))["W"]
+    beside = torch.empty(edges + 1, dtype=torch.int32, device=device)[1:]
+    beside.copy_(on_device["indices_W_1"])
+    for index in (on_device["indices_W_1"], beside):  # as it is, and off the 16-byte boundaries
+        actual = hip_vjp("sasaw", dict(on_device, indices_W_1=index))["W"].cpu().numpy()
+        same, terms = (other, None) if dtype == np.float32 else (None, other)
+        support.assert_calibrated(actual, exact, dtype, f"{components} grad_W", same, terms)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 def test_senders_outside_the_tensor_count_as_zero(oracle, device, dtype):
     case = support.sasaw_case(7, dtype, E=300, nA=9, L=20, n_nodes=12, n2=9, n3=9, N=120)
     lost = np.random.default_rng(1).integers(0, 300, 40)
