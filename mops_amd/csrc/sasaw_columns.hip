@@ -27,14 +27,20 @@
 //
 // with G_i[:, :, l] of the receiver in the registers of the lane: both come from
 // the same multiply-adds and ONE look at the rows of W; the sum over the columns
-// is taken across lanes (DPP and permlane swaps). grad_W is the sum of the
+// is taken across lanes (DPP and permlane swaps). Of up to 9 components a lane has
+// all block rows, and two or four edges of a node are worked on side by side: no
+// sums across parts, no rows that fill the last part, and the sums over the columns
+// of several edges for the instructions of one (an edge of 9 components and 32
+// columns takes 72 vector instructions instead of 108 in float; 1 000 000 edges,
+// grad_A and grad_B, f32 / f64: 245 -> 215 / 458 -> 410 us, 16 columns 197 -> 122;
+// 60 000 edges 25.4 -> 22.2 / 36.2 -> 30.6). grad_W is the sum of the
 // forward pass over the edges of a sender, with the roles of W and grad_output,
 // m2 and m3 exchanged.
 //
 // Whole calls against one per-node sum on the matrix cores each, 9 components, 32
 // columns, the same buffers every call, f32 / f64, us: 1 000 000 edges, forward 315
-// -> 200 / 391 -> 366, vjp 1184 -> 507 / 1397 -> 895; 60 000 edges, 20.2 -> 19.6 /
-// 29.2 -> 25.1 and 58.5 -> 54 / 99 -> 69; 128 columns there, vjp 247 -> 114 / 360
+// -> 200 / 391 -> 369, vjp 1184 -> 478 / 1397 -> 854; 60 000 edges, 20.2 -> 20.2 /
+// 29.2 -> 25.0 and 58.5 -> 52 / 99 -> 65; 128 columns there, vjp 247 -> 114 / 360
 // -> 223; 600 edges, 12.6 -> 7.5 / 14.0 -> 8.5 and 25.1 -> 11.8 / 31.7 -> 12.8. At a
 // million edges 1.3 GB (float; 2.6 in double) come through the memory side of L2 in
 // the forward pass, rows of W in no order for the most part, at 6.4 (7.1) TB/s: the
@@ -45,6 +51,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "device_common.hpp"
 #include "mfma.hpp"
@@ -62,9 +69,12 @@ constexpr int WAVES = THREADS / WAVE;
 
 /// The sums of a lane for N components of A and N block rows: all components
 /// times M2 block rows, a PARTS-th of them: part, part + PARTS, ... (so that the
-/// parts together load consecutive rows).
-template <int N, int COLUMNS> struct Sums {
-    static constexpr int PARTS = WAVE / COLUMNS;
+/// parts together load consecutive rows). With EDGES > 1 the lanes work on that many
+/// edges side by side instead, and every lane has all rows.
+template <int N_, int COLUMNS_, int EDGES_ = 1> struct Sums {
+    static constexpr int N = N_, COLUMNS = COLUMNS_, EDGES = EDGES_;
+    static constexpr int PARTS = WAVE / COLUMNS / EDGES;
+    static_assert(EDGES == 1 || PARTS == 1, "parts or edges");
     static constexpr int M2 = (N + PARTS - 1) / PARTS;
     static constexpr bool EXACT = PARTS * M2 == N;
     static constexpr int MC = N == 4 ? 4 : N == 9 ? 3 : 2; // components of A that go through LDS at a time
@@ -91,12 +101,10 @@ struct Dense {
     const int32_t* Pout; // [N] row of the result
     int32_t entries, n_out;
 };
-template <int N, int COLUMNS, bool SPREAD> constexpr int table_slots() {
-    using S = Sums<N, COLUMNS>;
+template <typename S, bool SPREAD> constexpr int table_slots() {
     return S::CHUNKS * (SPREAD ? S::TILES * 4 : S::STEPS) * WAVE;
 }
-template <int N, int COLUMNS, bool SPREAD> __device__ __forceinline__ int32_t slot_of(int32_t m1, int32_t m2, int32_t o) {
-    using S = Sums<N, COLUMNS>;
+template <typename S, bool SPREAD> __device__ __forceinline__ int32_t slot_of(int32_t m1, int32_t m2, int32_t o) {
     const int32_t chunk = m1 / S::MC;
     const int32_t pair = m2 % S::PARTS * S::VALUES + m1 % S::MC * S::M2 + m2 / S::PARTS;
     return SPREAD ? ((chunk * S::TILES + (pair >> 4)) * 4 + (o >> 2)) * WAVE + 16 * (o & 3) + (pair & 15)
@@ -106,10 +114,10 @@ template <int N, int COLUMNS, bool SPREAD> __device__ __forceinline__ int32_t sl
 /// Called by all threads of a workgroup, which is in step afterwards. The
 /// entries of one slot are added in ascending order: every round the smallest
 /// pending one of each slot (`owner`: as many integers as the table has slots).
-template <typename T, int N, int COLUMNS, bool SPREAD>
+template <typename T, typename S, bool SPREAD>
 __device__ void build(T* __restrict__ table, int32_t* __restrict__ owner, const T* __restrict__ C, const Dense& t) {
     constexpr int ENTRIES = 4; // of a thread at a time
-    for (int32_t s = threadIdx.x; s < table_slots<N, COLUMNS, SPREAD>(); s += THREADS) {
+    for (int32_t s = threadIdx.x; s < table_slots<S, SPREAD>(); s += THREADS) {
         table[s] = T(0);
         owner[s] = NOBODY;
     }
@@ -129,8 +137,8 @@ __device__ void build(T* __restrict__ table, int32_t* __restrict__ owner, const 
         for (int k = 0; k < ENTRIES; k++) {
             const int32_t n = first + threadIdx.x + k * THREADS;
             const bool inside =
-                n < t.entries && in_bounds(m1[k], N) && in_bounds(c[k], N) && in_bounds(o[k], t.n_out);
-            slot[k] = slot_of<N, COLUMNS, SPREAD>(m1[k], c[k], o[k]);
+                n < t.entries && in_bounds(m1[k], S::N) && in_bounds(c[k], S::N) && in_bounds(o[k], t.n_out);
+            slot[k] = slot_of<S, SPREAD>(m1[k], c[k], o[k]);
             pending |= inside ? 1u << k : 0u;
         }
         __syncthreads();
@@ -219,6 +227,39 @@ template <typename T> __device__ __forceinline__ T sum_of_row(T x) {
     return x;
 }
 
+/// body(integral_constant 0), body(integral_constant 1), ..
+template <typename Body, int... I>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, Body&& body) {
+    (body(std::integral_constant<int, I>{}), ...);
+}
+
+/// Sums over the COLUMNS lanes of an edge of COUNT values at once: every level adds up pairs of lanes, and where
+/// there are two values, one half of the pairs goes on with the one and the other half with the other (three
+/// instructions for two values; the sum of each on its own in all lanes is two, but then all the levels
+/// after it are twice the work). The lane whose bits, in the order of the levels, are those of i ends with value i.
+template <int COLUMNS, int COUNT, int LEVEL = COLUMNS == 32 ? 0 : 1, typename T, int SIZE>
+__device__ __forceinline__ T folded(T (&value)[SIZE], const bool (&bit)[4]) {
+    if constexpr (LEVEL == 5) {
+        static_assert(COUNT == 1, "as many levels as it takes");
+        return value[0];
+    } else {
+        // pairs of rows, mirrors of a row and of its halves, lanes two and one apart
+        constexpr int CONTROL = LEVEL == 1 ? 0x140 : LEVEL == 2 ? 0x141 : LEVEL == 3 ? 0x4e : 0xb1;
+#pragma unroll
+        for (int k = 0; k < (COUNT + 1) / 2; k++) {
+            const bool two = 2 * k + 1 < COUNT;
+            const T x = value[2 * k], y = value[two ? 2 * k + 1 : 2 * k];
+            if constexpr (LEVEL == 0) {
+                value[k] = sum_rows(x, y);
+            } else {
+                const bool mine = bit[LEVEL - 1];
+                value[k] = two ? (mine ? y : x) + rotated<CONTROL>(mine ? x : y) : x + rotated<CONTROL>(x);
+            }
+        }
+        return folded<COLUMNS, (COUNT + 1) / 2, LEVEL + 1>(value, bit);
+    }
+}
+
 /// First position of the sorted index (n entries) whose value is not below `value`.
 __device__ __forceinline__ int32_t lower_bound(const int32_t* __restrict__ index, int32_t n, int32_t value, int lane) {
     int32_t low = 0, high = n;
@@ -295,14 +336,13 @@ template <typename T> struct Window {
 };
 
 /// A lane's place, and the rows of an edge it works on.
-template <typename T, int N, int COLUMNS> struct Columns {
-    using S = Sums<N, COLUMNS>;
-    static constexpr int M2 = S::M2;
-    /// Edges whose operands are on their way while one is worked on.
+template <typename T, typename S> struct Columns {
+    static constexpr int N = S::N, COLUMNS = S::COLUMNS, EDGES = S::EDGES, M2 = S::M2;
+    /// Edges whose operands are on their way while one is worked on (of each of the EDGES).
     static constexpr int AHEAD = (M2 + 1) * sizeof(T) <= 32 ? 4 : 2;
 
     const Walk<T>& p;
-    int lane, c, part;
+    int lane, c, part, slot;
     int32_t column;
     bool column_inside;
     uint32_t column_bytes;
@@ -321,7 +361,8 @@ template <typename T, int N, int COLUMNS> struct Columns {
     __device__ __forceinline__ explicit Columns(const Walk<T>& walk) : p(walk) {
         lane = threadIdx.x & (WAVE - 1);
         c = lane & (COLUMNS - 1);
-        part = lane / COLUMNS;
+        part = EDGES == 1 ? lane / COLUMNS : 0;
+        slot = EDGES == 1 ? 0 : lane / COLUMNS;
         row_bytes = static_cast<uint32_t>(p.L) * sizeof(T);
         block_bytes = N * row_bytes;
         B.set(p.B, static_cast<uint32_t>(p.n_edges) * row_bytes);
@@ -372,9 +413,10 @@ template <typename T, int N, int COLUMNS> struct Columns {
     /// wait is for all of them).
     ///
     /// A_BATCH: the rows of A asked for at once, while as many are worked on.
-    template <int A_BATCH, typename EdgeOf, typename Ask, typename Each>
+    /// `meanwhile()`: what there is to do while the first operands are on their way.
+    template <int A_BATCH, typename EdgeOf, typename Ask, typename Meanwhile, typename Each>
     __device__ __forceinline__ void
-    over(int32_t sources, int32_t n, EdgeOf&& edge_of, Ask&& ask_more, Each&& each) const {
+    over(int32_t sources, int32_t n, EdgeOf&& edge_of, Ask&& ask_more, Meanwhile&& meanwhile, Each&& each) const {
         Operands ring[AHEAD];
         auto ask = [&](Operands& to, int32_t k) {
             k = min(k, n - 1);
@@ -395,6 +437,7 @@ template <typename T, int N, int COLUMNS> struct Columns {
         for (int d = 0; d < AHEAD; d++) {
             ask(ring[d], d);
         }
+        meanwhile();
         auto step = [&](int d, int32_t k) {
             T(&rows)[A_BATCH][N] = a[d / A_BATCH & 1];
             if (d % A_BATCH == 0) {
@@ -424,6 +467,64 @@ template <typename T, int N, int COLUMNS> struct Columns {
             if (d + AHEAD < STEPS - 1) {
                 ask(ring[d % AHEAD], first + d + AHEAD);
             }
+        }
+    }
+
+    /// EDGES > 1: `each(operands, first, valid)` for the edges at positions `first` to first + EDGES, one per slot,
+    /// of the n <= 64 from `begin` on, whose sources the lanes hold; `valid`: whether the lane's is one of them.
+    /// (Loads are counted as in `over`. An edge's row of A comes as an element per lane of every row of 16 lanes,
+    /// from where the multiply-adds take it.)
+    struct Side {
+        T a, b, more;
+        T w[M2];
+    };
+    template <typename Ask, typename Meanwhile, typename Each>
+    __device__ __forceinline__ void side_by_side(
+        const BufferOf<T>& A, const BufferOf<T>& rows, int32_t sources, int32_t begin, int32_t n, Ask&& ask_more,
+        Meanwhile&& meanwhile, Each&& each
+    ) const {
+        const uint32_t a_at = static_cast<uint32_t>(slot * N + min(lane & 15, N - 1)) * static_cast<uint32_t>(sizeof(T));
+        const uint32_t b_at = static_cast<uint32_t>(slot) * row_bytes + column_bytes;
+        // (a source outside the tensor: an offset beyond it, also with what is added)
+        const uint32_t block = static_cast<uint32_t>(sources) * block_bytes | unless(in_bounds(sources, p.n_blocks));
+        const int32_t groups = (n + EDGES - 1) / EDGES;
+        Side ring[AHEAD];
+        auto ask = [&](Side& to, int32_t group) {
+            const int32_t k = min(group, groups - 1) * EDGES;
+            const uint32_t edge = static_cast<uint32_t>(begin + k);
+            const uint32_t of_edge = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute((k + slot) << 2, static_cast<int>(block)));
+            const uint32_t at = __builtin_elementwise_add_sat(of_edge, column_bytes);
+#pragma unroll
+            for (int m = 0; m < M2; m++) {
+                to.w[m] = rows.load(at, m * row_bytes);
+            }
+            to.b = B.load(b_at, edge * row_bytes);
+            to.a = A.load(a_at, edge * static_cast<uint32_t>(N * sizeof(T)));
+            ask_more(to, edge);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+            ask(ring[d], d);
+        }
+        meanwhile();
+        auto step = [&](int d, int32_t group) {
+            each(ring[d], static_cast<uint32_t>(begin + group * EDGES), group * EDGES + slot < n);
+        };
+        int32_t first = 0;
+        for (; first + AHEAD <= groups; first += AHEAD) {
+#pragma unroll
+            for (int d = 0; d < AHEAD; d++) {
+                step(d, first + d);
+                ask(ring[d], first + d + AHEAD);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < AHEAD - 1; d++) {
+            if (first + d >= groups) { // (uniform)
+                return;
+            }
+            step(d, first + d);
         }
     }
 
@@ -485,8 +586,8 @@ template <typename T, int N, int COLUMNS> constexpr int contract_waves() {
 }
 template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
     using S = Sums<N, COLUMNS>;
-    return table_slots<N, COLUMNS, false>() * sizeof(T) +
-           std::max(table_slots<N, COLUMNS, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
+    return table_slots<Sums<N, COLUMNS>, false>() * sizeof(T) +
+           std::max(table_slots<Sums<N, COLUMNS>, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
 }
 
 /// SHARED: a workgroup has one node, whose edges its wavefronts share; else every wavefront has a range of
@@ -503,14 +604,14 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
     constexpr int ROWS_OF_A = contract_rows_of_A<T, N>();
     const Walk<T>& p = args.walk;
     T* table = reinterpret_cast<T*>(lds);
-    T* stages = table + table_slots<N, COLUMNS, false>();
+    T* stages = table + table_slots<Sums<N, COLUMNS>, false>();
     int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
     T* stage = stages + wave * STAGE;
 
-    Columns<T, N, COLUMNS> columns_of(p);
+    Columns<T, S> columns_of(p);
     const int lane = columns_of.lane;
-    build<T, N, COLUMNS, false>(table, owner, p.C, p.table);
+    build<T, S, false>(table, owner, p.C, p.table);
     for (int32_t k = lane; k < STAGE; k += WAVE) {
         stage[k] = T(0); // (rows of a step that stand for no pair stay zero)
     }
@@ -542,6 +643,7 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
     };
 
     auto nothing = [](auto&, int32_t) {};
+    auto not_now = [] {};
 
     // O = D Z, MC components of A at a time through LDS
     const int row16 = lane >> 4;
@@ -640,7 +742,7 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
                 n = SHARED ? min(WAVE, to - at) : window.edges_of(args, node, at);
                 const ContractWindow<T, LISTS> next(args, at + n, lane);
                 if (n > 0) {
-                    columns_of.template over<ROWS_OF_A>(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, add);
+                    columns_of.template over<ROWS_OF_A>(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, not_now, add);
                 }
                 at += n;
                 window = next;
@@ -653,7 +755,7 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
             auto hand_on = [&](int32_t edge, int32_t n) {
                 const int32_t sources = p.gather[edge];
                 columns_of.template over<ROWS_OF_A>(
-                    sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, add
+                    sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, not_now, add
                 );
             };
             auto look_through_index = [&] {
@@ -733,31 +835,34 @@ template <typename T> struct EdgeArgs {
     int32_t shares;       // wavefronts per node, each with a share of its edges (0: a share of all edges)
 };
 
+/// How a wavefront shares out its lanes: several edges side by side where G fits the registers of a lane.
+template <int N, int COLUMNS> using EdgeSums = Sums<N, COLUMNS, N == 16 ? 1 : WAVE / COLUMNS>;
 /// Wavefronts per SIMD.
 template <typename T, int N, int COLUMNS> constexpr int edge_waves() {
-    constexpr int REGISTERS = (N * Sums<N, COLUMNS>::M2 + N + 44) * static_cast<int>(sizeof(T)) / 4;
+    constexpr int REGISTERS = (N * EdgeSums<N, COLUMNS>::M2 + N + 44) * static_cast<int>(sizeof(T)) / 4;
     return REGISTERS <= 100 ? 4 : REGISTERS <= 140 ? 3 : 2;
 }
 template <typename T, int N, int COLUMNS> constexpr size_t edge_lds() {
-    return table_slots<N, COLUMNS, true>() * sizeof(T) +
-           std::max(table_slots<N, COLUMNS, true>() * sizeof(int32_t), WAVES * Sums<N, COLUMNS>::TILES * 16 * pitch<COLUMNS>() * sizeof(T));
+    using S = EdgeSums<N, COLUMNS>;
+    return table_slots<S, true>() * sizeof(T) +
+           std::max(table_slots<S, true>() * sizeof(int32_t), WAVES * S::TILES * 16 * pitch<COLUMNS>() * sizeof(T));
 }
 
 template <typename T, int N, int COLUMNS>
 __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* lds, const int32_t block) {
     using M = Mfma<T>;
-    using S = Sums<N, COLUMNS>;
-    constexpr int M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::TILES * 16 * PITCH;
+    using S = EdgeSums<N, COLUMNS>;
+    constexpr int EDGES = S::EDGES, M2 = S::M2, PITCH = pitch<COLUMNS>(), STAGE = S::TILES * 16 * PITCH;
     const Walk<T>& p = args.walk;
     T* table = reinterpret_cast<T*>(lds);
-    T* stages = table + table_slots<N, COLUMNS, true>();
+    T* stages = table + table_slots<S, true>();
     int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
     T* stage = stages + wave * STAGE;
 
-    Columns<T, N, COLUMNS> columns_of(p);
+    Columns<T, S> columns_of(p);
     const int lane = columns_of.lane;
-    build<T, N, COLUMNS, true>(table, owner, p.C, p.table);
+    build<T, S, true>(table, owner, p.C, p.table);
 
     const int32_t range = block * WAVES + wave;
     if (range >= p.ranges) {
@@ -778,21 +883,33 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
     G.set(args.grad_output, static_cast<uint32_t>(p.n_blocks) * g_block_bytes);
     const int row16 = lane >> 4, sub = lane & 15;
     constexpr int FOLDED = (N + 3) / 4;
+    // (with registers to spare for grad_output and the operands at once)
+    constexpr bool MEANWHILE = N * M2 * sizeof(T) <= 400;
     constexpr uint32_t A_ROW_BYTES = N * sizeof(T);
-    const int32_t component = 4 * sub + ((row16 & 1) << 1 | row16 >> 1);
+    // the component of A whose gradient ends up in this lane, and where in an edge's (or EDGES edges') rows it goes
+    const bool bit[4] = {(lane & 8) != 0, (lane & 4) != 0, (lane & 2) != 0, (lane & 1) != 0};
+    const int32_t of_row = bit[0] + 2 * bit[1] + 4 * bit[2];
+    const int32_t component = EDGES == 1      ? 4 * sub + ((row16 & 1) << 1 | row16 >> 1)
+                              : COLUMNS == 32 ? 2 * of_row + (row16 & 1)
+                                              : of_row + 8 * bit[3];
+    const bool holds = component < N && (EDGES == 1 ? sub < FOLDED : COLUMNS == 16 || !bit[3]);
     const uint32_t a_at =
-        static_cast<uint32_t>(component) * static_cast<uint32_t>(sizeof(T)) | unless(sub < FOLDED && component < N);
+        static_cast<uint32_t>(columns_of.slot * N + component) * static_cast<uint32_t>(sizeof(T)) | unless(holds);
     // (a gradient that is not wanted: a tensor of no bytes, which stores do not reach)
     BufferOf<T> to_A, to_B;
     to_A.set(args.grad_A, args.grad_A != nullptr ? static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES : 0);
     to_B.set(args.grad_B, args.grad_B != nullptr ? static_cast<uint32_t>(p.n_edges) * columns_of.row_bytes : 0);
+    BufferOf<T> A, rows; // (EDGES > 1)
+    A.set(p.A, static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES);
+    rows.set(p.rows, static_cast<uint32_t>(p.n_blocks) * columns_of.block_bytes);
     const T* spread_from = stage + columns_of.part * S::VALUES * PITCH + columns_of.c;
 
     for (int32_t tile = 0; tile < p.column_tiles; tile++) {
         columns_of.set_tile(tile);
         // what this lane stores of an edge's gradients, if anything: an element of grad_B, and a
         // component of grad_A, to which the columns of the tiles before are added
-        const uint32_t b_at = columns_of.column_bytes | unless(columns_of.part == 0 && columns_of.column_inside);
+        const uint32_t b_at = (static_cast<uint32_t>(columns_of.slot) * columns_of.row_bytes + columns_of.column_bytes) |
+                              unless(columns_of.part == 0 && columns_of.column_inside);
         BufferOf<T> from_A;
         from_A.set(args.grad_A, tile == 0 || args.grad_A == nullptr ? 0 : static_cast<uint32_t>(p.n_edges) * A_ROW_BYTES);
         int32_t at = begin;
@@ -800,22 +917,25 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
         while (at < end) {
             const int32_t node = __builtin_amdgcn_readfirstlane(window.receiver);
             T g[N * M2];
-            // G = D^T grad_output of the node, MC components of A at a time through LDS
-            auto spread = [&] {
-                T upstream[COLUMNS / 16][4];
+            // G = D^T grad_output of the node, MC components of A at a time through LDS; grad_output is asked
+            // for before, and G made while, the operands of the first edges are on their way
+            const bool exists = in_bounds(node, p.n_blocks);
+            T upstream[COLUMNS / 16][4];
 #pragma unroll
-                for (int t = 0; t < COLUMNS / 16; t++) {
+            for (int t = 0; t < COLUMNS / 16; t++) {
 #pragma unroll
-                    for (int s3 = 0; s3 < 4; s3++) {
-                        const int32_t o = 4 * s3 + row16, column = tile * COLUMNS + 16 * t + sub;
-                        upstream[t][s3] = G.load(
-                            (static_cast<uint32_t>(node) * g_block_bytes + static_cast<uint32_t>(o) * columns_of.row_bytes +
-                             static_cast<uint32_t>(column) * static_cast<uint32_t>(sizeof(T))) |
-                                unless(o < p.table.n_out && column < p.L),
-                            0
-                        );
-                    }
+                for (int s3 = 0; s3 < 4; s3++) {
+                    const int32_t o = 4 * s3 + row16, column = tile * COLUMNS + 16 * t + sub;
+                    upstream[t][s3] = G.load(
+                        (static_cast<uint32_t>(node) * g_block_bytes + static_cast<uint32_t>(o) * columns_of.row_bytes +
+                         static_cast<uint32_t>(column) * static_cast<uint32_t>(sizeof(T))) |
+                            unless(exists && o < p.table.n_out && column < p.L),
+                        0
+                    );
                 }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            auto spread = [&] {
 #pragma unroll
                 for (int chunk = 0; chunk < S::CHUNKS; chunk++) {
 #pragma unroll
@@ -899,22 +1019,56 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
                     to_A.store(mine + operands.more, a_at, edge * A_ROW_BYTES);
                 };
             };
-            const bool exists = in_bounds(node, p.n_blocks);
-            if (exists) {
-                spread();
+            // (EDGES > 1: of the lane's edge)
+            auto gradients_of_its_own = [&](const auto& operands, uint32_t edge, bool valid) {
+                const T b = columns_of.column_inside ? operands.b : T(0);
+                T sum = T(0), term[N];
+                unrolled(std::make_integer_sequence<int, N>{}, [&](auto i) {
+                    T u = g[i * M2] * operands.w[0];
+#pragma unroll
+                    for (int m = 1; m < M2; m++) {
+                        u += g[i * M2 + m] * operands.w[m];
+                    }
+                    term[i] = u * b;
+                    sum += rotated<0x150 + i>(operands.a) * u; // (row_newbcast: element i of the row of A)
+                });
+                const uint32_t lost = unless(valid);
+                to_B.store(sum, b_at | lost, edge * columns_of.row_bytes);
+                to_A.store(folded<COLUMNS, N>(term, bit) + operands.more, a_at | lost, edge * A_ROW_BYTES);
+            };
+            bool spread_out = false;
+            if constexpr (!MEANWHILE) {
+                if (exists) {
+                    spread();
+                    spread_out = true;
+                }
             }
+            auto spread_once = [&] {
+                if (MEANWHILE && !spread_out) { // (uniform)
+                    spread();
+                    spread_out = true;
+                }
+            };
             int32_t n;
             do {
                 n = min(window.edges_of(node), end - at);
                 const Window<T> next(p, at + n, lane);
-                if (exists && n > 0) {
+                if constexpr (EDGES > 1) {
+                    if (exists && n > 0) {
+                        columns_of.side_by_side(
+                            A, rows, window.source, at, n,
+                            [&](auto& operands, uint32_t edge) { operands.more = from_A.load(a_at, edge * A_ROW_BYTES); },
+                            spread_once, gradients_of_its_own
+                        );
+                    }
+                } else if (exists && n > 0) {
                     const int32_t first = at;
                     columns_of.template over<1>(
                         window.source, n, [&](int32_t k) { return first + k; },
                         [&](auto& operands, int32_t k) {
                             operands.more = from_A.load(a_at, static_cast<uint32_t>(first + k) * A_ROW_BYTES);
                         },
-                        gradients(first)
+                        spread_once, gradients(first)
                     );
                 }
                 at += n;
@@ -953,22 +1107,26 @@ small_kernel(const ContractArgs<T> of_nodes, const EdgeArgs<T> of_edges, int32_t
 /// instructions' worth of everything else.
 template <int N, int COLUMNS> constexpr int cost() { return (N + 1) * Sums<N, COLUMNS>::M2 + 8; }
 
-/// body(N, COLUMNS): the cheapest tiles.
-template <typename T, typename Body> void with_layout(const Shape& s, bool narrow, Body&& body) {
+/// body(N, COLUMNS): the cheapest tiles. EDGES: for the gradients by edge, in double of 32 columns at most for 9
+/// components (60 000 edges, 64 columns, grad_A and grad_B with 64 / 32 at a time 66 / 56 us, 300 000 259 / 248; in float
+/// 31 / 37 and 128 / 132). `more`: what a tile costs beside that.
+template <typename T, bool EDGES, typename Body> void with_layout(const Shape& s, Body&& body, int more = 0) {
     auto with_columns = [&](auto n) {
         constexpr int N = decltype(n)::value;
         // (sums that fit the registers of a lane)
-        constexpr int MOST = N == 16 ? (sizeof(T) == 4 ? 32 : 16) : 64;
-        int best = 16, least = (s.L + 15) / 16 * cost<N, 16>();
-        if (const int c = (s.L + 31) / 32 * cost<N, 32>(); MOST >= 32 && c <= least) {
+        constexpr int MOST = N == 16                            ? (sizeof(T) == 4 ? 32 : 16)
+                             : EDGES && N == 9 && sizeof(T) == 8 ? 32
+                                                                 : 64;
+        int best = 16, least = (s.L + 15) / 16 * (cost<N, 16>() + more);
+        if (const int c = (s.L + 31) / 32 * (cost<N, 32>() + more); MOST >= 32 && c <= least) {
             best = 32;
             least = c;
         }
-        if (const int c = (s.L + 63) / 64 * cost<N, 64>(); MOST >= 64 && c <= least) {
+        if (const int c = (s.L + 63) / 64 * (cost<N, 64>() + more); MOST >= 64 && c <= least) {
             best = 64;
         }
         // (few nodes: more, narrower tiles, which the contraction takes as wavefronts of their own)
-        if (narrow && static_cast<int64_t>(s.n_nodes) * ((s.L + best - 1) / best) < 4 * compute_units()) {
+        if (!EDGES && static_cast<int64_t>(s.n_nodes) * ((s.L + best - 1) / best) < 4 * compute_units()) {
             best = 16;
         }
         if (best == 16) {
@@ -1022,7 +1180,7 @@ Walk<T> walk_of(
 }
 
 template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Shape& s, hipStream_t stream) {
-    with_layout<T>(s, true, [&](auto n, auto columns) {
+    with_layout<T, false>(s, [&](auto n, auto columns) {
         constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
         Walk<T>& w = args.walk;
         constexpr size_t lds = contract_lds<T, N, COLUMNS>();
@@ -1136,7 +1294,7 @@ void edge_gradients(
 ) {
     EdgeArgs<T> args = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
     MainKernelTimer timer(stream);
-    with_layout<T>(s, false, [&](auto components, auto columns) {
+    with_layout<T, true>(s, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
         constexpr size_t lds = edge_lds<T, N, COLUMNS>();
         const size_t blocks = share_out<T, N, COLUMNS>(args, s);
@@ -1163,7 +1321,7 @@ void small_vjp(
     ContractArgs<T> nodes = of_senders(grad_W, grad_output, A, B, C, indices, s);
     EdgeArgs<T> edges = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
     MainKernelTimer timer(stream);
-    with_layout<T>(s, false, [&](auto components, auto columns) {
+    with_layout<T, true>(s, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
         constexpr size_t lds = std::max(edge_lds<T, N, COLUMNS>(), contract_lds<T, N, COLUMNS>());
         nodes.walk.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
@@ -1173,7 +1331,9 @@ void small_vjp(
         auto kernel = small_kernel<T, N, COLUMNS>;
         allow_lds(kernel, lds);
         kernel<<<static_cast<unsigned>(of_nodes + of_edges), THREADS, lds, stream>>>(nodes, edges, static_cast<int32_t>(of_nodes));
-    });
+        // (tiles are one after the other for the edges' wavefronts, and little else bounds a small graph: 2000 edges
+        // of 60 nodes, 40 columns, f64, with 16 / 32 at a time 18.7 / 15.5 us)
+    }, 4);
     MOPS_HIP_CHECK(hipGetLastError());
 }
 

@@ -60,6 +60,17 @@ def test_against_the_oracle(oracle, device, shape, dtype):
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize(
     "shape",
+    [(2, 1, 9, 30, 16), (700, 300, 9, 60, 16), (700, 300, 4, 24, 13), (501, 200, 9, 250, 32), (300, 200, 4, 30, 33), (1999, 31, 9, 250, 40), (20001, 9000, 9, 250, 32)],
+    ids=lambda s: "x".join(map(str, s)),
+)  # fmt: skip
+def test_edges_side_by_side(oracle, device, shape, dtype):
+    """Two or four edges of a node at a time: nodes with fewer, and with any remainder; several tiles of columns."""
+    test_against_the_oracle(oracle, device, shape, dtype)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize(
+    "shape",
     [  # edges, nodes, components, columns: a node by a workgroup (up to 512 to 1024 nodes), a range of them by a wavefront
         (7, 3, 9, 32),
         (700, 3, 9, 33),
