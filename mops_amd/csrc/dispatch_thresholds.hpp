@@ -167,12 +167,6 @@ constexpr int32_t ARRIVAL_NODES = 4000;
 /// Edges up to which OPSAW lists by arrival; beyond, the counting sort (see
 /// opsa.hip).
 constexpr int32_t ARRIVAL_EDGES = 500000;
-/// Edges x nodes from which a counting sort of the edges by sender replaces the
-/// slots where the kernels of sasaw_columns.hip use them (four lookers at the
-/// index per 16 nodes against three short launches). grad_W alone, f32, 9
-/// components, 32 columns, slots / sort: 4000 nodes of 30 edges 44.7 / 52.0 us,
-/// of 46 edges 56.0 / 64.5, 6000 of 30 70.8 / about 66, 11 000 of 10 65.5 / 59.
-constexpr size_t SLOT_PRODUCT = 1000u * 1000 * 1000;
 
 // ---- SASAW (sasaw_columns.hip) ------------------------------------------------
 /// Edges from which the forward pass of a shape that fills the matrix cores (16

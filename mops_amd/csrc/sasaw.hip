@@ -758,7 +758,12 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
         const sasaw_mfma::Indices indices{
             indices_A.data, indices_W_1.data, indices_W_2.data, indices_output_1.data, indices_output_2.data
         };
-        const size_t bytes = sasaw_segments::vjp_workspace_bytes(shape, sizeof(scalar_t), want_W);
+        // (a call that is captured by a thread with a smaller block takes the way that needs less)
+        size_t bytes = sasaw_segments::vjp_workspace_bytes(shape, sizeof(scalar_t), want_W, true);
+        const bool shares = scratch_ready(bytes);
+        if (!shares) {
+            bytes = sasaw_segments::vjp_workspace_bytes(shape, sizeof(scalar_t), want_W, false);
+        }
         void* workspace = bytes > 0 ? scratch(bytes) : nullptr;
         std::optional<ScratchCounters> taken; // (until the end of this call, finish_call included)
         if (bytes > 0) {
@@ -767,7 +772,7 @@ void sparse_accumulation_scatter_add_with_weights_vjp(MOPS_SASAW_VJP_PARAMS(MOPS
         int32_t* counters = taken ? taken->data() : nullptr;
         sasaw_segments::vjp<scalar_t>(
             grad_A.data, grad_B.data, grad_W.data, grad_output.data, A.data, B.data, C.data, W.data, indices,
-            shape, workspace, counters, true, stream
+            shape, workspace, shares, counters, true, stream
         );
         finish_call(operation);
         return;
@@ -951,13 +956,17 @@ void sasaw_vjp_no_alloc(
         // (the same kernels as the existing entry point takes for these shapes)
         // (the places of the senders' edges or their order, then the counters; the array is shared with
         // the kernels of other shapes, so the counters are cleared by a launch in front)
-        const size_t places = sasaw_segments::vjp_workspace_bytes(shape, sizeof(float), want_W);
+        size_t places = sasaw_segments::vjp_workspace_bytes(shape, sizeof(float), want_W, true);
+        const bool shares = places <= NO_ALLOC_SCRATCH_BYTES;
+        if (!shares) {
+            places = sasaw_segments::vjp_workspace_bytes(shape, sizeof(float), want_W, false);
+        }
         const size_t needed = places + sasaw_segments::vjp_counters(shape, sizeof(float), want_W) * sizeof(int32_t);
         if (needed <= NO_ALLOC_SCRATCH_BYTES) {
             char* const array = static_cast<char*>(no_alloc_scratch_of_current_device());
             sasaw_segments::vjp<float>(
                 grad_A.data, grad_B.data, grad_W.data, grad_output.data, A.data, B.data, C.data, W.data, indices, shape,
-                array, reinterpret_cast<int32_t*>(array + places), false, stream
+                array, shares, reinterpret_cast<int32_t*>(array + places), false, stream
             );
             finish_call(operation);
             return;

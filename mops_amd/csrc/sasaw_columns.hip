@@ -58,6 +58,7 @@
 #include "runtime.hpp"
 #include "sasaw_table.hpp"
 #include "sender_buckets.hpp"
+#include "sender_shares.hpp"
 
 namespace mops::amd::sasaw_columns {
 namespace {
@@ -114,8 +115,11 @@ template <typename S, bool SPREAD> __device__ __forceinline__ int32_t slot_of(in
 /// Called by all threads of a workgroup, which is in step afterwards. The
 /// entries of one slot are added in ascending order: every round the smallest
 /// pending one of each slot (`owner`: as many integers as the table has slots).
-template <typename T, typename S, bool SPREAD>
-__device__ void build(T* __restrict__ table, int32_t* __restrict__ owner, const T* __restrict__ C, const Dense& t) {
+/// `meanwhile()`: what there is to do while the first entries are on their way.
+template <typename T, typename S, bool SPREAD, typename Meanwhile>
+__device__ __forceinline__ void build(
+    T* __restrict__ table, int32_t* __restrict__ owner, const T* __restrict__ C, const Dense& t, Meanwhile&& meanwhile
+) {
     constexpr int ENTRIES = 4; // of a thread at a time
     for (int32_t s = threadIdx.x; s < table_slots<S, SPREAD>(); s += THREADS) {
         table[s] = T(0);
@@ -131,6 +135,9 @@ __device__ void build(T* __restrict__ table, int32_t* __restrict__ owner, const 
             c[k] = t.Pred[safe];
             o[k] = t.Pout[safe];
             coefficient[k] = C[safe];
+        }
+        if (first == 0) {
+            meanwhile();
         }
         uint32_t pending = 0;
 #pragma unroll
@@ -541,37 +548,15 @@ template <typename T, typename S> struct Columns {
 template <typename T> struct ContractArgs {
     Walk<T> walk;
     T* result; // [n_blocks][n_out][L]
-    // the edges of every sender: LISTS == SLOTS, and what they were made from
-    SenderSlots slots;
-    const int32_t* senders; // [n_edges]
-    // LISTS == ORDERED
-    EdgesBySender ordered;
+    const int32_t* senders; // [n_edges] LISTS == LOOKED_FOR
+    EdgesBySender ordered;  // LISTS == ORDERED
+    Shares shares;          // LISTS == BUCKETS
+    SharePlan plan;
 };
 
-/// Where the edges of a node are: next to each other in the (sorted) index, or in lists.
-enum Lists { SEGMENTS, SLOTS, ORDERED };
-
-/// The next 64 edges, one per lane: at positions of the index, or of the ordered lists.
-template <typename T, Lists LISTS> struct ContractWindow : Window<T> {
-    __device__ __forceinline__ ContractWindow(const ContractArgs<T>& args, int32_t at, int32_t lane)
-        : Window<T>(args.walk, at, lane) {}
-    __device__ __forceinline__ int32_t edges_of(const ContractArgs<T>&, int32_t node, int32_t) const {
-        return Window<T>::edges_of(node);
-    }
-    static __device__ __forceinline__ int32_t edge(int32_t at, int32_t k) { return at + k; }
-};
-template <typename T> struct ContractWindow<T, ORDERED> {
-    int32_t listed, source;
-
-    __device__ __forceinline__ ContractWindow(const ContractArgs<T>& args, int32_t at, int32_t lane) {
-        listed = args.ordered.edge[min(at + lane, args.walk.n_edges - 1)];
-        source = args.walk.gather[listed];
-    }
-    __device__ __forceinline__ int32_t edges_of(const ContractArgs<T>& args, int32_t node, int32_t at) const {
-        return min(args.ordered.offsets[node + 1] - at, WAVE);
-    }
-    __device__ __forceinline__ int32_t edge(int32_t, int32_t k) const { return __builtin_amdgcn_readlane(listed, k); }
-};
+/// Where the edges of a node are: next to each other in the (sorted) index, in a list of all edges by node, in a
+/// bucket that the workgroup fetches first, or anywhere in a short index that the workgroup looks through.
+enum Lists { SEGMENTS, ORDERED, BUCKETS, LOOKED_FOR };
 
 /// Rows of A in scalar registers at once, where they fit without others being moved out of the way:
 /// 1 000 000 edges, 32 columns, 4 components, f32 / f64, 94.9 -> 92.7 / 198 -> 188 us, sums over
@@ -586,8 +571,17 @@ template <typename T, int N, int COLUMNS> constexpr int contract_waves() {
 }
 template <typename T, int N, int COLUMNS> constexpr size_t contract_lds() {
     using S = Sums<N, COLUMNS>;
-    return table_slots<Sums<N, COLUMNS>, false>() * sizeof(T) +
-           std::max(table_slots<Sums<N, COLUMNS>, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
+    return table_slots<S, false>() * sizeof(T) +
+           std::max(table_slots<S, false>() * sizeof(int32_t), WAVES * S::STEPS * 4 * pitch<COLUMNS>() * sizeof(T));
+}
+/// The same with a bucket's edges between the table and the stages, and what fetching them takes where the stages are.
+__host__ __device__ constexpr size_t kept_of_bucket(int32_t per_bucket) {
+    return (static_cast<size_t>(bucket_lds(per_bucket)) + 3) / 4 * 4 * sizeof(int32_t);
+}
+template <typename T, int N, int COLUMNS> constexpr size_t contract_lds(int32_t per_bucket) {
+    constexpr size_t table = table_slots<Sums<N, COLUMNS>, false>() * sizeof(T);
+    return table + kept_of_bucket(per_bucket) +
+           std::max(contract_lds<T, N, COLUMNS>() - table, gather_lds<THREADS>(per_bucket) * sizeof(int32_t));
 }
 
 /// SHARED: a workgroup has one node, whose edges its wavefronts share; else every wavefront has a range of
@@ -604,27 +598,43 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
     constexpr int ROWS_OF_A = contract_rows_of_A<T, N>();
     const Walk<T>& p = args.walk;
     T* table = reinterpret_cast<T*>(lds);
-    T* stages = table + table_slots<Sums<N, COLUMNS>, false>();
-    int32_t* owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
+    T* stages = table + table_slots<S, false>();
+    int32_t* const kept = reinterpret_cast<int32_t*>(stages);
+    if constexpr (LISTS == BUCKETS) {
+        stages = reinterpret_cast<T*>(reinterpret_cast<char*>(stages) + kept_of_bucket(args.plan.per_bucket));
+    }
+    int32_t* const owner = reinterpret_cast<int32_t*>(stages); // (while the table is built)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
     T* stage = stages + wave * STAGE;
 
     Columns<T, S> columns_of(p);
     const int lane = columns_of.lane;
-    build<T, S, false>(table, owner, p.C, p.table);
+    BucketEdges bucket{};
+    // SHARED: (range, tile) by workgroup; of a bucket, its nodes and their tiles as wavefronts are done with the ones
+    // before; else (range, tile) by wavefront.
+    const int32_t unit = SHARED ? block : LISTS == BUCKETS ? block * p.column_tiles : block * WAVES + wave;
+    const int32_t range = unit / p.column_tiles;
+    int32_t tile = unit % p.column_tiles;
+    if constexpr (LISTS == BUCKETS) {
+        BucketFetch fetch(args.shares, args.plan, range);
+        build<T, S, false>(table, owner, p.C, p.table, [&] { fetch.ask(); });
+        bucket = gather_bucket<THREADS>(kept, owner, fetch, args.shares, args.plan, range, tile);
+    } else {
+        build<T, S, false>(table, owner, p.C, p.table, [] {});
+    }
     for (int32_t k = lane; k < STAGE; k += WAVE) {
         stage[k] = T(0); // (rows of a step that stand for no pair stay zero)
     }
     wave_sync();
-
-    const int32_t unit = SHARED ? block : block * WAVES + wave;
-    const int32_t tile = unit % p.column_tiles, range = unit / p.column_tiles;
     if (range >= p.ranges) {
         return;
     }
+    const int32_t node0 = LISTS == BUCKETS ? args.plan.first_of(range)
+                                           : static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * range / p.ranges);
+    const int32_t node1 = LISTS == BUCKETS
+                              ? args.plan.first_of(range + 1)
+                              : static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * (range + 1) / p.ranges);
     columns_of.set_tile(tile);
-    const int32_t node0 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * range / p.ranges);
-    const int32_t node1 = static_cast<int32_t>(static_cast<int64_t>(p.n_blocks) * (range + 1) / p.ranges);
 
     T z[N * M2];
     auto add = [&](const T (&a)[N], const auto& operands, int32_t) {
@@ -718,103 +728,158 @@ __device__ __forceinline__ void contract(const ContractArgs<T>& args, char* lds,
         }
     };
 
-    if constexpr (LISTS != SLOTS) {
-        int32_t at, to = INT32_MAX;
+    if constexpr (LISTS == LOOKED_FOR) {
+        clear();
+        const int32_t share = (p.n_edges + WAVES - 1) / WAVES, begin = min(wave * share, p.n_edges);
+        edges_of_sender<4>(
+            args.senders, p.n_edges, begin, min(begin + share, p.n_edges), node0, lane,
+            [&](int32_t edge, int32_t n) {
+                columns_of.template over<ROWS_OF_A>(
+                    p.gather[edge], n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, not_now, add
+                );
+            }
+        );
+        finish(node0);
+    } else {
+        // Positions of the index or of a list from `at` on, one per lane, asked for while the ones before are worked
+        // on: what is there (a node, or an edge), and the block of the edge.
+        struct Positions {
+            int32_t name, source;
+            bool inside;
+        };
+        auto positions = [&](int32_t at) {
+            Positions here;
+            const int32_t last = LISTS == BUCKETS ? max(bucket.n, 1) : p.n_edges;
+            const int32_t position = min(at + lane, last - 1);
+            here.inside = at + lane < last;
+            if constexpr (LISTS == SEGMENTS) {
+                here.name = p.sorted[position];
+                here.source = p.gather[position];
+            } else {
+                if constexpr (LISTS == ORDERED) {
+                    here.name = args.ordered.edge[position];
+                } else {
+                    here.name = bucket.fits ? bucket.list[position] : bucket.in_memory[position];
+                }
+                here.source = p.gather[here.name];
+            }
+            return here;
+        };
+        auto begin_of = [&](int32_t node) { // (of a list)
+            return LISTS == ORDERED ? args.ordered.offsets[node]
+                                    : __builtin_amdgcn_readfirstlane(bucket.offsets[node - node0]);
+        };
+        // the sum over n edges at `at`, and what lies at `next`
+        auto add_up = [&](Positions& here, int32_t at, int32_t n, int32_t next) {
+            const Positions there = positions(next);
+            if (n > 0) {
+                columns_of.template over<ROWS_OF_A>(
+                    here.source, n,
+                    [&](int32_t k) { return LISTS == SEGMENTS ? at + k : __builtin_amdgcn_readlane(here.name, k); },
+                    nothing, not_now, add
+                );
+            }
+            here = there;
+        };
         if constexpr (SHARED) { // the wavefront's quarter of the node's edges
             int32_t first, last;
-            if constexpr (LISTS == ORDERED) {
-                first = args.ordered.offsets[node0];
-                last = args.ordered.offsets[node0 + 1];
-            } else {
+            if constexpr (LISTS == SEGMENTS) {
                 bounds_of(p.sorted, p.n_edges, node0, lane, first, last);
-            }
-            at = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * wave / WAVES);
-            to = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * (wave + 1) / WAVES);
-        } else {
-            at = LISTS == ORDERED ? args.ordered.offsets[node0] : lower_bound(p.sorted, p.n_edges, node0, lane);
-        }
-        // positions at .. at + 64 of the index or of the lists, and the blocks of their edges
-        ContractWindow<T, LISTS> window(args, at, lane);
-        for (int32_t node = node0; node < node1; node++) {
-            clear();
-            int32_t n;
-            do {
-                n = SHARED ? min(WAVE, to - at) : window.edges_of(args, node, at);
-                const ContractWindow<T, LISTS> next(args, at + n, lane);
-                if (n > 0) {
-                    columns_of.template over<ROWS_OF_A>(window.source, n, [&](int32_t k) { return window.edge(at, k); }, nothing, not_now, add);
-                }
-                at += n;
-                window = next;
-            } while (n == WAVE);
-            finish(node);
-        }
-    } else {
-        for (int32_t node = node0; node < node1; node++) {
-            clear();
-            auto hand_on = [&](int32_t edge, int32_t n) {
-                const int32_t sources = p.gather[edge];
-                columns_of.template over<ROWS_OF_A>(
-                    sources, n, [&](int32_t k) { return __builtin_amdgcn_readlane(edge, k); }, nothing, not_now, add
-                );
-            };
-            auto look_through_index = [&] {
-                const int32_t share = (p.n_edges + WAVES - 1) / WAVES, begin = min(wave * share, p.n_edges);
-                edges_of_sender<4>(args.senders, p.n_edges, begin, min(begin + share, p.n_edges), node, lane, hand_on);
-            };
-            if constexpr (SHARED) {
-                if (args.slots.edges == nullptr) { // a short index: its quarters looked at as they are
-                    look_through_index();
-                    finish(node);
-                    continue;
-                }
-            }
-            const int32_t* places = args.slots.edges + static_cast<size_t>(node) * SLOT_CAPACITY;
-            int32_t first_half = places[lane], second_half = places[lane + WAVE];
-            static_assert(SLOT_PARTS == 4 && SLOT_CAPACITY == 2 * WAVE, "four parts of a node's places in two registers");
-            const int4 counts = reinterpret_cast<const int4*>(args.slots.counts)[node];
-            const int32_t c0 = __builtin_amdgcn_readfirstlane(counts.x), c1 = __builtin_amdgcn_readfirstlane(counts.y);
-            const int32_t c2 = __builtin_amdgcn_readfirstlane(counts.z), c3 = __builtin_amdgcn_readfirstlane(counts.w);
-            const int32_t count = c0 + c1 + c2 + c3;
-            const bool listed = max(max(c0, c1), max(c2, c3)) <= SLOT_PART_CAPACITY;
-            // the parts moved together: position k of the list is in part `part`, place k - before
-            const int32_t low = first_half, high = second_half;
-            auto edge_at = [&](int32_t position) {
-                const int32_t part =
-                    (position >= c0 ? 1 : 0) + (position >= c0 + c1 ? 1 : 0) + (position >= c0 + c1 + c2 ? 1 : 0);
-                const int32_t before = part == 0 ? 0 : part == 1 ? c0 : part == 2 ? c0 + c1 : c0 + c1 + c2;
-                const int32_t place = part * SLOT_PART_CAPACITY + position - before;
-                const int32_t from_low = __shfl(low, place & (WAVE - 1));
-                const int32_t from_high = __shfl(high, place & (WAVE - 1));
-                return place < WAVE ? from_low : from_high;
-            };
-            if (listed) {
-                first_half = edge_at(lane);
-                second_half = count > WAVE ? edge_at(lane + WAVE) : 0;
-            }
-            if (listed && SHARED) {
-                // (at most 32 of the 128 places)
-                const int32_t from = count * wave / WAVES, n = count * (wave + 1) / WAVES - from;
-                const int32_t place = from + lane;
-                const int32_t low = __shfl(first_half, place & (WAVE - 1)), high = __shfl(second_half, place & (WAVE - 1));
-                if (n > 0) {
-                    hand_on(lane < n ? (place < WAVE ? low : high) : 0, n);
-                }
-            } else if (listed) {
-                if (count > 0) {
-                    hand_on(lane < count ? first_half : 0, min(count, WAVE));
-                }
-                if (count > WAVE) {
-                    hand_on(lane + WAVE < count ? second_half : 0, count - WAVE);
-                }
-            } else if (SHARED) {
-                look_through_index();
             } else {
-                // more edges than places (a hub of a sparse graph): this wavefront reads the index itself
-                // (3000 nodes of 30 edges, one of them of 300, f32, whole vjp 250 us; a load at a time 674; without it 71)
-                edges_of_sender<4>(args.senders, p.n_edges, 0, p.n_edges, node, lane, hand_on);
+                first = begin_of(node0);
+                last = begin_of(node0 + 1);
             }
-            finish(node);
+            int32_t at = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * wave / WAVES), n;
+            const int32_t to = first + static_cast<int32_t>(static_cast<int64_t>(last - first) * (wave + 1) / WAVES);
+            Positions here = positions(at);
+            clear();
+            do {
+                n = min(WAVE, to - at);
+                add_up(here, at, n, at + n);
+                at += n;
+            } while (n == WAVE);
+            finish(node0);
+        } else if constexpr (LISTS == BUCKETS) {
+            // One tile: whichever node is next when a wavefront is done with one. Several: up to four of them (step) of
+            // a node at the same time, which share the lines that gathered rows lie on; each wavefront has every
+            // WAVES / step-th node then. Three tiles leave a wavefront over: it has the last quarter of the nodes,
+            // a tile of them after the other (of fewer than four nodes: as with one tile). 16 components, f32, W alone, 300 000
+            // edges of 10 000 nodes, 40 columns: whichever is next 235 us, the third tile by itself 237, this 213;
+            // 9 components, 32 columns, 1 000 000 edges: a quarter of the nodes each 250, whichever is next 241.
+            struct Unit {
+                int32_t node, tile, step;
+            };
+            const int32_t last_quarter = node1 - (node1 - node0) / 4;
+            auto alone = [&](const Unit& unit) { return unit.step == 3 && wave == 3; };
+            const bool any = p.column_tiles == 1 || (p.column_tiles == 3 && node1 - node0 < 4);
+            auto nth = [&](int32_t k) { return Unit{node0 + k / p.column_tiles, k % p.column_tiles, 1}; };
+            auto begin_tiles = [&](int32_t tile) { // (the first unit of this or of a later group of tiles)
+                for (;;) {
+                    const int32_t left = p.column_tiles - tile, step = min(left, 4);
+                    const bool of_last = step == 3 && wave == 3;
+                    const Unit unit{
+                        of_last ? last_quarter : node0 + wave / max(step, 1), of_last ? tile : tile + wave % max(step, 1), step};
+                    if (left <= 0 || unit.node < node1) {
+                        return unit;
+                    }
+                    tile += step;
+                }
+            };
+            auto exists = [&](const Unit& unit) { return unit.node < node1 && unit.tile < p.column_tiles; };
+            Unit unit = any ? nth(wave) : begin_tiles(0);
+            int32_t at = exists(unit) ? begin_of(unit.node) : 0, n;
+            Positions here = positions(at);
+            while (exists(unit)) {
+                Unit next = unit;
+                if (any) {
+                    int32_t taken = 0;
+                    if (lane == 0) {
+                        taken = atomicAdd(bucket.counter, 1);
+                    }
+                    next = nth(WAVES + __builtin_amdgcn_readfirstlane(taken));
+                } else {
+                    // (a group of three tiles is the last one)
+                    const int32_t first = alone(unit) ? p.column_tiles - 3 : unit.tile - wave % unit.step;
+                    if (alone(unit) && unit.tile < first + 2) {
+                        next.tile++;
+                    } else {
+                        next.node += WAVES / unit.step;
+                        next.tile = alone(unit) ? first : unit.tile;
+                        if (next.node >= (unit.step == 3 && wave < 3 ? last_quarter : node1)) {
+                            next = begin_tiles(first + unit.step);
+                        }
+                    }
+                }
+                const int32_t after = exists(next) ? begin_of(next.node) : 0;
+                tile = unit.tile;
+                columns_of.set_tile(tile);
+                clear();
+                do {
+                    n = min(WAVE, begin_of(unit.node + 1) - at);
+                    add_up(here, at, n, n == WAVE ? at + n : after);
+                    at += n;
+                } while (n == WAVE);
+                finish(unit.node);
+                unit = next;
+                at = after;
+            }
+        } else {
+            int32_t at = LISTS == ORDERED ? begin_of(node0) : lower_bound(p.sorted, p.n_edges, node0, lane), n;
+            Positions here = positions(at);
+            for (int32_t node = node0; node < node1; node++) {
+                clear();
+                do {
+                    if constexpr (LISTS == SEGMENTS) {
+                        const unsigned long long others = __ballot(!here.inside || here.name != node);
+                        n = others == 0 ? WAVE : __ffsll(others) - 1;
+                    } else {
+                        n = min(WAVE, begin_of(node + 1) - at);
+                    }
+                    add_up(here, at, n, at + n);
+                    at += n;
+                } while (n == WAVE);
+                finish(node);
+            }
         }
     }
 }
@@ -833,6 +898,7 @@ template <typename T> struct EdgeArgs {
     T* grad_A;            // [n_edges][nA], may be null
     T* grad_B;            // [n_edges][L], may be null
     int32_t shares;       // wavefronts per node, each with a share of its edges (0: a share of all edges)
+    int32_t late, less;   // the first `late` shares of all edges have `less` edges less than the others
 };
 
 /// How a wavefront shares out its lanes: several edges side by side where G fits the registers of a lane.
@@ -862,7 +928,7 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
 
     Columns<T, S> columns_of(p);
     const int lane = columns_of.lane;
-    build<T, S, true>(table, owner, p.C, p.table);
+    build<T, S, true>(table, owner, p.C, p.table, [] {});
 
     const int32_t range = block * WAVES + wave;
     if (range >= p.ranges) {
@@ -876,8 +942,11 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
         bounds_of(p.sorted, p.n_edges, range / args.shares, lane, first, last);
         n_all = last - first;
     }
-    const int32_t begin = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * share / shares);
-    const int32_t end = first + static_cast<int32_t>(static_cast<int64_t>(n_all) * (share + 1) / shares);
+    auto begin_of = [&](int32_t which) {
+        const int32_t less = args.less * min(which, args.late);
+        return first + static_cast<int32_t>((static_cast<int64_t>(n_all) + args.less * args.late) * which / shares) - less;
+    };
+    const int32_t begin = begin_of(share), end = begin_of(share + 1);
     BufferOf<T> G;
     const uint32_t g_block_bytes = static_cast<uint32_t>(p.table.n_out) * columns_of.row_bytes;
     G.set(args.grad_output, static_cast<uint32_t>(p.n_blocks) * g_block_bytes);
@@ -1078,10 +1147,16 @@ __device__ __forceinline__ void edge_gradients(const EdgeArgs<T>& args, char* ld
     }
 }
 
+/// The first plan.shares workgroups split `senders` before their part of the edges, which is the smaller for it.
 template <typename T, int N, int COLUMNS>
 __global__ __launch_bounds__(THREADS)
-__attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void edge_kernel(const EdgeArgs<T> args) {
+__attribute__((amdgpu_waves_per_eu(edge_waves<T, N, COLUMNS>()))) void
+edge_kernel(const EdgeArgs<T> args, const Shares shares, const SharePlan plan, const int32_t* __restrict__ senders) {
     extern __shared__ __align__(16) char lds[];
+    if (static_cast<int32_t>(blockIdx.x) < plan.shares) { // (uniform)
+        split_share<THREADS>(reinterpret_cast<int32_t*>(lds), shares, plan, senders, blockIdx.x);
+        __syncthreads();
+    }
     edge_gradients<T, N, COLUMNS>(args, lds, blockIdx.x);
 }
 
@@ -1096,7 +1171,7 @@ __attribute__((amdgpu_waves_per_eu(std::min(contract_waves<T, N, COLUMNS>(), edg
 small_kernel(const ContractArgs<T> of_nodes, const EdgeArgs<T> of_edges, int32_t nodes) {
     extern __shared__ __align__(16) char lds[];
     if (static_cast<int32_t>(blockIdx.x) < nodes) { // (uniform)
-        contract<T, N, COLUMNS, SLOTS, true>(of_nodes, lds, blockIdx.x);
+        contract<T, N, COLUMNS, LOOKED_FOR, true>(of_nodes, lds, blockIdx.x);
     } else {
         edge_gradients<T, N, COLUMNS>(of_edges, lds, blockIdx.x - nodes);
     }
@@ -1179,23 +1254,32 @@ Walk<T> walk_of(
     return w;
 }
 
+/// Workgroups of a sum on the device at a time.
+template <typename T, int N, int COLUMNS> int64_t resident_sums() {
+    return static_cast<int64_t>(compute_units()) * contract_waves<T, N, COLUMNS>();
+}
+
 template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Shape& s, hipStream_t stream) {
     with_layout<T, false>(s, [&](auto n, auto columns) {
         constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
         Walk<T>& w = args.walk;
-        constexpr size_t lds = contract_lds<T, N, COLUMNS>();
+        const size_t lds = LISTS == BUCKETS ? contract_lds<T, N, COLUMNS>(args.plan.per_bucket) : contract_lds<T, N, COLUMNS>();
         w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
-        const int64_t resident = static_cast<int64_t>(compute_units()) * contract_waves<T, N, COLUMNS>(); // workgroups
         auto launch = [&](auto kernel, int64_t ranges, int waves_per_range) {
             w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, std::max<int64_t>(1, ranges)));
-            const size_t waves = static_cast<size_t>(w.ranges) * w.column_tiles * waves_per_range;
+            const size_t waves = static_cast<size_t>(w.ranges) * waves_per_range;
             allow_lds(kernel, lds);
             kernel<<<static_cast<unsigned>(ceil_div(waves, WAVES)), THREADS, lds, stream>>>(args);
         };
-        if (static_cast<int64_t>(s.n_nodes) * w.column_tiles <= resident) {
-            launch(contract_kernel<T, N, COLUMNS, LISTS, true>, s.n_nodes, WAVES);
+        const int64_t resident = resident_sums<T, N, COLUMNS>();
+        const bool shared = LISTS == BUCKETS ? args.plan.multiplier == 0
+                                             : static_cast<int64_t>(s.n_nodes) * w.column_tiles <= resident;
+        if (shared) {
+            launch(contract_kernel<T, N, COLUMNS, LISTS, true>, s.n_nodes, WAVES * w.column_tiles);
+        } else if (LISTS == BUCKETS) {
+            launch(contract_kernel<T, N, COLUMNS, LISTS, false>, args.plan.buckets, WAVES);
         } else {
-            launch(contract_kernel<T, N, COLUMNS, LISTS, false>, resident * WAVES / w.column_tiles, 1);
+            launch(contract_kernel<T, N, COLUMNS, LISTS, false>, resident * WAVES / w.column_tiles, w.column_tiles);
         }
     });
     MOPS_HIP_CHECK(hipGetLastError());
@@ -1274,15 +1358,34 @@ template <typename T, int N, int COLUMNS> size_t share_out(EdgeArgs<T>& args, co
 
 } // namespace
 
+template <typename T> SenderLists plan_lists(const Shape& s) {
+    SenderLists lists{};
+    with_layout<T, false>(s, [&](auto n, auto columns) {
+        constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
+        const int32_t tiles = (s.L + COLUMNS - 1) / COLUMNS;
+        const int64_t resident = resident_sums<T, N, COLUMNS>();
+        // A node by a workgroup for each of its tiles if there are no more of them than run at a time; else as many
+        // buckets as workgroups run at a time (fewer would leave some idle), or twice or four times as many.
+        const bool shared = static_cast<int64_t>(s.n_nodes) * tiles <= resident;
+        for (int64_t buckets = shared ? s.n_nodes : std::min<int64_t>(resident, s.n_nodes);
+             buckets <= MOST_SHARE_BUCKETS && !lists.in_shares; buckets *= 2) {
+            lists.in_shares = plan_shares(lists.plan, s.n_nodes, s.n_edges, static_cast<int32_t>(buckets));
+        }
+        lists.copies = lists.plan.multiplier == 0 ? tiles : 1;
+    });
+    return lists;
+}
+
 template <typename T>
 void weight_gradient(
     T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& s,
-    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+    const SenderLists* lists, void* workspace, const EdgesBySender* ordered, hipStream_t stream
 ) {
     ContractArgs<T> args = of_senders(grad_W, grad_output, A, B, C, indices, s);
-    if (slots != nullptr) {
-        args.slots = *slots;
-        contract<T, SLOTS>(args, s, stream);
+    if (lists != nullptr) {
+        args.plan = lists->plan;
+        args.shares = shares_in(workspace, lists->plan);
+        contract<T, BUCKETS>(args, s, stream);
     } else {
         args.ordered = *ordered;
         contract<T, ORDERED>(args, s, stream);
@@ -1292,17 +1395,29 @@ void weight_gradient(
 template <typename T>
 void edge_gradients(
     T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
-    const Shape& s, hipStream_t stream
+    const Shape& s, const SenderLists* lists, void* workspace, hipStream_t stream
 ) {
     EdgeArgs<T> args = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
+    SharePlan plan{};
+    Shares shares{};
+    if (lists != nullptr) {
+        plan = lists->plan;
+        shares = shares_in(workspace, plan);
+    }
     MainKernelTimer timer(stream);
     with_layout<T, true>(s, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
-        constexpr size_t lds = edge_lds<T, N, COLUMNS>();
-        const size_t blocks = share_out<T, N, COLUMNS>(args, s);
+        const size_t lds =
+            std::max(edge_lds<T, N, COLUMNS>(), split_lds<THREADS>(plan.buckets) * sizeof(int32_t));
+        const size_t blocks = std::max(share_out<T, N, COLUMNS>(args, s), static_cast<size_t>(plan.shares));
+        if (args.shares == 0) {
+            // (splitting 1024 edges takes as long as some six edges of a wavefront's part, 4096 as 18)
+            args.late = std::min(plan.shares * WAVES, args.walk.ranges);
+            args.less = std::min(2 + plan.share / 256, s.n_edges / args.walk.ranges / 2);
+        }
         auto kernel = edge_kernel<T, N, COLUMNS>;
         allow_lds(kernel, lds);
-        kernel<<<static_cast<unsigned>(blocks), THREADS, lds, stream>>>(args);
+        kernel<<<static_cast<unsigned>(blocks), THREADS, lds, stream>>>(args, shares, plan, indices.W_1);
     });
     MOPS_HIP_CHECK(hipGetLastError());
 }
@@ -1344,10 +1459,11 @@ void small_vjp(
         T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t      \
     );                                                                                             \
     template void edge_gradients<T>(                                                               \
-        T*, T*, const T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t \
+        T*, T*, const T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, const SenderLists*, void*, hipStream_t \
     );                                                                                             \
+    template SenderLists plan_lists<T>(const Shape&);                                              \
     template void weight_gradient<T>(                                                              \
-        T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, const SenderSlots*, const EdgesBySender*, hipStream_t \
+        T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, const SenderLists*, void*, const EdgesBySender*, hipStream_t \
     );                                                                                             \
     template void small_vjp<T>(                                                                    \
         T*, T*, T*, const T*, const T*, const T*, const T*, const T*, const Indices&, const Shape&, hipStream_t \

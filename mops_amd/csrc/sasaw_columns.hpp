@@ -12,6 +12,7 @@
 #include "dispatch_thresholds.hpp"
 #include "sasaw_mfma.hpp"
 #include "sender_buckets.hpp"
+#include "sender_shares.hpp"
 
 namespace mops::amd::sasaw_columns {
 
@@ -36,19 +37,29 @@ void forward(
     hipStream_t stream
 );
 
-/// grad_A, grad_B: either may be null.
+/// How the edges of every sender are found for grad_W: in shares and buckets (sender_shares.hpp) which
+/// the launch for grad_A and grad_B splits the index into, or, if not in_shares, by a counting sort.
+struct SenderLists {
+    SharePlan plan;
+    int32_t copies; // workgroups with the same bucket
+    bool in_shares;
+    size_t bytes() const { return shares_bytes(plan, copies); }
+};
+template <typename T> SenderLists plan_lists(const Shape& shape);
+
+/// grad_A, grad_B: either may be null, but not both. `lists`: those to begin in `workspace`, or null.
 template <typename T>
 void edge_gradients(
     T* grad_A, T* grad_B, const T* grad_output, const T* A, const T* B, const T* C, const T* W, const Indices& indices,
-    const Shape& shape, hipStream_t stream
+    const Shape& shape, const SenderLists* lists, void* workspace, hipStream_t stream
 );
 
-/// The edges of every sender in slots, or in the order of their senders: one of
-/// the two is null.
+/// The edges of every sender in the lists begun in `workspace`, or in the order of their senders: one of the
+/// two is null.
 template <typename T>
 void weight_gradient(
     T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const Indices& indices, const Shape& shape,
-    const SenderSlots* slots, const EdgesBySender* ordered, hipStream_t stream
+    const SenderLists* lists, void* workspace, const EdgesBySender* ordered, hipStream_t stream
 );
 
 /// Whether a graph is small enough that all its gradients are one launch, in which every sender's edges are

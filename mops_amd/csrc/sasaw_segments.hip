@@ -1517,17 +1517,18 @@ bool vjp_supported(const Shape& s, size_t element_size, bool want_grad_W) {
            (!want_grad_W || static_cast<size_t>(s.n_edges) <= static_cast<size_t>(s.n_nodes) * thresholds::ARRIVAL_MEAN_EDGES);
 }
 
-/// Whether grad_W of vjp_by_columns() gets its edges by a counting sort and not in slots.
-static bool columns_in_order(const Shape& s) {
-    return dense_for_slots(s) || static_cast<size_t>(s.n_nodes) * s.n_edges > thresholds::SLOT_PRODUCT;
+/// How grad_W of vjp_by_columns() finds a sender's edges.
+static sasaw_columns::SenderLists column_lists(const Shape& s, size_t element_size) {
+    return element_size == 4 ? sasaw_columns::plan_lists<float>(s) : sasaw_columns::plan_lists<double>(s);
 }
 
-size_t vjp_workspace_bytes(const Shape& s, size_t element_size, bool want_grad_W) {
-    if (vjp_by_columns(s, element_size) && sasaw_columns::small(s, element_size)) {
-        return 0;
-    }
-    if (want_grad_W && vjp_by_columns(s, element_size) && columns_in_order(s)) {
-        return edges_by_sender_bytes(s.n_nodes, s.n_edges, false);
+size_t vjp_workspace_bytes(const Shape& s, size_t element_size, bool want_grad_W, bool shares) {
+    if (vjp_by_columns(s, element_size)) {
+        if (!want_grad_W || sasaw_columns::small(s, element_size)) {
+            return 0;
+        }
+        const sasaw_columns::SenderLists lists = column_lists(s, element_size);
+        return shares && lists.in_shares ? lists.bytes() : edges_by_sender_bytes(s.n_nodes, s.n_edges, false);
     }
     return want_grad_W ? sender_slots_bytes(s.n_nodes) : 0; // (enough for either way of listing)
 }
@@ -1664,7 +1665,7 @@ void launch_gradients(
 template <typename T>
 void vjp(
     T* grad_A, T* grad_B, T* grad_W, const T* grad_output, const T* A, const T* B, const T* C, const T* W,
-    const Indices& indices, const Shape& s, void* workspace, int32_t* counters, bool counters_are_zero,
+    const Indices& indices, const Shape& s, void* workspace, bool shares, int32_t* counters, bool counters_are_zero,
     hipStream_t stream
 ) {
     GradientArgs<T> args{};
@@ -1686,18 +1687,29 @@ void vjp(
         return;
     }
     if (vjp_by_columns(s, sizeof(T))) {
-        if (grad_A != nullptr || grad_B != nullptr) {
-            sasaw_columns::edge_gradients<T>(grad_A, grad_B, grad_output, A, B, C, W, indices, s, stream);
+        const bool want_edges = grad_A != nullptr || grad_B != nullptr;
+        sasaw_columns::SenderLists plan{};
+        const sasaw_columns::SenderLists* lists = nullptr;
+        if (grad_W != nullptr && shares) {
+            plan = sasaw_columns::plan_lists<T>(s);
+            lists = plan.in_shares ? &plan : nullptr;
         }
-        if (grad_W != nullptr && columns_in_order(s)) {
-            const EdgesBySender ordered =
-                order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, false, workspace, stream);
+        if (want_edges) {
+            sasaw_columns::edge_gradients<T>(
+                grad_A, grad_B, grad_output, A, B, C, W, indices, s, lists, workspace, stream
+            );
+        } else if (lists != nullptr) {
+            split_shares(shares_in(workspace, plan.plan), plan.plan, indices.W_1, stream);
+        }
+        if (grad_W != nullptr) {
+            EdgesBySender ordered{};
+            if (lists == nullptr) {
+                ordered = order_edges_by_sender(indices.W_1, s.n_edges, s.n_nodes, false, workspace, stream);
+            }
             test_failure_point("sasaw_vjp_after_listing");
-            sasaw_columns::weight_gradient<T>(grad_W, grad_output, A, B, C, indices, s, nullptr, &ordered, stream);
-        } else if (grad_W != nullptr) {
-            const SenderSlots slots = list_edges_in_slots(indices.W_1, s.n_edges, s.n_nodes, workspace, stream);
-            test_failure_point("sasaw_vjp_after_listing");
-            sasaw_columns::weight_gradient<T>(grad_W, grad_output, A, B, C, indices, s, &slots, nullptr, stream);
+            sasaw_columns::weight_gradient<T>(
+                grad_W, grad_output, A, B, C, indices, s, lists, workspace, lists == nullptr ? &ordered : nullptr, stream
+            );
         }
         return;
     }
@@ -1759,11 +1771,11 @@ template void forward<double>(
 );
 template void vjp<float>(
     float*, float*, float*, const float*, const float*, const float*, const float*, const float*, const Indices&,
-    const Shape&, void*, int32_t*, bool, hipStream_t
+    const Shape&, void*, bool, int32_t*, bool, hipStream_t
 );
 template void vjp<double>(
     double*, double*, double*, const double*, const double*, const double*, const double*, const double*,
-    const Indices&, const Shape&, void*, int32_t*, bool, hipStream_t
+    const Indices&, const Shape&, void*, bool, int32_t*, bool, hipStream_t
 );
 
 } // namespace mops::amd::sasaw_segments

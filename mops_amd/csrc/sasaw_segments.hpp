@@ -33,9 +33,10 @@ void forward(
 /// Whether vjp() serves the shape (grad_W needs a sparse graph: at most 48
 /// edges per node on average), the device scratch it needs and the number of
 /// 32-bit counters (see SenderArrivals in sender_buckets.hpp). vjp() makes no
-/// allocation and uses no second stream.
+/// allocation and uses no second stream. `shares`: whether the senders' edges may be
+/// listed in shares (sender_shares.hpp), the faster way, which can need more scratch.
 bool vjp_supported(const Shape& shape, size_t element_size, bool want_grad_W);
-size_t vjp_workspace_bytes(const Shape& shape, size_t element_size, bool want_grad_W);
+size_t vjp_workspace_bytes(const Shape& shape, size_t element_size, bool want_grad_W, bool shares);
 size_t vjp_counters(const Shape& shape, size_t element_size, bool want_grad_W);
 
 /// Any of grad_A, grad_B, grad_W may be null (not all). `counters`: the
@@ -45,8 +46,8 @@ size_t vjp_counters(const Shape& shape, size_t element_size, bool want_grad_W);
 template <typename T>
 void vjp(
     T* grad_A, T* grad_B, T* grad_W, const T* grad_output, const T* A, const T* B, const T* C,
-    const T* W, const Indices& indices, const Shape& shape, void* workspace, int32_t* counters,
-    bool counters_are_zero, hipStream_t stream
+    const T* W, const Indices& indices, const Shape& shape, void* workspace, bool shares,
+    int32_t* counters, bool counters_are_zero, hipStream_t stream
 );
 
 } // namespace mops::amd::sasaw_segments

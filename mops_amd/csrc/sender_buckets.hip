@@ -4,6 +4,8 @@
 #include <type_traits>
 
 #include "runtime.hpp"
+#include "sender_shares.hpp"
+#include "wave_sort.hpp"
 
 namespace mops::amd {
 
@@ -22,179 +24,10 @@ namespace {
 // over 10 000: 27; what they wait for is one dependent load after the other.
 constexpr int SORT_THREADS = 1024;
 constexpr int32_t MOST_BUCKETS = 512;
-constexpr int32_t MOST_SHARES = 256;         // workgroups of the first level
 constexpr int32_t SENDERS_AT_A_TIME = 4096;  // of the second level: counters in LDS
 
 constexpr int HELD = 4;                      // positions a lane keeps from counting to placing
 constexpr int32_t STAGED = 5120;             // edges of a bucket that are put in order in LDS
-constexpr int BATCH = 4;                     // positions beyond those that it asks for at once
-
-/// What lies at a position: an edge, its sender, and what it is sorted by (negative: it is not).
-struct Item {
-    int32_t key, edge, sender;
-};
-
-/// The lanes of a wavefront with the same key, and how many of them are below this one.
-struct Ranked {
-    uint64_t same;
-    uint32_t before;
-};
-__device__ __forceinline__ Ranked rank_in_wave(int32_t key, bool valid, int bits, int lane) {
-    uint64_t same = __ballot(valid);
-    for (int b = 0; b < bits; b++) {
-        const bool set = (key >> b & 1) != 0;
-        const uint64_t with = __ballot(set);
-        same &= set ? with : ~with;
-    }
-    return Ranked{same, static_cast<uint32_t>(__popcll(same & ((uint64_t(1) << lane) - 1)))};
-}
-
-/// A wavefront's share [begin, end) of the positions a workgroup has.
-struct Share {
-    int32_t begin, end;
-    __device__ __forceinline__ Share(int32_t first, int32_t last, int wave, int waves) {
-        const int32_t each = ((last - first + waves - 1) / waves + WAVE - 1) / WAVE * WAVE;
-        begin = min(first + wave * each, last);
-        end = min(begin + each, last);
-    }
-};
-
-/// The first HELD items of a lane: those of most shares all told, so that they are read once.
-template <int HELD, typename ItemAt>
-__device__ __forceinline__ void hold_items(Item (&held)[HELD], const Share& share, int lane, ItemAt&& item_at) {
-#pragma unroll
-    for (int u = 0; u < HELD; u++) {
-        held[u] = item_at(max(min(share.begin + u * WAVE + lane, share.end - 1), 0));
-    }
-}
-
-/// counters[wavefront][key] := how many of the wavefront's items have the key.
-template <int HELD, typename ItemAt>
-__device__ __forceinline__ void count_keys(
-    const Item (&held)[HELD], int32_t* counters, int32_t keys, const Share& share, int wave, int waves, int lane,
-    ItemAt&& item_at
-) {
-    for (int32_t i = threadIdx.x; i < waves * keys; i += blockDim.x) {
-        counters[i] = 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < HELD; u++) {
-        if (share.begin + u * WAVE + lane < share.end && held[u].key >= 0) {
-            atomicAdd(&counters[wave * keys + held[u].key], 1);
-        }
-    }
-    for (int32_t at = share.begin + HELD * WAVE + lane; at - lane < share.end; at += BATCH * WAVE) {
-        int32_t key[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; u++) {
-            key[u] = item_at(min(at + u * WAVE, share.end - 1)).key;
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; u++) {
-            if (at + u * WAVE < share.end && key[u] >= 0) {
-                atomicAdd(&counters[wave * keys + key[u]], 1);
-            }
-        }
-    }
-    __syncthreads();
-}
-
-/// put(place, item) for every item that has a key, items of one key in ascending places:
-/// counters[wavefront][key] is the place of the wavefront's first one.
-template <int HELD, typename ItemAt, typename Put>
-__device__ __forceinline__ void place_keys(
-    const Item (&held)[HELD], int32_t* counters, int32_t keys, int bits, const Share& share, int wave, int lane,
-    ItemAt&& item_at, Put&& put
-) {
-    int32_t* mine = counters + static_cast<size_t>(wave) * keys;
-    auto place_one = [&](const Item& item, int32_t at) {
-        const bool valid = at < share.end && item.key >= 0;
-        const Ranked ranked = rank_in_wave(item.key, valid, bits, lane);
-        const int32_t place = valid ? mine[item.key] + static_cast<int32_t>(ranked.before) : 0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (valid && ranked.before == 0) {
-            mine[item.key] += __popcll(ranked.same);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (valid) {
-            put(place, item);
-        }
-    };
-#pragma unroll
-    for (int u = 0; u < HELD; u++) {
-        if (share.begin + u * WAVE < share.end) { // (uniform)
-            place_one(held[u], share.begin + u * WAVE + lane);
-        }
-    }
-    for (int32_t at = share.begin + HELD * WAVE + lane; at - lane < share.end; at += BATCH * WAVE) {
-        Item item[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; u++) {
-            item[u] = item_at(min(at + u * WAVE, share.end - 1));
-        }
-#pragma unroll
-        for (int u = 0; u < BATCH; u++) {
-            place_one(item[u], at + u * WAVE);
-        }
-    }
-}
-
-/// Turns counters[wavefront][key] into the place of the wavefront's first of each key:
-/// start_of(key) and what the wavefronts before have. All threads.
-template <int WAVES, typename StartOf>
-__device__ __forceinline__ void starts_of_waves(int32_t* counters, int32_t keys, StartOf&& start_of) {
-    for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
-        int32_t here[WAVES];
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            here[w] = counters[w * keys + key];
-        }
-        int32_t place = start_of(key);
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            counters[w * keys + key] = place;
-            place += here[w];
-        }
-    }
-    __syncthreads();
-}
-
-/// values[0 .. n) := `first` + the sum of those before; returns `first` + the sum of all. All
-/// threads; `of_wave`: an integer per wavefront.
-template <int WAVES>
-__device__ __forceinline__ int32_t scan_in_place(int32_t* values, int32_t n, int32_t first, int32_t* of_wave) {
-    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-    int32_t carry = first;
-    for (int32_t base = 0; base < n; base += blockDim.x) {
-        const int32_t i = base + threadIdx.x;
-        const int32_t value = i < n ? values[i] : 0;
-        int32_t sum = value;
-#pragma unroll
-        for (int step = 1; step < WAVE; step <<= 1) {
-            const int32_t other = __shfl_up(sum, step);
-            sum += lane >= step ? other : 0;
-        }
-        if (lane == WAVE - 1) {
-            of_wave[wave] = sum;
-        }
-        __syncthreads();
-        int32_t ahead = carry;
-#pragma unroll
-        for (int w = 0; w < WAVES; w++) {
-            ahead += w < wave ? of_wave[w] : 0;
-            carry += of_wave[w];
-        }
-        if (i < n) {
-            values[i] = ahead + sum - value;
-        }
-        __syncthreads();
-    }
-    return carry;
-}
 
 /// counts[workgroup][pitch]: how many in every bucket of the workgroup's share of the edges.
 __global__ __launch_bounds__(SORT_THREADS) void count_buckets_kernel(
@@ -244,7 +77,7 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
     int32_t* of_wave = total + pitch;
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     const int32_t first = blockIdx.x * share, last = first + min(share, n_edges - first);
-    const Share mine(first, last, wave, WAVES);
+    const WaveShare mine(first, last, wave, WAVES);
     auto item_at = [&](int32_t e) {
         const int32_t sender = senders[e];
         return Item{in_bounds(sender, n_nodes) ? sender >> shift : -1, e, sender};
@@ -253,9 +86,8 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
         before[b] = 0;
         total[b] = 0;
     }
-    Item held[HELD];
-    hold_items(held, mine, lane, item_at);
-    count_keys(held, counters, pitch, mine, wave, WAVES, lane, item_at);
+    const Held<HELD> held(mine, lane, item_at);
+    count_keys<4>(held, counters, pitch, mine, wave, WAVES, lane, item_at);
     // what the workgroups before have of every bucket, and all of them: several threads per bucket
     // (of a single workgroup, the counts it has just made)
     const int32_t* all_counts = gridDim.x > 1 ? counts : counters;
@@ -302,7 +134,7 @@ __global__ __launch_bounds__(SORT_THREADS) void fill_buckets_kernel(
     starts_of_waves<WAVES>(counters, pitch, [&](int32_t bucket) { return total[bucket] + before[bucket]; });
     // (two levels: the sender's place in its bucket beside the edge, where both go into one word)
     const int32_t of_bucket = (1 << shift) - 1;
-    place_keys(held, counters, pitch, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+    place_keys<4>(held, counters, pitch, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
         edge_of_place[place] = packed_above < 32 ? item.edge | (item.sender & of_bucket) << packed_above : item.edge;
         if (sender_of_place != nullptr) {
             sender_of_place[place] = item.sender;
@@ -335,7 +167,7 @@ __global__ __launch_bounds__(WAVES* WAVE) void sort_buckets_kernel(
     int32_t* of_wave = start + at_a_time;
     int32_t* staged = of_wave + WAVES;
     const int32_t begin = bucket_offsets[blockIdx.x], end = bucket_offsets[blockIdx.x + 1];
-    const Share mine(begin, end, wave, WAVES);
+    const WaveShare mine(begin, end, wave, WAVES);
     const int32_t node0 = static_cast<int32_t>(blockIdx.x) << shift;
     const int32_t nodes = min(1 << shift, n_nodes - node0);
     const bool packed = packed_above < 32;
@@ -351,9 +183,8 @@ __global__ __launch_bounds__(WAVES* WAVE) void sort_buckets_kernel(
             const int32_t key = of_bucket - base;
             return Item{in_bounds(key, keys) ? key : -1, static_cast<int32_t>(word & edge_mask), node0 + of_bucket};
         };
-        Item held[HELD];
-        hold_items(held, mine, lane, item_at);
-        count_keys(held, counters, keys, mine, wave, WAVES, lane, item_at);
+        const Held<HELD> held(mine, lane, item_at);
+        count_keys<4>(held, counters, keys, mine, wave, WAVES, lane, item_at);
         for (int32_t key = threadIdx.x; key < keys; key += blockDim.x) {
             int32_t sum = 0;
 #pragma unroll
@@ -368,7 +199,7 @@ __global__ __launch_bounds__(WAVES* WAVE) void sort_buckets_kernel(
             offsets[node0 + base + key] = start[key];
         }
         starts_of_waves<WAVES>(counters, keys, [&](int32_t key) { return start[key]; });
-        place_keys(held, counters, keys, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+        place_keys<4>(held, counters, keys, bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
             if (in_lds) {
                 staged[place - begin] = item.edge | item.key << packed_above;
             } else {
@@ -400,6 +231,14 @@ __global__ __launch_bounds__(WAVES* WAVE) void sort_buckets_kernel(
             }
         }
     }
+}
+
+constexpr int SPLIT_THREADS = 512;
+
+__global__ __launch_bounds__(SPLIT_THREADS) void
+split_shares_kernel(const Shares to, const SharePlan plan, const int32_t* __restrict__ senders) {
+    extern __shared__ int32_t lds[];
+    split_share<SPLIT_THREADS>(lds, to, plan, senders, blockIdx.x);
 }
 
 // Sparse graphs: one launch of list_in_slots_block (sender_buckets.hpp), four
@@ -519,6 +358,54 @@ SortPlan sort_plan(int32_t n_nodes, int32_t n_edges) {
     return plan;
 }
 } // namespace
+
+bool plan_shares(SharePlan& plan, int32_t n_nodes, int32_t n_edges, int32_t buckets) {
+    if (n_nodes < 1 || n_edges < 1 || buckets < 1 || buckets > n_nodes || buckets > MOST_SHARE_BUCKETS) {
+        return false;
+    }
+    plan.n_edges = n_edges;
+    plan.n_nodes = n_nodes;
+    const size_t each = ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(MOST_SHARES) * SHARE_STEP);
+    plan.share = static_cast<int32_t>(each) * SHARE_STEP;
+    plan.shares = static_cast<int32_t>(ceil_div(static_cast<size_t>(n_edges), static_cast<size_t>(plan.share)));
+    plan.buckets = buckets;
+    plan.multiplier = 0;
+    plan.senders_each = 0;
+    plan.per_bucket = 1;
+    if (buckets < n_nodes) {
+        plan.multiplier = static_cast<uint32_t>((static_cast<uint64_t>(buckets) << 32) / static_cast<uint64_t>(n_nodes));
+        plan.senders_each = 4294967296.0 / plan.multiplier;
+        plan.per_bucket = static_cast<int32_t>((uint64_t(1) << 32) / plan.multiplier + 1);
+    }
+    plan.bucket_bits = bits_for(buckets);
+    plan.sender_bits = bits_for(plan.per_bucket);
+    return each * SHARE_STEP <= MOST_SHARE_EDGES && plan.per_bucket <= MOST_PER_BUCKET &&
+           bits_for(n_edges) + plan.sender_bits <= 32 &&
+           static_cast<int64_t>(n_edges) <= static_cast<int64_t>(buckets) * BUCKET_EDGES / 4 * 3;
+}
+
+size_t shares_bytes(const SharePlan& plan, int32_t copies) {
+    return align256(static_cast<size_t>(plan.shares) * plan.share * 4) +
+           align256(static_cast<size_t>(plan.buckets) * MOST_SHARES * 4) +
+           static_cast<size_t>(copies) * plan.n_edges * 4;
+}
+
+Shares shares_in(void* workspace, const SharePlan& plan) {
+    char* at = static_cast<char*>(workspace);
+    Shares shares;
+    shares.words = reinterpret_cast<uint32_t*>(at);
+    at += align256(static_cast<size_t>(plan.shares) * plan.share * 4);
+    shares.starts = reinterpret_cast<uint32_t*>(at);
+    at += align256(static_cast<size_t>(plan.buckets) * MOST_SHARES * 4);
+    shares.lists = reinterpret_cast<int32_t*>(at);
+    return shares;
+}
+
+void split_shares(const Shares& to, const SharePlan& plan, const int32_t* senders, hipStream_t stream) {
+    const size_t lds = static_cast<size_t>(split_lds<SPLIT_THREADS>(plan.buckets)) * sizeof(int32_t);
+    split_shares_kernel<<<plan.shares, SPLIT_THREADS, lds, stream>>>(to, plan, senders);
+    MOPS_HIP_CHECK(hipGetLastError());
+}
 
 size_t edges_by_sender_bytes(int32_t n_nodes, int32_t n_edges, bool with_senders) {
     if (n_nodes < 1) {

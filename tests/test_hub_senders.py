@@ -5,8 +5,8 @@ the oracle.
 The hubs are the first and the last sender, two next to each other and one alone; the index is longer
 than the 1024 positions that are looked at together and does not come out even in quarters; the
 per-edge rows have one, two and four columns per lane; edges in slots and by arrival, below and above
-48 edges per sender on average. (`slots` of SASAW: one launch that looks through the index for every sender,
-but for 16 components in double; lists in slots that a workgroup shares: test_sasaw_columns.py.)
+48 edges per sender on average. (SASAW lists its senders' edges otherwise, but where it looks through the index
+for every sender, in `slots` here but for 16 components in double; see test_sasaw_columns.py.)
 """
 import numpy as np
 import pytest

@@ -113,10 +113,43 @@ def test_one_node_has_a_third_of_the_edges(oracle, device, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize(
+    "shape",
+    [  # edges, nodes, components, columns, edges of one sender
+        (17003, 401, 9, 16, 3000),  # a sender by a workgroup, more of its edges than fit into LDS
+        (60007, 2003, 9, 32, 2500),  # two to four to a bucket
+        (60007, 2003, 16, 40, 5),  # three tiles of columns and few nodes, more than three tiles
+        (90001, 4503, 9, 70, 2100),
+        (90001, 4503, 4, 200, 5),
+        (262144, 5003, 4, 3, 40000),  # as many shares as there can be, a sender with edges in all of them
+        (262145, 40009, 4, 2, 5),  # fewer, larger shares
+        (150001, 70001, 4, 3, 2100),  # senders beyond 16 bits, most of them with one edge or two
+    ],
+    ids=lambda s: "x".join(map(str, s)),
+)
+def test_buckets_of_senders(oracle, device, shape, dtype):
+    """The senders' edges in shares and buckets (mops_amd/csrc/sender_shares.hpp), split by the launch for the other
+    gradients and by one of its own."""
+    edges, nodes, n, columns, of_hub = shape
+    case = support.sasaw_case(
+        edges + columns, dtype, E=edges, nA=n, L=columns, n_nodes=nodes, n2=n, n3=n, N=40, allow_empty=True
+    )
+    hub = np.random.default_rng(3).permutation(edges)[:of_hub]
+    case["indices_W_1"][hub] = nodes - 3
+    exact = cpu_vjp(oracle, "sasaw", support.in_float64(case))["W"]
+    other = cpu_vjp(oracle, "sasaw", case if dtype == np.float32 else support.magnitudes(case))["W"]
+    on_device = to_device(case, device)
+    together, alone = hip_vjp("sasaw", on_device)["W"], hip_vjp("sasaw", on_device, wanted=["W"])["W"]
+    assert (together == alone).all()
+    same, terms = (other, None) if dtype == np.float32 else (None, other)
+    support.assert_calibrated(together.cpu().numpy(), exact, dtype, f"{shape} grad_W", same, terms)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("components", [4, 9, 16])
 def test_listed_senders_shared_by_a_workgroup(oracle, device, components, dtype):
-    """Lists in slots whose entries the wavefronts of a workgroup share (more than 16 384 edges, no more nodes
-    than workgroups at a time): around 64 and 128 entries, parts that overflow, senders outside the tensor."""
+    """Lists whose entries the wavefronts of a workgroup share (more than 16 384 edges, no more nodes
+    than workgroups at a time): around 64 and 128 entries, senders outside the tensor."""
     import torch
 
     edges, nodes, columns = 17003, 401, 16
