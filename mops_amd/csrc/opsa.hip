@@ -49,6 +49,7 @@
 #include "opsa_edges.hpp"
 #include "segment_walk.hpp"
 #include "sender_buckets.hpp"
+#include "sender_shares.hpp"
 #include "sender_gather.hpp"
 
 namespace mops::amd {
@@ -1553,20 +1554,14 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_slotted_rows_kernel(
 // of a row per lane, any number of rows of columns). What bounds it is the gather
 // of the rows, BATCH loads in flight: 1 000 000 rows of 32 floats, 53.9 us with a
 // row per load, 26.4 us with two.
-template <typename T, int PARTS, int COLUMNS>
-__global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_listed_rows_kernel(
-    T* __restrict__ grad_W, const T* __restrict__ edge_W, const int32_t* __restrict__ offsets,
-    const int32_t* __restrict__ edge_of_position, int32_t n_nodes, int32_t L
+template <typename T, int PARTS, int COLUMNS, typename EdgeAt>
+__device__ __forceinline__ void sum_listed_rows(
+    T* __restrict__ grad_W, const T* __restrict__ edge_W, int32_t node, int32_t begin, int32_t end, int32_t L, int lane,
+    EdgeAt&& edge_at
 ) {
     constexpr int WIDTH = WAVE / PARTS;
     constexpr int BATCH = 16 / (COLUMNS * static_cast<int>(sizeof(T) / 4)); // (of PARTS rows)
-    const int lane = threadIdx.x & (WAVE - 1), part = lane / WIDTH;
-    const int32_t node = __builtin_amdgcn_readfirstlane(blockIdx.x * LISTED_WAVES + (threadIdx.x >> 6));
-    if (node >= n_nodes) {
-        return;
-    }
-    const int32_t begin = offsets[node];
-    const int32_t end = offsets[node + 1];
+    const int part = lane / WIDTH;
     T sum[COLUMNS];
     int32_t column[COLUMNS];
 #pragma unroll
@@ -1576,7 +1571,7 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_listed_rows_kernel(
     }
     for (int32_t p0 = begin; p0 < end; p0 += WAVE) {
         const int32_t n = min(WAVE, end - p0);
-        const int32_t my_edge = edge_of_position[p0 + min(lane, n - 1)];
+        const int32_t my_edge = edge_at(p0 + min(lane, n - 1));
 #pragma unroll 1
         for (int32_t k0 = 0; k0 < n; k0 += BATCH * PARTS) {
             T values[BATCH][COLUMNS];
@@ -1612,6 +1607,55 @@ __global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_listed_rows_kernel(
         if (part == 0 && l < L) {
             grad_W[static_cast<size_t>(node) * L + l] = sum[c];
         }
+    }
+}
+
+template <typename T, int PARTS, int COLUMNS>
+__global__ __launch_bounds__(LISTED_WAVES* WAVE) void sum_listed_rows_kernel(
+    T* __restrict__ grad_W, const T* __restrict__ edge_W, const int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ edge_of_position, int32_t n_nodes, int32_t L
+) {
+    const int32_t node = __builtin_amdgcn_readfirstlane(blockIdx.x * LISTED_WAVES + (threadIdx.x >> 6));
+    if (node < n_nodes) {
+        sum_listed_rows<T, PARTS, COLUMNS>(
+            grad_W, edge_W, node, offsets[node], offsets[node + 1], L, threadIdx.x & (WAVE - 1),
+            [&](int32_t position) { return edge_of_position[position]; }
+        );
+    }
+}
+
+// And over lists that a workgroup gathers from shares first (sender_shares.hpp), a bucket of senders each: its
+// wavefronts take a sender when they are done with the one before.
+constexpr int BUCKET_THREADS = 512;
+
+template <typename T, int PARTS, int COLUMNS>
+__global__ __launch_bounds__(BUCKET_THREADS) void sum_bucket_rows_kernel(
+    T* __restrict__ grad_W, const T* __restrict__ edge_W, const Shares shares, const SharePlan plan, int32_t L
+) {
+    extern __shared__ int32_t bucket_area[];
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int32_t number = swizzled(blockIdx.x, plan.buckets);
+    if (number >= plan.buckets) {
+        return;
+    }
+    BucketFetch fetch(shares, plan, number);
+    fetch.ask();
+    const BucketEdges bucket = gather_bucket<BUCKET_THREADS>(
+        bucket_area, bucket_area + bucket_lds(plan.per_bucket), fetch, shares, plan, number, 0
+    );
+    const int32_t node0 = plan.first_of(number), nodes = plan.first_of(number + 1) - node0;
+    int32_t which = wave;
+    while (which < nodes) {
+        const int32_t begin = __builtin_amdgcn_readfirstlane(bucket.offsets[which]);
+        const int32_t end = __builtin_amdgcn_readfirstlane(bucket.offsets[which + 1]);
+        sum_listed_rows<T, PARTS, COLUMNS>(grad_W, edge_W, node0 + which, begin, end, L, lane, [&](int32_t position) {
+            return bucket.fits ? bucket.list[position] : bucket.in_memory[position];
+        });
+        int32_t taken = 0;
+        if (lane == 0) {
+            taken = atomicAdd(bucket.counter, 1);
+        }
+        which = BUCKET_THREADS / WAVE + __builtin_amdgcn_readfirstlane(taken);
     }
 }
 
@@ -1934,8 +1978,17 @@ void launch_vjp(
     // graphs with more edges per sender keep the gather)
     const bool slotted = want_W && gather_in_kernel && sparse && !by_arrival;
     const size_t slots_bytes = slotted ? sender_slots_bytes(n_output) : by_arrival ? sender_arrivals_bytes(n_output) : 0;
-    const size_t buckets_bytes =
+    size_t buckets_bytes =
         want_W && !gather_in_kernel && !by_arrival ? edges_by_sender_bytes(n_output, n_edges, false) : slots_bytes;
+    // many edges: shares split by the per-edge kernel itself, and gathered by the workgroups of the sum (not in a call
+    // that is captured by a thread whose scratch block is smaller)
+    SharePlan plan{};
+    const bool in_shares = want_W && !gather_in_kernel && !by_arrival && narrow_rows && L > 0 && K > 0 &&
+                           plan_shares(plan, n_output, n_edges, std::min(n_output, MOST_SHARE_BUCKETS)) &&
+                           scratch_ready(edge_w_bytes + shares_bytes(plan, 1));
+    if (in_shares) {
+        buckets_bytes = shares_bytes(plan, 1);
+    }
     char* workspace =
         want_W ? static_cast<char*>(scratch(edge_w_bytes + buckets_bytes)) : nullptr;
     T* edge_W = want_W ? reinterpret_cast<T*>(workspace) : nullptr;
@@ -1950,7 +2003,9 @@ void launch_vjp(
     }
     const bool use_buckets = want_W && n_output > 0 && L > 0 && !gather_in_kernel && !by_arrival;
     bool listed = false; // the slots are being filled by a kernel that is already enqueued
-    if (use_buckets) {
+    const Shares shares = in_shares ? shares_in(workspace + edge_w_bytes, plan) : Shares{};
+    bool split = false; // by a kernel that is already enqueued
+    if (use_buckets && !in_shares) {
         // (beside the per-edge kernel on a stream of its own the sort gains nothing: both want all CUs)
         by_sender = order_edges_by_sender(indices_W, n_edges, n_output, false, workspace + edge_w_bytes, stream);
     }
@@ -2007,8 +2062,10 @@ void launch_vjp(
                 opsa_edges::Tensors<T>{
                     grad_A.data, grad_B.data, edge_W, grad_output.data, A.data, B.data, W, indices_output.data, indices_W,
                     n_edges, n_output, K, L},
-                const_cast<int32_t*>(slots.edges), const_cast<int32_t*>(slots.counts), list_blocks, stream
+                const_cast<int32_t*>(slots.edges), const_cast<int32_t*>(slots.counts), list_blocks,
+                in_shares ? &plan : nullptr, shares, stream
             );
+            split = in_shares;
         } else if (lds > 64 * 1024 && K > thresholds::OPSA_VJP_ROWS_IN_REGISTERS) {
             const unsigned blocks = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_edges), WIDE_WAVES));
             vjp_wide_kernel<T, WEIGHTED><<<blocks, WIDE_WAVES * WAVE, 0, stream>>>(
@@ -2159,23 +2216,37 @@ void launch_vjp(
             grad_W.data, edge_W, indices_W, n_edges, n_output, L, aligned
         );
     } else if (use_buckets) {
+        if (in_shares && !split) {
+            split_shares(shares, plan, indices_W, stream);
+        }
         if (narrow_rows) {
             const unsigned blocks = static_cast<unsigned>(ceil_div(static_cast<size_t>(n_output), LISTED_WAVES));
-            auto sum = [&](auto kernel) {
-                kernel<<<blocks, LISTED_WAVES * WAVE, 0, stream>>>(
-                    grad_W.data, edge_W, by_sender.offsets, by_sender.edge, n_output, L
-                );
+            const size_t lds = static_cast<size_t>(bucket_lds(plan.per_bucket) + gather_lds<BUCKET_THREADS>(plan.per_bucket)) *
+                               sizeof(int32_t);
+            auto sum = [&](auto parts, auto columns) {
+                constexpr int PARTS = decltype(parts)::value, COLUMNS = decltype(columns)::value;
+                if (in_shares) {
+                    sum_bucket_rows_kernel<T, PARTS, COLUMNS>
+                        <<<swizzled_blocks(plan.buckets), BUCKET_THREADS, lds, stream>>>(grad_W.data, edge_W, shares, plan, L);
+                } else {
+                    sum_listed_rows_kernel<T, PARTS, COLUMNS><<<blocks, LISTED_WAVES * WAVE, 0, stream>>>(
+                        grad_W.data, edge_W, by_sender.offsets, by_sender.edge, n_output, L
+                    );
+                }
             };
+            const std::integral_constant<int, 1> one;
+            const std::integral_constant<int, 2> two;
+            const std::integral_constant<int, 4> four;
             if (L <= 16) {
-                sum(sum_listed_rows_kernel<T, 4, 1>);
+                sum(four, one);
             } else if (L <= 32) {
-                sum(sum_listed_rows_kernel<T, 2, 1>);
+                sum(two, one);
             } else if (L <= WAVE) {
-                sum(sum_listed_rows_kernel<T, 1, 1>);
+                sum(one, one);
             } else if (L <= 2 * WAVE) {
-                sum(sum_listed_rows_kernel<T, 1, 2>);
+                sum(one, two);
             } else {
-                sum(sum_listed_rows_kernel<T, 1, 4>);
+                sum(one, four);
             }
         } else {
             int threads = std::min(256, round_up_wave(L));

@@ -67,6 +67,9 @@ template <typename T> struct Arguments {
     int32_t* slot_counts;
     int32_t list_blocks; // (none, but slots: every edge takes a place of its sender, see SenderArrivals)
     bool aligned_senders;
+    SharePlan plan; // (no shares: the senders are not split)
+    Shares shares;
+    int32_t late, less; // the first `late` ranges have `less` edges less than the others
 };
 
 /// A tensor's rows first .. first + n, as elements 64 t + lane of one piece; n = 0: nothing.
@@ -92,6 +95,13 @@ __global__ __launch_bounds__(THREADS) void edge_kernel(const Arguments<T> p) {
             return;
         }
     }
+    if constexpr (WEIGHTED) {
+        // (a share of the senders first; the ranges of these workgroups are the shorter for it)
+        if (static_cast<int32_t>(blockIdx.x) < p.plan.shares) {
+            split_share<THREADS>(reinterpret_cast<int32_t*>(lds), p.shares, p.plan, p.t.senders, blockIdx.x);
+            __syncthreads();
+        }
+    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE); // (uniform, and known to be)
     const int lane = threadIdx.x & (WAVE - 1), i = lane & 15, q = lane >> 4;
     const int32_t range = (static_cast<int32_t>(blockIdx.x) - p.list_blocks) * WAVES + wave;
@@ -107,7 +117,11 @@ __global__ __launch_bounds__(THREADS) void edge_kernel(const Arguments<T> p) {
     }
     wave_sync();
 
-    const int32_t begin = range * p.range_edges, end = begin + min(p.range_edges, p.t.n_edges - begin);
+    auto begin_of = [&](int32_t which) {
+        const int64_t at = static_cast<int64_t>(which) * p.range_edges - p.less * min(which, p.late);
+        return static_cast<int32_t>(at < p.t.n_edges ? at : p.t.n_edges);
+    };
+    const int32_t begin = begin_of(range), end = begin_of(range + 1);
     const bool want_A = p.t.grad_A != nullptr, want_U = p.t.grad_B != nullptr || (WEIGHTED && p.t.edge_W != nullptr);
     BufferOf<T> W;
     W.set(p.t.W, WEIGHTED ? static_cast<uint32_t>(p.t.n_nodes) * static_cast<uint32_t>(L) * ES : 0);
@@ -355,9 +369,16 @@ __global__ __launch_bounds__(THREADS) void edge_kernel(const Arguments<T> p) {
 }
 
 template <typename T, int KT, int LT, bool WEIGHTED>
-void launch_with(const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, hipStream_t stream) {
+void launch_with(
+    const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, const SharePlan* plan,
+    const Shares& shares, hipStream_t stream
+) {
     Arguments<T> p{};
     p.t = t;
+    if (plan != nullptr) {
+        p.plan = *plan;
+        p.shares = shares;
+    }
     p.slots = slots;
     p.slot_counts = slot_counts;
     p.list_blocks = static_cast<int32_t>(list_blocks);
@@ -371,6 +392,9 @@ void launch_with(const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsi
     if (list_blocks > 0) {
         lds = std::max(lds, sizeof(SlotLists));
     }
+    if (plan != nullptr) {
+        lds = std::max(lds, split_lds<THREADS>(plan->buckets) * sizeof(int32_t));
+    }
     auto kernel = edge_kernel<T, KT, LT, WEIGHTED>;
     if (lds > 64 * 1024) {
         MOPS_HIP_CHECK(hipFuncSetAttribute(
@@ -382,8 +406,18 @@ void launch_with(const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsi
     const int64_t tiles = (static_cast<int64_t>(t.n_edges) + 15) / 16;
     const int64_t per_range = (tiles + resident - 1) / resident;
     p.range_edges = static_cast<int32_t>(std::min<int64_t>(16 * per_range, 1 << 30));
-    p.ranges = static_cast<int32_t>((static_cast<int64_t>(t.n_edges) + p.range_edges - 1) / p.range_edges);
-    const unsigned blocks = list_blocks + static_cast<unsigned>((p.ranges + WAVES - 1) / WAVES);
+    if (plan != nullptr) {
+        p.late = static_cast<int32_t>(std::min<int64_t>(plan->shares * WAVES, resident));
+        // (splitting 1024 edges takes as long as what moves some 15 000 bytes of a wavefront's range)
+        const int64_t edge_bytes = static_cast<int64_t>(2 * t.K + 5 * t.L) * static_cast<int64_t>(sizeof(T));
+        p.less = static_cast<int32_t>(std::min(15000 * (plan->share / 1024) / edge_bytes, t.n_edges / resident / 2));
+        p.range_edges = static_cast<int32_t>((t.n_edges + static_cast<int64_t>(p.late) * p.less + resident - 1) / resident);
+    }
+    p.ranges = static_cast<int32_t>(
+        (static_cast<int64_t>(t.n_edges) + static_cast<int64_t>(p.late) * p.less + p.range_edges - 1) / p.range_edges
+    );
+    const unsigned blocks =
+        std::max(list_blocks + static_cast<unsigned>((p.ranges + WAVES - 1) / WAVES), static_cast<unsigned>(p.plan.shares));
     kernel<<<blocks, THREADS, lds, stream>>>(p);
     MOPS_HIP_CHECK(hipGetLastError());
 }
@@ -397,14 +431,15 @@ bool covers(int32_t n_nodes, int32_t K, int32_t L, size_t element_size) {
 
 template <typename T>
 void launch(
-    const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, hipStream_t stream
+    const Tensors<T>& t, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, const SharePlan* plan,
+    const Shares& shares, hipStream_t stream
 ) {
     auto with_columns = [&](auto kt, auto lt) {
         constexpr int KT = decltype(kt)::value, LT = decltype(lt)::value;
         if (t.W != nullptr) {
-            launch_with<T, KT, LT, true>(t, slots, slot_counts, list_blocks, stream);
+            launch_with<T, KT, LT, true>(t, slots, slot_counts, list_blocks, plan, shares, stream);
         } else {
-            launch_with<T, KT, LT, false>(t, slots, slot_counts, list_blocks, stream);
+            launch_with<T, KT, LT, false>(t, slots, slot_counts, list_blocks, plan, shares, stream);
         }
     };
     auto with_rows = [&](auto kt) {
@@ -425,7 +460,7 @@ void launch(
     }
 }
 
-template void launch<float>(const Tensors<float>&, int32_t*, int32_t*, unsigned, hipStream_t);
-template void launch<double>(const Tensors<double>&, int32_t*, int32_t*, unsigned, hipStream_t);
+template void launch<float>(const Tensors<float>&, int32_t*, int32_t*, unsigned, const SharePlan*, const Shares&, hipStream_t);
+template void launch<double>(const Tensors<double>&, int32_t*, int32_t*, unsigned, const SharePlan*, const Shares&, hipStream_t);
 
 } // namespace mops::amd::opsa_edges

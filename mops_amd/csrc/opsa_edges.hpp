@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "sender_shares.hpp"
+
 namespace mops::amd::opsa_edges {
 
 template <typename T> struct Tensors {
@@ -27,10 +29,11 @@ bool covers(int32_t n_nodes, int32_t K, int32_t L, size_t element_size);
 
 /// With `slots` and `slot_counts`, the edges of every sender are listed as well: by `list_blocks`
 /// workgroups (sender_slots_blocks()) beside the others, or, if that is 0, by arrival
-/// (SenderArrivals, one copy of the counters).
+/// (SenderArrivals, one copy of the counters). With `plan` (or null), the senders are split into `shares`.
 template <typename T>
 void launch(
-    const Tensors<T>& tensors, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, hipStream_t stream
+    const Tensors<T>& tensors, int32_t* slots, int32_t* slot_counts, unsigned list_blocks, const SharePlan* plan,
+    const Shares& shares, hipStream_t stream
 );
 
 } // namespace mops::amd::opsa_edges

@@ -888,7 +888,15 @@ template <typename T, int N, int COLUMNS, Lists LISTS, bool SHARED>
 __global__ __launch_bounds__(THREADS)
 __attribute__((amdgpu_waves_per_eu(contract_waves<T, N, COLUMNS>()))) void contract_kernel(const ContractArgs<T> args) {
     extern __shared__ __align__(16) char lds[];
-    contract<T, N, COLUMNS, LISTS, SHARED>(args, lds, blockIdx.x);
+    int32_t block = blockIdx.x;
+    if constexpr (LISTS == BUCKETS) {
+        const int32_t blocks = args.walk.ranges * (SHARED ? args.walk.column_tiles : 1);
+        block = swizzled(block, blocks);
+        if (block >= blocks) {
+            return;
+        }
+    }
+    contract<T, N, COLUMNS, LISTS, SHARED>(args, lds, block);
 }
 
 // ---------------------------------------------------------------- gradients --
@@ -1267,9 +1275,9 @@ template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Sha
         w.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
         auto launch = [&](auto kernel, int64_t ranges, int waves_per_range) {
             w.ranges = static_cast<int32_t>(std::min<int64_t>(s.n_nodes, std::max<int64_t>(1, ranges)));
-            const size_t waves = static_cast<size_t>(w.ranges) * waves_per_range;
+            const int32_t blocks = static_cast<int32_t>(ceil_div(static_cast<size_t>(w.ranges) * waves_per_range, WAVES));
             allow_lds(kernel, lds);
-            kernel<<<static_cast<unsigned>(ceil_div(waves, WAVES)), THREADS, lds, stream>>>(args);
+            kernel<<<LISTS == BUCKETS ? swizzled_blocks(blocks) : blocks, THREADS, lds, stream>>>(args);
         };
         const int64_t resident = resident_sums<T, N, COLUMNS>();
         const bool shared = LISTS == BUCKETS ? args.plan.multiplier == 0

@@ -377,7 +377,6 @@ bool plan_shares(SharePlan& plan, int32_t n_nodes, int32_t n_edges, int32_t buck
         plan.senders_each = 4294967296.0 / plan.multiplier;
         plan.per_bucket = static_cast<int32_t>((uint64_t(1) << 32) / plan.multiplier + 1);
     }
-    plan.bucket_bits = bits_for(buckets);
     plan.sender_bits = bits_for(plan.per_bucket);
     return each * SHARE_STEP <= MOST_SHARE_EDGES && plan.per_bucket <= MOST_PER_BUCKET &&
            bits_for(n_edges) + plan.sender_bits <= 32 &&

@@ -47,7 +47,7 @@ struct SharePlan {
     int32_t buckets, per_bucket;  // of senders, and how many senders at most
     uint32_t multiplier;          // floor(2^32 buckets / n_nodes); 0: a bucket per sender
     double senders_each;          // 2^32 / multiplier
-    int bucket_bits, sender_bits; // of a bucket's number, and of a sender's place in its bucket
+    int sender_bits; // of a sender's place in its bucket
 
     __device__ __forceinline__ int32_t bucket_of(int32_t sender) const {
         return multiplier == 0 ? sender : static_cast<int32_t>(__umulhi(static_cast<uint32_t>(sender), multiplier));
@@ -61,6 +61,15 @@ struct SharePlan {
 
 /// The plan with so many buckets; false: a graph for order_edges_by_sender.
 bool plan_shares(SharePlan& plan, int32_t n_nodes, int32_t n_edges, int32_t buckets);
+
+/// Consecutive numbers to the workgroups of one die (which get every eighth workgroup): what consecutive buckets
+/// have of a share lies on the same lines, eight buckets to a line of 128 bytes if they have four edges each.
+/// Workgroups below `count` only; of a launch of swizzled_blocks(count).
+constexpr int32_t DIES = 8;
+__device__ __forceinline__ int32_t swizzled(int32_t block, int32_t count) {
+    return block % DIES * ((count + DIES - 1) / DIES) + block / DIES;
+}
+inline int32_t swizzled_blocks(int32_t count) { return (count + DIES - 1) / DIES * DIES; }
 
 /// What the first half leaves behind.
 struct Shares {
@@ -83,7 +92,7 @@ template <int THREADS> __host__ __device__ constexpr int32_t split_lds(int32_t b
 template <int THREADS>
 __device__ __forceinline__ void
 split_share(int32_t* lds, const Shares& to, const SharePlan& plan, const int32_t* __restrict__ senders, int32_t which) {
-    constexpr int WAVES = THREADS / WAVE, HELD = SHARE_STEP / THREADS < 4 ? SHARE_STEP / THREADS : 4;
+    constexpr int WAVES = THREADS / WAVE, BATCH = SHARE_STEP / THREADS < 8 ? SHARE_STEP / THREADS : 8;
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int32_t* counters = lds;
     int32_t* start = counters + WAVES * plan.buckets;
@@ -95,8 +104,7 @@ split_share(int32_t* lds, const Shares& to, const SharePlan& plan, const int32_t
         const int32_t bucket = plan.bucket_of(sender);
         return Item{in_bounds(sender, plan.n_nodes) ? bucket : -1, e, sender};
     };
-    const Held<HELD> held(mine, lane, item_at);
-    count_keys<4>(held, counters, plan.buckets, mine, wave, WAVES, lane, item_at);
+    count_keys<BATCH>(Held<0>{}, counters, plan.buckets, mine, wave, WAVES, lane, item_at);
     for (int32_t bucket = threadIdx.x; bucket < plan.buckets; bucket += THREADS) {
         int32_t sum = 0;
 #pragma unroll
@@ -120,7 +128,7 @@ split_share(int32_t* lds, const Shares& to, const SharePlan& plan, const int32_t
     }
     __syncthreads();
     uint32_t* const words = to.words + first;
-    place_keys<4>(held, counters, plan.buckets, plan.bucket_bits, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
+    place_rare_keys<BATCH>(counters, plan.buckets, mine, wave, lane, item_at, [&](int32_t place, const Item& item) {
         words[place] = static_cast<uint32_t>(item.edge - first) | static_cast<uint32_t>(item.sender) << 16;
     });
 }

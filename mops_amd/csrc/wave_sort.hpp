@@ -137,6 +137,49 @@ __device__ __forceinline__ void place_keys(
     }
 }
 
+/// The same for many keys, of which few are named twice among 64 items: the places come from atomics on the counters,
+/// which lanes with the same key are given in no particular order; those are found by their places and put in
+/// theirs. BATCH x 64 items wait for LDS together. (1 000 000 senders in shares of 4096 over 1024 buckets, two
+/// wavefronts each, beside the edges' gradients of OPSAW: 4 us of the launch instead of 9.)
+template <int BATCH, typename ItemAt, typename Put>
+__device__ __forceinline__ void place_rare_keys(
+    int32_t* counters, int32_t keys, const WaveShare& share, int wave, int lane, ItemAt&& item_at, Put&& put
+) {
+    int32_t* mine = counters + static_cast<size_t>(wave) * keys;
+#pragma unroll 1
+    for (int32_t at = share.begin + lane; at - lane < share.end; at += BATCH * WAVE) {
+        Item item[BATCH];
+        int32_t place[BATCH], given[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            item[u] = item_at(min(at + u * WAVE, share.end - 1));
+            item[u].key = at + u * WAVE < share.end ? item[u].key : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) { // (LDS operations of one wavefront happen in program order)
+            place[u] = given[u] = 0;
+            if (item[u].key >= 0) {
+                place[u] = __hip_atomic_load(&mine[item[u].key], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                given[u] = atomicAdd(&mine[item[u].key], 1);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < BATCH; u++) {
+            uint64_t others = __ballot(given[u] != place[u]);
+            while (others != 0) { // (uniform)
+                const int32_t key = __builtin_amdgcn_readlane(item[u].key, __builtin_ctzll(others));
+                const uint64_t same = __ballot(item[u].key == key);
+                const int32_t before = __popcll(same & ((uint64_t(1) << lane) - 1));
+                place[u] += item[u].key == key ? before : 0;
+                others &= ~same;
+            }
+            if (item[u].key >= 0) {
+                put(place[u], item[u]);
+            }
+        }
+    }
+}
+
 /// Turns counters[wavefront][key] into the place of the wavefront's first of each key:
 /// start_of(key) and what the wavefronts before have. All threads.
 template <int WAVES, typename StartOf>
