@@ -140,14 +140,16 @@ constexpr size_t SENDER_SCAN_LIMIT = 100u * 1000 * 1000;
 /// reading the whole index). OPSAW, 60 000 edges over 2000 senders, L = 32,
 /// f32: 33 -> 22 us for the whole vjp.
 constexpr int32_t SLOT_MEAN_EDGES = 48;
-/// Edges up to which SASAW's gradients with a lane per column are one launch, where every node's workgroup
-/// looks through the whole index of senders (with up to two nodes and 32 columns per compute unit). That / a
-/// launch that lists the edges and one for each kind of gradient, f32, f64, 9 components unless it says
-/// otherwise: 600 edges of 20 nodes, 32 columns 11.8 / 24.0, 12.8 / 26.6 us; 8000 of 260 15.4 / 29, 26.7 / 33;
-/// 16 000 of 500 27.7 / 34.1, 36.0 / 39.3; 16 000 of 250, 64 columns 28.5 / 39.1, 54.7 / 60.7; 24 000 of 500
-/// 30.5 / 37.1, 43.6 / 46.7. Half as many where nodes have more than SLOT_MEAN_EDGES each (24 000 of 40 63.7 /
-/// 52.2, 67.6 / 59.0), and for 16 components in double, then also half as many nodes (12 000 of 500 70 / 62;
-/// 5000 of 200 40.8 / 53).
+/// Edges up to which SASAW's gradients with a lane per column are one launch, where every node's workgroup looks
+/// through the whole index of senders (three quarters of it for 16 components in float, half in double), with no more
+/// nodes and tiles of columns than workgroups at a time. Beyond, an index that is read often or in several rounds, and
+/// sums that take the registers of the edges, cost more than a second launch; grad_W alone comes to this first, and
+/// its bits are not to depend on what else is wanted. One launch / two, us, whole vjp and grad_W alone, 32 columns. 9
+/// components, f32 (768 workgroups): 12 000 edges of 400 nodes 23.0 / 26.6, 16.5 / 17.0; 16 000 of 533 26.2 / 29.6, 19.1 /
+/// 18.9; 10 000 of 1000 26.0 / 29.0, 23.9 / 19.1; 24 000 of 800 34.4 / 33.6, 32.7 / 21.2; f64 (512): 16 000 of 250 29.2 / 32.3,
+/// 20.9 / 18.7, of 533 34.3 / 38.1, 31.6 / 23.2. 4 components, f32 (1024): 16 000 of 533 15.2 / 20.0, 14.1 / 13.8; 24 000 of 800
+/// 19.6 / 22.2, 18.2 / 14.8. 16 components, f32 (512): 12 000 of 400 39.6 / 41.3, 23.8 / 23.4; 16 000 of 250 41.8 / 39.3, 25.3 /
+/// 20.9; f64 (two tiles): 5000 of 100 29.3 / 44.1; 16 000 of 250 63.5 / 59.2.
 constexpr int32_t COLUMNS_EDGES_AS_THEY_ARE = 16384;
 /// Edges per sender on average up to which lists are made by arrival (128 places
 /// per sender). SASAW, 1000 nodes x 60 edges, whole vjp 87.6 -> 76.6 us (f32), 143.8

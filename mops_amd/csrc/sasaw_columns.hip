@@ -1168,6 +1168,10 @@ edge_kernel(const EdgeArgs<T> args, const Shares shares, const SharePlan plan, c
     edge_gradients<T, N, COLUMNS>(args, lds, blockIdx.x);
 }
 
+template <typename T, int N, int COLUMNS> constexpr int small_waves() {
+    return std::min(contract_waves<T, N, COLUMNS>(), edge_waves<T, N, COLUMNS>());
+}
+
 /// All gradients of a small graph in one launch: the first `nodes` workgroups have a node and a tile of
 /// columns of grad_W each, and look through the index for its edges themselves; the others grad_A and grad_B.
 /// Bound by the launch and one chain of loads. Against the listing of the edges, grad_A and grad_B, and grad_W
@@ -1175,7 +1179,7 @@ edge_kernel(const EdgeArgs<T> args, const Shares shares, const SharePlan plan, c
 /// of 200 nodes 27.0 -> 14.9 / 31.3 -> 17.0.
 template <typename T, int N, int COLUMNS>
 __global__ __launch_bounds__(THREADS)
-__attribute__((amdgpu_waves_per_eu(std::min(contract_waves<T, N, COLUMNS>(), edge_waves<T, N, COLUMNS>())))) void
+__attribute__((amdgpu_waves_per_eu(small_waves<T, N, COLUMNS>()))) void
 small_kernel(const ContractArgs<T> of_nodes, const EdgeArgs<T> of_edges, int32_t nodes) {
     extern __shared__ __align__(16) char lds[];
     if (static_cast<int32_t>(blockIdx.x) < nodes) { // (uniform)
@@ -1190,15 +1194,21 @@ small_kernel(const ContractArgs<T> of_nodes, const EdgeArgs<T> of_edges, int32_t
 /// instructions' worth of everything else.
 template <int N, int COLUMNS> constexpr int cost() { return (N + 1) * Sums<N, COLUMNS>::M2 + 8; }
 
+/// Workgroups of a sum on the device at a time.
+template <typename T, int N, int COLUMNS> int64_t resident_sums() {
+    return static_cast<int64_t>(compute_units()) * contract_waves<T, N, COLUMNS>();
+}
+
 /// body(N, COLUMNS): the cheapest tiles. EDGES: for the gradients by edge, in double of 32 columns at most for 9
 /// components (60 000 edges, 64 columns, grad_A and grad_B with 64 / 32 at a time 66 / 56 us, 300 000 259 / 248; in float
 /// 31 / 37 and 128 / 132). `more`: what a tile costs beside that.
-template <typename T, bool EDGES, typename Body> void with_layout(const Shape& s, Body&& body, int more = 0) {
+enum Of { EDGES, SUMS, BUCKETED };
+template <typename T, Of OF, typename Body> void with_layout(const Shape& s, Body&& body, int more = 0) {
     auto with_columns = [&](auto n) {
         constexpr int N = decltype(n)::value;
         // (sums that fit the registers of a lane)
         constexpr int MOST = N == 16                            ? (sizeof(T) == 4 ? 32 : 16)
-                             : EDGES && N == 9 && sizeof(T) == 8 ? 32
+                             : OF == EDGES && N == 9 && sizeof(T) == 8 ? 32
                                                                  : 64;
         int best = 16, least = (s.L + 15) / 16 * (cost<N, 16>() + more);
         if (const int c = (s.L + 31) / 32 * (cost<N, 32>() + more); MOST >= 32 && c <= least) {
@@ -1208,8 +1218,17 @@ template <typename T, bool EDGES, typename Body> void with_layout(const Shape& s
         if (const int c = (s.L + 63) / 64 * (cost<N, 64>() + more); MOST >= 64 && c <= least) {
             best = 64;
         }
-        // (few nodes: more, narrower tiles, which the contraction takes as wavefronts of their own)
-        if (!EDGES && static_cast<int64_t>(s.n_nodes) * ((s.L + best - 1) / best) < 4 * compute_units()) {
+        // The sums of few nodes take more, narrower tiles, which are wavefronts of their own. Where a workgroup gathers a
+        // bucket first, it is better used for a node and all of the columns that fit its registers, if no more nodes
+        // than run at a time leave it a node to itself (grad_W with grad_A and grad_B, 9 components, f32: 30 000 edges of
+        // 1000 nodes, 32 columns, 16 / 32 at a time 40.3 / 35.3 us; of 600, 64 columns, 50.9 / 44.6; but 9000 of 300 in
+        // double 46.8 / 51.7).
+        const int64_t nodes = s.n_nodes;
+        const bool wide = OF == BUCKETED && best > 16 && nodes * ((s.L + 15) / 16) > resident_sums<T, N, 16>() &&
+                          (best == 32   ? nodes * ((s.L + 31) / 32) <= resident_sums<T, N, MOST >= 32 ? 32 : 16>()
+                           : sizeof(T) == 4 ? nodes * ((s.L + 63) / 64) <= resident_sums<T, N, MOST >= 64 ? 64 : 16>()
+                                            : false);
+        if (OF != EDGES && !wide && nodes * ((s.L + best - 1) / best) < 4 * compute_units()) {
             best = 16;
         }
         if (best == 16) {
@@ -1262,13 +1281,8 @@ Walk<T> walk_of(
     return w;
 }
 
-/// Workgroups of a sum on the device at a time.
-template <typename T, int N, int COLUMNS> int64_t resident_sums() {
-    return static_cast<int64_t>(compute_units()) * contract_waves<T, N, COLUMNS>();
-}
-
 template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Shape& s, hipStream_t stream) {
-    with_layout<T, false>(s, [&](auto n, auto columns) {
+    with_layout<T, LISTS == BUCKETS ? BUCKETED : SUMS>(s, [&](auto n, auto columns) {
         constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
         Walk<T>& w = args.walk;
         const size_t lds = LISTS == BUCKETS ? contract_lds<T, N, COLUMNS>(args.plan.per_bucket) : contract_lds<T, N, COLUMNS>();
@@ -1280,8 +1294,7 @@ template <typename T, Lists LISTS> void contract(ContractArgs<T> args, const Sha
             kernel<<<LISTS == BUCKETS ? swizzled_blocks(blocks) : blocks, THREADS, lds, stream>>>(args);
         };
         const int64_t resident = resident_sums<T, N, COLUMNS>();
-        const bool shared = LISTS == BUCKETS ? args.plan.multiplier == 0
-                                             : static_cast<int64_t>(s.n_nodes) * w.column_tiles <= resident;
+        const bool shared = static_cast<int64_t>(s.n_nodes) * w.column_tiles <= resident;
         if (shared) {
             launch(contract_kernel<T, N, COLUMNS, LISTS, true>, s.n_nodes, WAVES * w.column_tiles);
         } else if (LISTS == BUCKETS) {
@@ -1368,18 +1381,21 @@ template <typename T, int N, int COLUMNS> size_t share_out(EdgeArgs<T>& args, co
 
 template <typename T> SenderLists plan_lists(const Shape& s) {
     SenderLists lists{};
-    with_layout<T, false>(s, [&](auto n, auto columns) {
+    with_layout<T, BUCKETED>(s, [&](auto n, auto columns) {
         constexpr int N = decltype(n)::value, COLUMNS = decltype(columns)::value;
         const int32_t tiles = (s.L + COLUMNS - 1) / COLUMNS;
         const int64_t resident = resident_sums<T, N, COLUMNS>();
         // A node by a workgroup for each of its tiles if there are no more of them than run at a time; else as many
         // buckets as workgroups run at a time (fewer would leave some idle), or twice or four times as many.
         const bool shared = static_cast<int64_t>(s.n_nodes) * tiles <= resident;
-        for (int64_t buckets = shared ? s.n_nodes : std::min<int64_t>(resident, s.n_nodes);
+        // (of few nodes no more buckets than leave each wavefront a node and tile: grad_W alone, 10 000 edges of 1000 nodes,
+        // 16 components, f32, with a bucket per two nodes / per four 25.6 / 21.9 us, 9 in double 22.5 / 20.1)
+        const int64_t units = static_cast<int64_t>(s.n_nodes) * std::min(tiles, WAVES);
+        for (int64_t buckets = shared ? s.n_nodes : std::min<int64_t>(resident, (units + WAVES - 1) / WAVES);
              buckets <= MOST_SHARE_BUCKETS && !lists.in_shares; buckets *= 2) {
             lists.in_shares = plan_shares(lists.plan, s.n_nodes, s.n_edges, static_cast<int32_t>(buckets));
         }
-        lists.copies = lists.plan.multiplier == 0 ? tiles : 1;
+        lists.copies = shared ? tiles : 1;
     });
     return lists;
 }
@@ -1413,7 +1429,7 @@ void edge_gradients(
         shares = shares_in(workspace, plan);
     }
     MainKernelTimer timer(stream);
-    with_layout<T, true>(s, [&](auto components, auto columns) {
+    with_layout<T, EDGES>(s, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
         const size_t lds =
             std::max(edge_lds<T, N, COLUMNS>(), split_lds<THREADS>(plan.buckets) * sizeof(int32_t));
@@ -1430,13 +1446,28 @@ void edge_gradients(
     MOPS_HIP_CHECK(hipGetLastError());
 }
 
-bool small(const Shape& s, size_t element_size) {
-    const bool sums_fill_the_registers = s.nA == 16 && element_size == 8;
-    const bool dense = s.n_edges > static_cast<int64_t>(s.n_nodes) * thresholds::SLOT_MEAN_EDGES;
-    const int32_t edges = thresholds::COLUMNS_EDGES_AS_THEY_ARE / (sums_fill_the_registers || dense ? 2 : 1);
-    return s.n_edges <= edges &&
-           static_cast<int64_t>(s.n_nodes) * ((s.L + 31) / 32) <= (sums_fill_the_registers ? 1 : 2) * compute_units();
+namespace {
+
+/// What a tile costs a small graph beside its columns: tiles are one after the other for the edges' wavefronts,
+/// and little else bounds it (2000 edges of 60 nodes, 40 columns, f64, with 16 / 32 at a time 18.7 / 15.5 us).
+constexpr int SMALL_TILE_COST = 4;
+
+template <typename T> bool is_small(const Shape& s) {
+    bool result = false;
+    with_layout<T, EDGES>(s, [&](auto n, auto columns) {
+        constexpr int WAVES_PER_SIMD = small_waves<T, decltype(n)::value, decltype(columns)::value>();
+        const int32_t tiles = (s.L + decltype(columns)::value - 1) / decltype(columns)::value;
+        const int64_t resident = static_cast<int64_t>(compute_units()) * WAVES_PER_SIMD; // workgroups
+        const int32_t edges = thresholds::COLUMNS_EDGES_AS_THEY_ARE;
+        result = s.n_edges <= (s.nA < 16 ? edges : sizeof(T) == 4 ? edges / 4 * 3 : edges / 2) &&
+                 static_cast<int64_t>(s.n_nodes) * tiles <= resident;
+    }, SMALL_TILE_COST);
+    return result;
 }
+
+} // namespace
+
+bool small(const Shape& s, size_t element_size) { return element_size == 4 ? is_small<float>(s) : is_small<double>(s); }
 
 template <typename T>
 void small_vjp(
@@ -1446,7 +1477,7 @@ void small_vjp(
     ContractArgs<T> nodes = of_senders(grad_W, grad_output, A, B, C, indices, s);
     EdgeArgs<T> edges = of_edges(grad_A, grad_B, grad_output, A, B, C, W, indices, s);
     MainKernelTimer timer(stream);
-    with_layout<T, true>(s, [&](auto components, auto columns) {
+    with_layout<T, EDGES>(s, [&](auto components, auto columns) {
         constexpr int N = decltype(components)::value, COLUMNS = decltype(columns)::value;
         constexpr size_t lds = std::max(edge_lds<T, N, COLUMNS>(), contract_lds<T, N, COLUMNS>());
         nodes.walk.column_tiles = (s.L + COLUMNS - 1) / COLUMNS;
@@ -1456,9 +1487,7 @@ void small_vjp(
         auto kernel = small_kernel<T, N, COLUMNS>;
         allow_lds(kernel, lds);
         kernel<<<static_cast<unsigned>(of_nodes + of_edges), THREADS, lds, stream>>>(nodes, edges, static_cast<int32_t>(of_nodes));
-        // (tiles are one after the other for the edges' wavefronts, and little else bounds a small graph: 2000 edges
-        // of 60 nodes, 40 columns, f64, with 16 / 32 at a time 18.7 / 15.5 us)
-    }, 4);
+    }, SMALL_TILE_COST);
     MOPS_HIP_CHECK(hipGetLastError());
 }
 

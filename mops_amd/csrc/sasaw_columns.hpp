@@ -63,7 +63,8 @@ void weight_gradient(
 );
 
 /// Whether a graph is small enough that all its gradients are one launch, in which every sender's edges are
-/// looked for in the index as it is.
+/// looked for in the index as it is. Whichever of the gradients are wanted, so that the bits
+/// of one do not depend on the others.
 bool small(const Shape& shape, size_t element_size);
 
 /// Of a small graph: any of grad_A, grad_B, grad_W may be null, but not all.

@@ -1682,12 +1682,12 @@ void vjp(
     args.lda = s.nA;
     args.w_stride_rows = s.n2;
     args.g_stride_rows = s.n3;
+    const bool want_edges = grad_A != nullptr || grad_B != nullptr;
     if (vjp_by_columns(s, sizeof(T)) && sasaw_columns::small(s, sizeof(T))) {
         sasaw_columns::small_vjp<T>(grad_A, grad_B, grad_W, grad_output, A, B, C, W, indices, s, stream);
         return;
     }
     if (vjp_by_columns(s, sizeof(T))) {
-        const bool want_edges = grad_A != nullptr || grad_B != nullptr;
         sasaw_columns::SenderLists plan{};
         const sasaw_columns::SenderLists* lists = nullptr;
         if (grad_W != nullptr && shares) {
