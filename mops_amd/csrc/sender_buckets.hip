@@ -385,7 +385,7 @@ bool plan_shares(SharePlan& plan, int32_t n_nodes, int32_t n_edges, int32_t buck
 
 size_t shares_bytes(const SharePlan& plan, int32_t copies) {
     return align256(static_cast<size_t>(plan.shares) * plan.share * 4) +
-           align256(static_cast<size_t>(plan.buckets) * MOST_SHARES * 4) +
+           align256(static_cast<size_t>(plan.buckets) * plan.shares * 4) +
            static_cast<size_t>(copies) * plan.n_edges * 4;
 }
 
@@ -395,7 +395,7 @@ Shares shares_in(void* workspace, const SharePlan& plan) {
     shares.words = reinterpret_cast<uint32_t*>(at);
     at += align256(static_cast<size_t>(plan.shares) * plan.share * 4);
     shares.starts = reinterpret_cast<uint32_t*>(at);
-    at += align256(static_cast<size_t>(plan.buckets) * MOST_SHARES * 4);
+    at += align256(static_cast<size_t>(plan.buckets) * plan.shares * 4);
     shares.lists = reinterpret_cast<int32_t*>(at);
     return shares;
 }

@@ -35,7 +35,7 @@ namespace mops::amd {
 constexpr int32_t MOST_SHARES = 256;
 constexpr int32_t SHARE_STEP = 1024;        // edges of a share: a multiple of this
 constexpr int32_t MOST_SHARE_EDGES = 32768; // (places in a share take 16 bits)
-constexpr int32_t MOST_SHARE_BUCKETS = 1024; // counters in LDS
+constexpr int32_t MOST_SHARE_BUCKETS = 1024; // counters in LDS, of every wavefront
 /// Edges of a bucket that fit into LDS. Larger ones (of a few senders with many more
 /// edges than the others: on average buckets are at most three quarters of it) are sorted in global memory.
 constexpr int32_t BUCKET_EDGES = 2048;
@@ -74,7 +74,7 @@ inline int32_t swizzled_blocks(int32_t count) { return (count + DIES - 1) / DIES
 /// What the first half leaves behind.
 struct Shares {
     uint32_t* words;  // [shares][share] edge in the share | lower half of its sender << 16, by bucket
-    uint32_t* starts; // [buckets][MOST_SHARES] first of the bucket's places in the share | how many << 16
+    uint32_t* starts; // [shares][buckets] first of the bucket's places in the share | how many << 16
     int32_t* lists;   // [copies][n_edges] for buckets that do not fit into LDS
 };
 /// Bytes of scratch memory: `copies` workgroups gather the same bucket.
@@ -85,7 +85,7 @@ void split_shares(const Shares& to, const SharePlan& plan, const int32_t* sender
 
 /// Integers of LDS that split_share takes.
 template <int THREADS> __host__ __device__ constexpr int32_t split_lds(int32_t buckets) {
-    return (THREADS / WAVE + 1) * buckets + THREADS / WAVE;
+    return THREADS / WAVE * buckets + THREADS + THREADS / WAVE;
 }
 
 /// All threads of a workgroup of THREADS.
@@ -95,8 +95,8 @@ split_share(int32_t* lds, const Shares& to, const SharePlan& plan, const int32_t
     constexpr int WAVES = THREADS / WAVE, BATCH = SHARE_STEP / THREADS < 8 ? SHARE_STEP / THREADS : 8;
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     int32_t* counters = lds;
-    int32_t* start = counters + WAVES * plan.buckets;
-    int32_t* of_wave = start + plan.buckets;
+    int32_t* of_thread = counters + WAVES * plan.buckets;
+    int32_t* of_wave = of_thread + THREADS;
     const int32_t first = which * plan.share, last = first + min(plan.share, plan.n_edges - first);
     const WaveShare mine(first, last, wave, WAVES);
     auto item_at = [&](int32_t e) {
@@ -105,26 +105,30 @@ split_share(int32_t* lds, const Shares& to, const SharePlan& plan, const int32_t
         return Item{in_bounds(sender, plan.n_nodes) ? bucket : -1, e, sender};
     };
     count_keys<BATCH>(Held<0>{}, counters, plan.buckets, mine, wave, WAVES, lane, item_at);
-    for (int32_t bucket = threadIdx.x; bucket < plan.buckets; bucket += THREADS) {
-        int32_t sum = 0;
+    // every thread has as many consecutive buckets
+    const int32_t each = (plan.buckets + THREADS - 1) / THREADS;
+    const int32_t begin = min(static_cast<int32_t>(threadIdx.x) * each, plan.buckets), end = min(begin + each, plan.buckets);
+    int32_t sum = 0;
+    for (int32_t bucket = begin; bucket < end; bucket++) {
 #pragma unroll
         for (int w = 0; w < WAVES; w++) {
             sum += counters[w * plan.buckets + bucket];
         }
-        start[bucket] = sum;
     }
+    of_thread[threadIdx.x] = sum;
     __syncthreads();
-    scan_in_place<WAVES>(start, plan.buckets, 0, of_wave);
-    for (int32_t bucket = threadIdx.x; bucket < plan.buckets; bucket += THREADS) {
-        const int32_t begin = start[bucket];
-        int32_t place = begin;
+    scan_in_place<WAVES>(of_thread, THREADS, 0, of_wave);
+    uint32_t* const starts = to.starts + static_cast<size_t>(which) * plan.buckets;
+    int32_t place = of_thread[threadIdx.x];
+    for (int32_t bucket = begin; bucket < end; bucket++) {
+        const int32_t start = place;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) {
             const int32_t here = counters[w * plan.buckets + bucket];
             counters[w * plan.buckets + bucket] = place;
             place += here;
         }
-        to.starts[static_cast<size_t>(bucket) * MOST_SHARES + which] = static_cast<uint32_t>(begin | (place - begin) << 16);
+        starts[bucket] = static_cast<uint32_t>(start | (place - start) << 16);
     }
     __syncthreads();
     uint32_t* const words = to.words + first;
@@ -160,7 +164,7 @@ struct BucketFetch {
 
     __device__ __forceinline__ BucketFetch(const Shares& from, const SharePlan& plan, int32_t bucket) {
         const int32_t share = min(static_cast<int32_t>(threadIdx.x), plan.shares - 1);
-        const uint32_t found = from.starts[static_cast<size_t>(bucket) * MOST_SHARES + share];
+        const uint32_t found = from.starts[static_cast<size_t>(share) * plan.buckets + bucket];
         start = static_cast<int32_t>(threadIdx.x) < plan.shares ? static_cast<int32_t>(found & 0xffff) : 0;
         count = static_cast<int32_t>(threadIdx.x) < plan.shares ? static_cast<int32_t>(found >> 16) : 0;
         words = from.words + static_cast<size_t>(share) * plan.share;
@@ -286,7 +290,7 @@ __device__ __forceinline__ BucketEdges gather_bucket(
                 for (int step = MOST_SHARES / 2; step > 0; step /= 2) {
                     which += before[which + step] <= place ? step : 0;
                 }
-                const uint32_t of_share = from.starts[static_cast<size_t>(bucket) * MOST_SHARES + which] & 0xffff;
+                const uint32_t of_share = from.starts[static_cast<size_t>(which) * plan.buckets + bucket] & 0xffff;
                 const uint32_t word =
                     from.words[static_cast<size_t>(which) * plan.share + of_share + (place - before[which])];
                 return Item{static_cast<int32_t>(key_of(word)), which * plan.share + static_cast<int32_t>(word & 0xffff), 0};
