@@ -12,11 +12,16 @@
 // table costs an instruction per factor and no scalar loads.
 //
 // What bounds these kernels is LDS: order (forward) or order * (order - 1)
-// (gradients) values per row and monomial. A term of a gradient reads the
+// (gradients) values per row and monomial, and that the features which a pass of 16-byte
+// reads brings for four teams are as often as not on the same quarter of the banks (of
+// 1000 rows, 2000 features, 100 000 monomials of order 4, float, 0.48 of the gradients' 71 us
+// of LDS are such conflicts; the best order of a record's factors would leave nine tenths
+// of that time, the best places of four records as well four fifths). A term of a gradient reads the
 // order - 1 OTHER factors and adds up in registers; nothing is added in LDS.
 // For that the table is first turned round (feature -> the terms it is a
 // factor of, `records_kernel`), deterministically and without atomics on
-// shared counters: a stable counting sort (8 us for 400 000 factors).
+// shared counters: a stable counting sort (5 us for the counts and 24 for
+// the records of 400 000 factors).
 //
 // 1000 rows, 2000 features, 100 000 monomials of order 4, whole calls: forward
 // 91 -> 37 us (float), 98 -> 61 (double), of which LDS at 128 bytes per clock

@@ -39,12 +39,13 @@
 //
 // Whole calls against one per-node sum on the matrix cores each, 9 components, 32
 // columns, the same buffers every call, f32 / f64, us: 1 000 000 edges, forward 315
-// -> 200 / 391 -> 369, vjp 1184 -> 478 / 1397 -> 854; 60 000 edges, 20.2 -> 20.2 /
-// 29.2 -> 25.0 and 58.5 -> 52 / 99 -> 65; 128 columns there, vjp 247 -> 114 / 360
-// -> 223; 600 edges, 12.6 -> 7.5 / 14.0 -> 8.5 and 25.1 -> 11.8 / 31.7 -> 12.8. At a
+// -> 200 / 391 -> 370, vjp 1184 -> 447 / 1397 -> 812; 60 000 edges, 20.2 -> 20.2 /
+// 29.2 -> 25.1 and 58.5 -> 46 / 99 -> 59.5; 128 columns there, vjp 247 -> 108 / 360
+// -> 201; 600 edges, 12.6 -> 7.4 / 14.0 -> 8.2 and 25.1 -> 11.0 / 31.7 -> 12.1. At a
 // million edges 1.3 GB (float; 2.6 in double) come through the memory side of L2 in
 // the forward pass, rows of W in no order for the most part, at 6.4 (7.1) TB/s: the
-// same loads with nothing done to what they bring take 175 of the 200 us.
+// same loads with nothing done to what they bring take 175 of the 200 us, and with
+// twice as many on their way the time is the same.
 //
 // Every sum has one fixed order; no atomics on floating point.
 #include "sasaw_columns.hpp"

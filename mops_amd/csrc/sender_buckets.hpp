@@ -308,7 +308,8 @@ __device__ __forceinline__ void arrivals_in_order(
 }
 
 /// The edges of [begin, end) that name `sender`, in ascending order, found by one wavefront that
-/// reads this piece of the index itself: for a sender with more edges than it has places.
+/// reads this piece of the index itself: for a sender with more edges than it has places, and for every
+/// sender of a small graph (sasaw_columns.hip: small_kernel).
 /// `hand_on(edge, n)` gets up to 64 of them at a time, lane k < n holding the k-th (the other lanes
 /// hold 0). AHEAD loads of 256 positions are on their way together, and the edges wait in a register
 /// until there are 64, so that neither the index nor the rows are read one round trip at a time.
