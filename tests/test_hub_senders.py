@@ -5,7 +5,7 @@ the oracle.
 The hubs are the first and the last sender, two next to each other and one alone; the index is longer
 than the 1024 positions that are looked at together and does not come out even in quarters; the
 per-edge rows have one, two and four columns per lane; edges in slots and by arrival, below and above
-48 edges per sender on average. (SASAW lists its senders' edges otherwise, but where it looks through the index
+48 edges per sender on average, and in shares. (SASAW lists its senders' edges otherwise, but where it looks through the index
 for every sender, in `slots` here but for 16 components in double; see test_sasaw_columns.py.)
 """
 import numpy as np
@@ -58,6 +58,26 @@ def test_opsaw(oracle, device, size, columns, dtype):
     edges, senders, of_hub = SIZES[size]
     case = support.opsaw_case(edges + columns, dtype, E=edges, K=2, L=columns, n_nodes=senders, allow_empty=True)
     compare(oracle, device, "opsaw", with_hubs(case, "indices_W", senders, of_hub, columns), "indices_W", dtype, f"{size} grad_W")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize(
+    "shape",
+    [  # edges, senders, K, L, edges of a hub: one to four columns per lane, senders split by a launch of its own
+        (60007, 26701, 65, 3, 2200),
+        (60007, 26701, 65, 20, 2200),
+        (60007, 26701, 65, 50, 2200),
+        (60007, 26701, 65, 100, 2200),
+        (60007, 26701, 65, 140, 2200),
+        (330007, 5001, 17, 33, 3000),  # split by the edges' kernel
+    ],
+    ids=lambda s: "x".join(map(str, s)),
+)
+def test_opsaw_in_shares(oracle, device, shape, dtype):
+    """Senders in shares and buckets (mops_amd/csrc/sender_shares.hpp), some with more edges than a bucket's place in LDS."""
+    edges, senders, rows, columns, of_hub = shape
+    case = support.opsaw_case(edges + columns, dtype, E=edges, K=rows, L=columns, n_nodes=senders, allow_empty=True)
+    compare(oracle, device, "opsaw", with_hubs(case, "indices_W", senders, of_hub, columns), "indices_W", dtype, f"{shape} grad_W")
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
